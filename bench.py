@@ -312,18 +312,18 @@ STAGE_KERNELS = {
     "refine_vertex_pos_quad": r"k_final<{s}, \w+, {multi}, false>",
     "refine_vertex_quad": r"k_level<true, {s},",
     "refine_vertex_poly": r"k_level<false, {s},",
-    "facepoints_quad": r"k_faces<true, true, false>",
-    "facepoints_poly": r"k_faces<false, true, false>",
-    "gather": r"k_gather",
-    "count_quad": r"k_count<true>",
-    "count_poly": r"k_count<false>",
+    "facepoints_quad": r"k_faces<true>",
+    "facepoints_poly": r"k_faces<false>",
+    "gather": r"k_gather<",  # the gather, count and transpose stages are one launch
+    "count_quad": r"k_gather<true>",
+    "count_poly": r"k_gather<false>",
     "lak_form": r"k_lak_form",
-    "transpose_quad": r"k_transpose<true>",
-    "transpose_poly": r"k_transpose<false>",
-    "spgemm_symbolic_quad": r"k_symbolic<true, {s},",
-    "spgemm_symbolic_poly": r"k_symbolic<false, {s},",
-    "number_facepoints_quad": r"k_number_faces<true, {s},",
-    "number_facepoints_poly": r"k_number_faces<false, {s},",
+    "transpose_quad": r"k_gather<true>",
+    "transpose_poly": r"k_gather<false>",
+    "spgemm_symbolic_quad": r"k_symbolic<true, {s}>",
+    "spgemm_symbolic_poly": r"k_symbolic<false, {s}>",
+    "number_facepoints_quad": r"k_number_faces<true, {s}>",
+    "number_facepoints_poly": r"k_number_faces<false, {s}>",
 }
 PMC_WORKLOADS = ("cfg4", "cfg2", "cfg3")
 

@@ -122,6 +122,12 @@ __device__ __forceinline__ int seg_of_wave(const int64_t* base, int n, int64_t x
   return k;
 }
 
+constexpr int kBlockItems = 256;  // threads (items) per block of the level kernels
+
+// M^T row slots per vertex while the first level's rows are built
+constexpr int kRowSlots = 8;
+constexpr int kTilesPerGroup = 64;
+
 struct LevelView {
   const int32_t* ids;
   const int32_t* fptr;   // poly levels
@@ -130,13 +136,26 @@ struct LevelView {
   int32_t nv;
   int32_t nf;
   int64_t nnz;
-  const int32_t* tptr;
-  int32_t* tids;         // M^T corners (first level: transposed, rows sorted on use)
-  int2* trow;            // sorted rows with in-neighbours (written by the symbolic pass), or null
-  int32_t* mpos;         // M^T storage position of every corner (SLAK, symbolic pass), or null
-  int32_t* ecnt;
-  int32_t* hist_rows;    // zeroed histogram copies of row lengths (symbolic pass), or null
-  const int32_t* eptr;
+  int32_t* tptr;
+  // first-level rows while they are built: cnt[v] corners of vertex v, the
+  // first kRowSlots of them in slots[kRowSlots v ..] (unsorted); longer rows
+  // continue in a linked list (head[v], next[corner]) until the symbolic pass
+  // gathers them into a run of tids (handed out by *pool) and leaves the run's
+  // position in the row's first slot
+  int32_t* cnt;
+  int32_t* slots;
+  int32_t* head;
+  int32_t* next;
+  int32_t* tids;
+  int32_t* pool;
+  int32_t* ecnt;         // edges each vertex owns (symbolic pass)
+  uint64_t* tile_sum;    // packed (corners, owned edges) of each kBlockItems vertices
+  uint64_t* group_sum;   // and of each kTilesPerGroup tiles (zeroed before)
+  int32_t* bounds;       // owned edges before each mesh (several meshes)
+  int2* trow;            // sorted rows with in-neighbours (written by the number pass)
+  int32_t* mpos;         // M^T storage position of every corner (SLAK, number pass), or null
+  int32_t* hist_rows;    // zeroed histogram copies of row lengths (symbolic pass)
+  int32_t* eptr;         // owned edges before each vertex
   int32_t* ci;           // (edge id, twin) pairs per corner, written by the number pass
   int32_t* bnd;          // union edge boundary flags (number pass), or null: closed level
   int32_t* E_ids;   // LAK edge matrix rows (SpGEMM operator)
@@ -149,8 +168,9 @@ struct LevelView {
   int32_t* D_ids;
   int32_t* D_vals;
   int64_t ne_cap;  // E capacity of the SpGEMM operator
-  int32_t rows_per_block;  // first-level row kernels: M^T rows per block (64, 128 or 256)
-  int32_t tile_entries;    // first-level row kernels: entries of the block's LDS row tile
+  int32_t row_cap;         // rows up to this length are processed in registers (4 or 8)
+  int32_t rows_per_block;  // numbering: M^T rows per block (64, 128 or 256)
+  int32_t tile_entries;    // numbering: entries of the block's LDS row tile
 };
 
 __device__ __forceinline__ float4 f4add(float4 a, float4 b) {
@@ -193,6 +213,7 @@ __device__ __forceinline__ void rloop(int n, Fn&& fn) {
 // predecessor's corner; jm/im pair each out-half-edge with its twin.
 template <int CAP, bool QUAD>
 struct RegRow {
+  static_assert(CAP % 2 == 0 && CAP <= kRowSlots, "pairs of a row's slots");
   static constexpr int kCap = CAP;
   int n;
   int32_t t_[CAP], f_[CAP], w_[CAP], u_[CAP], tp_[CAP];
@@ -200,12 +221,21 @@ struct RegRow {
   int32_t fj_[CAP], tpj_[CAP];  // face / predecessor corner of the twin of out-half-edge i
   int8_t rko_[CAP], rki_[CAP];  // LAK: rank of w_i / u_j among the owned lower neighbours
 
-  __device__ __forceinline__ void load(const LevelView& L, int32_t s, int cnt) { load(L, L.tids + s, cnt); }
-  // row: the row's unsorted corners (global memory, or the block's LDS copy)
-  __device__ __forceinline__ void load(const LevelView& L, const int32_t* row, int cnt) {
+  // slots: the row's kRowSlots slots (32 bytes, aligned), n <= CAP of them in
+  // use, unsorted: read as whole 16-byte pieces
+  __device__ __forceinline__ void load_slots(const LevelView& L, const int32_t* slots, int cnt) {
     n = cnt;
+    const int4* __restrict__ q = reinterpret_cast<const int4*>(slots);
 #pragma unroll
-    for (int i = 0; i < CAP; ++i) t_[i] = (i < n) ? row[i] : 0x7fffffff;
+    for (int i = 0; i < CAP; i += 4) {
+      const int4 x = n > i ? q[i >> 2] : make_int4(0, 0, 0, 0);
+      t_[i] = i < n ? x.x : 0x7fffffff;
+      t_[i + 1] = i + 1 < n ? x.y : 0x7fffffff;
+      if (i + 3 < CAP) {
+        t_[i + 2] = i + 2 < n ? x.z : 0x7fffffff;
+        t_[i + 3] = i + 3 < n ? x.w : 0x7fffffff;
+      }
+    }
     // odd-even transposition network: canonical (ascending corner) order
 #pragma unroll
     for (int p = 0; p < CAP; ++p) {
@@ -238,26 +268,6 @@ struct RegRow {
         w_[i] = -1 - i;
         u_[i] = -100 - i;
       }
-    }
-    pair();
-  }
-  // The same row from the symbolic pass's output: corners already sorted,
-  // each with its in-neighbour, so only the out-neighbours are gathered.
-  __device__ __forceinline__ void load_sorted(const LevelView& L, const int2* __restrict__ row, int cnt) {
-    n = cnt;
-#pragma unroll
-    for (int i = 0; i < CAP; ++i) {
-      const int2 e = (i < n) ? row[i] : make_int2(0x7fffffff, -100 - i);
-      t_[i] = e.x;
-      u_[i] = e.y;
-    }
-#pragma unroll
-    for (int i = 0; i < CAP; ++i) {
-      int32_t f = 0, tn = 0, tp = 0;
-      if (i < n) corner_geo<QUAD>(L, t_[i], f, tn, tp);
-      f_[i] = f;
-      tp_[i] = tp;
-      w_[i] = (i < n) ? L.ids[tn] : -1 - i;
     }
     pair();
   }
@@ -318,20 +328,19 @@ struct RegRow {
 };
 
 // The same row read from global memory (rows longer than the register
-// capacity). The row must already be sorted in tids.
+// capacity). The row must already be sorted.
 template <bool QUAD>
 struct MemRow {
   static constexpr int kCap = 0;
   const int32_t* ids;
   const int32_t* fptr;
   const int32_t* cface;
-  const int32_t* tids;
-  int32_t s;
+  const int32_t* row;
   int n;
-  __device__ __forceinline__ MemRow(const LevelView& L, int32_t s_, int n_)
-      : ids(L.ids), fptr(L.fptr), cface(L.cface), tids(L.tids), s(s_), n(n_) {}
+  __device__ __forceinline__ MemRow(const LevelView& L, const int32_t* row_, int n_)
+      : ids(L.ids), fptr(L.fptr), cface(L.cface), row(row_), n(n_) {}
   __device__ __forceinline__ void geo(int i, int32_t& f, int32_t& tn, int32_t& tp) const {
-    int32_t t = tids[s + i];
+    int32_t t = row[i];
     if (QUAD) {
       f = t >> 2;
       int32_t b = t & ~3;
@@ -344,7 +353,7 @@ struct MemRow {
       tp = (t == a) ? e - 1 : t - 1;
     }
   }
-  __device__ __forceinline__ int32_t T(int i) const { return tids[s + i]; }
+  __device__ __forceinline__ int32_t T(int i) const { return row[i]; }
   __device__ __forceinline__ int32_t F(int i) const {
     int32_t f, a, b;
     geo(i, f, a, b);
@@ -435,9 +444,10 @@ __device__ __forceinline__ void row_symbolic(const Row& r, int32_t v, int32_t& c
 // (LAK: column v of E, spgemm.cuh:71-100; SLAK: flagged out-half-edges in
 // corner order, CatmullClarkKernels.cuh:147-236) and the twin corner, stored
 // as (edge id, twin) at both of its half-edges' corners, and the boundary
-// flag of every owned edge by union edge index.
+// flag of every owned edge by union edge index. edges_before: the union's
+// edges owned by the vertices before v.
 template <int SCHEME, class Row>
-__device__ __forceinline__ void row_number(Row& r, const LevelView& L, int32_t v) {
+__device__ __forceinline__ void row_number(Row& r, const LevelView& L, int32_t v, int32_t edges_before) {
   constexpr int C = Row::kCap;
   const int k = seg_of_wave(L.seg.vbase, L.seg.n, v);
   const SegDesc* __restrict__ S = L.seg.d + k;
@@ -446,7 +456,7 @@ __device__ __forceinline__ void row_number(Row& r, const LevelView& L, int32_t v
   int32_t* __restrict__ ci = L.ci;
   int32_t* __restrict__ bnd = L.bnd;
   int* flags = L.flags;
-  const int32_t e0 = L.eptr[v] - L.eptr[S->vb];  // mesh-local edge base of v
+  const int32_t e0 = edges_before - (int32_t)eb;  // mesh-local edge base of v
   const int n = r.n;
   // Edge ids beyond the segment's edges are clamped (and flagged) so that
   // every later index stays inside the mesh's ranges.
@@ -525,8 +535,6 @@ struct RefineView {
 // two levels before the output and the positions of its refinement M1 (whose
 // structure is never written): M's bases in the union arrays of its level,
 // its sizes, its M1 positions and its outputs.
-constexpr int kBlockItems = 256;  // threads (items) per block of the level kernels
-
 struct FinalSeg {
   int64_t cb, vb, eb;    // union bases of M's corners, vertices, edges
   int32_t nv, nf, ne;    // M sizes

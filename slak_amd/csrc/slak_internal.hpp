@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include <exception>
+#include <initializer_list>
 #include <mutex>
 #include <stdexcept>
 #include <string>
@@ -38,18 +39,21 @@ struct Error : std::runtime_error {
 // reads SLAK_XCD_REMAP once and sets the device-side option (call before capture)
 void init_device_options();
 void launch_fill_i32(int32_t* p, int64_t n, int32_t value, hipStream_t st);
-// also zeroes zero[0..nzero) (the counters of the analysis that follows) and,
-// when hist_faces is set, adds the face orders to that zeroed histogram block
-// (kHistCopies copies of 17 bins; the host sums the copies)
-void launch_gather(const SegTable& seg, int32_t nf_total, bool use_vals, int32_t* ids_pos, int32_t* fptr,
-                   int32_t* cface, int* flags, int32_t* zero, int32_t nzero, int32_t* hist_faces, hipStream_t st);
+// copies `bytes` (a multiple of 16) of pinned host memory to the device and
+// zeroes zero[0 .. nzero) (a multiple of 4 ints) in one launch; either may be empty
+void launch_setup(const void* src_pinned, void* dst, int64_t bytes, int32_t* zero, int64_t nzero, hipStream_t st);
+// validates the caller's faces, gathers them into the union (ids_pos, L.fptr,
+// L.cface), counts the valences and places the corners in the rows of M^T
+// (L.cnt zeroed before, L.slots, L.head, L.next)
+void launch_gather(bool quad, const SegTable& seg, bool use_vals, int32_t* ids_pos, const LevelView& L,
+                   hipStream_t st);
 void launch_gather_verts(const SegTable& seg, int32_t nv_total, float4* P, hipStream_t st);
 constexpr int kRowHistBins = 17;  // row lengths 0..15, 16 = longer
-// LDS tile of the first level's row kernels, in M^T entries (sized per level
-// by the plan, at most this): a block's rows are staged through it when their
+// LDS tile of the first level's numbering, in M^T entries (sized per level by
+// the plan, at most this): a block's rows are stored through it when their
 // total length fits
 constexpr int kRowTileMax = 2560;
-// Each histogram is kept as kHistCopies copies, one 128-byte line apart; block
+// The histogram is kept as kHistCopies copies, one 128-byte line apart; block
 // b adds its counts to copy b % kHistCopies. A single copy takes one
 // device-scope atomic per block on the same address, and those serialize: on
 // a 4096-block launch they cost about 35 us.
@@ -58,25 +62,24 @@ constexpr int kHistStride = 32;  // ints per copy
 constexpr int kHistInts = kHistCopies * kHistStride;
 // The plan's state block (int32, zeroed before the gather), read back from
 // its start after the first level's analysis:
-// [flags | pad | row hist copies | face hist copies | edge bounds (nseg + 1) | mesh flags (nseg)]
+// [flags | pad | row hist copies | edge bounds (nseg + 1) | mesh flags (nseg)]
+// followed by [pool | group sums | valence counters] (a single mesh's host adds up
+// its edges from the group sums)
 constexpr int kStateRowHist = 32;
-constexpr int kStateFaceHist = kStateRowHist + kHistInts;
-constexpr int kStateBounds = kStateFaceHist + kHistInts;
-// bounds[k] = eptr[vbase[k]], k = 0..nseg
-void launch_seg_bounds(const int64_t* vbase, int32_t nseg, const int32_t* eptr, int32_t* bounds, hipStream_t st);
+constexpr int kStateBounds = kStateRowHist + kHistInts;
 void launch_copy_probe(const float4* a, float4* b, int64_t n, hipStream_t st);
 // *out = order-sensitive 64-bit digest of bytes at p (out: device, 8 bytes)
 void launch_digest(const void* p, int64_t bytes, uint64_t* out, hipStream_t st);
-// guard (or null): the kernel does nothing when it holds an input-validation flag
-void launch_faces(bool quad, bool fp, bool count, const int32_t* ids, const int32_t* fptr, const float4* P, int32_t nf,
-                  const SegTable& seg, int32_t* cnt, const int* guard, hipStream_t st);
-void launch_transpose(bool quad, const int32_t* ids, const int32_t* fptr, int32_t nf, const int32_t* tptr,
-                      int32_t* cnt, int32_t* tids, const int* guard, hipStream_t st);
-void launch_symbolic(bool quad, int scheme, int cap, const LevelView& L, hipStream_t st);
-// first level: edge numbering and (faces set) face points in one launch; the
-// rows come from the symbolic pass (L.trow sorted with in-neighbours, L.tids
-// sorted in place for rows above the register capacity)
-void launch_number_faces(bool quad, int scheme, int cap, const LevelView& L, bool faces, hipStream_t st);
+void launch_faces(bool quad, const int32_t* ids, const int32_t* fptr, const float4* P, int32_t nf, const SegTable& seg,
+                  hipStream_t st);
+// validates and sizes the rows the gather has placed: owned edges per vertex
+// (L.ecnt) and the sums of tiles and groups (L.pool and L.group_sum zeroed before)
+void launch_symbolic(bool quad, int scheme, const LevelView& L, hipStream_t st);
+// L.bounds of several meshes, from the symbolic pass's sums
+void launch_seg_bounds(const LevelView& L, hipStream_t st);
+// first level: row offsets, sorted rows, edge numbering and (faces set) face
+// points in one launch, after the symbolic pass
+void launch_number_faces(bool quad, int scheme, const LevelView& L, bool faces, hipStream_t st);
 void launch_spgemm_fde(bool quad, const LevelView& L, hipStream_t st);
 // refine (per corner) and vertex (per vertex) items of a level in one launch;
 // the refine items also write the LAK form of the segments with dst_ptr set
@@ -107,9 +110,8 @@ struct NoAllocScratch {
 NoAllocScratch noalloc_scratch();
 // largest scan the scratch holds the partials of
 int64_t noalloc_scan_max_items();
-// out[i] = sum(in[0..i)), out[n] = total (also to *total_out when given)
-void launch_scan(const int32_t* in, int32_t* out, int64_t n, int64_t* partial, int* flags, hipStream_t st,
-                 int32_t* total_out = nullptr);
+// out[i] = sum(in[0..i)), out[n] = total
+void launch_scan(const int32_t* in, int32_t* out, int64_t n, int64_t* partial, int* flags, hipStream_t st);
 
 // ---------------------------------------------------------------------------
 // caching device allocator (one per device)
@@ -175,12 +177,20 @@ class Arena {
 // when enabled, every launch site records an event pair on its stream and the
 // stage's algorithmic bytes (compulsory reads + writes of distinct arrays).
 
+// A launch that runs several stages records them all; the report shares its
+// time among them in proportion to their algorithmic bytes.
+
+struct StageBytes {
+  const char* name;
+  double bytes;
+};
+
 class Profiler {
  public:
   static Profiler& get();
   bool enabled() const { return enabled_; }
   void set_enabled(bool on) { enabled_ = on; }
-  void begin(hipStream_t st, const char* name, double bytes);
+  void begin(hipStream_t st, std::vector<StageBytes> stages);
   void end(hipStream_t st);
   // adds `bytes` to the latest record of stage `name` (names compare by text)
   void amend_last(const char* name, double bytes);
@@ -189,8 +199,7 @@ class Profiler {
 
  private:
   struct Rec {
-    const char* name;
-    double bytes;
+    std::vector<StageBytes> stages;
     hipEvent_t a, b;
   };
   hipEvent_t event();
@@ -203,8 +212,9 @@ class Profiler {
 struct ProfScope {
   hipStream_t st;
   bool on;
-  ProfScope(hipStream_t s, const char* name, double bytes) : st(s), on(Profiler::get().enabled()) {
-    if (on) Profiler::get().begin(st, name, bytes);
+  ProfScope(hipStream_t s, const char* name, double bytes) : ProfScope(s, {{name, bytes}}) {}
+  ProfScope(hipStream_t s, std::initializer_list<StageBytes> stages) : st(s), on(Profiler::get().enabled()) {
+    if (on) Profiler::get().begin(st, stages);
   }
   ~ProfScope() {
     if (on) Profiler::get().end(st);

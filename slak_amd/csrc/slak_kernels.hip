@@ -1,13 +1,14 @@
 // HIP kernels of the Catmull-Clark level pipeline for gfx950 (MI355X).
 //
 // First level (the caller's mesh):
-//   validate      check the input and bring corners into position order
-//                 (sortKeyValuePairsSegmentedInPlace, LAKCatmullClarkKernels.cuh:147-180)
-//   count         valence per vertex (spmv_right with ones, LAKCatmullClarkImpl.cu:347-356)
-//   scan          exclusive scan (cub_wrappers.cuh:30-43)
-//   transpose     M -> M^T by counting sort (csr2cscEx2, LAKCatmullClarkImpl.cu:381-423)
-//   symbolic      row sizing of the mapped SpGEMM -> edges owned per vertex;
-//                 rows sorted and stored with their in-neighbours
+//   gather        check the input and bring corners into position order
+//                 (sortKeyValuePairsSegmentedInPlace, LAKCatmullClarkKernels.cuh:147-180);
+//                 valence per vertex (spmv_right with ones, LAKCatmullClarkImpl.cu:347-356)
+//                 and the corners of M^T's rows into fixed slots per vertex
+//   symbolic      M^T (csr2cscEx2, LAKCatmullClarkImpl.cu:381-423) and row sizing
+//                 of the mapped SpGEMM -> edges owned per vertex; rows sorted and
+//                 stored with their in-neighbours at offsets scanned in the same
+//                 pass (scan_exclusive, cub_wrappers.cuh:30-43)
 //   number        mapped SpGEMM rows -> E numbering: edge id and twin of
 //                 every corner's half-edge, boundary flags
 // Every level:
@@ -37,6 +38,7 @@
 #include <climits>
 #include <cstdlib>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "slak_device.hpp"
@@ -47,7 +49,6 @@ namespace slak {
 namespace {
 
 constexpr int kBlock = kBlockItems;
-constexpr int kRowCap = 8;  // M^T rows up to this length stay in registers
 
 // Workgroups are dispatched round-robin over the 8 XCDs, each with its own L2.
 // With the remap, consecutive tiles (which gather from neighbouring parts of
@@ -82,6 +83,16 @@ __global__ void k_fill_i32(int32_t* __restrict__ p, int64_t n, int32_t value) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (; i < n; i += stride) p[i] = value;
+}
+
+// A plan's start in one launch: its tables from pinned host memory (read
+// across the bus by the kernel itself) and its zeroed state.
+__global__ void __launch_bounds__(kBlock) k_setup(const int4* __restrict__ src, int4* __restrict__ dst, int64_t n,
+                                                  int4* __restrict__ zero, int64_t nzero) {
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  const int64_t i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  for (int64_t i = i0; i < n; i += stride) dst[i] = src[i];
+  for (int64_t i = i0; i < nzero; i += stride) zero[i] = make_int4(0, 0, 0, 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -171,27 +182,120 @@ struct BlockHist {
   }
 };
 
-__device__ void gather_face(const SegTable& seg, int32_t f, int32_t nf_total, int use_vals, int32_t* __restrict__ ids_pos,
-                            int32_t* __restrict__ fptr, int32_t* __restrict__ cface, int* __restrict__ flags,
-                            int32_t* hist);
+// What the gather hands on of one face to the row building: the corners of
+// the union (first corner c0) and their union vertices, in storage order for
+// the corners kept in registers (v[i] < 0: none, or an invalid corner).
+constexpr int kGatherRegs = 8;
 
+template <int REGS>
+struct FaceCorners {
+  int32_t v[REGS];
+  int32_t c[REGS];
+};
+
+// M^T rows under construction (first level): cnt[v] corners of vertex v so
+// far, the first kRowSlots of them in slots[kRowSlots v ..], the others in a
+// linked list (head[v], then next[corner]) of cnt[v] - kRowSlots entries.
+struct RowBuild {
+  int32_t* cnt;
+  int32_t* slots;
+  int32_t* head;
+  int32_t* next;
+};
+
+__device__ __forceinline__ void put_row(const RowBuild& rb, int32_t v, int32_t slot, int32_t c) {
+  if (slot < kRowSlots)
+    rb.slots[(int64_t)kRowSlots * v + slot] = c;
+  else
+    rb.next[c] = atomicExch(&rb.head[v], c);
+}
+
+template <bool QUAD>
+__device__ __forceinline__ void gather_face(const SegTable& seg, int32_t f, int32_t nf_total, int use_vals,
+                                            int32_t* __restrict__ ids_pos, int32_t* __restrict__ fptr,
+                                            int32_t* __restrict__ cface, int* __restrict__ flags,
+                                            const RowBuild& rb, FaceCorners<QUAD ? 4 : kGatherRegs>& out);
+
+// min / max over the block (mm: kBlock / 64 LDS entries)
+__device__ __forceinline__ int2 block_minmax(int lo, int hi, int2* mm) {
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) {
+    lo = min(lo, __shfl_xor(lo, d));
+    hi = max(hi, __shfl_xor(hi, d));
+  }
+  if ((threadIdx.x & 63) == 0) mm[threadIdx.x >> 6] = make_int2(lo, hi);
+  __syncthreads();
+  int2 r = mm[0];
+#pragma unroll
+  for (int w = 1; w < kBlock / 64; ++w) r = make_int2(min(r.x, mm[w].x), max(r.y, mm[w].y));
+  return r;
+}
+
+// The corners of a block's 256 faces usually reference a narrow range of
+// vertex ids (grids, refined meshes, each mesh of a batch): the block then
+// counts into LDS over [vmin, vmax] and reserves each touched vertex's row
+// slots with one device atomic. A block whose range is wider than
+// kCountWindow vertices takes one per corner (device-scope atomics are what
+// the row building costs).
+constexpr int kCountWindow = 2048;
+
+// Gather, valence count and row placement in one pass over the caller's
+// faces: the corners of a face are in registers when they are placed, and a
+// row needs no offset while its corners go to fixed slots, so no scan stands
+// between the count and the placement.
+template <bool QUAD>
 __global__ void __launch_bounds__(kBlock) k_gather(SegTable seg, int32_t nf_total, int use_vals, int32_t* __restrict__ ids_pos,
                          int32_t* __restrict__ fptr, int32_t* __restrict__ cface, int* __restrict__ flags,
-                         int32_t* __restrict__ zero, int32_t nzero, int32_t* __restrict__ hist_faces) {
-  __shared__ int32_t h[kHistBins];
-  BlockHist bh{h};
-  if (hist_faces) bh.init();
+                         RowBuild rb, int window) {
+  constexpr int REGS = QUAD ? 4 : kGatherRegs;
+  __shared__ int32_t win[kCountWindow];
+  __shared__ int2 mm[kBlock / 64];
   const int32_t f = (int32_t)(block_index() * blockDim.x + threadIdx.x);
-  if (f < nzero) zero[f] = 0;  // counters of the analysis that follows
-  if (f < nf_total) gather_face(seg, f, nf_total, use_vals, ids_pos, fptr, cface, flags, hist_faces ? h : nullptr);
-  if (hist_faces) bh.flush(hist_faces);
+  FaceCorners<REGS> fc;
+#pragma unroll
+  for (int i = 0; i < REGS; ++i) fc.v[i] = -1;
+  if (f < nf_total) gather_face<QUAD>(seg, f, nf_total, use_vals, ids_pos, fptr, cface, flags, rb, fc);
+  int lo = INT_MAX, hi = INT_MIN;
+#pragma unroll
+  for (int i = 0; i < REGS; ++i)
+    if (fc.v[i] >= 0) {
+      lo = min(lo, fc.v[i]);
+      hi = max(hi, fc.v[i]);
+    }
+  const int2 w = block_minmax(lo, hi, mm);
+  const int64_t n = (int64_t)w.y - w.x + 1;  // <= 0 when no corner is placed
+  if (window && n <= kCountWindow) {          // block-uniform
+    for (int i = threadIdx.x; i < n; i += kBlock) win[i] = 0;
+    __syncthreads();
+    int32_t rank[REGS];
+#pragma unroll
+    for (int i = 0; i < REGS; ++i)
+      if (fc.v[i] >= 0) rank[i] = atomicAdd(&win[fc.v[i] - w.x], 1);
+    __syncthreads();
+    for (int i = threadIdx.x; i < n; i += kBlock) {
+      const int32_t k = win[i];
+      if (k) win[i] = atomicAdd(&rb.cnt[w.x + i], k);  // the first slot of the block's corners
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < REGS; ++i)
+      if (fc.v[i] >= 0) put_row(rb, fc.v[i], win[fc.v[i] - w.x] + rank[i], fc.c[i]);
+  } else {
+#pragma unroll
+    for (int i = 0; i < REGS; ++i)
+      if (fc.v[i] >= 0) put_row(rb, fc.v[i], atomicAdd(&rb.cnt[fc.v[i]], 1), fc.c[i]);
+  }
 }
 
 // first level: validate caller face f and gather it into the union in
-// position order; face order into the block's LDS histogram (hist, or null)
-__device__ void gather_face(const SegTable& seg, int32_t f, int32_t nf_total, int use_vals, int32_t* __restrict__ ids_pos,
-                            int32_t* __restrict__ fptr, int32_t* __restrict__ cface, int* __restrict__ flags,
-                            int32_t* hist) {
+// position order. out: the face's
+// valid corners for the row building; the corners of a longer face beyond
+// the registers are placed here, one device atomic each.
+template <bool QUAD>
+__device__ __forceinline__ void gather_face(const SegTable& seg, int32_t f, int32_t nf_total, int use_vals,
+                                            int32_t* __restrict__ ids_pos, int32_t* __restrict__ fptr,
+                                            int32_t* __restrict__ cface, int* __restrict__ flags,
+                                            const RowBuild& rb, FaceCorners<QUAD ? 4 : kGatherRegs>& out) {
   const int k = seg_of_wave(seg.fbase, seg.n, f);
   const SegDesc* S = seg.d + k;
   const int32_t lf = (int32_t)(f - S->fb);
@@ -211,7 +315,6 @@ __device__ void gather_face(const SegTable& seg, int32_t f, int32_t nf_total, in
     return;
   }
   const int32_t order = (int32_t)(e - s);
-  if (hist) hist_add_wave(hist, order < kHistBins - 1 ? order : kHistBins - 1);
   if (order < 3) bad |= kFlagBadOrder;
   if (S->require_quad && (order != 4 || s != 4ll * lf)) bad |= kFlagBadQuad;
   const int64_t cb = S->cb;
@@ -260,23 +363,32 @@ __device__ void gather_face(const SegTable& seg, int32_t f, int32_t nf_total, in
         atomicOr(seg.mflags + k, bad);
         atomicOr(flags, bad);
       }
+      const int32_t c0 = (int32_t)(cb + s);
+      out.v[0] = o.x;
+      out.v[1] = o.y;
+      out.v[2] = o.z;
+      out.v[3] = o.w;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) out.c[i] = c0 + i;
       return;
     }
   }
-  // any other face: its first kGatherRegs corners are loaded before the
+  // any other face: its first REGS corners are loaded before the
   // first store (a load issued after a store would wait for it), the rest
   // one by one
-  constexpr int kGatherRegs = 8;
+  constexpr int REGS = QUAD ? 4 : kGatherRegs;
   const int32_t snv = S->nv;
   uint32_t mask = 0;
-  auto corner = [&](int64_t c, int32_t id, int32_t pos) __attribute__((always_inline)) {
-    if (id < 0 || id >= snv) {
+  // returns whether the corner can be placed in its vertex's row
+  auto corner = [&](int64_t c, int32_t id, int32_t pos) __attribute__((always_inline)) -> bool {
+    const bool known = id >= 0 && id < snv;
+    if (!known) {
       bad |= kFlagBadId;
       id = 0;
     }
     if (pos < 1 || pos > order) {
       bad |= kFlagBadVals;
-      return;
+      return false;
     }
     if (order <= 32) {
       uint32_t bit = 1u << (pos - 1);
@@ -288,18 +400,26 @@ __device__ void gather_face(const SegTable& seg, int32_t f, int32_t nf_total, in
     }
     ids_pos[cb + s + pos - 1] = vb + id;
     if (cface) cface[cb + c] = f;
+    return known;
   };
-  int32_t rid[kGatherRegs], rpos[kGatherRegs];
+  int32_t rid[REGS], rpos[REGS];
 #pragma unroll
-  for (int i = 0; i < kGatherRegs; ++i)
+  for (int i = 0; i < REGS; ++i)
     if (i < order) {
       rid[i] = sid[s + i];
       rpos[i] = sval ? sval[s + i] : i + 1;
     }
 #pragma unroll
-  for (int i = 0; i < kGatherRegs; ++i)
-    if (i < order) corner(s + i, rid[i], rpos[i]);
-  for (int64_t c = s + kGatherRegs; c < e; ++c) corner(c, sid[c], sval ? sval[c] : (int32_t)(c - s + 1));
+  for (int i = 0; i < REGS; ++i)
+    if (i < order && corner(s + i, rid[i], rpos[i])) {
+      out.v[i] = vb + rid[i];
+      out.c[i] = (int32_t)(cb + s + rpos[i] - 1);
+    }
+  for (int64_t c = s + REGS; c < e; ++c) {
+    const int32_t id = sid[c], pos = sval ? sval[c] : (int32_t)(c - s + 1);
+    if (corner(c, id, pos))
+      put_row(rb, vb + id, atomicAdd(&rb.cnt[vb + id], 1), (int32_t)(cb + s + pos - 1));
+  }
   if (fptr) {
     fptr[f] = (int32_t)(cb + s);
     if (f == nf_total - 1) fptr[nf_total] = (int32_t)(cb + e);
@@ -318,215 +438,51 @@ __global__ void k_gather_verts(SegTable seg, int32_t nv_total, float4* __restric
   P[v] = to_global(S->src_verts)[v - S->vb];
 }
 
-// eptr at every segment's first vertex: bounds[k] = eptr[vbase[k]], k = 0..n
-// (multi-mesh plans; a single mesh takes its total from the scan)
-__global__ void k_seg_bounds(const int64_t* __restrict__ vbase, int32_t n, const int32_t* __restrict__ eptr,
-                             int32_t* __restrict__ bounds) {
-  const int32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k <= n) bounds[k] = eptr[vbase[k]];
-}
-
 // ---------------------------------------------------------------------------
-// valence count (+ face points into each segment's destination)
+// face points into each segment's destination
 
-template <bool QUAD, bool FP, bool COUNT>
+template <bool QUAD>
 __device__ __forceinline__ void faces_item(const int32_t* __restrict__ ids, const int32_t* __restrict__ fptr,
-                                           const float4* __restrict__ P, int32_t nf, const SegTable& seg,
-                                           int32_t* __restrict__ cnt, const int* __restrict__ guard, int32_t f) {
+                                           const float4* __restrict__ P, int32_t nf, const SegTable& seg, int32_t f) {
   if (f >= nf) return;
-  if (guard && (*guard & kFlagsInput)) return;
-  float4* dst = nullptr;
-  if (FP) {
-    const SegDesc* S = seg.d + seg_of_wave(seg.fbase, seg.n, f);
-    dst = to_global(S->dst_verts) + S->nv + (f - S->fb);
-  }
+  const SegDesc* S = seg.d + seg_of_wave(seg.fbase, seg.n, f);
+  float4* const dst = to_global(S->dst_verts) + S->nv + (f - S->fb);
   if (QUAD) {
     int4 c = reinterpret_cast<const int4*>(ids)[f];
-    if (FP) *dst = f4div(f4add(f4add(f4add(P[c.x], P[c.y]), P[c.z]), P[c.w]), 4.0f);
-    if (COUNT) {
-      atomicAdd(&cnt[c.x], 1);
-      atomicAdd(&cnt[c.y], 1);
-      atomicAdd(&cnt[c.z], 1);
-      atomicAdd(&cnt[c.w], 1);
-    }
+    *dst = f4div(f4add(f4add(f4add(P[c.x], P[c.y]), P[c.z]), P[c.w]), 4.0f);
   } else {
     int32_t s = fptr[f], e = fptr[f + 1];
     float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int32_t c = s; c < e; ++c) {
-      int32_t v = ids[c];
-      if (FP) acc = f4add(acc, P[v]);
-      if (COUNT) atomicAdd(&cnt[v], 1);
-    }
-    if (FP) *dst = f4div(acc, (float)(e - s));
+    for (int32_t c = s; c < e; ++c) acc = f4add(acc, P[ids[c]]);
+    *dst = f4div(acc, (float)(e - s));
   }
 }
 
-template <bool QUAD, bool FP, bool COUNT>
+template <bool QUAD>
 __global__ void k_faces(const int32_t* __restrict__ ids, const int32_t* __restrict__ fptr, const float4* __restrict__ P,
-                        int32_t nf, SegTable seg, int32_t* __restrict__ cnt, const int* __restrict__ guard) {
-  faces_item<QUAD, FP, COUNT>(ids, fptr, P, nf, seg, cnt, guard, (int32_t)(block_index() * blockDim.x + threadIdx.x));
+                        int32_t nf, SegTable seg) {
+  faces_item<QUAD>(ids, fptr, P, nf, seg, (int32_t)(block_index() * blockDim.x + threadIdx.x));
 }
 
-// ---------------------------------------------------------------------------
-// Valence count and transpose through a block-local vertex window. The corners
-// of a block's faces usually reference a narrow range of vertex ids (grids,
-// refined meshes, each mesh of a batch): the block then counts into LDS over
-// [vmin, vmax] and adds each touched vertex's count with one device atomic,
-// and the transpose reserves each touched vertex's slots with one atomic and
-// hands them out by LDS atomics. Device-scope atomics are what both passes
-// cost (one per corner otherwise); a block whose window is wider than
-// kCountWindow vertices takes one per corner.
-constexpr int kCountWindow = 2048;
-
-// min / max over the block (mm: kBlock / 64 LDS entries)
-__device__ __forceinline__ int2 block_minmax(int lo, int hi, int2* mm) {
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) {
-    lo = min(lo, __shfl_xor(lo, d));
-    hi = max(hi, __shfl_xor(hi, d));
-  }
-  if ((threadIdx.x & 63) == 0) mm[threadIdx.x >> 6] = make_int2(lo, hi);
-  __syncthreads();
-  int2 r = mm[0];
-#pragma unroll
-  for (int w = 1; w < kBlock / 64; ++w) r = make_int2(min(r.x, mm[w].x), max(r.y, mm[w].y));
-  return r;
+// 64-bit lane exchange by DPP (row_shr / row_bcast); lanes without a source,
+// and rows outside ROWMASK, read 0.
+template <int CTRL, int ROWMASK>
+__device__ __forceinline__ int64_t dpp64(int64_t x) {
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)x, CTRL, ROWMASK, 0xF, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(x >> 32), CTRL, ROWMASK, 0xF, false);
+  return (int64_t)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
 }
-
-// the vertex range of face f's corners (quad: c holds them)
-template <bool QUAD>
-__device__ __forceinline__ int2 face_range(const int32_t* __restrict__ ids, const int32_t* __restrict__ fptr,
-                                           int32_t f, int4& c, int32_t& s, int32_t& e) {
-  if (QUAD) {
-    c = reinterpret_cast<const int4*>(ids)[f];
-    return make_int2(min(min(c.x, c.y), min(c.z, c.w)), max(max(c.x, c.y), max(c.z, c.w)));
-  }
-  s = fptr[f];
-  e = fptr[f + 1];
-  int lo = INT_MAX, hi = INT_MIN;
-  for (int32_t k = s; k < e; ++k) {
-    const int32_t v = ids[k];
-    lo = min(lo, v);
-    hi = max(hi, v);
-  }
-  return make_int2(lo, hi);
-}
-
-// cnt[v] += valence of v over the faces [0, nf) (cnt zeroed before)
-template <bool QUAD>
-__global__ void __launch_bounds__(kBlock) k_count(const int32_t* __restrict__ ids, const int32_t* __restrict__ fptr,
-                                                  int32_t nf, int32_t* __restrict__ cnt, const int* __restrict__ guard) {
-  __shared__ int32_t win[kCountWindow];
-  __shared__ int2 mm[kBlock / 64];
-  if (guard && (*guard & kFlagsInput)) return;  // block-uniform
-  const int32_t f = (int32_t)(block_index() * blockDim.x + threadIdx.x);
-  const bool act = f < nf;
-  int4 c = make_int4(0, 0, 0, 0);
-  int32_t s = 0, e = 0;
-  int2 r = make_int2(INT_MAX, INT_MIN);
-  if (act) r = face_range<QUAD>(ids, fptr, f, c, s, e);
-  const int2 w = block_minmax(r.x, r.y, mm);
-  const int64_t n = (int64_t)w.y - w.x + 1;  // <= 0 when no lane is active
-  if (n <= kCountWindow) {                    // block-uniform
-    for (int i = threadIdx.x; i < n; i += blockDim.x) win[i] = 0;
-    __syncthreads();
-    if (act) {
-      if (QUAD) {
-        atomicAdd(&win[c.x - w.x], 1);
-        atomicAdd(&win[c.y - w.x], 1);
-        atomicAdd(&win[c.z - w.x], 1);
-        atomicAdd(&win[c.w - w.x], 1);
-      } else {
-        for (int32_t k = s; k < e; ++k) atomicAdd(&win[ids[k] - w.x], 1);
-      }
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-      const int32_t k = win[i];
-      if (k) atomicAdd(&cnt[w.x + i], k);
-    }
-  } else if (act) {
-    if (QUAD) {
-      atomicAdd(&cnt[c.x], 1);
-      atomicAdd(&cnt[c.y], 1);
-      atomicAdd(&cnt[c.z], 1);
-      atomicAdd(&cnt[c.w], 1);
-    } else {
-      for (int32_t k = s; k < e; ++k) atomicAdd(&cnt[ids[k]], 1);
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// transpose scatter: tids[tptr[v] + slot] = corner; cnt[] counts back to zero
-// (slot order within a row is arbitrary: the row-sizing pass sorts the rows)
-
-template <bool QUAD>
-__global__ void __launch_bounds__(kBlock) k_transpose(const int32_t* __restrict__ ids, const int32_t* __restrict__ fptr,
-                                                      int32_t nf, const int32_t* __restrict__ tptr,
-                                                      int32_t* __restrict__ cnt, int32_t* __restrict__ tids,
-                                                      const int* __restrict__ guard, int window) {
-  __shared__ int32_t lc[kCountWindow];    // the block's corners per window vertex, then counted back
-  __shared__ int32_t base[kCountWindow];  // the first tids slot the block reserved for each
-  __shared__ int2 mm[kBlock / 64];
-  if (guard && (*guard & kFlagsInput)) return;  // block-uniform
-  const int32_t f = (int32_t)(block_index() * blockDim.x + threadIdx.x);
-  const bool act = f < nf;
-  int4 c = make_int4(0, 0, 0, 0);
-  int32_t s = 0, e = 0;
-  int2 r = make_int2(INT_MAX, INT_MIN);
-  if (act) r = face_range<QUAD>(ids, fptr, f, c, s, e);
-  const int2 w = block_minmax(r.x, r.y, mm);
-  const int64_t n = (int64_t)w.y - w.x + 1;
-  if (window && n <= kCountWindow) {  // block-uniform
-    for (int i = threadIdx.x; i < n; i += blockDim.x) lc[i] = 0;
-    __syncthreads();
-    if (act) {
-      if (QUAD) {
-        atomicAdd(&lc[c.x - w.x], 1);
-        atomicAdd(&lc[c.y - w.x], 1);
-        atomicAdd(&lc[c.z - w.x], 1);
-        atomicAdd(&lc[c.w - w.x], 1);
-      } else {
-        for (int32_t k = s; k < e; ++k) atomicAdd(&lc[ids[k] - w.x], 1);
-      }
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-      const int32_t k = lc[i];
-      if (k) base[i] = tptr[w.x + i] + atomicSub(&cnt[w.x + i], k) - k;
-    }
-    __syncthreads();
-    if (act) {
-      if (QUAD) {
-        const int32_t t = 4 * f;
-        tids[base[c.x - w.x] + atomicSub(&lc[c.x - w.x], 1) - 1] = t;
-        tids[base[c.y - w.x] + atomicSub(&lc[c.y - w.x], 1) - 1] = t + 1;
-        tids[base[c.z - w.x] + atomicSub(&lc[c.z - w.x], 1) - 1] = t + 2;
-        tids[base[c.w - w.x] + atomicSub(&lc[c.w - w.x], 1) - 1] = t + 3;
-      } else {
-        for (int32_t k = s; k < e; ++k) {
-          const int32_t i = ids[k] - w.x;
-          tids[base[i] + atomicSub(&lc[i], 1) - 1] = k;
-        }
-      }
-    }
-    return;
-  }
-  if (!act) return;
-  if (QUAD) {
-    int4 c = reinterpret_cast<const int4*>(ids)[f];
-    int32_t t = 4 * f;
-    tids[tptr[c.x] + atomicSub(&cnt[c.x], 1) - 1] = t;
-    tids[tptr[c.y] + atomicSub(&cnt[c.y], 1) - 1] = t + 1;
-    tids[tptr[c.z] + atomicSub(&cnt[c.z], 1) - 1] = t + 2;
-    tids[tptr[c.w] + atomicSub(&cnt[c.w], 1) - 1] = t + 3;
-  } else {
-    for (int32_t k = fptr[f]; k < fptr[f + 1]; ++k) {
-      int32_t v = ids[k];
-      tids[tptr[v] + atomicSub(&cnt[v], 1) - 1] = k;
-    }
-  }
+// Inclusive scan over the 64 lanes of a wave: shifts by 1, 2, 4, 8 inside
+// each row of 16 lanes, then lane 15 of rows 0 / 2 into rows 1 / 3 and lane
+// 31 into rows 2 and 3.
+__device__ __forceinline__ int64_t wave_scan64(int64_t x) {
+  x += dpp64<0x111, 0xF>(x);
+  x += dpp64<0x112, 0xF>(x);
+  x += dpp64<0x114, 0xF>(x);
+  x += dpp64<0x118, 0xF>(x);
+  x += dpp64<0x142, 0xA>(x);
+  x += dpp64<0x143, 0xC>(x);
+  return x;
 }
 
 // ---------------------------------------------------------------------------
@@ -544,162 +500,227 @@ __device__ void sort_row_in_place(int32_t* a, int n) {
   }
 }
 
-// The M^T rows of a block's R consecutive vertices (R = L.rows_per_block:
-// 256, 128 or 64) are one contiguous segment [tptr[v0], tptr[v0 + R]) of tids
-// (and of trow): when it fits the block's LDS tile (L.tile_entries entries,
-// dynamic LDS; the plan sizes R and the tile from the row lengths) it is read
-// in with all 256 lanes on consecutive entries, the rows are taken from LDS
-// (one lane per row), and the sorted rows with their in-neighbours go back out
-// the same way. Longer segments use global memory.
-extern __shared__ __align__(16) unsigned char row_tile_lds[];
+// The unsorted corners of vertex v's row of n: its slots, or (more than
+// kRowSlots) the run of the tids pool that slot 0 points to once k_symbolic
+// has gathered the row there.
+__device__ __forceinline__ int32_t* row_corners(const LevelView& L, int32_t v, int n) {
+  int32_t* const slots = L.slots + (int64_t)kRowSlots * v;
+  return n <= kRowSlots ? slots : L.tids + slots[0];
+}
 
-template <bool QUAD, int SCHEME, int CAP, bool STAGED>
-__device__ __forceinline__ void symbolic_row(const LevelView& L, int32_t v, int32_t* hist, const int32_t* rows_in,
-                                             int2* rows_out, int32_t s0);
+// Row lengths and owned-edge counts are summed per tile of kBlock vertices
+// (packed: corners << 31 | edges; a level's totals stay below 2^31) and per
+// kTilesPerGroup tiles, so that any later block adds up the offsets of its
+// rows from a few hundred sums: no scan launches, and no block waits for
+// another. (A decoupled look-back in the sizing pass measured slower: its
+// ticket, one atomic per block on one address, takes about 20 ns a block --
+// 89 against 31 us on 4096 blocks.)
+__device__ __forceinline__ uint64_t pack_row(int32_t n, int32_t owned) {
+  return ((uint64_t)(uint32_t)n << 31) | (uint32_t)owned;
+}
+constexpr uint64_t kOwnedMask = (1ull << 31) - 1;
 
-template <bool QUAD, int SCHEME, int CAP>
+// sum over the block; lds: kBlock / 64 entries, free again after a barrier
+__device__ __forceinline__ uint64_t block_sum(uint64_t x, uint64_t* lds) {
+  for (int d = 32; d > 0; d >>= 1) x += __shfl_xor(x, d, 64);
+  if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = x;
+  __syncthreads();
+  uint64_t t = 0;
+#pragma unroll
+  for (int w = 0; w < kBlock / 64; ++w) t += lds[w];
+  return t;
+}
+
+// exclusive scan over the block; total: the block's sum
+__device__ __forceinline__ uint64_t block_scan_packed(uint64_t x, uint64_t* lds, uint64_t& total) {
+  const uint64_t inc = (uint64_t)wave_scan64((int64_t)x);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (lane == 63) lds[wave] = inc;
+  __syncthreads();
+  uint64_t off = 0;
+  total = 0;
+#pragma unroll
+  for (int w = 0; w < kBlock / 64; ++w) {
+    off += w < wave ? lds[w] : 0;
+    total += lds[w];
+  }
+  return off + inc - x;
+}
+
+// this thread's share of the packed sum of all tiles before `tile`
+__device__ __forceinline__ uint64_t tiles_before(const LevelView& L, int tile, int tid, int nthreads) {
+  const int group = tile / kTilesPerGroup;
+  uint64_t acc = 0;
+  for (int i = tid; i < group; i += nthreads) acc += L.group_sum[i];
+  for (int i = group * kTilesPerGroup + tid; i < tile; i += nthreads) acc += L.tile_sum[i];
+  return acc;
+}
+
+// Runs fn(row) on vertex v's row of n <= cap corners in registers, from its
+// slots. Sorting and pairing a row of capacity C costs about C^2 selects, so
+// each wave takes the smallest of three capacities that holds all of its rows.
+template <bool QUAD, class Fn>
+__device__ __forceinline__ void with_row(const LevelView& L, const int32_t* slots, int n, Fn&& fn) {
+  auto run = [&](auto row) __attribute__((always_inline)) {
+    row.load_slots(L, slots, n);
+    fn(row);
+  };
+  if (__any(n > 6))
+    run(RegRow<8, QUAD>{});
+  else if (__any(n > 4))
+    run(RegRow<6, QUAD>{});
+  else
+    run(RegRow<4, QUAD>{});
+}
+
+// Mapped-SpGEMM row sizing, one lane per vertex: the row's corners from their
+// slots, validated, the edges the vertex owns counted; a row longer than its
+// slots is gathered into a run of the pool, and rows beyond the register
+// capacity are sorted in place.
+template <bool QUAD, int SCHEME>
 __global__ void __launch_bounds__(kBlock) k_symbolic(LevelView L) {
   __shared__ int32_t h[kHistBins];
-  const int T = L.tile_entries;  // even: tile_out starts 8-byte aligned
-  int32_t* const tile_in = reinterpret_cast<int32_t*>(row_tile_lds);       // T corners
-  int2* const tile_out = reinterpret_cast<int2*>(row_tile_lds + 4 * T);  // T (corner, in-neighbour)
+  __shared__ uint64_t wave_sum[kBlock / 64];
+  if (*L.flags & kFlagsInput) return;  // set by the gather alone: the same for every block
   BlockHist bh{h};
-  if (L.hist_rows) bh.init();
-  const int R = L.rows_per_block;
-  const int64_t v0 = block_index() * R;
-  const int32_t v = (int32_t)(v0 + threadIdx.x);
-  const bool valid = !(*L.flags & kFlagsInput);
-  int32_t s0 = 0, len = 0;
-  if (valid && v0 < L.nv) {
-    s0 = L.tptr[v0];
-    len = L.tptr[min(v0 + (int64_t)R, (int64_t)L.nv)] - s0;
-  }
-  const bool staged = len > 0 && len <= T;  // block-uniform
-  if (staged)
-    for (int i = threadIdx.x; i < len; i += blockDim.x) tile_in[i] = L.tids[s0 + i];
-  __syncthreads();
-  // (staged or not as a template argument: a pointer that may address LDS
-  // or global memory makes every access through it a FLAT instruction)
-  if ((int)threadIdx.x < R && v < L.nv && valid) {
-    if (staged)
-      symbolic_row<QUAD, SCHEME, CAP, true>(L, v, L.hist_rows ? h : nullptr, tile_in, L.trow ? tile_out : nullptr, s0);
-    else
-      symbolic_row<QUAD, SCHEME, CAP, false>(L, v, L.hist_rows ? h : nullptr, nullptr, nullptr, s0);
-  }
-  __syncthreads();
-  if (staged && L.trow)
-    for (int i = threadIdx.x; i < len; i += blockDim.x) L.trow[s0 + i] = tile_out[i];
-  if (L.hist_rows) bh.flush(L.hist_rows);
-}
-
-// mapped-SpGEMM row sizing of vertex v (edges it owns), validation, the
-// sorted row with in-neighbours; row length into the block histogram.
-// STAGED: rows_in / rows_out are the block's LDS tiles from position s0
-// (rows_out null: no sorted rows wanted); else both null
-template <bool QUAD, int SCHEME, int CAP, bool STAGED>
-__device__ __forceinline__ void symbolic_row(const LevelView& L, int32_t v, int32_t* hist, const int32_t* rows_in,
-                                             int2* rows_out, int32_t s0) {
-  int32_t s = L.tptr[v];
-  int n = L.tptr[v + 1] - s;
-  if (hist) hist_add_wave(hist, n < kHistBins - 1 ? n : kHistBins - 1);
-  int32_t count = 0, bcount = 0;
+  bh.init();
+  const int tile = (int)block_index();
+  const int32_t v = tile * kBlock + (int32_t)threadIdx.x;
+  int32_t n = 0, owned = 0, bcount = 0;
   int bad = 0;
-  // the sorted row goes to the block's LDS tile (or straight to trow)
-  auto put = [&](int i, int2 x) __attribute__((always_inline)) {
-    if (STAGED) {
-      if (rows_out) rows_out[s - s0 + i] = x;
-    } else if (L.trow) {
-      L.trow[s + i] = x;
+  if (v < L.nv) {
+    n = L.cnt[v];
+    hist_add_wave(h, n < kHistBins - 1 ? n : kHistBins - 1);
+    int32_t* row = L.slots + (int64_t)kRowSlots * v;
+    if (n <= L.row_cap) {
+      with_row<QUAD>(L, row, n, [&](auto& r) __attribute__((always_inline)) {
+        row_symbolic<SCHEME>(r, v, owned, bcount, bad);
+      });
+    } else {
+      if (n > kRowSlots) {  // the whole row to a run of the pool
+        int32_t* const run = L.tids + atomicAdd(L.pool, n);
+        for (int i = 0; i < kRowSlots; ++i) run[i] = row[i];
+        int32_t c = L.head[v];
+        for (int i = kRowSlots; i < n; ++i) {
+          run[i] = c;
+          c = L.next[c];
+        }
+        row[0] = (int32_t)(run - L.tids);
+        row = run;
+      }
+      sort_row_in_place(row, n);
+      const MemRow<QUAD> r(L, row, n);
+      row_symbolic<SCHEME>(r, v, owned, bcount, bad);
     }
-  };
-  if (n <= CAP) {
-    RegRow<CAP, QUAD> r;
-    if (STAGED)
-      r.load(L, rows_in + (s - s0), n);
-    else
-      r.load(L, L.tids + s, n);
-    row_symbolic<SCHEME>(r, v, count, bcount, bad);
-#pragma unroll
-    for (int i = 0; i < CAP; ++i)
-      if (i < n) put(i, make_int2(r.T(i), r.U(i)));
-    if (L.mpos)
-#pragma unroll
-      for (int i = 0; i < CAP; ++i)
-        if (i < n) L.mpos[r.T(i)] = s + i;
-  } else {
-    sort_row_in_place(L.tids + s, n);
-    MemRow<QUAD> r(L, s, n);
-    row_symbolic<SCHEME>(r, v, count, bcount, bad);
-    for (int i = 0; i < n; ++i) put(i, make_int2(r.T(i), r.U(i)));
-    if (L.mpos)
-      for (int i = 0; i < n; ++i) L.mpos[r.T(i)] = s + i;
+    (void)bcount;
+    L.ecnt[v] = owned;
+    if (bad) {
+      atomicOr(L.flags, bad);
+      if (L.seg.mflags) atomicOr(L.seg.mflags + seg_of(L.seg.vbase, L.seg.n, v), bad);
+    }
   }
-  L.ecnt[v] = count;
-  (void)bcount;
-  if (bad) {
-    atomicOr(L.flags, bad);
-    if (L.seg.mflags) atomicOr(L.seg.mflags + seg_of(L.seg.vbase, L.seg.n, v), bad);
+  const uint64_t sum = block_sum(pack_row(n, owned), wave_sum);
+  if (threadIdx.x == 0) {
+    L.tile_sum[tile] = sum;
+    atomicAdd(reinterpret_cast<unsigned long long*>(L.group_sum) + tile / kTilesPerGroup, (unsigned long long)sum);
   }
+  bh.flush(L.hist_rows);
 }
 
-template <bool QUAD, int SCHEME, int CAP, bool STAGED>
-__device__ __forceinline__ void number_row(const LevelView& L, int32_t v, const int2* rows, int32_t s0);
-template <bool QUAD, bool FP, bool COUNT>
-__device__ __forceinline__ void faces_item(const int32_t* __restrict__ ids, const int32_t* __restrict__ fptr,
-                                           const float4* __restrict__ P, int32_t nf, const SegTable& seg,
-                                           int32_t* __restrict__ cnt, const int* __restrict__ guard, int32_t f);
+// bounds[k] = owned edges before mesh k, k = 0 .. n (several meshes), one
+// wave each
+__global__ void __launch_bounds__(kBlock) k_seg_bounds(LevelView L) {
+  if (*L.flags & kFlagsInput) return;
+  const int32_t k = (int32_t)((blockIdx.x * kBlock + threadIdx.x) >> 6);
+  if (k > L.seg.n) return;  // wave-uniform
+  const int lane = threadIdx.x & 63;
+  const int32_t b = (int32_t)L.seg.vbase[k];
+  const int tile = b / kBlock;
+  uint64_t acc = tiles_before(L, tile, lane, 64) & kOwnedMask;
+  for (int32_t v = tile * kBlock + lane; v < b; v += 64) acc += (uint64_t)L.ecnt[v];
+  for (int d = 32; d > 0; d >>= 1) acc += __shfl_xor(acc, d, 64);
+  if (lane == 0) L.bounds[k] = (int32_t)acc;
+}
 
-// First level: the edge numbering (blocks [0, nbn)) and the face points (the
-// other blocks) are independent; one launch runs both.
-template <bool QUAD, int SCHEME, int CAP>
+// First level, blocks [0, nbn): the rows of R = L.rows_per_block vertices (a
+// part of a sizing tile), one lane per row. The block forms its rows' offsets
+// from the tile sums, writes them and the sorted rows with their
+// in-neighbours (through its LDS tile when they fit: L.tile_entries entries
+// of dynamic LDS), and numbers the edges its vertices own. The other blocks
+// form the face points, which are independent.
+extern __shared__ __align__(16) unsigned char row_tile_lds[];
+
+template <bool QUAD, int SCHEME>
 __global__ void __launch_bounds__(kBlock) k_number_faces(LevelView L, int32_t nbn) {
+  __shared__ uint64_t wave_sum[2][kBlock / 64];
+  __shared__ uint64_t row_at[kBlock + 1];
+  // an invalid mesh: its ids, rows and counts were not (all) written; a
+  // single mesh's numbering is launched before the host has read the flags
+  if (*L.flags & kFlagsInput) return;
   const int64_t b = block_index();
-  if (b < nbn) {
-    // the block's sorted rows through LDS, as in k_symbolic
-    int2* const tile = reinterpret_cast<int2*>(row_tile_lds);  // L.tile_entries entries
-    const int R = L.rows_per_block;
-    const int64_t v0 = b * R;
-    int32_t s0 = 0, len = 0;
-    if (v0 < L.nv) {
-      s0 = L.tptr[v0];
-      len = L.tptr[min(v0 + (int64_t)R, (int64_t)L.nv)] - s0;
-    }
-    const bool staged = len > 0 && len <= L.tile_entries;  // block-uniform
-    if (staged)
-      for (int i = threadIdx.x; i < len; i += blockDim.x) tile[i] = L.trow[s0 + i];
-    __syncthreads();
-    if ((int)threadIdx.x < R) {
-      if (staged)
-        number_row<QUAD, SCHEME, CAP, true>(L, (int32_t)(v0 + threadIdx.x), tile, s0);
-      else
-        number_row<QUAD, SCHEME, CAP, false>(L, (int32_t)(v0 + threadIdx.x), nullptr, s0);
-    }
-  } else
-    faces_item<QUAD, true, false>(L.ids, L.fptr, L.P, L.nf, L.seg, nullptr, nullptr,
-                                  (int32_t)((b - nbn) * blockDim.x + threadIdx.x));
-}
-
-// STAGED: rows is the block's LDS copy of trow from position s0 (else null)
-template <bool QUAD, int SCHEME, int CAP, bool STAGED>
-__device__ __forceinline__ void number_row(const LevelView& L, int32_t v, const int2* rows, int32_t s0) {
-  if (v >= L.nv) return;
-  int32_t s = L.tptr[v];
-  int n = L.tptr[v + 1] - s;
-  if (n <= CAP) {
-    RegRow<CAP, QUAD> r;
-    // the symbolic pass's sorted rows
-    if (STAGED)
-      r.load_sorted(L, rows + (s - s0), n);
-    else
-      r.load_sorted(L, L.trow + s, n);
-    row_number<SCHEME>(r, L, v);
-  } else {
-    // the symbolic pass sorted every row longer than its own capacity; the
-    // in-memory path needs this one sorted whatever that capacity was (idempotent)
-    sort_row_in_place(L.tids + s, n);
-    MemRow<QUAD> r(L, s, n);
-    row_number<SCHEME>(r, L, v);
+  if (b >= nbn) {
+    faces_item<QUAD>(L.ids, L.fptr, L.P, L.nf, L.seg, (int32_t)((b - nbn) * blockDim.x + threadIdx.x));
+    return;
   }
+  int2* const tile_out = reinterpret_cast<int2*>(row_tile_lds);  // (corner, in-neighbour)
+  const int R = L.rows_per_block;
+  const int32_t v0 = (int32_t)b * R;
+  const int tile = v0 / kBlock, r0 = v0 - tile * kBlock;  // the block's rows [r0, r0 + R) of the tile
+  {
+    const int32_t tv = tile * kBlock + (int32_t)threadIdx.x;
+    const uint64_t own = tv < L.nv ? pack_row(L.cnt[tv], L.ecnt[tv]) : 0;
+    const uint64_t before = block_sum(tiles_before(L, tile, threadIdx.x, kBlock), wave_sum[0]);
+    uint64_t total;
+    const uint64_t ex = block_scan_packed(own, wave_sum[1], total);
+    row_at[threadIdx.x] = before + ex;
+    if (threadIdx.x == 0) row_at[kBlock] = before + total;
+  }
+  __syncthreads();
+  const int32_t s0 = (int32_t)(row_at[r0] >> 31);
+  const int32_t len = (int32_t)(row_at[r0 + R] >> 31) - s0;  // 0 rows beyond the last vertex
+  const bool staged = len <= L.tile_entries;                 // block-uniform
+  const int32_t v = v0 + (int32_t)threadIdx.x;
+  if ((int)threadIdx.x < R && v < L.nv) {
+    const uint64_t at = row_at[r0 + threadIdx.x];
+    const int32_t s = (int32_t)(at >> 31), e0 = (int32_t)(at & kOwnedMask);
+    const int n = (int)((int32_t)(row_at[r0 + threadIdx.x + 1] >> 31) - s);
+    L.tptr[v] = s;
+    L.eptr[v] = e0;
+    if (v == L.nv - 1) {
+      L.tptr[L.nv] = s + n;
+      L.eptr[L.nv] = (int32_t)(row_at[r0 + threadIdx.x + 1] & kOwnedMask);
+    }
+    // the sorted row to the LDS tile, or straight to its place
+    // (by a branch around each store: a pointer that may address LDS or
+    // global memory makes every access through it a FLAT instruction)
+    auto put = [&](int i, int32_t t, int32_t u) __attribute__((always_inline)) {
+      if (staged)
+        tile_out[s - s0 + i] = make_int2(t, u);
+      else
+        L.trow[s + i] = make_int2(t, u);
+      if (SCHEME == kSLAK) L.mpos[t] = s + i;
+    };
+    if (n <= L.row_cap) {
+      with_row<QUAD>(L, L.slots + (int64_t)kRowSlots * v, n, [&](auto& r) __attribute__((always_inline)) {
+        constexpr int C = std::decay_t<decltype(r)>::kCap;
+#pragma unroll
+        for (int i = 0; i < C; ++i)
+          if (i < n) put(i, r.T(i), r.U(i));
+        row_number<SCHEME>(r, L, v, e0);
+      });
+    } else {
+      // the sizing pass sorted every row longer than its own capacity; this
+      // one must be sorted whatever that capacity was (idempotent)
+      int32_t* const row = row_corners(L, v, n);
+      sort_row_in_place(row, n);
+      MemRow<QUAD> r(L, row, n);
+      for (int i = 0; i < n; ++i) put(i, r.T(i), r.U(i));
+      row_number<SCHEME>(r, L, v, e0);
+    }
+  }
+  __syncthreads();
+  if (staged)
+    for (int i = threadIdx.x; i < len; i += kBlock) L.trow[s0 + i] = tile_out[i];
 }
 
 template <bool QUAD>
@@ -708,12 +729,12 @@ __global__ void __launch_bounds__(kBlock) k_spgemm_fde(LevelView L) {
   if (v >= L.nv) return;
   int32_t s = L.tptr[v];
   int n = L.tptr[v + 1] - s;
-  if (n <= kRowCap) {
-    RegRow<kRowCap, QUAD> r;
-    r.load(L, s, n);
+  if (n <= kRowSlots) {
+    RegRow<kRowSlots, QUAD> r;
+    r.load_slots(L, L.slots + (int64_t)kRowSlots * v, n);
     row_fde(r, L, v);
   } else {
-    MemRow<QUAD> r(L, s, n);
+    MemRow<QUAD> r(L, row_corners(L, v, n), n);  // sorted by k_symbolic
     row_fde(r, L, v);
   }
 }
@@ -1743,34 +1764,12 @@ constexpr int kScanSmallRounds = 8;  // int4 loads per thread
 constexpr int kScanSmallRound = 4 * kScanSmallThreads;
 constexpr int64_t kScanSmall = (int64_t)kScanSmallRounds * kScanSmallRound;
 
-// 64-bit lane exchange by DPP (row_shr / row_bcast); lanes without a source,
-// and rows outside ROWMASK, read 0.
-template <int CTRL, int ROWMASK>
-__device__ __forceinline__ int64_t dpp64(int64_t x) {
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)x, CTRL, ROWMASK, 0xF, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(x >> 32), CTRL, ROWMASK, 0xF, false);
-  return (int64_t)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
-}
-// Inclusive scan over the 64 lanes of a wave: shifts by 1, 2, 4, 8 inside
-// each row of 16 lanes, then lane 15 of rows 0 / 2 into rows 1 / 3 and lane
-// 31 into rows 2 and 3.
-__device__ __forceinline__ int64_t wave_scan64(int64_t x) {
-  x += dpp64<0x111, 0xF>(x);
-  x += dpp64<0x112, 0xF>(x);
-  x += dpp64<0x114, 0xF>(x);
-  x += dpp64<0x118, 0xF>(x);
-  x += dpp64<0x142, 0xA>(x);
-  x += dpp64<0x143, 0xC>(x);
-  return x;
-}
-
 // Item (r, tid, j) = r * 4096 + 4 tid + j: every load and store instruction
 // of a wave covers 1 KB of consecutive ints, all loads are in flight before
 // the first add, the eight rounds are scanned side by side in registers, and
 // wave 0 scans the 128 wave totals (rounds major) between two barriers.
 __global__ void __launch_bounds__(kScanSmallThreads) k_scan_small(const int32_t* __restrict__ in, int64_t n,
-                                                                  int32_t* __restrict__ out, int* __restrict__ flags,
-                                                                  int32_t* __restrict__ total_out) {
+                                                                  int32_t* __restrict__ out, int* __restrict__ flags) {
   constexpr int kWaves = kScanSmallThreads / 64;
   static_assert(kScanSmallRounds * kWaves == 128, "wave 0 scans two wave totals per lane");
   __shared__ int64_t wsum[kScanSmallRounds * kWaves];
@@ -1829,7 +1828,6 @@ __global__ void __launch_bounds__(kScanSmallThreads) k_scan_small(const int32_t*
     const int64_t carry = total;
     if (carry > 0x7fffffffll) atomicOr(flags, kFlagOverflow);
     out[n] = (int32_t)carry;
-    if (total_out) *total_out = (int32_t)carry;
   }
 }
 
@@ -1864,8 +1862,7 @@ __global__ void __launch_bounds__(kBlock) k_scan_reduce(const int32_t* __restric
 }
 
 __global__ void __launch_bounds__(kBlock) k_scan_partials(int64_t* __restrict__ partial, int64_t ntiles,
-                                                          int32_t* __restrict__ out, int64_t n, int* __restrict__ flags,
-                                                          int32_t* __restrict__ total_out) {
+                                                          int32_t* __restrict__ out, int64_t n, int* __restrict__ flags) {
   __shared__ int64_t lds[kBlock / 64];
   int64_t carry = 0;
   for (int64_t b = 0; b < ntiles; b += kBlock) {
@@ -1879,19 +1876,17 @@ __global__ void __launch_bounds__(kBlock) k_scan_partials(int64_t* __restrict__ 
   if (threadIdx.x == 0) {
     if (carry > 0x7fffffffll) atomicOr(flags, kFlagOverflow);
     out[n] = (int32_t)carry;
-    if (total_out) *total_out = (int32_t)carry;
   }
 }
 
 // FOLD: partial holds the tile sums (no partials pass); each block adds up
 // the sums of the tiles before it, and block 0 also forms the total
-// (out[n], total_out, the overflow flag). Without FOLD partial holds the
+// (out[n], the overflow flag). Without FOLD partial holds the
 // exclusive tile prefixes.
 template <bool FOLD>
 __global__ void __launch_bounds__(kBlock) k_scan_down(const int32_t* __restrict__ in, int64_t n,
                                                       const int64_t* __restrict__ partial, int32_t* __restrict__ out,
-                                                      int64_t ntiles, int* __restrict__ flags,
-                                                      int32_t* __restrict__ total_out) {
+                                                      int64_t ntiles, int* __restrict__ flags) {
   constexpr int kWaves = kBlock / 64;
   __shared__ int64_t wsum[kScanRounds * kWaves];
   __shared__ int64_t red[kBlock / 64];
@@ -1907,13 +1902,11 @@ __global__ void __launch_bounds__(kBlock) k_scan_down(const int32_t* __restrict_
       if (threadIdx.x == 0) {
         if (carry > 0x7fffffffll) atomicOr(flags, kFlagOverflow);
         out[n] = (int32_t)carry;
-        if (total_out) *total_out = (int32_t)carry;
       }
     }
   } else {
     (void)ntiles;
     (void)flags;
-    (void)total_out;
   }
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const bool vin = (reinterpret_cast<uintptr_t>(in) & 15) == 0;
@@ -1979,21 +1972,43 @@ void launch_fill_i32(int32_t* p, int64_t n, int32_t value, hipStream_t st) {
   k_fill_i32<<<(unsigned)g, kBlock, 0, st>>>(p, n, value);
 }
 
-void launch_gather(const SegTable& seg, int32_t nf_total, bool use_vals, int32_t* ids_pos, int32_t* fptr,
-                   int32_t* cface, int* flags, int32_t* zero, int32_t nzero, int32_t* hist_faces, hipStream_t st) {
-  const int32_t n = std::max(nf_total, nzero);
-  if (n <= 0) return;
-  k_gather<<<grid_for(n), kBlock, 0, st>>>(seg, nf_total, use_vals ? 1 : 0, ids_pos, fptr, cface, flags, zero,
-                                          nzero, hist_faces);
+// row slots by the block's vertex window (default); SLAK_COUNT_WINDOW=0 takes
+// one device atomic per corner (read once)
+static bool count_window() {
+  static const bool on = [] {
+    const char* e = std::getenv("SLAK_COUNT_WINDOW");
+    return !e || std::atoi(e) != 0;
+  }();
+  return on;
+}
+
+void launch_gather(bool quad, const SegTable& seg, bool use_vals, int32_t* ids_pos, const LevelView& L,
+                   hipStream_t st) {
+  if (L.nf <= 0) return;
+  const RowBuild rb{L.cnt, L.slots, L.head, L.next};
+  const int vals = use_vals ? 1 : 0, window = count_window() ? 1 : 0;
+  int32_t* const fptr = const_cast<int32_t*>(L.fptr);
+  int32_t* const cface = const_cast<int32_t*>(L.cface);
+  if (quad)
+    k_gather<true><<<grid_for(L.nf), kBlock, 0, st>>>(seg, L.nf, vals, ids_pos, fptr, cface, L.flags, rb, window);
+  else
+    k_gather<false><<<grid_for(L.nf), kBlock, 0, st>>>(seg, L.nf, vals, ids_pos, fptr, cface, L.flags, rb, window);
+}
+
+void launch_setup(const void* src_pinned, void* dst, int64_t bytes, int32_t* zero, int64_t nzero, hipStream_t st) {
+  if (bytes <= 0 && nzero <= 0) return;
+  if ((bytes & 15) || (nzero & 3)) throw Error(5, "setup of partial 16-byte pieces");  // SLAK_ERR_INTERNAL
+  void* src = nullptr;
+  if (bytes > 0) SLAK_HIP_CHECK(hipHostGetDevicePointer(&src, const_cast<void*>(src_pinned), 0));
+  const int64_t n = bytes / 16, nz = nzero / 4;
+  const unsigned g = std::min<unsigned>(4096, grid_for(std::max(n, nz)));
+  k_setup<<<g, kBlock, 0, st>>>(static_cast<const int4*>(src), static_cast<int4*>(dst), n,
+                                reinterpret_cast<int4*>(zero), nz);
 }
 
 void launch_gather_verts(const SegTable& seg, int32_t nv_total, float4* P, hipStream_t st) {
   if (nv_total <= 0) return;
   k_gather_verts<<<grid_for(nv_total), kBlock, 0, st>>>(seg, nv_total, P);
-}
-
-void launch_seg_bounds(const int64_t* vbase, int32_t n, const int32_t* eptr, int32_t* bounds, hipStream_t st) {
-  k_seg_bounds<<<grid_for(n + 1), kBlock, 0, st>>>(vbase, n, eptr, bounds);
 }
 
 void launch_copy_probe(const float4* a, float4* b, int64_t n, hipStream_t st) {
@@ -2010,75 +2025,28 @@ void launch_digest(const void* p, int64_t bytes, uint64_t* out, hipStream_t st) 
   k_digest<<<g, kBlock, 0, st>>>(static_cast<const uint8_t*>(p), bytes, reinterpret_cast<unsigned long long*>(out));
 }
 
-// the valence count and transpose through the block's vertex window (default);
-// SLAK_COUNT_WINDOW=0 takes one device atomic per corner (read once)
-static bool count_window() {
-  static const bool on = [] {
-    const char* e = std::getenv("SLAK_COUNT_WINDOW");
-    return !e || std::atoi(e) != 0;
-  }();
-  return on;
-}
-
-void launch_faces(bool quad, bool fp, bool count, const int32_t* ids, const int32_t* fptr, const float4* P, int32_t nf,
-                  const SegTable& seg, int32_t* cnt, const int* guard, hipStream_t st) {
+void launch_faces(bool quad, const int32_t* ids, const int32_t* fptr, const float4* P, int32_t nf, const SegTable& seg,
+                  hipStream_t st) {
   if (nf <= 0) return;
-  unsigned g = grid_for(nf);
-  if (count && !fp && count_window()) {  // the valence count alone: through the block's vertex window
-    if (quad)
-      k_count<true><<<g, kBlock, 0, st>>>(ids, fptr, nf, cnt, guard);
-    else
-      k_count<false><<<g, kBlock, 0, st>>>(ids, fptr, nf, cnt, guard);
-    return;
-  }
-#define SLAK_FACES(Q, A, B) k_faces<Q, A, B><<<g, kBlock, 0, st>>>(ids, fptr, P, nf, seg, cnt, guard)
-  if (quad) {
-    if (fp && count) SLAK_FACES(true, true, true);
-    else if (fp) SLAK_FACES(true, true, false);
-    else if (count) SLAK_FACES(true, false, true);
-  } else {
-    if (fp && count) SLAK_FACES(false, true, true);
-    else if (fp) SLAK_FACES(false, true, false);
-    else if (count) SLAK_FACES(false, false, true);
-  }
-#undef SLAK_FACES
-}
-
-void launch_transpose(bool quad, const int32_t* ids, const int32_t* fptr, int32_t nf, const int32_t* tptr,
-                      int32_t* cnt, int32_t* tids, const int* guard, hipStream_t st) {
-  if (nf <= 0) return;
-  const int window = count_window() ? 1 : 0;
   if (quad)
-    k_transpose<true><<<grid_for(nf), kBlock, 0, st>>>(ids, fptr, nf, tptr, cnt, tids, guard, window);
+    k_faces<true><<<grid_for(nf), kBlock, 0, st>>>(ids, fptr, P, nf, seg);
   else
-    k_transpose<false><<<grid_for(nf), kBlock, 0, st>>>(ids, fptr, nf, tptr, cnt, tids, guard, window);
+    k_faces<false><<<grid_for(nf), kBlock, 0, st>>>(ids, fptr, P, nf, seg);
 }
 
-// cap: M^T row length held in registers (4 or 8); longer rows take the
-// in-memory path. Chosen per level from the row-length histogram.
-#define SLAK_ROW_DISPATCH(KERNEL, quad, scheme, cap, g, smem, L, st)                  \
+#define SLAK_ROW_DISPATCH(KERNEL, quad, scheme, g, smem, st, ...)                      \
   do {                                                                                \
     if (quad) {                                                                       \
-      if (scheme == kLAK) {                                                           \
-        if (cap <= 4) KERNEL<true, kLAK, 4><<<g, kBlock, smem, st>>>(L);              \
-        else KERNEL<true, kLAK, 8><<<g, kBlock, smem, st>>>(L);                       \
-      } else {                                                                        \
-        if (cap <= 4) KERNEL<true, kSLAK, 4><<<g, kBlock, smem, st>>>(L);             \
-        else KERNEL<true, kSLAK, 8><<<g, kBlock, smem, st>>>(L);                      \
-      }                                                                               \
+      if (scheme == kLAK) KERNEL<true, kLAK><<<g, kBlock, smem, st>>>(__VA_ARGS__);   \
+      else KERNEL<true, kSLAK><<<g, kBlock, smem, st>>>(__VA_ARGS__);                 \
     } else {                                                                          \
-      if (scheme == kLAK) {                                                           \
-        if (cap <= 4) KERNEL<false, kLAK, 4><<<g, kBlock, smem, st>>>(L);             \
-        else KERNEL<false, kLAK, 8><<<g, kBlock, smem, st>>>(L);                      \
-      } else {                                                                        \
-        if (cap <= 4) KERNEL<false, kSLAK, 4><<<g, kBlock, smem, st>>>(L);            \
-        else KERNEL<false, kSLAK, 8><<<g, kBlock, smem, st>>>(L);                     \
-      }                                                                               \
+      if (scheme == kLAK) KERNEL<false, kLAK><<<g, kBlock, smem, st>>>(__VA_ARGS__);  \
+      else KERNEL<false, kSLAK><<<g, kBlock, smem, st>>>(__VA_ARGS__);                \
     }                                                                                 \
   } while (0)
 
 // rows per block (64, 128 or 256) and LDS tile (even, 256..kRowTileMax
-// entries) of the first level's row kernels
+// entries) of the numbering
 static void check_row_tiling(const LevelView& L) {
   if (L.rows_per_block != 64 && L.rows_per_block != 128 && L.rows_per_block != kBlock)
     throw Error(5, "rows per block must be 64, 128 or 256");  // SLAK_ERR_INTERNAL
@@ -2086,39 +2054,25 @@ static void check_row_tiling(const LevelView& L) {
     throw Error(5, "row tile out of range");  // SLAK_ERR_INTERNAL
 }
 
-void launch_symbolic(bool quad, int scheme, int cap, const LevelView& L, hipStream_t st) {
+void launch_symbolic(bool quad, int scheme, const LevelView& L, hipStream_t st) {
   if (L.nv <= 0) return;
-  check_row_tiling(L);
-  unsigned g = grid_for(L.nv, L.rows_per_block);
-  const size_t smem = (size_t)L.tile_entries * (sizeof(int32_t) + sizeof(int2));
-  SLAK_ROW_DISPATCH(k_symbolic, quad, scheme, cap, g, smem, L, st);
+  const unsigned g = grid_for(L.nv);
+  SLAK_ROW_DISPATCH(k_symbolic, quad, scheme, g, 0, st, L);
 }
 
-void launch_number_faces(bool quad, int scheme, int cap, const LevelView& L, bool faces, hipStream_t st) {
-  if (!L.trow) throw Error(5, "edge numbering without the symbolic pass's rows");  // SLAK_ERR_INTERNAL
+void launch_seg_bounds(const LevelView& L, hipStream_t st) {
+  if (L.nv <= 0) return;
+  k_seg_bounds<<<grid_for((int64_t)(L.seg.n + 1) * 64), kBlock, 0, st>>>(L);
+}
+
+void launch_number_faces(bool quad, int scheme, const LevelView& L, bool faces, hipStream_t st) {
   check_row_tiling(L);
   const int32_t nbn = L.nv > 0 ? (int32_t)grid_for(L.nv, L.rows_per_block) : 0;
   const size_t smem = (size_t)L.tile_entries * sizeof(int2);
   const int32_t nbf = faces && L.nf > 0 ? (int32_t)grid_for(L.nf) : 0;
   if (nbn + nbf == 0) return;
   const unsigned g = (unsigned)(nbn + nbf);
-  if (quad) {
-    if (scheme == kLAK) {
-      if (cap <= 4) k_number_faces<true, kLAK, 4><<<g, kBlock, smem, st>>>(L, nbn);
-      else k_number_faces<true, kLAK, 8><<<g, kBlock, smem, st>>>(L, nbn);
-    } else {
-      if (cap <= 4) k_number_faces<true, kSLAK, 4><<<g, kBlock, smem, st>>>(L, nbn);
-      else k_number_faces<true, kSLAK, 8><<<g, kBlock, smem, st>>>(L, nbn);
-    }
-  } else {
-    if (scheme == kLAK) {
-      if (cap <= 4) k_number_faces<false, kLAK, 4><<<g, kBlock, smem, st>>>(L, nbn);
-      else k_number_faces<false, kLAK, 8><<<g, kBlock, smem, st>>>(L, nbn);
-    } else {
-      if (cap <= 4) k_number_faces<false, kSLAK, 4><<<g, kBlock, smem, st>>>(L, nbn);
-      else k_number_faces<false, kSLAK, 8><<<g, kBlock, smem, st>>>(L, nbn);
-    }
-  }
+  SLAK_ROW_DISPATCH(k_number_faces, quad, scheme, g, smem, st, L, nbn);
 }
 
 void launch_spgemm_fde(bool quad, const LevelView& L, hipStream_t st) {
@@ -2294,20 +2248,19 @@ int64_t noalloc_scan_max_items() {
   return (partials - 1) * kScanTile;  // scan_partials_len(n) <= partials
 }
 
-void launch_scan(const int32_t* in, int32_t* out, int64_t n, int64_t* partial, int* flags, hipStream_t st,
-                 int32_t* total_out) {
+void launch_scan(const int32_t* in, int32_t* out, int64_t n, int64_t* partial, int* flags, hipStream_t st) {
   if (n <= kScanSmall) {
-    k_scan_small<<<1, kScanSmallThreads, 0, st>>>(in, n, out, flags, total_out);
+    k_scan_small<<<1, kScanSmallThreads, 0, st>>>(in, n, out, flags);
     return;
   }
   int64_t ntiles = (n + kScanTile - 1) / kScanTile;
   k_scan_reduce<<<(unsigned)ntiles, kBlock, 0, st>>>(in, n, partial);
   if (ntiles <= kScanFoldTiles) {  // two launches: each tile adds up the sums before it
-    k_scan_down<true><<<(unsigned)ntiles, kBlock, 0, st>>>(in, n, partial, out, ntiles, flags, total_out);
+    k_scan_down<true><<<(unsigned)ntiles, kBlock, 0, st>>>(in, n, partial, out, ntiles, flags);
     return;
   }
-  k_scan_partials<<<1, kBlock, 0, st>>>(partial, ntiles, out, n, flags, total_out);
-  k_scan_down<false><<<(unsigned)ntiles, kBlock, 0, st>>>(in, n, partial, out, ntiles, flags, total_out);
+  k_scan_partials<<<1, kBlock, 0, st>>>(partial, ntiles, out, n, flags);
+  k_scan_down<false><<<(unsigned)ntiles, kBlock, 0, st>>>(in, n, partial, out, ntiles, flags);
 }
 
 }  // namespace slak

@@ -86,42 +86,22 @@ void check_i32(int64_t x, const std::string& what) {
 
 }  // namespace
 
-// Register capacity of the SpGEMM row kernels for a level with the given
-// row-length statistics. Rows above the capacity take the in-memory path
-// (correct for any length, slower); capacity 4 keeps the row state in half
-// the registers, which doubles occupancy. Pick 4 when every row fits or the
-// long rows are rare enough that the waves they stall cost less than the
-// occupancy gained; the threshold is a tuned constant (SLAK_CAP_THRESHOLD
-// overrides it, SLAK_ROW_CAP forces a capacity).
-int autotune_cap(bool quad, int64_t nv, int64_t long_rows, int max_row) {
-  const char* ef = std::getenv("SLAK_ROW_CAP");
-  const char* et = std::getenv("SLAK_CAP_THRESHOLD");
-  const int forced = ef ? std::atoi(ef) : 0;
-  const double thresh = et ? std::atof(et) : 0.02;
-  if (forced == 4 || forced == 8) return forced;
-  if (max_row <= 4) return 4;
-  if (nv <= 0) return 8;
-  double frac = (double)long_rows / (double)nv;
-  (void)quad;
-  return frac < thresh ? 4 : 8;
+// Register capacity of the first level's row kernels: rows up to it are
+// processed in registers, longer ones (correct for any length, slower) from
+// memory. SLAK_ROW_CAP=4 sends rows of 5 and more down the in-memory path.
+static int row_capacity() {
+  const char* e = std::getenv("SLAK_ROW_CAP");
+  return e && std::atoi(e) == 4 ? 4 : kRowSlots;
 }
 
-// Rows per block and LDS row tile of the first level's row kernels
-// (k_symbolic, the numbering of k_number_faces). A block of R rows needs
-// about R m + 3 sqrt(R) sigma tile entries, with m the mean row length
-// (corners over vertices) and sigma the spread of row lengths from the
+// Rows per block and LDS row tile of the first level's numbering. A block of
+// R rows needs about R m + 3 sqrt(R) sigma tile entries, with m the mean row
+// length (corners over vertices) and sigma the spread of row lengths from the
 // histogram (hist: kRowHistBins counts, the last bin "longer"; without one,
-// sigma = 1): R is the largest of 256, 128, 64 whose need fits kRowTileMax,
-// and the tile that need rounded up to 256 entries (at least 1024). A block
-// whose rows exceed the tile reads them from global memory. With rows
-// averaging more than 5 the numbering takes half as many rows per block (at
-// least 64). Medians of interleaved runs on a 1024 x 1024 triangle torus
-// (rows of 6): numbering 89.5 -> 72.5 us, while the sizing pass is fastest at
-// R = 256 (62.8 against 74.7 us at 128). With rows of about 4 the numbering
-// gains little or loses at R/2 (quad 1024 x 1024 torus 38.6 -> 35.0 us, the
-// 256 x 128 mixed torus 11.8 -> 13.5 us, the 4096-mesh batch 385 -> 450 us).
-// SLAK_ROWS_PER_BLOCK forces the sizing pass's R, SLAK_ROWS_NUMBER the
-// numbering's.
+// sigma = 1): R is the largest of 256, 128, 64 whose need fits kRowTileMax
+// (half of it when rows average more than 5), and the tile that need rounded
+// up to 256 entries (at least 1024). A block whose rows exceed the tile stores
+// them directly. SLAK_ROWS_NUMBER forces R.
 RowTiling autotune_rows(int64_t nv, int64_t nnz, const int64_t* hist) {
   double m = nv > 0 ? (double)nnz / (double)nv : 4.0;
   double sigma = 1.0;
@@ -140,18 +120,13 @@ RowTiling autotune_rows(int64_t nv, int64_t nnz, const int64_t* hist) {
       R = r;
       break;
     }
-  if (const char* e = std::getenv("SLAK_ROWS_PER_BLOCK")) {
+  if (m > 5.0) R = std::max(64, R / 2);
+  if (const char* e = std::getenv("SLAK_ROWS_NUMBER")) {
     const int forced = std::atoi(e);
     if (forced == 64 || forced == 128 || forced == 256) R = forced;
   }
   const double want = std::ceil(need(R) / 256.0) * 256.0;
-  const int tile = (int)std::min<double>(kRowTileMax, std::max(1024.0, want));
-  int Rn = m > 5.0 ? std::max(64, R / 2) : R;
-  if (const char* e = std::getenv("SLAK_ROWS_NUMBER")) {
-    const int forced = std::atoi(e);
-    if (forced == 64 || forced == 128 || forced == 256) Rn = forced;
-  }
-  return RowTiling{R, Rn, tile};
+  return RowTiling{R, (int)std::min<double>(kRowTileMax, std::max(1024.0, want))};
 }
 
 Plan::Plan(int scheme, std::vector<MeshJob> jobs, OutputMode mode, hipStream_t st)
@@ -211,7 +186,7 @@ int Plan::readback(const int32_t* src, int count, int64_t* dst, const std::funct
 // Uploads the segment tables (SegDesc, vertex, face and corner bases) of levels
 // [l0, l1) in one copy from a plan-owned staging buffer (one per call site,
 // so a pending copy never sees its source rewritten).
-void Plan::upload_tables(int l0, int l1, Staging& staging, int64_t state_ints) {
+void Plan::upload_tables(int l0, int l1, Staging& staging, bool zero_state) {
   auto align = [](size_t x) { return (x + 255) & ~(size_t)255; };
   size_t total = 0;
   std::vector<size_t> offs;
@@ -225,8 +200,6 @@ void Plan::upload_tables(int l0, int l1, Staging& staging, int64_t state_ints) {
     offs.push_back(total);
     total = align(total + n * sizeof(SegDesc)) + align(3 * (n + 1) * sizeof(int64_t)) + fin_bytes(levels_[l]);
   }
-  const size_t state_off = total;
-  total += align((size_t)state_ints * sizeof(int32_t));
   if (total == 0) return;
   if (staging.p) SLAK_HIP_CHECK(hipStreamSynchronize(st_));  // reused: an earlier copy may still read it
   if (staging.cap < total) {
@@ -235,10 +208,6 @@ void Plan::upload_tables(int l0, int l1, Staging& staging, int64_t state_ints) {
   }
   std::memset(staging.p, 0, total);
   char* d = arena_.get_n<char>((int64_t)total);
-  if (state_ints > 0) {  // the plan's state block, zeros
-    d_state_ = reinterpret_cast<int32_t*>(d + state_off);
-    d_flags_ = d_state_;
-  }
   for (int l = l0; l < l1; ++l) {
     LevelPlan& L = levels_[l];
     const size_t n = L.segs.size();
@@ -269,7 +238,7 @@ void Plan::upload_tables(int l0, int l1, Staging& staging, int64_t state_ints) {
       o = align(o + T->units.size() * sizeof(int4));
     }
   }
-  SLAK_HIP_CHECK(hipMemcpyAsync(d, staging.p, total, hipMemcpyHostToDevice, st_));
+  launch_setup(staging.p, d, (int64_t)total, zero_state ? d_state_ : nullptr, zero_state ? n_state_ : 0, st_);
 }
 
 std::string Plan::describe_failure(int fl) const {
@@ -332,17 +301,24 @@ void Plan::plan_first_level() {
   check_i32(L.nnz, "corners of the first level");
   check_i32(4 * L.nnz, "refined corners of the first level");
   const RowTiling rt = autotune_rows(L.nv, L.nnz, nullptr);
+  L.cap = row_capacity();
   L.rows = rt.rows;
-  L.rows_num = rt.rows_num;
   L.tile = rt.tile;
 
   // one arena block for the first level's buffers and the analysis state
   // that follows (the table upload, the scan partials, a single mesh's
   // boundary flags); anything beyond it comes from the pool as before
+  const int64_t nseg = (int64_t)L.segs.size();
+  const int64_t at_dev = (kStateBounds + 2 * nseg + 1 + 3) & ~(int64_t)3;  // 16-byte aligned
+  const int64_t ntiles = (L.nv + kBlockItems - 1) / kBlockItems, ngroups = (ntiles + kTilesPerGroup - 1) / kTilesPerGroup;
+  const int64_t at_groups = at_dev + 4;
+  const int64_t at_cnt = (at_groups + 2 * ngroups + 3) & ~(int64_t)3;
+  n_state_ = (at_cnt + L.nv + 3) & ~(int64_t)3;
   {
     auto line = [](int64_t n, size_t elem) { return ((size_t)std::max<int64_t>(n, 1) * elem + 255) & ~(size_t)255; };
-    size_t est = line(L.nnz, 4) + line(L.nv, 4) + line(L.nv + 1, 4) + line(L.nnz, 4) + 2 * line(L.nnz, 8) +
-                 line(L.nv, 4) + line(L.nv + 1, 4) + line(L.nnz, 4);
+    size_t est = 2 * line(L.nnz, 4) + 2 * line(L.nnz, 8) + line(L.nv, 4 * kRowSlots) + 2 * line(L.nv, 4) +
+                 2 * line(L.nv + 1, 4) + line(n_state_, 4) +
+                 line(ntiles, 8);
     if (!L.quad) est += line(L.nf + 1, 4) + line(L.nnz, 4);
     if (L.segs.size() != 1) est += line(L.nv, 16);
     if (scheme_ == kSLAK) est += line(L.nnz, 4);
@@ -361,64 +337,78 @@ void Plan::plan_first_level() {
     P1_ = arena_.get_n<float4>(L.nv);
     L.P = P1_;
   }
-  d_cnt_ = arena_.get_n<int32_t>(L.nv);
-  L.cnt = d_cnt_;
+  d_state_ = arena_.get_n<int32_t>(n_state_);
+  d_flags_ = d_state_;
+  L.pool = d_state_ + at_dev;
+  L.group_sum = reinterpret_cast<uint64_t*>(d_state_ + at_groups);
+  at_groups_ = at_groups;
+  n_groups_ = ngroups;
+  L.cnt = d_state_ + at_cnt;
+  L.slots = arena_.get_n<int32_t>(kRowSlots * L.nv);
+  L.head = arena_.get_n<int32_t>(L.nv);
+  L.ecnt = arena_.get_n<int32_t>(L.nv);
+  L.tile_sum = arena_.get_n<uint64_t>(ntiles);
   L.tptr = arena_.get_n<int32_t>(L.nv + 1);
   L.tids = arena_.get_n<int32_t>(L.nnz);
   L.trow = arena_.get_n<int2>(L.nnz);
   L.ci = arena_.get_n<int2>(L.nnz);
   if (scheme_ == kSLAK) L.mpos = arena_.get_n<int32_t>(L.nnz);
-  L.ecnt = arena_.get_n<int32_t>(L.nv);
   L.eptr = arena_.get_n<int32_t>(L.nv + 1);
 }
 
-// First-level analysis: M^T by counting sort, sorted rows with in-neighbours
-// and owned-edge counts (later levels receive their structure from the level
-// before).
+LevelView LevelPlan::view(int* flags) const {
+  LevelView V{};
+  V.ids = ids;
+  V.fptr = fptr;
+  V.cface = cface;
+  V.P = P;
+  V.nv = (int32_t)nv;
+  V.nf = (int32_t)nf;
+  V.nnz = nnz;
+  V.tptr = tptr;
+  V.cnt = cnt;
+  V.slots = slots;
+  V.head = head;
+  V.next = reinterpret_cast<int32_t*>(ci);  // free until the numbering writes the pairs
+  V.tids = tids;
+  V.pool = pool;
+  V.ecnt = ecnt;
+  V.tile_sum = tile_sum;
+  V.group_sum = group_sum;
+  V.row_cap = cap;
+  V.rows_per_block = rows;
+  V.trow = trow;
+  V.mpos = mpos;
+  V.eptr = eptr;
+  V.flags = flags;
+  V.seg = table();
+  V.tile_entries = tile;
+  return V;
+}
+
+// Validation, position order, valences and the rows' corners in one launch.
+void Plan::record_gather(LevelPlan& L) {
+  ProfScope ps(st_, {{"gather", 4.0 * (L.nf + 1) + 12.0 * L.nnz + (L.quad ? 0.0 : 8.0 * L.nnz + 4.0 * L.nf)},
+                     {L.quad ? "count_quad" : "count_poly", 4.0 * L.nnz + 8.0 * L.nv + (L.quad ? 0.0 : 4.0 * L.nf)},
+                     {L.quad ? "transpose_quad" : "transpose_poly",
+                      8.0 * L.nnz + 12.0 * L.nv + (L.quad ? 0.0 : 4.0 * L.nf)}});
+  launch_gather(L.quad, L.table(), scheme_ == kLAK, const_cast<int32_t*>(L.ids), L.view(d_flags_), st_);
+}
+
+// First-level analysis: sorted rows of M^T with in-neighbours and their
+// offsets, owned-edge counts and offsets (later levels receive their structure
+// from the level before).
 void Plan::record_analysis(LevelPlan& L) {
   const double poly_b = L.quad ? 0.0 : 4.0 * (L.nf + 1) + 4.0 * L.nnz;
-  {
-    ProfScope ps(st_, L.quad ? "count_quad" : "count_poly", 4.0 * L.nnz + 8.0 * L.nv + (L.quad ? 0.0 : 4.0 * L.nf));
-    launch_faces(L.quad, false, true, L.ids, L.fptr, L.P, (int32_t)L.nf, L.table(), L.cnt, d_flags_, st_);
-  }
-  {
-    ProfScope ps(st_, "scan", 8.0 * L.nv + 4);
-    launch_scan(L.cnt, L.tptr, L.nv, d_partial_, d_flags_, st_);
-  }
-  {
-    ProfScope ps(st_, L.quad ? "transpose_quad" : "transpose_poly",
-                 8.0 * L.nnz + 12.0 * L.nv + (L.quad ? 0.0 : 4.0 * L.nf));
-    launch_transpose(L.quad, L.ids, L.fptr, (int32_t)L.nf, L.tptr, L.cnt, L.tids, d_flags_, st_);
-  }
-  LevelView V{};
-  V.ids = L.ids;
-  V.fptr = L.fptr;
-  V.cface = L.cface;
-  V.P = L.P;
-  V.nv = (int32_t)L.nv;
-  V.nf = (int32_t)L.nf;
-  V.nnz = L.nnz;
-  V.tptr = L.tptr;
-  V.tids = L.tids;
-  V.trow = L.trow;
-  V.mpos = L.mpos;
-  V.ecnt = L.ecnt;
+  LevelView V = L.view(d_flags_);
   V.hist_rows = d_state_ + kStateRowHist;
-  V.rows_per_block = L.rows;
-  V.tile_entries = L.tile;
-  V.flags = d_flags_;
-  V.seg = L.table();
-  {
-    ProfScope ps(st_, L.quad ? "spgemm_symbolic_quad" : "spgemm_symbolic_poly",
-                 8.0 * L.nnz + 8.0 * L.nv + 8.0 * L.nnz + poly_b);
-    launch_symbolic(L.quad, scheme_, L.cap, V, st_);
-  }
-  {
-    // a single mesh's edge total goes straight to its read-back slot
-    int32_t* bounds = d_state_ + kStateBounds;
-    ProfScope ps(st_, "scan", 8.0 * L.nv + 4);
-    launch_scan(L.ecnt, L.eptr, L.nv, d_partial_, d_flags_, st_, L.segs.size() == 1 ? bounds + 1 : nullptr);
-  }
+  V.bounds = d_state_ + kStateBounds;
+  ProfScope ps(st_, {{"scan", 8.0 * L.nv + 4},
+                     {L.quad ? "spgemm_symbolic_quad" : "spgemm_symbolic_poly",
+                      8.0 * L.nnz + 8.0 * L.nv + 8.0 * L.nnz + poly_b},
+                     {"scan", 8.0 * L.nv + 4}});
+  launch_symbolic(L.quad, scheme_, V, st_);
+  if (L.segs.size() > 1) launch_seg_bounds(V, st_);
 }
 
 void Plan::prepare() {
@@ -468,19 +458,10 @@ void Plan::prepare() {
       L1.segs[0].dst_verts = early_p1_;
     }
   }
-  n_state_ = kStateBounds + (nseg + 1) + nseg;
-  upload_tables(0, 1, staging_first_, n_state_);
-  int64_t need = scan_partials_len(L1.nv);
-  d_partial_ = arena_.get_n<int64_t>(need);
-  partial_len_ = need;
+  upload_tables(0, 1, staging_first_, true);
 
-  // 1. validate + gather (the state block arrived zeroed with the tables)
-  {
-    ProfScope ps(st_, "gather", 4.0 * (L1.nf + 1) + 12.0 * L1.nnz + (L1.quad ? 0.0 : 8.0 * L1.nnz + 4.0 * L1.nf));
-    launch_gather(L1.table(), (int32_t)L1.nf, scheme_ == kLAK, const_cast<int32_t*>(L1.ids),
-                  const_cast<int32_t*>(L1.fptr), const_cast<int32_t*>(L1.cface), d_flags_, d_cnt_, (int32_t)L1.nv,
-                  d_state_ + kStateFaceHist, st_);
-  }
+  // 1. validate + gather (the state block is zeroed with the table upload)
+  record_gather(L1);
   if (P1_) launch_gather_verts(L1.table(), (int32_t)L1.nv, P1_, st_);
   auto fail_if = [&](int fl) {
     if (!fl) return;
@@ -498,53 +479,35 @@ void Plan::prepare() {
   // (its kernels do nothing on an input the gather flagged; the flags come
   // back with the edge counts in one round trip)
   record_analysis(L1);
-  int32_t* d_bounds = d_state_ + kStateBounds;
-  if (nseg > 1) launch_seg_bounds(L1.d_vbase, nseg, L1.eptr, d_bounds, st_);
-  std::vector<int64_t> hb(2 * kRowHistBins + nseg + 1, 0);
+  std::vector<int64_t> hb(kRowHistBins + nseg + 1, 0);
   bool have_hist = false;
   if (!all_known) {
     std::function<void()> overlap;
     if (early) overlap = [this, &L1] { launch_number(L1, early_p1_ != nullptr); };
     // state ints 1 .. kStateBounds + nseg: flags, the histogram copies, the edge bounds
-    std::vector<int64_t> sb((size_t)kStateBounds + nseg, 0);
-    fail_if(readback(nullptr, kStateBounds + nseg, sb.data(), overlap));
+    // (a single mesh: up to its group sums, whose edges make its total)
+    const int nread = nseg == 1 ? (int)(at_groups_ + 2 * n_groups_ - 1) : kStateBounds + nseg;
+    std::vector<int64_t> sb((size_t)nread, 0);
+    fail_if(readback(nullptr, nread, sb.data(), overlap));
     for (int c = 0; c < kHistCopies; ++c)
-      for (int b = 0; b < kRowHistBins; ++b) {
-        hb[b] += sb[kStateRowHist - 1 + c * kHistStride + b];
-        hb[kRowHistBins + b] += sb[kStateFaceHist - 1 + c * kHistStride + b];
-      }
-    for (int k = 0; k <= nseg; ++k) hb[2 * kRowHistBins + k] = sb[kStateBounds - 1 + k];
+      for (int b = 0; b < kRowHistBins; ++b) hb[b] += sb[kStateRowHist - 1 + c * kHistStride + b];
+    for (int k = 0; k <= nseg; ++k) hb[kRowHistBins + k] = sb[kStateBounds - 1 + k];
+    if (nseg == 1)
+      for (int64_t g = 0; g < n_groups_; ++g)
+        hb[kRowHistBins + 1] += sb[at_groups_ - 1 + 2 * g] & 0x7fffffff;  // (corners << 31 | edges)
     // the early numbering was recorded before its edge count was known: its
     // boundary-flag writes (4 bytes per edge) join its algorithmic bytes now
     if (early && Profiler::get().enabled())
       Profiler::get().amend_last(L1.quad ? "number_facepoints_quad" : "number_facepoints_poly",
-                                 4.0 * (double)hb[2 * kRowHistBins + 1]);
+                                 4.0 * (double)hb[kRowHistBins + 1]);
     number_early_ = early;
     early_faces_ = early && early_p1_ != nullptr;
     have_hist = true;
   } else {
     if (!all_trusted) fail_if(readback(nullptr, 0, nullptr));
-    for (int k = 0; k < nseg; ++k) hb[2 * kRowHistBins + k + 1] = hb[2 * kRowHistBins + k] + jobs_[L1.jobs[k]].known_ne;
+    for (int k = 0; k < nseg; ++k) hb[kRowHistBins + k + 1] = hb[kRowHistBins + k] + jobs_[L1.jobs[k]].known_ne;
   }
-  const int64_t* bounds = hb.data() + 2 * kRowHistBins;
-  // row-length statistics of every level, predicted from the first level:
-  // original vertices keep their valence, face points take the face order,
-  // edge points have 4 (2 on the boundary), later face points 4.
-  int64_t vlong = 0, flong = 0;
-  int vmax = 0, fmax = 0;
-  if (have_hist) {
-    const int64_t* hv = hb.data();
-    const int64_t* hf = hv + kRowHistBins;
-    for (int b = 0; b < kRowHistBins; ++b) {
-      if (b > 4) {
-        vlong += hv[b];
-        flong += hf[b];
-      }
-      if (hv[b]) vmax = b;
-      if (hf[b]) fmax = b;
-    }
-  }
-
+  const int64_t* bounds = hb.data() + kRowHistBins;
   // 3. closed-form sizes of every later level
   int Lmax = 0;
   for (int k = 0; k < nseg; ++k) {
@@ -851,22 +814,11 @@ void Plan::prepare() {
       partial_len_ = need2;
     }
   }
-  for (int l = 1; l <= Lmax; ++l) {
-    LevelPlan& L = levels_[l - 1];
-    if (!have_hist) {
-      L.cap = 8;
-      continue;
-    }
-    L.long_rows = l == 1 ? vlong : vlong + flong;
-    L.max_row = l == 1 ? vmax : std::max(std::max(vmax, fmax), 4);
-    L.cap = autotune_cap(L.quad, L.nv, L.long_rows, L.max_row);  // used by the first level's row kernels
-  }
   // the first level's rows per block, now with the row-length spread (the
   // numbering after the read-back and every graph replay use it)
   {
     const RowTiling rt = autotune_rows(levels_[0].nv, levels_[0].nnz, have_hist ? hb.data() : nullptr);
     levels_[0].rows = rt.rows;
-    levels_[0].rows_num = rt.rows_num;
     levels_[0].tile = rt.tile;
   }
   // k_final tables: per fused mesh, its segment of M (the level before's
@@ -917,28 +869,13 @@ void Plan::prepare() {
 void Plan::launch_number(LevelPlan& L, bool faces) {
   const double poly_b = L.quad ? 0.0 : 4.0 * (L.nf + 1) + 4.0 * L.nnz;
   const double ne = (double)L.ne;
-  LevelView V{};
-  V.ids = L.ids;
-  V.fptr = L.fptr;
-  V.cface = L.cface;
-  V.P = L.P;
-  V.nv = (int32_t)L.nv;
-  V.nf = (int32_t)L.nf;
-  V.nnz = L.nnz;
-  V.tptr = L.tptr;
-  V.tids = L.tids;
-  V.trow = L.trow;  // sorted rows with in-neighbours (symbolic pass)
-  V.eptr = L.eptr;
+  LevelView V = L.view(d_flags_);
   V.ci = reinterpret_cast<int32_t*>(L.ci);
   V.bnd = L.bnd;
-  V.flags = d_flags_;
-  V.seg = L.table();
-  V.rows_per_block = L.rows_num;
-  V.tile_entries = L.tile;
   ProfScope ps(st_, faces ? (L.quad ? "number_facepoints_quad" : "number_facepoints_poly") : "number",
                12.0 * L.nv + 12.0 * L.nnz + 8.0 * L.nnz + (L.bnd ? 4.0 * ne : 0.0) + poly_b +
                    (faces ? 4.0 * L.nnz + 16.0 * L.nv + 16.0 * L.nf : 0.0));
-  launch_number_faces(L.quad, scheme_, L.cap, V, faces, st_);
+  launch_number_faces(L.quad, scheme_, V, faces, st_);
 }
 
 // Vertex classes of the mesh two levels before job J's level l (the mesh M
@@ -1108,7 +1045,7 @@ void Plan::record_level(int l) {
   if (l == 1 && number_early_ && !early_faces_) {
     ProfScope ps(st_, L.quad ? "facepoints_quad" : "facepoints_poly",
                  4.0 * L.nnz + 16.0 * L.nv + 16.0 * L.nf + (L.quad ? 0.0 : 4.0 * (L.nf + 1)));
-    launch_faces(L.quad, true, false, L.ids, L.fptr, L.P, (int32_t)L.nf, L.table(), nullptr, nullptr, st_);
+    launch_faces(L.quad, L.ids, L.fptr, L.P, (int32_t)L.nf, L.table(), st_);
   }
   if (L.blk) {
     ProfScope ps(st_, "scan", 8.0 * ne + 4);
@@ -1118,7 +1055,7 @@ void Plan::record_level(int l) {
   if (l > 1) {
     ProfScope ps(st_, L.quad ? "facepoints_quad" : "facepoints_poly",
                  4.0 * L.nnz + 16.0 * L.nv + 16.0 * L.nf + (L.quad ? 0.0 : 4.0 * (L.nf + 1)));
-    launch_faces(L.quad, true, false, L.ids, L.fptr, L.P, (int32_t)L.nf, L.table(), nullptr, nullptr, st_);
+    launch_faces(L.quad, L.ids, L.fptr, L.P, (int32_t)L.nf, L.table(), st_);
   }
   RefineView R{};
   R.ids = L.ids;
@@ -1185,13 +1122,8 @@ void Plan::launch(bool include_analysis) {
   if (include_analysis) number_early_ = false;  // the analysis runs again: number in order
   LevelPlan& L1 = levels_[0];
   if (include_analysis) {
-    launch_fill_i32(d_state_, n_state_, 0, st_);  // a fill kernel: graph-safe
-    {
-      ProfScope ps(st_, "gather", 4.0 * (L1.nf + 1) + 12.0 * L1.nnz + (L1.quad ? 0.0 : 8.0 * L1.nnz + 4.0 * L1.nf));
-      launch_gather(L1.table(), (int32_t)L1.nf, scheme_ == kLAK, const_cast<int32_t*>(L1.ids),
-                    const_cast<int32_t*>(L1.fptr), const_cast<int32_t*>(L1.cface), d_flags_, d_cnt_,
-                    (int32_t)L1.nv, d_state_ + kStateFaceHist, st_);
-    }
+    launch_setup(nullptr, nullptr, 0, d_state_, n_state_, st_);  // a fill kernel: graph-safe
+    record_gather(L1);
     if (P1_) {
       ProfScope ps(st_, "gather_verts", 32.0 * L1.nv);
       launch_gather_verts(L1.table(), (int32_t)L1.nv, P1_, st_);

@@ -55,10 +55,9 @@ struct FinalTable {
   bool empty() const { return segs.empty(); }
 };
 
-// rows per block and LDS row tile (entries) of the first level's row kernels
+// rows per block and LDS row tile (entries) of the first level's numbering
 struct RowTiling {
-  int rows;      // k_symbolic
-  int rows_num;  // the numbering of k_number_faces
+  int rows;
   int tile;
 };
 
@@ -71,14 +70,13 @@ struct LevelPlan {
   const float4* P = nullptr;
   int64_t ne = 0;           // union edges
   bool boundary = false;    // some mesh of the level has boundary edges
-  int cap = 8;              // first level: M^T row length held in registers (autotuned)
-  int rows = 256;           // first level: M^T rows per block of k_symbolic (autotuned)
-  int rows_num = 128;       // first level: M^T rows per block of the numbering (autotuned)
-  int tile = 1536;          // first level: LDS row tile of the row kernels, entries (autotuned)
-  int64_t long_rows = -1;   // rows longer than 4 (from the first level's histogram)
-  int max_row = -1;
-  // first-level analysis scratch
-  int32_t *cnt = nullptr, *tids = nullptr, *ecnt = nullptr, *eptr = nullptr;
+  int cap = kRowSlots;      // first level: M^T row length held in registers
+  int rows = 256;           // first level: M^T rows per block of the numbering (autotuned)
+  int tile = 1536;          // first level: its LDS row tile, entries (autotuned)
+  // first-level analysis scratch (see LevelView)
+  int32_t *cnt = nullptr, *slots = nullptr, *head = nullptr, *tids = nullptr, *eptr = nullptr;
+  int32_t *pool = nullptr, *ecnt = nullptr;
+  uint64_t *tile_sum = nullptr, *group_sum = nullptr;
   // the level's structure: M^T rows with in-neighbours, (edge id, twin) per
   // corner, boundary flags per edge and their scan (boundary levels)
   int32_t* tptr = nullptr;
@@ -113,6 +111,7 @@ struct LevelPlan {
   int64_t* d_fbase = nullptr;
   int64_t* d_cbase = nullptr;
   int* d_mflags = nullptr;
+  LevelView view(int* flags) const;  // the first level's inputs and analysis arrays
   SegTable table() const { return SegTable{d_segs, d_vbase, d_fbase, (int32_t)segs.size(), d_mflags, d_cbase}; }
 };
 
@@ -156,14 +155,15 @@ class Plan {
   void plan_first_level();
   void record_analysis(LevelPlan& L);
   void record_level(int l);
-  // state_ints > 0: also carries the plan's zeroed state block (first upload)
+  // zero_state: also zeroes the plan's state block (first upload)
   // pinned host staging of a table upload (recycled through a process-wide
   // pool; released once the plan's stream has passed the copy)
   struct Staging {
     char* p = nullptr;
     size_t cap = 0;
   };
-  void upload_tables(int l0, int l1, Staging& staging, int64_t state_ints = 0);
+  void upload_tables(int l0, int l1, Staging& staging, bool zero_state = false);
+  void record_gather(LevelPlan& L);
   // overlap: work enqueued after the copy and before the wait (the host then
   // waits for the copy only)
   int readback(const int32_t* src, int count, int64_t* dst, const std::function<void()>& overlap = {});
@@ -178,11 +178,11 @@ class Plan {
   int* d_flags_ = nullptr;
   int64_t* d_partial_ = nullptr;
   int64_t partial_len_ = 0;
-  // per-plan device state, zeroed by the first table upload:
-  // [flags | row hist (17) | face hist (17) | edge bounds (nseg + 1) | mesh flags (nseg)]
+  // per-plan device state, zeroed before each run of the analysis:
+  // [flags | row hist | edge bounds (nseg + 1) | mesh flags (nseg)],
+  // then [pool | group sums | valence counters] (n_state_ ints in all)
   int32_t* d_state_ = nullptr;
-  int64_t n_state_ = 0;
-  int32_t* d_cnt_ = nullptr;  // first level: valence counters (zeroed by the gather)
+  int64_t n_state_ = 0, at_groups_ = 0, n_groups_ = 0;
   Staging staging_first_, staging_all_;  // segment table uploads
   // first-level union gather (multi-mesh)
   float4* P1_ = nullptr;

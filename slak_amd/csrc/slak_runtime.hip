@@ -166,9 +166,9 @@ hipEvent_t Profiler::event() {
   return e;
 }
 
-void Profiler::begin(hipStream_t st, const char* name, double bytes) {
+void Profiler::begin(hipStream_t st, std::vector<StageBytes> stages) {
   std::lock_guard<std::mutex> g(mu_);
-  Rec r{name, bytes, event(), event()};
+  Rec r{std::move(stages), event(), event()};
   SLAK_HIP_CHECK(hipEventRecord(r.a, st));
   recs_.push_back(r);
 }
@@ -181,10 +181,11 @@ void Profiler::end(hipStream_t st) {
 void Profiler::amend_last(const char* name, double bytes) {
   std::lock_guard<std::mutex> g(mu_);
   for (auto it = recs_.rbegin(); it != recs_.rend(); ++it)
-    if (std::strcmp(it->name, name) == 0) {
-      it->bytes += bytes;
-      return;
-    }
+    for (StageBytes& s : it->stages)
+      if (std::strcmp(s.name, name) == 0) {
+        s.bytes += bytes;
+        return;
+      }
 }
 
 void Profiler::reset() {
@@ -208,14 +209,18 @@ std::string Profiler::report() {
     SLAK_HIP_CHECK(hipEventSynchronize(r.b));
     float ms = 0;
     SLAK_HIP_CHECK(hipEventElapsedTime(&ms, r.a, r.b));
-    auto it = std::find_if(agg.begin(), agg.end(), [&](auto& kv) { return kv.first == r.name; });
-    if (it == agg.end()) {
-      agg.push_back({r.name, Agg{}});
-      it = agg.end() - 1;
+    double all = 0;
+    for (const StageBytes& x : r.stages) all += x.bytes;
+    for (const StageBytes& x : r.stages) {
+      auto it = std::find_if(agg.begin(), agg.end(), [&](auto& kv) { return kv.first == x.name; });
+      if (it == agg.end()) {
+        agg.push_back({x.name, Agg{}});
+        it = agg.end() - 1;
+      }
+      it->second.n += 1;
+      it->second.ms += all > 0 ? ms * x.bytes / all : ms / r.stages.size();
+      it->second.bytes += x.bytes;
     }
-    it->second.n += 1;
-    it->second.ms += ms;
-    it->second.bytes += r.bytes;
   }
   std::string js = "{\"stages\": [";
   for (size_t i = 0; i < agg.size(); ++i) {
@@ -306,19 +311,7 @@ void spgemm_operator(const slak_mesh& cmesh, int32_t** F_ptr, int32_t** F_ids, i
     SLAK_HIP_CHECK(hipMemcpyAsync(fptr, L.tptr, (nv + 1) * 4, hipMemcpyDeviceToDevice, st));
     SLAK_HIP_CHECK(hipMemcpyAsync(dptr, L.tptr, (nv + 1) * 4, hipMemcpyDeviceToDevice, st));
     SLAK_HIP_CHECK(hipMemcpyAsync(eptr, L.eptr, (nv + 1) * 4, hipMemcpyDeviceToDevice, st));
-    LevelView V{};
-    V.ids = L.ids;
-    V.fptr = L.fptr;
-    V.cface = L.cface;
-    V.P = L.P;
-    V.nv = (int32_t)nv;
-    V.nf = (int32_t)L.nf;
-    V.nnz = nnz;
-    V.tptr = L.tptr;
-    V.tids = L.tids;
-    V.eptr = L.eptr;
-    V.flags = plan.flags();
-    V.seg = L.table();
+    LevelView V = L.view(plan.flags());
     V.ne_cap = ne;
     V.F_ids = take(nnz);
     V.F_vals = take(nnz);
