@@ -43,6 +43,8 @@ enum : int {
 // the invalid mesh)
 constexpr int kFlagsInput = kFlagBadPtr | kFlagBadOrder | kFlagBadId | kFlagBadVals | kFlagBadQuad;
 
+constexpr int kBlockItems = 256;  // threads (items) per block of the level kernels
+
 // One mesh of a level's union.
 struct SegDesc {
   int64_t vb, fb, cb;      // union bases: vertices, faces, corners
@@ -68,13 +70,17 @@ struct SegDesc {
   int32_t dst_final;       // 1: the destination is the caller's output (stored non-temporally)
 };
 
+// The meshes of a level. A single mesh (n == 1) is described by `one`, in the
+// kernel's arguments; several by device tables: the descriptors, the union
+// bases (n + 1 each) and, per block of kBlockItems vertices, faces and
+// corners, the mesh its first item belongs to.
 struct SegTable {
   const SegDesc* d;
-  const int64_t* vbase;  // n + 1 vertex bases
-  const int64_t* fbase;  // n + 1 face bases
+  const int64_t *vbase, *fbase, *cbase;
+  const int32_t *vblk, *fblk, *cblk;
   int32_t n;
-  int* mflags;           // per-segment validation flags
-  const int64_t* cbase;  // n + 1 corner bases
+  int* mflags;  // per-mesh validation flags
+  SegDesc one;
 };
 
 // A pointer read from device memory (a mesh table entry) is generic to the
@@ -104,25 +110,33 @@ __device__ __forceinline__ int seg_of(const int64_t* base, int n, int64_t x) {
   return lo;
 }
 
-// seg_of for items that rise with the lane (item = first + lane within a
-// wave): one wave-uniform binary search for the first active lane's item
-// (scalar loads), then a few steps forward per lane. Falls back to the
-// per-lane search when an item lies before the first lane's or more than 8
-// segments after it.
-__device__ __forceinline__ int seg_of_wave(const int64_t* base, int n, int64_t x) {
-  if (n <= 1) return 0;
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)x);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)((uint64_t)x >> 32));
-  const int64_t x0 = (int64_t)(((uint64_t)hi << 32) | lo);
-  if (x < x0) return seg_of(base, n, x);
-  int k = seg_of(base, n, x0);
-#pragma unroll 1
-  for (int it = 0; it < 8 && k + 1 < n && base[k + 1] <= x; ++it) ++k;
-  if (k + 1 < n && base[k + 1] <= x) k = seg_of(base, n, x);
+// Segment of an item, for items that rise with the lane: from the mesh of the
+// first item of the wave's block (blk, one scalar load) a few wave-uniform
+// steps to the first lane's mesh, then a few per lane. (A search over the
+// bases of 4096 meshes instead takes 12 dependent loads per wave; see
+// k_level.)
+__device__ __forceinline__ int seg_of_wave(const int64_t* base, const int32_t* blk, int n, int32_t x) {
+  const int32_t x0 = __builtin_amdgcn_readfirstlane(x);
+  int k = __builtin_amdgcn_readfirstlane(blk[x0 / kBlockItems]);
+  while (k + 1 < n && base[k + 1] <= x0) ++k;
+  while (k + 1 < n && base[k + 1] <= x) ++k;
   return k;
 }
 
-constexpr int kBlockItems = 256;  // threads (items) per block of the level kernels
+// Descriptor of the mesh of a vertex, face or corner of the union. ONE: the
+// level holds one mesh.
+template <bool ONE>
+__device__ __forceinline__ const SegDesc* vertex_seg(const SegTable& seg, int32_t v) {
+  return ONE ? &seg.one : seg.d + seg_of_wave(seg.vbase, seg.vblk, seg.n, v);
+}
+template <bool ONE>
+__device__ __forceinline__ const SegDesc* face_seg(const SegTable& seg, int32_t f) {
+  return ONE ? &seg.one : seg.d + seg_of_wave(seg.fbase, seg.fblk, seg.n, f);
+}
+template <bool ONE>
+__device__ __forceinline__ const SegDesc* corner_seg(const SegTable& seg, int32_t t) {
+  return ONE ? &seg.one : seg.d + seg_of_wave(seg.cbase, seg.cblk, seg.n, t);
+}
 
 // M^T row slots per vertex while the first level's rows are built
 constexpr int kRowSlots = 8;
@@ -161,6 +175,11 @@ struct LevelView {
   int32_t* E_ids;   // LAK edge matrix rows (SpGEMM operator)
   int32_t* E_vals;  // LAK edge matrix values (+-(id+1))
   int* flags;
+  int* late;        // host word for what goes wrong after the flags were read
+  // host words the analysis reports to (or null): [done | flags | row-length
+  // histogram | bounds (n + 1)], done set last
+  int32_t* report;
+  int32_t ngroups;
   SegTable seg;
   // mapped SpGEMM operator outputs (F, D rows share M^T's row offsets)
   int32_t* F_ids;
@@ -446,23 +465,22 @@ __device__ __forceinline__ void row_symbolic(const Row& r, int32_t v, int32_t& c
 // as (edge id, twin) at both of its half-edges' corners, and the boundary
 // flag of every owned edge by union edge index. edges_before: the union's
 // edges owned by the vertices before v.
-template <int SCHEME, class Row>
+template <int SCHEME, bool ONE, class Row>
 __device__ __forceinline__ void row_number(Row& r, const LevelView& L, int32_t v, int32_t edges_before) {
   constexpr int C = Row::kCap;
-  const int k = seg_of_wave(L.seg.vbase, L.seg.n, v);
-  const SegDesc* __restrict__ S = L.seg.d + k;
+  const SegDesc* __restrict__ S = vertex_seg<ONE>(L.seg, v);
   const int64_t ne_cap = S->ne;
   const int64_t eb = S->eb;
   int32_t* __restrict__ ci = L.ci;
   int32_t* __restrict__ bnd = L.bnd;
-  int* flags = L.flags;
+  int* late = L.late;
   const int32_t e0 = edges_before - (int32_t)eb;  // mesh-local edge base of v
   const int n = r.n;
   // Edge ids beyond the segment's edges are clamped (and flagged) so that
   // every later index stays inside the mesh's ranges.
-  auto cap = [flags, ne_cap](int32_t e) __attribute__((always_inline)) {
+  auto cap = [late, ne_cap](int32_t e) __attribute__((always_inline)) {
     if (e >= ne_cap) {
-      atomicOr(flags, kFlagOverflow);
+      *late = kFlagOverflow;
       return (int32_t)(ne_cap > 0 ? ne_cap - 1 : 0);
     }
     return e;

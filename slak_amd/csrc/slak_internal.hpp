@@ -60,11 +60,9 @@ constexpr int kRowTileMax = 2560;
 constexpr int kHistCopies = 32;
 constexpr int kHistStride = 32;  // ints per copy
 constexpr int kHistInts = kHistCopies * kHistStride;
-// The plan's state block (int32, zeroed before the gather), read back from
-// its start after the first level's analysis:
+// The plan's state block (int32, zeroed before the gather):
 // [flags | pad | row hist copies | edge bounds (nseg + 1) | mesh flags (nseg)]
-// followed by [pool | group sums | valence counters] (a single mesh's host adds up
-// its edges from the group sums)
+// followed by [pool | group sums | valence counters]
 constexpr int kStateRowHist = 32;
 constexpr int kStateBounds = kStateRowHist + kHistInts;
 void launch_copy_probe(const float4* a, float4* b, int64_t n, hipStream_t st);
@@ -78,7 +76,9 @@ void launch_symbolic(bool quad, int scheme, const LevelView& L, hipStream_t st);
 // L.bounds of several meshes, from the symbolic pass's sums
 void launch_seg_bounds(const LevelView& L, hipStream_t st);
 // first level: row offsets, sorted rows, edge numbering and (faces set) face
-// points in one launch, after the symbolic pass
+// points in one launch, after the symbolic pass; a single mesh's launch also
+// fills L.report (if set), which several meshes take from launch_report
+void launch_report(const LevelView& L, hipStream_t st);
 void launch_number_faces(bool quad, int scheme, const LevelView& L, bool faces, hipStream_t st);
 void launch_spgemm_fde(bool quad, const LevelView& L, hipStream_t st);
 // refine (per corner) and vertex (per vertex) items of a level in one launch;

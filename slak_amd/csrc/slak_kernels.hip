@@ -210,7 +210,7 @@ __device__ __forceinline__ void put_row(const RowBuild& rb, int32_t v, int32_t s
     rb.next[c] = atomicExch(&rb.head[v], c);
 }
 
-template <bool QUAD>
+template <bool QUAD, bool ONE>
 __device__ __forceinline__ void gather_face(const SegTable& seg, int32_t f, int32_t nf_total, int use_vals,
                                             int32_t* __restrict__ ids_pos, int32_t* __restrict__ fptr,
                                             int32_t* __restrict__ cface, int* __restrict__ flags,
@@ -243,7 +243,7 @@ constexpr int kCountWindow = 2048;
 // faces: the corners of a face are in registers when they are placed, and a
 // row needs no offset while its corners go to fixed slots, so no scan stands
 // between the count and the placement.
-template <bool QUAD>
+template <bool QUAD, bool ONE>
 __global__ void __launch_bounds__(kBlock) k_gather(SegTable seg, int32_t nf_total, int use_vals, int32_t* __restrict__ ids_pos,
                          int32_t* __restrict__ fptr, int32_t* __restrict__ cface, int* __restrict__ flags,
                          RowBuild rb, int window) {
@@ -254,7 +254,7 @@ __global__ void __launch_bounds__(kBlock) k_gather(SegTable seg, int32_t nf_tota
   FaceCorners<REGS> fc;
 #pragma unroll
   for (int i = 0; i < REGS; ++i) fc.v[i] = -1;
-  if (f < nf_total) gather_face<QUAD>(seg, f, nf_total, use_vals, ids_pos, fptr, cface, flags, rb, fc);
+  if (f < nf_total) gather_face<QUAD, ONE>(seg, f, nf_total, use_vals, ids_pos, fptr, cface, flags, rb, fc);
   int lo = INT_MAX, hi = INT_MIN;
 #pragma unroll
   for (int i = 0; i < REGS; ++i)
@@ -291,13 +291,13 @@ __global__ void __launch_bounds__(kBlock) k_gather(SegTable seg, int32_t nf_tota
 // position order. out: the face's
 // valid corners for the row building; the corners of a longer face beyond
 // the registers are placed here, one device atomic each.
-template <bool QUAD>
+template <bool QUAD, bool ONE>
 __device__ __forceinline__ void gather_face(const SegTable& seg, int32_t f, int32_t nf_total, int use_vals,
                                             int32_t* __restrict__ ids_pos, int32_t* __restrict__ fptr,
                                             int32_t* __restrict__ cface, int* __restrict__ flags,
                                             const RowBuild& rb, FaceCorners<QUAD ? 4 : kGatherRegs>& out) {
-  const int k = seg_of_wave(seg.fbase, seg.n, f);
-  const SegDesc* S = seg.d + k;
+  const SegDesc* S = face_seg<ONE>(seg, f);
+  int* const mflags = seg.mflags + (ONE ? 0 : S - seg.d);
   const int32_t lf = (int32_t)(f - S->fb);
   const int32_t* sp = to_global(S->src_ptr);
   const int32_t* sid = to_global(S->src_ids);
@@ -310,7 +310,7 @@ __device__ __forceinline__ void gather_face(const SegTable& seg, int32_t f, int3
   if (lf == S->nf - 1 && e != snnz) bad |= kFlagBadPtr;
   if (s < 0 || e < s || e > snnz) {
     bad |= kFlagBadPtr;
-    atomicOr(seg.mflags + k, bad);
+    atomicOr(mflags, bad);
     atomicOr(flags, bad);
     return;
   }
@@ -360,7 +360,7 @@ __device__ __forceinline__ void gather_face(const SegTable& seg, int32_t f, int3
         if (f == nf_total - 1) fptr[nf_total] = (int32_t)(cb + e);
       }
       if (bad) {
-        atomicOr(seg.mflags + k, bad);
+        atomicOr(mflags, bad);
         atomicOr(flags, bad);
       }
       const int32_t c0 = (int32_t)(cb + s);
@@ -425,7 +425,7 @@ __device__ __forceinline__ void gather_face(const SegTable& seg, int32_t f, int3
     if (f == nf_total - 1) fptr[nf_total] = (int32_t)(cb + e);
   }
   if (bad) {
-    atomicOr(seg.mflags + k, bad);
+    atomicOr(mflags, bad);
     atomicOr(flags, bad);
   }
 }
@@ -433,19 +433,18 @@ __device__ __forceinline__ void gather_face(const SegTable& seg, int32_t f, int3
 __global__ void k_gather_verts(SegTable seg, int32_t nv_total, float4* __restrict__ P) {
   int32_t v = (int32_t)(block_index() * blockDim.x + threadIdx.x);
   if (v >= nv_total) return;
-  const int k = seg_of_wave(seg.vbase, seg.n, v);
-  const SegDesc* S = seg.d + k;
+  const SegDesc* S = vertex_seg<false>(seg, v);
   P[v] = to_global(S->src_verts)[v - S->vb];
 }
 
 // ---------------------------------------------------------------------------
 // face points into each segment's destination
 
-template <bool QUAD>
+template <bool QUAD, bool ONE>
 __device__ __forceinline__ void faces_item(const int32_t* __restrict__ ids, const int32_t* __restrict__ fptr,
                                            const float4* __restrict__ P, int32_t nf, const SegTable& seg, int32_t f) {
   if (f >= nf) return;
-  const SegDesc* S = seg.d + seg_of_wave(seg.fbase, seg.n, f);
+  const SegDesc* S = face_seg<ONE>(seg, f);
   float4* const dst = to_global(S->dst_verts) + S->nv + (f - S->fb);
   if (QUAD) {
     int4 c = reinterpret_cast<const int4*>(ids)[f];
@@ -458,10 +457,10 @@ __device__ __forceinline__ void faces_item(const int32_t* __restrict__ ids, cons
   }
 }
 
-template <bool QUAD>
+template <bool QUAD, bool ONE>
 __global__ void k_faces(const int32_t* __restrict__ ids, const int32_t* __restrict__ fptr, const float4* __restrict__ P,
                         int32_t nf, SegTable seg) {
-  faces_item<QUAD>(ids, fptr, P, nf, seg, (int32_t)(block_index() * blockDim.x + threadIdx.x));
+  faces_item<QUAD, ONE>(ids, fptr, P, nf, seg, (int32_t)(block_index() * blockDim.x + threadIdx.x));
 }
 
 // 64-bit lane exchange by DPP (row_shr / row_bcast); lanes without a source,
@@ -616,7 +615,7 @@ __global__ void __launch_bounds__(kBlock) k_symbolic(LevelView L) {
     L.ecnt[v] = owned;
     if (bad) {
       atomicOr(L.flags, bad);
-      if (L.seg.mflags) atomicOr(L.seg.mflags + seg_of(L.seg.vbase, L.seg.n, v), bad);
+      atomicOr(L.seg.mflags + seg_of(L.seg.vbase, L.seg.n, v), bad);
     }
   }
   const uint64_t sum = block_sum(pack_row(n, owned), wave_sum);
@@ -642,6 +641,40 @@ __global__ void __launch_bounds__(kBlock) k_seg_bounds(LevelView L) {
   if (lane == 0) L.bounds[k] = (int32_t)acc;
 }
 
+// What the host waits for, written straight to its memory by one block (a
+// copy and an event after the analysis cost 5 us more a call): the flags, the
+// row-length histogram, the owned edges before each mesh; then the done word.
+__device__ void report(const LevelView& L, uint64_t* lds) {
+  int32_t* const out = L.report;
+  const int tid = threadIdx.x;
+  if (tid == 0) out[1] = *L.flags;
+  if (tid < kRowHistBins) {
+    int32_t x = 0;
+    for (int c = 0; c < kHistCopies; ++c) x += L.hist_rows[c * kHistStride + tid];
+    out[2 + tid] = x;
+  }
+  int32_t* const bounds = out + 2 + kRowHistBins;
+  if (L.seg.n > 1) {
+    for (int k = tid; k <= L.seg.n; k += kBlock) bounds[k] = L.bounds[k];
+  } else {
+    uint64_t acc = 0;
+    for (int i = tid; i < L.ngroups; i += kBlock) acc += L.group_sum[i];
+    const uint64_t sum = block_sum(acc, lds);
+    if (tid == 0) {
+      bounds[0] = 0;
+      bounds[1] = (int32_t)(sum & kOwnedMask);
+    }
+  }
+  __threadfence_system();
+  __syncthreads();
+  if (tid == 0) __hip_atomic_store(out, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+__global__ void __launch_bounds__(kBlock) k_report(LevelView L) {
+  __shared__ uint64_t lds[kBlock / 64];
+  report(L, lds);
+}
+
 // First level, blocks [0, nbn): the rows of R = L.rows_per_block vertices (a
 // part of a sizing tile), one lane per row. The block forms its rows' offsets
 // from the tile sums, writes them and the sorted rows with their
@@ -650,16 +683,21 @@ __global__ void __launch_bounds__(kBlock) k_seg_bounds(LevelView L) {
 // form the face points, which are independent.
 extern __shared__ __align__(16) unsigned char row_tile_lds[];
 
-template <bool QUAD, int SCHEME>
+template <bool QUAD, int SCHEME, bool ONE>
 __global__ void __launch_bounds__(kBlock) k_number_faces(LevelView L, int32_t nbn) {
   __shared__ uint64_t wave_sum[2][kBlock / 64];
   __shared__ uint64_t row_at[kBlock + 1];
   // an invalid mesh: its ids, rows and counts were not (all) written; a
   // single mesh's numbering is launched before the host has read the flags
+  const bool reports = ONE && L.report;
+  if (reports && blockIdx.x == 0) {
+    report(L, wave_sum[0]);
+    return;
+  }
   if (*L.flags & kFlagsInput) return;
-  const int64_t b = block_index();
+  const int64_t b = block_index() - (reports ? 1 : 0);
   if (b >= nbn) {
-    faces_item<QUAD>(L.ids, L.fptr, L.P, L.nf, L.seg, (int32_t)((b - nbn) * blockDim.x + threadIdx.x));
+    faces_item<QUAD, ONE>(L.ids, L.fptr, L.P, L.nf, L.seg, (int32_t)((b - nbn) * blockDim.x + threadIdx.x));
     return;
   }
   int2* const tile_out = reinterpret_cast<int2*>(row_tile_lds);  // (corner, in-neighbour)
@@ -706,7 +744,7 @@ __global__ void __launch_bounds__(kBlock) k_number_faces(LevelView L, int32_t nb
 #pragma unroll
         for (int i = 0; i < C; ++i)
           if (i < n) put(i, r.T(i), r.U(i));
-        row_number<SCHEME>(r, L, v, e0);
+        row_number<SCHEME, ONE>(r, L, v, e0);
       });
     } else {
       // the sizing pass sorted every row longer than its own capacity; this
@@ -715,7 +753,7 @@ __global__ void __launch_bounds__(kBlock) k_number_faces(LevelView L, int32_t nb
       sort_row_in_place(row, n);
       MemRow<QUAD> r(L, row, n);
       for (int i = 0; i < n; ++i) put(i, r.T(i), r.U(i));
-      row_number<SCHEME>(r, L, v, e0);
+      row_number<SCHEME, ONE>(r, L, v, e0);
     }
   }
   __syncthreads();
@@ -805,9 +843,10 @@ struct SegK {
   bool next, dst_final;
 };
 
-__device__ __forceinline__ SegK seg_consts(const SegTable& seg, int32_t f) {
+template <bool ONE>
+__device__ __forceinline__ SegK seg_consts(const SegTable& seg, int32_t t) {
   SegK K;
-  const SegDesc* __restrict__ S = seg.d + seg_of_wave(seg.fbase, seg.n, f);
+  const SegDesc* __restrict__ S = corner_seg<ONE>(seg, t);
   K.vb = (int32_t)S->vb;
   K.fb = (int32_t)S->fb;
   K.cb = (int32_t)S->cb;
@@ -1031,13 +1070,13 @@ __device__ __forceinline__ void corner_store(const RefineView& R, const SegK& K,
 // per corner, so that each store instruction of a wave covers contiguous
 // memory; every load is issued before the first store.
 
-template <bool QUAD, int SCHEME>
+template <bool QUAD, int SCHEME, bool ONE>
 __device__ __forceinline__ void refine_item(const RefineView& R, int64_t t64) {
   if (t64 >= R.nnz) return;
   CornerIn c;
   c.t = (int32_t)t64;
   corner_nbrs<QUAD>(R.fptr, R.cface, c.t, c.f, c.tn, c.tp);
-  const SegK K = seg_consts(R.seg, c.f);
+  const SegK K = seg_consts<ONE>(R.seg, c.t);
   if (R.ntptr && t64 == R.nnz - 1) R.ntptr[R.next_nv] = R.next_nnz;  // end of the next level's M^T
   c.v = R.ids[c.t];
   const int2 c1 = R.ci[c.t];
@@ -1076,12 +1115,12 @@ __device__ __forceinline__ void refine_item(const RefineView& R, int64_t t64) {
 // are loaded before any store; longer rows loop.
 constexpr int kVertexRegs = 4;
 
-template <bool QUAD, int SCHEME, bool NEXT, bool BND>
+template <bool QUAD, int SCHEME, bool NEXT, bool BND, bool ONE>
 __device__ __forceinline__ void vertex_item(const RefineView& R, int32_t v) {
   if (v >= R.nv) return;
   // the segment's constants, all read before the first store (a table read
   // issued after a store would wait for that store)
-  const SegDesc* __restrict__ S = R.seg.d + seg_of_wave(R.seg.vbase, R.seg.n, v);
+  const SegDesc* __restrict__ S = vertex_seg<ONE>(R.seg, v);
   const int32_t vb = (int32_t)S->vb, fb = (int32_t)S->fb, cb = (int32_t)S->cb;
   const int32_t snv = S->nv, snf = S->nf;
   const int32_t semax = S->ne > 0 ? (int32_t)S->ne - 1 : 0;
@@ -1190,7 +1229,7 @@ __device__ __forceinline__ void vertex_item(const RefineView& R, int32_t v) {
 // machine. Block b is a vertex block when floor((b+1) nbv / T) > floor(b nbv / T)
 // (T = nbr + nbv): vertex block floor(b nbv / T), else refine block
 // b - floor(b nbv / T); a bijection onto both block ranges.
-template <bool QUAD, int SCHEME, bool NEXT, bool BND>
+template <bool QUAD, int SCHEME, bool NEXT, bool BND, bool ONE>
 __global__ void __launch_bounds__(kBlock) k_level(RefineView R, int32_t nbr, int32_t nbv) {
   const int64_t b = NEXT ? block_index<kRemapLevel>() : block_index<kRemapPositions>();
   const int64_t T = (int64_t)nbr + nbv;
@@ -1210,9 +1249,9 @@ __global__ void __launch_bounds__(kBlock) k_level(RefineView R, int32_t nbr, int
       rest -= nb;
     }
     const int64_t v = (int64_t)R.vseg[s] + u * blockDim.x + threadIdx.x;
-    vertex_item<QUAD, SCHEME, NEXT, BND>(R, v < R.vseg[s + 1] ? (int32_t)v : R.nv);
+    vertex_item<QUAD, SCHEME, NEXT, BND, ONE>(R, v < R.vseg[s + 1] ? (int32_t)v : R.nv);
   } else {
-    refine_item<QUAD, SCHEME>(R, (b - before) * blockDim.x + threadIdx.x);
+    refine_item<QUAD, SCHEME, ONE>(R, (b - before) * blockDim.x + threadIdx.x);
   }
 }
 
@@ -1826,7 +1865,7 @@ __global__ void __launch_bounds__(kScanSmallThreads) k_scan_small(const int32_t*
   }
   if (tid == 0) {
     const int64_t carry = total;
-    if (carry > 0x7fffffffll) atomicOr(flags, kFlagOverflow);
+    if (carry > 0x7fffffffll) *flags = kFlagOverflow;
     out[n] = (int32_t)carry;
   }
 }
@@ -1874,7 +1913,7 @@ __global__ void __launch_bounds__(kBlock) k_scan_partials(int64_t* __restrict__ 
     carry += tot;
   }
   if (threadIdx.x == 0) {
-    if (carry > 0x7fffffffll) atomicOr(flags, kFlagOverflow);
+    if (carry > 0x7fffffffll) *flags = kFlagOverflow;
     out[n] = (int32_t)carry;
   }
 }
@@ -1900,7 +1939,7 @@ __global__ void __launch_bounds__(kBlock) k_scan_down(const int32_t* __restrict_
       for (int64_t i = threadIdx.x; i < ntiles; i += kBlock) all += partial[i];
       block_exclusive_scan(all, red, carry);
       if (threadIdx.x == 0) {
-        if (carry > 0x7fffffffll) atomicOr(flags, kFlagOverflow);
+        if (carry > 0x7fffffffll) *flags = kFlagOverflow;
         out[n] = (int32_t)carry;
       }
     }
@@ -1989,10 +2028,17 @@ void launch_gather(bool quad, const SegTable& seg, bool use_vals, int32_t* ids_p
   const int vals = use_vals ? 1 : 0, window = count_window() ? 1 : 0;
   int32_t* const fptr = const_cast<int32_t*>(L.fptr);
   int32_t* const cface = const_cast<int32_t*>(L.cface);
-  if (quad)
-    k_gather<true><<<grid_for(L.nf), kBlock, 0, st>>>(seg, L.nf, vals, ids_pos, fptr, cface, L.flags, rb, window);
-  else
-    k_gather<false><<<grid_for(L.nf), kBlock, 0, st>>>(seg, L.nf, vals, ids_pos, fptr, cface, L.flags, rb, window);
+  const bool one = seg.n == 1;
+#define SLAK_GATHER(Q, O) \
+  k_gather<Q, O><<<grid_for(L.nf), kBlock, 0, st>>>(seg, L.nf, vals, ids_pos, fptr, cface, L.flags, rb, window)
+  if (quad) {
+    if (one) SLAK_GATHER(true, true);
+    else SLAK_GATHER(true, false);
+  } else {
+    if (one) SLAK_GATHER(false, true);
+    else SLAK_GATHER(false, false);
+  }
+#undef SLAK_GATHER
 }
 
 void launch_setup(const void* src_pinned, void* dst, int64_t bytes, int32_t* zero, int64_t nzero, hipStream_t st) {
@@ -2028,22 +2074,15 @@ void launch_digest(const void* p, int64_t bytes, uint64_t* out, hipStream_t st) 
 void launch_faces(bool quad, const int32_t* ids, const int32_t* fptr, const float4* P, int32_t nf, const SegTable& seg,
                   hipStream_t st) {
   if (nf <= 0) return;
-  if (quad)
-    k_faces<true><<<grid_for(nf), kBlock, 0, st>>>(ids, fptr, P, nf, seg);
-  else
-    k_faces<false><<<grid_for(nf), kBlock, 0, st>>>(ids, fptr, P, nf, seg);
+  const bool one = seg.n == 1;
+  if (quad) {
+    if (one) k_faces<true, true><<<grid_for(nf), kBlock, 0, st>>>(ids, fptr, P, nf, seg);
+    else k_faces<true, false><<<grid_for(nf), kBlock, 0, st>>>(ids, fptr, P, nf, seg);
+  } else {
+    if (one) k_faces<false, true><<<grid_for(nf), kBlock, 0, st>>>(ids, fptr, P, nf, seg);
+    else k_faces<false, false><<<grid_for(nf), kBlock, 0, st>>>(ids, fptr, P, nf, seg);
+  }
 }
-
-#define SLAK_ROW_DISPATCH(KERNEL, quad, scheme, g, smem, st, ...)                      \
-  do {                                                                                \
-    if (quad) {                                                                       \
-      if (scheme == kLAK) KERNEL<true, kLAK><<<g, kBlock, smem, st>>>(__VA_ARGS__);   \
-      else KERNEL<true, kSLAK><<<g, kBlock, smem, st>>>(__VA_ARGS__);                 \
-    } else {                                                                          \
-      if (scheme == kLAK) KERNEL<false, kLAK><<<g, kBlock, smem, st>>>(__VA_ARGS__);  \
-      else KERNEL<false, kSLAK><<<g, kBlock, smem, st>>>(__VA_ARGS__);                \
-    }                                                                                 \
-  } while (0)
 
 // rows per block (64, 128 or 256) and LDS tile (even, 256..kRowTileMax
 // entries) of the numbering
@@ -2057,7 +2096,13 @@ static void check_row_tiling(const LevelView& L) {
 void launch_symbolic(bool quad, int scheme, const LevelView& L, hipStream_t st) {
   if (L.nv <= 0) return;
   const unsigned g = grid_for(L.nv);
-  SLAK_ROW_DISPATCH(k_symbolic, quad, scheme, g, 0, st, L);
+  if (quad) {
+    if (scheme == kLAK) k_symbolic<true, kLAK><<<g, kBlock, 0, st>>>(L);
+    else k_symbolic<true, kSLAK><<<g, kBlock, 0, st>>>(L);
+  } else {
+    if (scheme == kLAK) k_symbolic<false, kLAK><<<g, kBlock, 0, st>>>(L);
+    else k_symbolic<false, kSLAK><<<g, kBlock, 0, st>>>(L);
+  }
 }
 
 void launch_seg_bounds(const LevelView& L, hipStream_t st) {
@@ -2070,10 +2115,25 @@ void launch_number_faces(bool quad, int scheme, const LevelView& L, bool faces, 
   const int32_t nbn = L.nv > 0 ? (int32_t)grid_for(L.nv, L.rows_per_block) : 0;
   const size_t smem = (size_t)L.tile_entries * sizeof(int2);
   const int32_t nbf = faces && L.nf > 0 ? (int32_t)grid_for(L.nf) : 0;
-  if (nbn + nbf == 0) return;
-  const unsigned g = (unsigned)(nbn + nbf);
-  SLAK_ROW_DISPATCH(k_number_faces, quad, scheme, g, smem, st, L, nbn);
+  const bool one = L.seg.n == 1;
+  const unsigned g = (unsigned)(nbn + nbf + (one && L.report ? 1 : 0));  // the first block reports
+  if (g == 0) return;
+#define SLAK_NUMBER(Q, S)                                                    \
+  do {                                                                       \
+    if (one) k_number_faces<Q, S, true><<<g, kBlock, smem, st>>>(L, nbn);    \
+    else k_number_faces<Q, S, false><<<g, kBlock, smem, st>>>(L, nbn);       \
+  } while (0)
+  if (quad) {
+    if (scheme == kLAK) SLAK_NUMBER(true, kLAK);
+    else SLAK_NUMBER(true, kSLAK);
+  } else {
+    if (scheme == kLAK) SLAK_NUMBER(false, kLAK);
+    else SLAK_NUMBER(false, kSLAK);
+  }
+#undef SLAK_NUMBER
 }
+
+void launch_report(const LevelView& L, hipStream_t st) { k_report<<<1, kBlock, 0, st>>>(L); }
 
 void launch_spgemm_fde(bool quad, const LevelView& L, hipStream_t st) {
   if (L.nv <= 0) return;
@@ -2083,16 +2143,22 @@ void launch_spgemm_fde(bool quad, const LevelView& L, hipStream_t st) {
     k_spgemm_fde<false><<<grid_for(L.nv), kBlock, 0, st>>>(L);
 }
 
-template <bool QUAD, int SCHEME>
+template <bool QUAD, int SCHEME, bool ONE>
 void launch_level_t(const RefineView& R, unsigned g, int32_t nbr, int32_t nbv, hipStream_t st) {
   const bool next = R.ntptr != nullptr, bnd = R.blk != nullptr;
   if (next) {
-    if (bnd) k_level<QUAD, SCHEME, true, true><<<g, kBlock, 0, st>>>(R, nbr, nbv);
-    else k_level<QUAD, SCHEME, true, false><<<g, kBlock, 0, st>>>(R, nbr, nbv);
+    if (bnd) k_level<QUAD, SCHEME, true, true, ONE><<<g, kBlock, 0, st>>>(R, nbr, nbv);
+    else k_level<QUAD, SCHEME, true, false, ONE><<<g, kBlock, 0, st>>>(R, nbr, nbv);
   } else {
-    if (bnd) k_level<QUAD, SCHEME, false, true><<<g, kBlock, 0, st>>>(R, nbr, nbv);
-    else k_level<QUAD, SCHEME, false, false><<<g, kBlock, 0, st>>>(R, nbr, nbv);
+    if (bnd) k_level<QUAD, SCHEME, false, true, ONE><<<g, kBlock, 0, st>>>(R, nbr, nbv);
+    else k_level<QUAD, SCHEME, false, false, ONE><<<g, kBlock, 0, st>>>(R, nbr, nbv);
   }
+}
+
+template <bool QUAD, int SCHEME>
+void launch_level_t(const RefineView& R, unsigned g, int32_t nbr, int32_t nbv, hipStream_t st) {
+  if (R.seg.n == 1) launch_level_t<QUAD, SCHEME, true>(R, g, nbr, nbv, st);
+  else launch_level_t<QUAD, SCHEME, false>(R, g, nbr, nbv, st);
 }
 
 void launch_level(bool quad, int scheme, const RefineView& R0, hipStream_t st) {

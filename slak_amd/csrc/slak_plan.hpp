@@ -110,9 +110,23 @@ struct LevelPlan {
   int64_t* d_vbase = nullptr;
   int64_t* d_fbase = nullptr;
   int64_t* d_cbase = nullptr;
+  int32_t *d_vblk = nullptr, *d_fblk = nullptr, *d_cblk = nullptr;
   int* d_mflags = nullptr;
-  LevelView view(int* flags) const;  // the first level's inputs and analysis arrays
-  SegTable table() const { return SegTable{d_segs, d_vbase, d_fbase, (int32_t)segs.size(), d_mflags, d_cbase}; }
+  LevelView view(int* flags, int* late) const;  // the first level's inputs and analysis arrays
+  SegTable table() const {
+    SegTable T{};
+    T.d = d_segs;
+    T.vbase = d_vbase;
+    T.fbase = d_fbase;
+    T.cbase = d_cbase;
+    T.vblk = d_vblk;
+    T.fblk = d_fblk;
+    T.cblk = d_cblk;
+    T.n = (int32_t)segs.size();
+    T.mflags = d_mflags;
+    if (T.n == 1) T.one = segs[0];
+    return T;
+  }
 };
 
 enum class OutputMode {
@@ -144,6 +158,7 @@ class Plan {
   std::vector<MeshJob>& jobs() { return jobs_; }
   LevelPlan& level(int i) { return levels_[i]; }
   int* flags() { return d_flags_; }
+  int* late() { return late_; }
   Arena& arena() { return arena_; }
   int syncs() const { return syncs_; }
   hipStream_t stream() const { return st_; }
@@ -164,10 +179,9 @@ class Plan {
   };
   void upload_tables(int l0, int l1, Staging& staging, bool zero_state = false);
   void record_gather(LevelPlan& L);
-  // overlap: work enqueued after the copy and before the wait (the host then
-  // waits for the copy only)
-  int readback(const int32_t* src, int count, int64_t* dst, const std::function<void()>& overlap = {});
-  void launch_number(LevelPlan& L, bool faces);
+  int read_flags();
+  void wait_report();
+  void launch_number(LevelPlan& L, bool faces, bool rep = false);
 
   int scheme_;
   std::vector<MeshJob> jobs_;
@@ -182,8 +196,13 @@ class Plan {
   // [flags | row hist | edge bounds (nseg + 1) | mesh flags (nseg)],
   // then [pool | group sums | valence counters] (n_state_ ints in all)
   int32_t* d_state_ = nullptr;
-  int64_t n_state_ = 0, at_groups_ = 0, n_groups_ = 0;
+  int64_t n_state_ = 0, n_groups_ = 0;
   Staging staging_first_, staging_all_;  // segment table uploads
+  // pinned words the device writes: [late flags | pad | report] (see LevelView)
+  Staging host_words_;
+  int32_t* late_ = nullptr;
+  int32_t* report_ = nullptr;
+  bool replayed_ = false;  // the last launch ran the analysis again
   // first-level union gather (multi-mesh)
   float4* P1_ = nullptr;
   bool prepared_ = false;

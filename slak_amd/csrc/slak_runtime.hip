@@ -311,7 +311,7 @@ void spgemm_operator(const slak_mesh& cmesh, int32_t** F_ptr, int32_t** F_ids, i
     SLAK_HIP_CHECK(hipMemcpyAsync(fptr, L.tptr, (nv + 1) * 4, hipMemcpyDeviceToDevice, st));
     SLAK_HIP_CHECK(hipMemcpyAsync(dptr, L.tptr, (nv + 1) * 4, hipMemcpyDeviceToDevice, st));
     SLAK_HIP_CHECK(hipMemcpyAsync(eptr, L.eptr, (nv + 1) * 4, hipMemcpyDeviceToDevice, st));
-    LevelView V = L.view(plan.flags());
+    LevelView V = L.view(plan.flags(), plan.late());
     V.ne_cap = ne;
     V.F_ids = take(nnz);
     V.F_vals = take(nnz);
