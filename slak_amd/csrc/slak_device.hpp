@@ -68,6 +68,8 @@ struct SegDesc {
   int32_t src_stride;
   int32_t require_quad;
   int32_t dst_final;       // 1: the destination is the caller's output (stored non-temporally)
+  int64_t next_own;        // base of the refined mesh's edges in the next level's edge owners
+                           // (a multiple of 4), or -1: not wanted
 };
 
 // The meshes of a level. A single mesh (n == 1) is described by `one`, in the
@@ -515,8 +517,46 @@ __device__ __forceinline__ void row_number(Row& r, const LevelView& L, int32_t v
   }
 }
 
+// Spreads the blocks of several lists over a launch in proportion: of the
+// first b of T blocks, share(b) = ceil-ratio(n / T) * b belong to a list of n,
+// so block b is the list's share(b)-th when share(b + 1) > share(b), else block
+// b - share(b) of the rest. With ratio = ceil(n 2^32 / T) and T < 2^31, share
+// rises by 0 or 1 per block and ends at n: the lists are covered exactly. (A
+// 64-bit division in its place is more than a hundred scalar instructions.)
+inline uint64_t share_ratio(int64_t n, int64_t T) {
+  return T > 0 ? (uint64_t)((((__uint128_t)n << 32) + (__uint128_t)(T - 1)) / (__uint128_t)T) : 0;
+}
+__device__ __forceinline__ int32_t share_of(int32_t b, uint64_t ratio) {
+  return (int32_t)(((uint64_t)(uint32_t)b * ratio) >> 32);
+}
+
 // One level's refinement inputs and the next level's structure.
 constexpr int kMaxVSeg = 8;
+
+// Vertex items as up to kMaxVSeg class runs [first[s], first[s + 1]) of
+// nb[s] blocks; ratio[s]: run s among the runs from s on (see share_ratio).
+struct VertexRuns {
+  int32_t n;
+  int32_t blocks;  // of all runs
+  int32_t first[kMaxVSeg + 1];
+  int32_t nb[kMaxVSeg];
+  uint64_t ratio[kMaxVSeg];
+};
+
+// first vertex of vertex block u of the runs; end: of its run
+__device__ __forceinline__ int32_t run_block(const VertexRuns& R, int32_t u, int32_t& end) {
+  int s = 0;
+  for (; s + 1 < R.n; ++s) {
+    const int32_t lo = share_of(u, R.ratio[s]), hi = share_of(u + 1, R.ratio[s]);
+    if (hi > lo) {
+      u = lo;
+      break;
+    }
+    u -= lo;
+  }
+  end = R.first[s + 1];
+  return R.first[s] + u * kBlockItems;
+}
 
 struct RefineView {
   const int32_t* ids;
@@ -538,15 +578,14 @@ struct RefineView {
   int2* nci;
   int32_t* nbnd;         // next level's union edge boundary flags, or null: closed
   int32_t* nmpos;        // next level's M^T positions (SLAK)
+  int2* nown;            // next level's edge owners (owner corner, twin), for the meshes with next_own >= 0
   int32_t next_nv;       // next level's union vertices and corners (end of its M^T)
   int32_t next_nnz;
   int32_t next_rows_x;   // 1: the next level's M^T rows are corners only (int32 in ntrow)
-  // one mesh: its vertex items as up to kMaxVSeg class runs [vseg[s],
-  // vseg[s+1]) of vnb[s] blocks, each run spread in proportion over the
-  // launch (nvseg 0: one run)
-  int32_t nvseg;
-  int32_t vseg[kMaxVSeg + 1];
-  int32_t vnb[kMaxVSeg];
+  // the vertex items' runs (one mesh: its vertex classes, each spread in
+  // proportion over the launch; n 0: one run), and their share of the launch
+  VertexRuns runs;
+  uint64_t vratio;
 };
 
 // One mesh of a final level computed from the structure of the quad mesh M
@@ -557,7 +596,6 @@ struct FinalSeg {
   int64_t cb, vb, eb;    // union bases of M's corners, vertices, edges
   int32_t nv, nf, ne;    // M sizes
   int32_t nnz;
-  int32_t id_off;        // added to the output vertex ids (pooled outputs)
   const float4* P1;      // M1 positions = [M vertices | M face points | M edge points]
   float4* out_verts;     // output positions: [M1 vertices | M1 face points | M1 edge points]
   int32_t* out_ids;      // output quads: 4 per M1 corner, 16 per M corner
@@ -574,22 +612,23 @@ struct FinalView {
   const int32_t* trow_x; // or the rows' corners alone (int32), or null
   const int32_t* blk;    // exclusive scan of the boundary edge flags, or null (closed)
   const int32_t* mpos;   // M^T position per corner (SLAK)
+  const int2* own;       // k_final_deep, whose union and meshes are those of N, three levels before
+                         // the output: (owner corner, twin) per edge, from base eb of each mesh
   FinalSeg one;          // a single mesh (nseg == 1, no table)
   const FinalSeg* segs;  // several meshes: device table
   // several meshes: work units of one block each, (mesh, first mesh-local
   // item, count, kind): kind 0 consecutive corners of one mesh, kind 1
-  // consecutive vertices of one class of one mesh. Mesh by mesh, the corner
+  // consecutive vertices of one class of one mesh, kind 2 consecutive edges
+  // (k_final_deep). Mesh by mesh, the corner
   // units and every vertex class's units are interleaved by their relative
   // position, so a mesh's vertex items run beside its corner items.
   const int4* units;
   int32_t nunits;
   int32_t nseg;
   int64_t nnz, nv;       // corner and vertex items of the launch
-  // the vertex items as up to kMaxVSeg runs [vseg[s], vseg[s+1]) of vnb[s]
-  // blocks, each run spread in proportion over the launch (nvseg 0: one run)
-  int32_t nvseg;
-  int32_t vseg[kMaxVSeg + 1];
-  int32_t vnb[kMaxVSeg];
+  // the vertex items' runs (n 0: one run) and their share of the launch
+  VertexRuns runs;
+  uint64_t vratio;
 };
 
 // Face, successor and predecessor corner of corner t (quad: bit arithmetic;

@@ -87,6 +87,11 @@ void launch_level(bool quad, int scheme, const RefineView& R, hipStream_t st);
 // last level of one mesh or several (V.segs) from the quad mesh two levels
 // back; ids: also the output quads and LAK form (false: positions only)
 void launch_final(int scheme, const FinalView& V, bool ids, hipStream_t st);
+// last level of one closed LAK mesh or several (V.segs) from the quad mesh
+// three levels back, whose structure V holds, and the positions of the level
+// before the output
+void launch_final_deep(const FinalView& V, hipStream_t st);
+constexpr int kDeepEdgeUnit = 64;  // edges per work unit of the several-mesh form
 // the LAK form (ptr, vals) of a several-mesh output level, after its k_final
 // launch (which leaves it out)
 void launch_final_lak_form(const FinalView& V, hipStream_t st);

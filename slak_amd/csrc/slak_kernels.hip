@@ -840,6 +840,7 @@ struct SegK {
   int32_t* dst_ptr;
   int32_t* dst_vals;
   int32_t ncb, nvb, neb;  // next level's union bases (ncb < 0: the mesh finishes here)
+  int64_t own;  // base in the next level's edge owners, < 0: not wanted
   bool next, dst_final;
 };
 
@@ -865,6 +866,7 @@ __device__ __forceinline__ SegK seg_consts(const SegTable& seg, int32_t t) {
   K.neb = (int32_t)S->next_eb;
   K.next = S->next_cb >= 0;
   K.dst_final = S->dst_final != 0;
+  K.own = S->next_own;
   return K;
 }
 
@@ -1001,6 +1003,18 @@ __device__ __forceinline__ void corner_store(const RefineView& R, const SegK& K,
   if (SCHEME == kSLAK && nbnd) nbnd[neb + snnz + lt] = 0;  // face point edges are interior
   if (c.own) {
     R.ntptr[nep + c.e1] = row1;
+    if (SCHEME == kLAK && K.own >= 0 && c.s1 >= 0) {
+      // the half-edges of the refined edges 4 e1 + 0 .. 3 (closed mesh): to
+      // the lower and the higher end, to the lower and the higher face
+      const int32_t s4 = ncb + 4 * (c.s1 - cb), n4 = ncb + 4 * (c.n1 - cb), tn4 = ncb + 4 * (c.tn - cb);
+      auto pair = [](int32_t x, int32_t y) __attribute__((always_inline)) { return make_int2(min(x, y), max(x, y)); };
+      const int2 ev = pair(c4, n4 + 3), ew = pair(s4, tn4 + 3), ef = pair(c4 + 1, tn4 + 2), eg = pair(s4 + 1, n4 + 2);
+      const bool vw = c.v > c.w, fg = c.f > c.g1;
+      int4* __restrict__ o4 = reinterpret_cast<int4*>(R.nown + (K.own + 4 * (int64_t)c.e1));
+      const int2 l0 = vw ? ew : ev, l1 = vw ? ev : ew, l2 = fg ? eg : ef, l3 = fg ? ef : eg;
+      o4[0] = make_int4(l0.x, l0.y, l1.x, l1.y);
+      o4[1] = make_int4(l2.x, l2.y, l3.x, l3.y);
+    }
     int2 a0 = make_int2(c4 + 1, nvb + (c.v - K.vb));
     int2 a1 = make_int2(ncb + 4 * (c.tn - cb) + 3, nvb + snv + lf);
     if (a1.x < a0.x) {
@@ -1226,32 +1240,17 @@ __device__ __forceinline__ void vertex_item(const RefineView& R, int32_t v) {
 // items (one per vertex) are independent once the face points exist, and they
 // write disjoint outputs. Their blocks are interleaved in proportion over the
 // grid, so write-bound refine waves and gather-bound vertex waves share the
-// machine. Block b is a vertex block when floor((b+1) nbv / T) > floor(b nbv / T)
-// (T = nbr + nbv): vertex block floor(b nbv / T), else refine block
-// b - floor(b nbv / T); a bijection onto both block ranges.
+// machine (share_ratio).
 template <bool QUAD, int SCHEME, bool NEXT, bool BND, bool ONE>
-__global__ void __launch_bounds__(kBlock) k_level(RefineView R, int32_t nbr, int32_t nbv) {
-  const int64_t b = NEXT ? block_index<kRemapLevel>() : block_index<kRemapPositions>();
-  const int64_t T = (int64_t)nbr + nbv;
-  const int64_t before = b * nbv / T, after = (b + 1) * nbv / T;
+__global__ void __launch_bounds__(kBlock) k_level(RefineView R) {
+  const int32_t b = (int32_t)(NEXT ? block_index<kRemapLevel>() : block_index<kRemapPositions>());
+  const int32_t before = share_of(b, R.vratio), after = share_of(b + 1, R.vratio);
   if (after > before) {
-    // vertex block `before`: its class run and its block within the run
-    int64_t u = before, rest = nbv;
-    int s = 0;
-    for (; s + 1 < R.nvseg; ++s) {
-      const int64_t nb = R.vnb[s];
-      const int64_t lo = u * nb / rest, hi = (u + 1) * nb / rest;
-      if (hi > lo) {
-        u = lo;
-        break;
-      }
-      u -= lo;
-      rest -= nb;
-    }
-    const int64_t v = (int64_t)R.vseg[s] + u * blockDim.x + threadIdx.x;
-    vertex_item<QUAD, SCHEME, NEXT, BND, ONE>(R, v < R.vseg[s + 1] ? (int32_t)v : R.nv);
+    int32_t end;
+    const int32_t v = run_block(R.runs, before, end) + (int32_t)threadIdx.x;
+    vertex_item<QUAD, SCHEME, NEXT, BND, ONE>(R, v < end ? v : R.nv);
   } else {
-    refine_item<QUAD, SCHEME, ONE>(R, (b - before) * blockDim.x + threadIdx.x);
+    refine_item<QUAD, SCHEME, ONE>(R, (int64_t)(b - before) * kBlock + threadIdx.x);
   }
 }
 
@@ -1409,8 +1408,8 @@ __device__ __forceinline__ Quads4 final_corner(const FinalView& V, const FinalSe
   // the four output quads of M1 face t
   Quads4 q4{};
   if (IDS) {
-    const int32_t off = S.id_off, eb2 = epb2 + off;
-    const int32_t x0 = v + off, x1 = ep0 + e1 + off, x2 = nv + F + off, x3 = ep0 + e0 + off, fid = nv1 + t + off;
+    const int32_t eb2 = epb2;
+    const int32_t x0 = v, x1 = ep0 + e1, x2 = nv + F, x3 = ep0 + e0, fid = nv1 + t;
     // the block stages them in LDS and writes them out as 1 KB runs
     // (64-byte pieces per lane, stored directly, cost several times more)
     q4.a = make_int4(x0, eb2 + ex, fid, eb2 + ew);
@@ -1583,67 +1582,13 @@ __device__ __forceinline__ void final_vertex(const FinalView& V, const FinalSeg&
   S.out_verts[v] = q;
 }
 
-// Corner items and vertex items interleaved in proportion, as in k_level.
-// The vertex blocks are split the same way between the runs of V.vseg (run s
-// against the runs after it): the vertex classes of M (the original vertices,
-// then the face points and edge points of every earlier level), each numbered
-// in the order of the original faces it descends from, so that every run
-// advances over the same part of the surface as the corner blocks and the
-// positions they gather are fetched once for both. Several meshes take their
-// blocks from V.units, which interleaves each mesh's corner and vertex units
-// the same way. A corner block stages its 16 KB of output quads in LDS and
-// stores them with consecutive lanes on consecutive 16-byte pieces.
-template <int SCHEME, bool BND, bool MULTI, bool IDS>
-__global__ void __launch_bounds__(kBlock) k_final(FinalView V, int32_t nbc, int32_t nbv) {
-  const int64_t b = block_index<kRemapFinal>();
-  FinalSeg S;
-  int32_t t0, cnt;
-  if (MULTI) {  // work unit b (block-uniform): corners or vertices of one mesh
-    const int4 U = V.units[b];
-    S = V.segs[U.x];
-    S.P1 = to_global(S.P1);
-    S.out_verts = to_global(S.out_verts);
-    S.out_ids = to_global(S.out_ids);
-    S.out_ptr = to_global(S.out_ptr);
-    S.out_vals = to_global(S.out_vals);
-    if (U.w) {
-      if ((int)threadIdx.x < U.z) final_vertex<SCHEME, BND>(V, S, U.y + (int32_t)threadIdx.x);
-      return;
-    }
-    t0 = U.y;
-    cnt = U.z;
-  } else {
-    const int64_t T = (int64_t)nbc + nbv;
-    const int64_t before = b * nbv / T, after = (b + 1) * nbv / T;
-    if (after > before) {
-      int64_t u = before, rest = nbv;
-      int s = 0;
-      for (; s + 1 < V.nvseg; ++s) {
-        const int64_t nb = V.vnb[s];
-        const int64_t lo = u * nb / rest, hi = (u + 1) * nb / rest;
-        if (hi > lo) {
-          u = lo;
-          break;
-        }
-        u -= lo;
-        rest -= nb;
-      }
-      const int64_t v = (int64_t)V.vseg[s] + u * blockDim.x + threadIdx.x;
-      if (v < V.vseg[s + 1]) final_vertex<SCHEME, BND>(V, V.one, (int32_t)v);
-      return;
-    }
-    S = V.one;
-    t0 = (int32_t)((b - before) * kBlock);
-    cnt = (int32_t)min((int64_t)kBlock, V.nnz - t0);
-  }
+// The output quads of a block's corners t0 .. t0 + cnt (of nnz in the mesh):
+// staged in LDS and stored with consecutive lanes on consecutive 16-byte
+// pieces; one mesh: their LAK form too.
+template <bool MULTI>
+__device__ __forceinline__ void store_quads(const FinalSeg& S, const Quads4& q4, int4* stage, int32_t t0, int32_t cnt,
+                                            int32_t nnz) {
   const int32_t t = t0 + (int32_t)threadIdx.x;
-  if (!IDS) {  // positions only
-    if ((int)threadIdx.x < cnt) final_corner<SCHEME, BND, false, MULTI>(V, S, t);
-    return;
-  }
-  __shared__ int4 stage[kStageStride * kBlock];
-  Quads4 q4{};
-  if ((int)threadIdx.x < cnt) q4 = final_corner<SCHEME, BND, true, MULTI>(V, S, t);
   if ((int)threadIdx.x < cnt) {
     int4* __restrict__ o = stage + kStageStride * threadIdx.x;
     o[0] = q4.a;
@@ -1679,8 +1624,455 @@ __global__ void __launch_bounds__(kBlock) k_final(FinalView V, int32_t nbc, int3
   }
   if (S.out_ptr) {
     if ((int)threadIdx.x < cnt) store_nt(S.out_ptr + 4 * (int64_t)t, 16 * t, 16 * t + 4, 16 * t + 8, 16 * t + 12);
-    if (t == S.nnz - 1) store_nt(S.out_ptr + 4 * (int64_t)S.nnz, 16 * S.nnz);
+    if (t == nnz - 1) store_nt(S.out_ptr + 4 * (int64_t)nnz, 16 * nnz);
   }
+}
+
+// Corner items and vertex items interleaved in proportion, as in k_level.
+// The vertex blocks are split the same way between the runs of V.runs (run s
+// against the runs after it): the vertex classes of M (the original vertices,
+// then the face points and edge points of every earlier level), each numbered
+// in the order of the original faces it descends from, so that every run
+// advances over the same part of the surface as the corner blocks and the
+// positions they gather are fetched once for both. Several meshes take their
+// blocks from V.units, which interleaves each mesh's corner and vertex units
+// the same way. A corner block stages its 16 KB of output quads in LDS and
+// stores them with consecutive lanes on consecutive 16-byte pieces.
+template <int SCHEME, bool BND, bool MULTI, bool IDS>
+__global__ void __launch_bounds__(kBlock) k_final(FinalView V) {
+  const int32_t b = (int32_t)block_index<kRemapFinal>();
+  FinalSeg S;
+  int32_t t0, cnt;
+  if (MULTI) {  // work unit b (block-uniform): corners or vertices of one mesh
+    const int4 U = V.units[b];
+    S = V.segs[U.x];
+    S.P1 = to_global(S.P1);
+    S.out_verts = to_global(S.out_verts);
+    S.out_ids = to_global(S.out_ids);
+    S.out_ptr = to_global(S.out_ptr);
+    S.out_vals = to_global(S.out_vals);
+    if (U.w) {
+      if ((int)threadIdx.x < U.z) final_vertex<SCHEME, BND>(V, S, U.y + (int32_t)threadIdx.x);
+      return;
+    }
+    t0 = U.y;
+    cnt = U.z;
+  } else {
+    const int32_t before = share_of(b, V.vratio), after = share_of(b + 1, V.vratio);
+    if (after > before) {
+      int32_t end;
+      const int32_t v = run_block(V.runs, before, end) + (int32_t)threadIdx.x;
+      if (v < end) final_vertex<SCHEME, BND>(V, V.one, v);
+      return;
+    }
+    S = V.one;
+    t0 = (b - before) * kBlock;
+    cnt = (int32_t)min((int64_t)kBlock, V.nnz - t0);
+  }
+  const int32_t t = t0 + (int32_t)threadIdx.x;
+  if (!IDS) {  // positions only
+    if ((int)threadIdx.x < cnt) final_corner<SCHEME, BND, false, MULTI>(V, S, t);
+    return;
+  }
+  __shared__ int4 stage[kStageStride * kBlock];
+  Quads4 q4{};
+  if ((int)threadIdx.x < cnt) q4 = final_corner<SCHEME, BND, true, MULTI>(V, S, t);
+  store_quads<MULTI>(S, q4, stage, t0, cnt, S.nnz);
+}
+
+// ---------------------------------------------------------------------------
+// The output level of a closed mesh from three levels back (LAK): N is the
+// quad mesh three levels before the output, M = refine(N), M1 = refine(M),
+// the output refine(M1). Only N's structure and M1's positions P1 are read;
+// M's structure, which the refine items would have written and k_final reads,
+// is a function of N's:
+//   M corner 4t + k of N corner t (v -> w along e1, twin s1; u -> v along e0,
+//   twin s0; face f): vertices (v, ep(e1), fp(f), ep(e0)), out-edges
+//   4e1 + (v > w), 4e1 + 2 + (f > g1), 4e0 + 2 + (f > g0), 4e0 + (v > u),
+//   faces across them next(s1), next(t), prev(t), s0
+// so the level before the last two writes no structure at all, and what a
+// wave gathers is shared: k_final is bound by the number of lines its lanes
+// gather and scatter (without its vertex items and with neighbouring instead
+// of real partners it ran at 4.7 TB/s instead of 3.0), so the work is laid
+// out over rows of 16 lanes that hold everything around one face or one edge
+// of N.
+//   corner items  one lane per M corner, 16 lanes per N face: the face points
+//                 of M1, the vertex points of M's face points, and of M's
+//                 vertex fp(f) (its four corners are in the row)
+//   edge items    16 lanes per N edge: the four M edges at X = ep(e), four M1
+//                 edges around each: 16 edge points (one 256-byte run), the
+//                 vertex points of the four M edge points and of X
+//   vertex items  one lane per N vertex
+// Every sum adds the same terms in the same order as k_final's: same bits.
+
+template <int N>
+__device__ __forceinline__ int32_t row_ror_i(int32_t x) {  // lane i of a row of 16 reads lane i - N
+  return __builtin_amdgcn_mov_dpp(x, 0x120 + N, 0xF, 0xF, false);
+}
+template <int N>
+__device__ __forceinline__ float4 row_ror(float4 x) {
+  return make_float4(__int_as_float(row_ror_i<N>(__float_as_int(x.x))), __int_as_float(row_ror_i<N>(__float_as_int(x.y))),
+                     __int_as_float(row_ror_i<N>(__float_as_int(x.z))), __int_as_float(row_ror_i<N>(__float_as_int(x.w))));
+}
+template <int K>
+__device__ __forceinline__ int32_t quad_lane_i(int32_t x) {
+  return __builtin_amdgcn_mov_dpp(x, K * 0x55, 0xF, 0xF, false);
+}
+// sizes of N, M and M1 of one mesh, as vertex bases of the output
+struct DeepBase {
+  int32_t epN;   // M vertex ep(edge 0 of N) = N vertices + N faces
+  int32_t fM;    // M1 vertex fp(M face 0) = M vertices
+  int32_t eM;    // M1 vertex ep(M edge 0)
+  int32_t fM1;   // output vertex fp(M1 face 0) = M1 vertices
+  int32_t eM1;   // output vertex ep(M1 edge 0)
+  __device__ __forceinline__ explicit DeepBase(const FinalSeg& S) {
+    epN = S.nv + S.nf;
+    fM = epN + S.ne;
+    eM = fM + S.nnz;
+    fM1 = eM + 2 * S.nnz;
+    eM1 = fM1 + 4 * S.nnz;
+  }
+};
+
+// Lanes exchange positions through LDS (rows of 16 lanes, so inside one wave):
+// orders the accesses for the compiler, the hardware keeps a wave's in order.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// What the vector memory unit pays for is lines per four neighbouring lanes:
+// a gather whose every lane has its own line takes four times as long as one
+// whose quads of lanes read 64 contiguous bytes. So a row loads each position
+// it needs once, neighbouring lanes neighbouring positions where there are
+// any, and its lanes take their operands from LDS.
+
+// Corner items: lane 4j + k of a row holds corner k of M face t_j = 4f + j. The
+// row loads v_j, ep(e_j), fp(f), fp(t_j) (four lanes each) and, a quad per
+// j, the four M edge points around ep(e_j). ex: the row's exchange, kRowEx
+// float4. Returns the 16 output ids of M corner c.
+constexpr int kRowEx = 65;  // loaded 0-31, M1 face points 32-47, out-edge points 48-63, one pad
+
+__device__ __forceinline__ Quads4 deep_corner(const FinalView& V, const FinalSeg& S, int32_t c, float4* ex) {
+  const DeepBase B(S);
+  const int i = threadIdx.x & 15, k = i & 3, j = i >> 2, jp = (j + 3) & 3;
+  const int32_t t = c >> 2, f = c >> 4, q0 = t & ~3;
+  const int32_t tn = q0 | ((t + 1) & 3), tp = q0 | ((t + 3) & 3);
+  const int32_t cb = (int32_t)S.cb, vb = (int32_t)S.vb, emax = S.ne > 0 ? S.ne - 1 : 0;
+  const float4* __restrict__ P1 = S.P1;
+  float4* __restrict__ out = S.out_verts;
+  float* __restrict__ outf = reinterpret_cast<float*>(S.out_verts);
+  const int32_t v = V.ids[cb + t] - vb;
+  const int2 c1 = V.ci[cb + t];
+  const int32_t vk = V.ids[cb + q0 + k] - vb;  // corner k of the face, for the row's loads
+  const int32_t ek = clampi(V.ci[cb + q0 + k].x, emax);
+  const int32_t e1 = clampi(c1.x, emax), s1 = c1.y - cb;
+  const float4 p0 = P1[j == 0 ? vk : j == 1 ? B.epN + ek : j == 2 ? S.nv + f : B.fM + q0 + k];
+  const float4 p1 = P1[B.eM + 4 * e1 + k];
+  // the face's other corners are 4 lanes on in the row
+  const int32_t w = row_ror_i<12>(v), u = row_ror_i<4>(v);
+  const int32_t e0 = row_ror_i<4>(e1), s0 = row_ror_i<4>(s1);
+  const int32_t n1 = (s1 & ~3) | ((s1 + 1) & 3);
+  // vertex, out-edge and face across it of M corner c
+  const int32_t x = k == 0 ? v : k == 1 ? B.epN + e1 : k == 2 ? S.nv + f : B.epN + e0;
+  const int slot = k == 0   ? (v > w ? 1 : 0)
+                   : k == 1 ? 2 + (f > (s1 >> 2) ? 1 : 0)
+                   : k == 2 ? 2 + (f > (s0 >> 2) ? 1 : 0)
+                            : (v > u ? 1 : 0);
+  const int32_t E1 = 4 * (k < 2 ? e1 : e0) + slot;
+  const int32_t G1 = k == 0 ? n1 : k == 1 ? tn : k == 2 ? tp : s0;
+  const int32_t E0 = quad_prev_i(E1), G0 = quad_prev_i(G1), xn = quad_next_i(x), xp = quad_prev_i(x);
+  ex[i] = p0;
+  ex[16 + i] = p1;
+  wave_lds_fence();
+  const float4 Pv = ex[k == 0 ? j : k == 1 ? 4 + j : k == 2 ? 8 : 4 + jp];
+  const float4 PF = ex[12 + j];
+  const float4 Pe = ex[16 + 4 * (k < 2 ? j : jp) + slot];
+  const float4 fpt = face_point(Pv, Pe, PF, quad_prev(Pe));
+  ex[32 + i] = fpt;
+  ex[48 + i] = Pe;
+  wave_lds_fence();
+  const float* const xf = reinterpret_cast<const float*>(ex);
+  float sF = 0.f, sV = 0.f;  // component k of two vertex points
+  {  // M face t's face point: the quad's M1 faces and out-edge points in corner order
+    const float* const q = xf + 128 + 16 * j + k;
+    sF = sF + q[0];
+    sF = sF + q[4];
+    sF = sF + q[8];
+    sF = sF + q[12];
+    sF = sF + q[64];
+    sF = sF + q[68];
+    sF = sF + q[72];
+    sF = sF + q[76];
+    sF = (sF / 4.0f + xf[4 * (12 + j) + k] * 2.0f) / 4.0f;
+  }
+  {  // M's vertex fp(f), corners 4t + 2: lanes 2, 6, 10, 14; in-neighbours the out-edge points of the lanes before
+    const float* const q = xf + 128 + k;
+    sV = sV + q[8];
+    sV = sV + q[24];
+    sV = sV + q[40];
+    sV = sV + q[56];
+    sV = sV + q[64 + 4];
+    sV = sV + q[64 + 20];
+    sV = sV + q[64 + 36];
+    sV = sV + q[64 + 52];
+    sV = (sV / 4.0f + xf[32 + k] * 2.0f) / 4.0f;
+  }
+  out[B.fM1 + c] = fpt;
+  outf[4 * (int64_t)(B.fM + t) + k] = sF;
+  if (j == 0) outf[4 * (int64_t)(S.nv + f) + k] = sV;
+  // M1 edges of corners 4c .. 4c + 3, then the four output quads
+  const int32_t eX = B.eM1 + 4 * E1 + (x > xn ? 1 : 0), eY = B.eM1 + 4 * E1 + 2 + (t > G1 ? 1 : 0);
+  const int32_t eZ = B.eM1 + 4 * E0 + 2 + (t > G0 ? 1 : 0), eW = B.eM1 + 4 * E0 + (x > xp ? 1 : 0);
+  const int32_t fid = B.fM1 + c;
+  Quads4 q;
+  q.a = make_int4(x, eX, fid, eW);
+  q.b = make_int4(B.eM + E1, eY, fid, eX);
+  q.c = make_int4(B.fM + t, eZ, fid, eY);
+  q.d = make_int4(B.eM + E0, eW, fid, eZ);
+  return q;
+}
+
+// Edge items: 16 lanes per N edge e. Around X = ep(e), in turn: the M vertices
+// A_j = v, fp(f), w, fp(g) and the M faces Z_j = t, next(t), s, next(s) between
+// A_j and A_{j+1} (each passes A_j -> X -> A_{j+1}; t is the owner, so f < g and
+// t, next(t) < s, next(s)); Y_j is the edge point of the M edge A_j X, M edge
+// 4e + (v > w), 4e + 2, 4e + (w > v), 4e + 3. Around Y_j in turn: A_j, Z_j, X,
+// Z_{j-1}, with the M1 faces
+//   psi_0 = (A_j, Y_j, Z_j, Bin_j)        psi_1 = (X, Y_{j+1}, Z_j, Y_j)
+//   psi_2 = (X, Y_j, Z_{j-1}, Y_{j-1})    psi_3 = (A_j, Bout_j, Z_{j-1}, Y_j)
+// after each, Bin_j and Bout_j being the edge points of A_j's other M edges in
+// Z_j and Z_{j-1}. The row loads the four Y (64 contiguous bytes), Z, A and X, and
+// the eight Bin / Bout (pairs of neighbours). Lane 4j + m then forms psi_m and the
+// edge point of M1's edge from Y_j to its neighbour m, (neighbour + Y_j + psi_m +
+// psi_{m-1}) / 4; the vertex points of the Y_j and of X are formed one component
+// per lane, their terms picked in row order by address.
+constexpr int kRows = kBlock / 16;
+constexpr int kEdgeIter = kDeepEdgeUnit / kRows;  // edges per row and unit
+constexpr int kRowE = 33;                   // float4 of a row: p 0-15, psi 16-31, one pad (rows start 4 banks apart)
+constexpr int kRowX = 9 * kEdgeIter + 1;    // per edge: psi_1 and Y of j = 0 .. 3, X
+constexpr int kEdgeLds = (kRowE + kRowX) * kRows;  // float4
+
+__device__ __forceinline__ void deep_edges(const FinalView& V, const FinalSeg& S, int32_t first, int32_t cnt,
+                                           float4* lds) {
+  const DeepBase B(S);
+  const int32_t cb = (int32_t)S.cb, vb = (int32_t)S.vb, emax = S.ne > 0 ? S.ne - 1 : 0;
+  const float4* __restrict__ P1 = S.P1;
+  float4* __restrict__ out = S.out_verts;
+  float* __restrict__ outf = reinterpret_cast<float*>(S.out_verts);
+  const int row = threadIdx.x >> 4, i = threadIdx.x & 15, m = i & 3, j = i >> 2, jp = (j + 3) & 3;
+  const bool odd = (j & 1) != 0, side = (j & 2) != 0;
+  float4* const re = lds + row * kRowE;
+  float4* const rx = lds + kRows * kRowE + row * kRowX;
+  const float* const ref = reinterpret_cast<const float*>(re);
+  uint32_t order = 0;  // per edge: t before next(t), s before next(s)
+#pragma unroll
+  for (int it = 0; it < kEdgeIter; ++it) {
+    const int r = row + it * kRows;
+    if (r >= cnt) break;
+    const int32_t e = first + r;
+    const int2 o = V.own[S.eb + e];
+    const int32_t t = o.x - cb, s1 = o.y - cb;
+    const bool tt = (t & 3) != 3, ss = (s1 & 3) != 3;
+    order |= ((tt ? 1u : 0u) | (ss ? 2u : 0u)) << (2 * it);
+    // the row's halves hold the face of t and the face of its twin, each quad
+    // the face's corners from the half-edge's own on
+    const int32_t a = side ? s1 : t, h = a >> 2;
+    const int32_t corner = cb + ((a & ~3) | ((a + m) & 3));
+    const int32_t id = V.ids[corner] - vb;
+    const int2 cc = V.ci[corner];
+    const int32_t ce = clampi(cc.x, emax), cg = (cc.y - cb) >> 2;  // edge, face across it
+    const int32_t I0 = quad_lane_i<0>(id), I1 = quad_lane_i<1>(id), I2 = quad_lane_i<2>(id), I3 = quad_lane_i<3>(id);
+    const int32_t C1 = quad_lane_i<1>(ce), C3 = quad_lane_i<3>(ce);
+    const int32_t gc = quad_lane_i<1>(cg), gd = quad_lane_i<3>(cg);
+    const int32_t Zc = odd ? ((a & ~3) | ((a + 1) & 3)) : a;
+    const int32_t Y_id = 4 * e + (odd ? (side ? 3 : 2) : (I0 > I1 ? 1 : 0));
+    const int32_t across = row_ror_i<8>(4 * C1 + (I1 > I2 ? 1 : 0));  // the other half's
+    const int32_t Bin = odd ? 4 * C1 + 2 + (h > gc ? 1 : 0) : 4 * C3 + (I0 > I3 ? 1 : 0);
+    const int32_t Bout = odd ? 4 * C3 + 2 + (h > gd ? 1 : 0) : across;
+    const float4 p = P1[m == 0 ? (odd ? S.nv + h : I0) : m == 1 ? B.fM + Zc : m == 2 ? B.eM + Y_id : B.epN + e];
+    float4 b = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (m == 0 || m == 3) b = P1[B.eM + (m == 0 ? Bin : Bout)];
+    const float4 A = quad_lane<0>(p), Z = quad_lane<1>(p), Y = quad_lane<2>(p), X = quad_lane<3>(p);
+    const float4 Zp = row_ror<4>(Z), Yn = row_ror<12>(Y), Yp = row_ror<4>(Y);
+    const bool atA = m == 0 || m == 3;
+    const float4 psi = face_point(f4sel(atA, A, X), f4sel(m == 1, Yn, f4sel(m == 3, b, Y)), f4sel(m < 2, Z, Zp),
+                                  f4sel(m == 0, b, f4sel(m == 2, Yp, Y)));
+    const float4 nbr = f4sel(m == 0, A, f4sel(m == 1, Z, f4sel(m == 2, X, Zp)));
+    const bool zfirst = j == 0 || (j == 1 && !tt) || (j == 3 && !ss);  // Z_j before Z_{j-1}
+    const int32_t slot = m == 0 ? 0 : m == 2 ? 1 : ((m == 1) == zfirst ? 2 : 3);
+    re[i] = p;
+    re[16 + i] = psi;
+    if (m) rx[9 * it + (m == 3 ? 8 : m == 2 ? 4 + j : j)] = f4sel(m == 1, psi, p);
+    out[B.eM1 + 4 * Y_id + slot] = f4mul(f4add(f4add(f4add(nbr, Y), psi), quad_prev(psi)), 0.25f);
+    wave_lds_fence();
+    // vertex point of Y_j, component m: the row's corners are those of the
+    // lower M face first; in Z_j A_j's comes before X's, in Z_{j-1} when j is odd
+    {
+      const int f = 16 * j + m, g = 64 + f;
+      const int r0 = odd ? 8 : 12, r1 = odd ? 12 : 8;
+      const int z = 16 * jp + 4 + m;  // Z_{j-1}
+      const int n0 = odd ? f + 12 : z, n1 = odd ? z : f + 12;
+      float sum = 0.f;
+      sum = sum + ref[g + (zfirst ? 0 : r0)];
+      sum = sum + ref[g + (zfirst ? 4 : r1)];
+      sum = sum + ref[g + (zfirst ? r0 : 0)];
+      sum = sum + ref[g + (zfirst ? r1 : 4)];
+      sum = sum + ref[zfirst ? f : n0];
+      sum = sum + ref[zfirst ? f + 4 : n1];
+      sum = sum + ref[zfirst ? n0 : f];
+      sum = sum + ref[zfirst ? n1 : f + 4];
+      outf[4 * (int64_t)(B.eM + Y_id) + m] = (sum / 4.0f + ref[f + 8] * 2.0f) / 4.0f;
+    }
+    wave_lds_fence();  // read before the next edge writes
+  }
+  // vertex points of the X: lane i forms component m of the row's edge j
+  const int r = row + j * kRows;
+  if (r < cnt) {
+    const float* const x = reinterpret_cast<const float*>(rx + 9 * j) + m;
+    const int tt = (order >> (2 * j)) & 1 ? 0 : 4, ss = (order >> (2 * j)) & 2 ? 8 : 12;
+    float sum = 0.f;
+    sum = sum + x[tt];
+    sum = sum + x[4 - tt];
+    sum = sum + x[ss];
+    sum = sum + x[20 - ss];
+    sum = sum + x[16 + tt];
+    sum = sum + x[20 - tt];
+    sum = sum + x[16 + ss];
+    sum = sum + x[36 - ss];
+    outf[4 * (int64_t)(B.epN + first + r) + m] = (sum / 4.0f + x[32] * 2.0f) / 4.0f;
+  }
+}
+
+// vertex point of a vertex v of N in the output: M corners 4t of its row's
+// corners t, M1 faces (v, ep(4e1 + (v > w)), fp(M face t), ep(4e0 + (v > u)))
+__device__ __forceinline__ void deep_vertex(const FinalView& V, const FinalSeg& S, int32_t v) {
+  const DeepBase B(S);
+  const int32_t cb = (int32_t)S.cb, vb = (int32_t)S.vb;
+  const int32_t emax = S.ne > 0 ? S.ne - 1 : 0;
+  const float4* __restrict__ P1 = S.P1;
+  const int32_t* __restrict__ ids = V.ids + cb;
+  const int2* __restrict__ ci = V.ci + cb;
+  const int32_t p0 = V.tptr[vb + v];
+  const int n = V.tptr[vb + v + 1] - p0;
+  const int32_t* __restrict__ rx = V.trow_x ? V.trow_x + p0 : reinterpret_cast<const int32_t*>(V.trow + p0);
+  const int rs = V.trow_x ? 1 : 2;
+  const float4 Pv = P1[v];
+  // M edges leaving v into its M face 4t, and entering it
+  auto edges = [&](int32_t t, int32_t& out_e, int32_t& in_e) __attribute__((always_inline)) {
+    const int32_t q0 = t & ~3;
+    const int32_t tp = q0 | ((t + 3) & 3), tn = q0 | ((t + 1) & 3);
+    out_e = 4 * clampi(ci[t].x, emax) + (v > ids[tn] - vb ? 1 : 0);
+    in_e = 4 * clampi(ci[tp].x, emax) + (v > ids[tp] - vb ? 1 : 0);
+  };
+  int32_t tt[kVertexRegs], eo[kVertexRegs], ei[kVertexRegs];
+  float4 a[kVertexRegs], b[kVertexRegs];
+#pragma unroll
+  for (int i = 0; i < kVertexRegs; ++i)
+    if (i < n) tt[i] = rx[rs * i] - cb;
+#pragma unroll
+  for (int i = 0; i < kVertexRegs; ++i)
+    if (i < n) edges(tt[i], eo[i], ei[i]);
+#pragma unroll
+  for (int i = 0; i < kVertexRegs; ++i)
+    if (i < n) b[i] = P1[B.eM + ei[i]];
+  // the out-edge's point from an in-edge already loaded, as in final_vertex
+#pragma unroll
+  for (int i = 0; i < kVertexRegs; ++i)
+    if (i < n) {
+      int k = -1;
+#pragma unroll
+      for (int j = 0; j < kVertexRegs; ++j)
+        if (j < n && ei[j] == eo[i]) k = j;
+      float4 e1 = b[0];
+#pragma unroll
+      for (int j = 1; j < kVertexRegs; ++j) e1 = f4sel(k == j, b[j], e1);
+      if (k < 0) e1 = P1[B.eM + eo[i]];
+      a[i] = face_point(Pv, e1, P1[B.fM + tt[i]], b[i]);
+    }
+  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+  for (int i = 0; i < kVertexRegs; ++i)
+    if (i < n) s = f4add(s, a[i]);
+  for (int i = kVertexRegs; i < n; ++i) {
+    const int32_t t = rx[rs * i] - cb;
+    int32_t o, e;
+    edges(t, o, e);
+    s = f4add(s, face_point(Pv, P1[B.eM + o], P1[B.fM + t], P1[B.eM + e]));
+  }
+#pragma unroll
+  for (int i = 0; i < kVertexRegs; ++i)
+    if (i < n) s = f4add(s, b[i]);
+  for (int i = kVertexRegs; i < n; ++i) {
+    int32_t o, e;
+    edges(rx[rs * i] - cb, o, e);
+    s = f4add(s, P1[B.eM + e]);
+  }
+  const float nf = (float)n;
+  S.out_verts[v] = f4div(f4add(f4div(s, nf), f4mul(Pv, nf - 2.0f)), nf);
+}
+
+// Blocks of one kind each: 256 M corners, kDeepEdges N edges, 256 N vertices.
+// One mesh: groups of kDeepGroup blocks, 32 of corners, 16 of edges and 2 of
+// vertices (a closed quad mesh has 4 M corners per N corner, N edges half and
+// N vertices about a quarter of its corners), so that the kinds advance over
+// the mesh together; several meshes take their blocks from V.units.
+constexpr int kDeepEdges = kDeepEdgeUnit;
+constexpr int kDeepCornerBlocks = 32, kDeepEdgeBlocks = 16, kDeepVertexBlocks = 2;
+constexpr int kDeepGroup = kDeepCornerBlocks + kDeepEdgeBlocks + kDeepVertexBlocks;
+
+template <bool MULTI>
+__global__ void __launch_bounds__(kBlock) k_final_deep(FinalView V) {
+  const int32_t b = (int32_t)block_index<kRemapFinal>();
+  FinalSeg S;
+  int32_t first, cnt, kind;
+  if (MULTI) {
+    const int4 U = V.units[b];
+    S = V.segs[U.x];
+    S.P1 = to_global(S.P1);
+    S.out_verts = to_global(S.out_verts);
+    S.out_ids = to_global(S.out_ids);
+    first = U.y;
+    cnt = U.z;
+    kind = U.w;
+  } else {
+    S = V.one;
+    const int32_t g = b / kDeepGroup, r = b - g * kDeepGroup;
+    if (r < kDeepCornerBlocks) {
+      kind = 0;
+      first = (g * kDeepCornerBlocks + r) * kBlock;
+      cnt = min(kBlock, 4 * S.nnz - first);
+    } else if (r < kDeepCornerBlocks + kDeepEdgeBlocks) {
+      kind = 2;
+      first = (g * kDeepEdgeBlocks + (r - kDeepCornerBlocks)) * kDeepEdges;
+      cnt = min(kDeepEdges, S.ne - first);
+    } else {
+      kind = 1;
+      const int32_t u = g * kDeepVertexBlocks + (r - kDeepCornerBlocks - kDeepEdgeBlocks);
+      int32_t end = 0;
+      first = u < V.runs.blocks ? run_block(V.runs, u, end) : 0;
+      cnt = min(kBlock, end - first);
+    }
+    if (cnt <= 0) return;  // the last groups
+  }
+  if (kind == 1) {
+    if ((int)threadIdx.x < cnt) deep_vertex(V, S, first + (int32_t)threadIdx.x);
+    return;
+  }
+  __shared__ int4 stage[std::max(kStageStride * kBlock, kEdgeLds)];
+  if (kind == 2) {
+    static_assert(kEdgeIter == 4, "a quad of the row's lanes per edge of its X");
+    deep_edges(V, S, first, cnt, reinterpret_cast<float4*>(stage));
+    return;
+  }
+  Quads4 q4{};
+  // (the exchange of a wave's rows lies in the LDS that the wave's own lanes stage their quads in)
+  static_assert(4 * kRowEx <= 64 * kStageStride, "a wave's four rows in its staging area");
+  float4* const ex = reinterpret_cast<float4*>(stage) + (threadIdx.x >> 6) * 64 * kStageStride + ((threadIdx.x >> 4) & 3) * kRowEx;
+  if ((int)threadIdx.x < cnt) q4 = deep_corner(V, S, first + (int32_t)threadIdx.x, ex);
+  wave_lds_fence();  // read before the quads overwrite it
+  store_quads<MULTI>(S, q4, stage, first, cnt, 4 * S.nnz);
 }
 
 
@@ -1694,11 +2086,11 @@ __global__ void __launch_bounds__(kBlock) k_final(FinalView V, int32_t nbc, int3
 __global__ void __launch_bounds__(kBlock) k_lak_form(FinalView V) {
   for (int64_t u = block_index(); u < V.nunits; u += gridDim.x) {
     const int4 U = V.units[u];
-    if (U.w) continue;  // vertex unit
+    if (U.w) continue;  // vertex or edge unit
     const FinalSeg& Sg = V.segs[U.x];
     int32_t* const out_vals = to_global(Sg.out_vals);
     int32_t* const out_ptr = to_global(Sg.out_ptr);
-    const int32_t t0 = U.y, cnt = U.z, nnz = Sg.nnz;
+    const int32_t t0 = U.y, cnt = U.z, nnz = V.own ? 4 * Sg.nnz : Sg.nnz;  // corners of M
     const int32_t t = t0 + (int32_t)threadIdx.x;
     const int nq = 4 * cnt;
     if (out_vals) {
@@ -2143,22 +2535,44 @@ void launch_spgemm_fde(bool quad, const LevelView& L, hipStream_t st) {
     k_spgemm_fde<false><<<grid_for(L.nv), kBlock, 0, st>>>(L);
 }
 
+// block counts and ratios of vertex runs over nv vertices; one run when they
+// are not wanted or do not cover the vertices
+static void plan_runs(VertexRuns& R, bool wanted, int64_t nv) {
+  if (!wanted || R.n <= 0 || R.n > kMaxVSeg || R.first[0] != 0 || R.first[R.n] != nv) {
+    R.n = 1;
+    R.first[0] = 0;
+    R.first[1] = (int32_t)nv;
+  }
+  int64_t total = 0;
+  for (int s = 0; s < R.n; ++s) {
+    const int64_t n = (int64_t)R.first[s + 1] - R.first[s];
+    if (n < 0) throw Error(5, "vertex runs out of order");  // SLAK_ERR_INTERNAL
+    R.nb[s] = (int32_t)((n + kBlock - 1) / kBlock);
+    total += R.nb[s];
+  }
+  R.blocks = (int32_t)total;
+  for (int s = 0; s < R.n; ++s) {
+    R.ratio[s] = share_ratio(R.nb[s], total);
+    total -= R.nb[s];
+  }
+}
+
 template <bool QUAD, int SCHEME, bool ONE>
-void launch_level_t(const RefineView& R, unsigned g, int32_t nbr, int32_t nbv, hipStream_t st) {
+void launch_level_t(const RefineView& R, unsigned g, hipStream_t st) {
   const bool next = R.ntptr != nullptr, bnd = R.blk != nullptr;
   if (next) {
-    if (bnd) k_level<QUAD, SCHEME, true, true, ONE><<<g, kBlock, 0, st>>>(R, nbr, nbv);
-    else k_level<QUAD, SCHEME, true, false, ONE><<<g, kBlock, 0, st>>>(R, nbr, nbv);
+    if (bnd) k_level<QUAD, SCHEME, true, true, ONE><<<g, kBlock, 0, st>>>(R);
+    else k_level<QUAD, SCHEME, true, false, ONE><<<g, kBlock, 0, st>>>(R);
   } else {
-    if (bnd) k_level<QUAD, SCHEME, false, true, ONE><<<g, kBlock, 0, st>>>(R, nbr, nbv);
-    else k_level<QUAD, SCHEME, false, false, ONE><<<g, kBlock, 0, st>>>(R, nbr, nbv);
+    if (bnd) k_level<QUAD, SCHEME, false, true, ONE><<<g, kBlock, 0, st>>>(R);
+    else k_level<QUAD, SCHEME, false, false, ONE><<<g, kBlock, 0, st>>>(R);
   }
 }
 
 template <bool QUAD, int SCHEME>
-void launch_level_t(const RefineView& R, unsigned g, int32_t nbr, int32_t nbv, hipStream_t st) {
-  if (R.seg.n == 1) launch_level_t<QUAD, SCHEME, true>(R, g, nbr, nbv, st);
-  else launch_level_t<QUAD, SCHEME, false>(R, g, nbr, nbv, st);
+void launch_level_t(const RefineView& R, unsigned g, hipStream_t st) {
+  if (R.seg.n == 1) launch_level_t<QUAD, SCHEME, true>(R, g, st);
+  else launch_level_t<QUAD, SCHEME, false>(R, g, st);
 }
 
 void launch_level(bool quad, int scheme, const RefineView& R0, hipStream_t st) {
@@ -2167,28 +2581,18 @@ void launch_level(bool quad, int scheme, const RefineView& R0, hipStream_t st) {
     const char* e = std::getenv("SLAK_LEVEL_RUNS");
     return !e || std::atoi(e) != 0;
   }();
-  if (!runs || R.nvseg <= 0 || R.nvseg > kMaxVSeg || R.vseg[0] != 0 || R.vseg[R.nvseg] != R.nv) {
-    R.nvseg = 1;
-    R.vseg[0] = 0;
-    R.vseg[1] = R.nv;
-  }
-  const int32_t nbr = R.nnz > 0 ? (int32_t)grid_for(R.nnz) : 0;
-  int32_t nbv = 0;
-  for (int s = 0; s < R.nvseg; ++s) {
-    const int64_t n = (int64_t)R.vseg[s + 1] - R.vseg[s];
-    if (n < 0) throw Error(5, "level: vertex runs out of order");  // SLAK_ERR_INTERNAL
-    R.vnb[s] = (int32_t)((n + kBlock - 1) / kBlock);
-    nbv += R.vnb[s];
-  }
-  if (R.nv <= 0) nbv = 0;
-  if (nbr + nbv == 0) return;
-  const unsigned g = (unsigned)(nbr + nbv);
+  plan_runs(R.runs, runs, R.nv);
+  const int64_t nbr = R.nnz > 0 ? grid_for(R.nnz) : 0;
+  const int64_t T = nbr + R.runs.blocks;
+  if (T == 0) return;
+  R.vratio = share_ratio(R.runs.blocks, T);
+  const unsigned g = (unsigned)T;
   if (quad) {
-    if (scheme == kLAK) launch_level_t<true, kLAK>(R, g, nbr, nbv, st);
-    else launch_level_t<true, kSLAK>(R, g, nbr, nbv, st);
+    if (scheme == kLAK) launch_level_t<true, kLAK>(R, g, st);
+    else launch_level_t<true, kSLAK>(R, g, st);
   } else {
-    if (scheme == kLAK) launch_level_t<false, kLAK>(R, g, nbr, nbv, st);
-    else launch_level_t<false, kSLAK>(R, g, nbr, nbv, st);
+    if (scheme == kLAK) launch_level_t<false, kLAK>(R, g, st);
+    else launch_level_t<false, kSLAK>(R, g, st);
   }
 }
 
@@ -2207,33 +2611,22 @@ void launch_final(int scheme, const FinalView& V0, bool ids, hipStream_t st) {
     const char* e = std::getenv("SLAK_FINAL_RUNS");
     return !e || std::atoi(e) != 0;
   }();
-  if (multi || !runs || V.nvseg <= 0 || V.nvseg > kMaxVSeg || V.vseg[0] != 0 || V.vseg[V.nvseg] != V.nv) {
-    V.nvseg = 1;
-    V.vseg[0] = 0;
-    V.vseg[1] = (int32_t)V.nv;
-  }
-  int64_t nbv = 0;
-  for (int s = 0; s < V.nvseg; ++s) {
-    const int64_t n = (int64_t)V.vseg[s + 1] - V.vseg[s];
-    if (n < 0) throw Error(5, "final level: vertex runs out of order");  // SLAK_ERR_INTERNAL
-    V.vnb[s] = (int32_t)((n + kBlock - 1) / kBlock);
-    nbv += V.vnb[s];
-  }
-  int64_t nbc = grid_for(V.nnz);
+  plan_runs(V.runs, runs && !multi, V.nv);
+  int64_t nblocks = (int64_t)grid_for(V.nnz) + V.runs.blocks;
   if (multi) {  // one block per work unit of V.units
     if (!V.units || V.nunits <= 0) throw Error(5, "final level: no work units");  // SLAK_ERR_INTERNAL
-    nbc = V.nunits;
-    nbv = 0;
+    nblocks = V.nunits;
   }
-  if ((nbc + nbv) * kBlock > 0xffffffffll) throw Error(1, "level too large for one launch");
-  const unsigned g = (unsigned)(nbc + nbv);
+  if (nblocks * kBlock > 0xffffffffll) throw Error(1, "level too large for one launch");
+  V.vratio = share_ratio(V.runs.blocks, nblocks);
+  const unsigned g = (unsigned)nblocks;
   const bool bnd = V.blk != nullptr;
 #define SLAK_FINAL(S, B, M)                                                    \
   do {                                                                         \
     if (ids)                                                                   \
-      k_final<S, B, M, true><<<g, kBlock, 0, st>>>(V, (int32_t)nbc, (int32_t)nbv);  \
+      k_final<S, B, M, true><<<g, kBlock, 0, st>>>(V);  \
     else                                                                       \
-      k_final<S, B, M, false><<<g, kBlock, 0, st>>>(V, (int32_t)nbc, (int32_t)nbv); \
+      k_final<S, B, M, false><<<g, kBlock, 0, st>>>(V); \
   } while (0)
   if (scheme == kLAK) {
     if (multi) {
@@ -2255,6 +2648,25 @@ void launch_final(int scheme, const FinalView& V0, bool ids, hipStream_t st) {
 #undef SLAK_FINAL
 }
 
+
+void launch_final_deep(const FinalView& V0, hipStream_t st) {
+  FinalView V = V0;
+  if (!V.own || V.blk) throw Error(5, "deep final level: closed meshes with edge owners only");  // SLAK_ERR_INTERNAL
+  if (V.segs) {
+    if (!V.units || V.nunits <= 0) throw Error(5, "final level: no work units");  // SLAK_ERR_INTERNAL
+    k_final_deep<true><<<(unsigned)V.nunits, kBlock, 0, st>>>(V);
+    return;
+  }
+  const FinalSeg& S = V.one;
+  if (S.nnz <= 0 || (int64_t)S.nnz != 4 * (int64_t)S.nf || 2 * (int64_t)S.ne != S.nnz || 4ll * S.nnz > 0x7fffffff)
+    throw Error(5, "deep final level: a closed quad mesh expected");  // SLAK_ERR_INTERNAL
+  plan_runs(V.runs, true, S.nv);
+  auto groups = [](int64_t blocks, int per) { return (blocks + per - 1) / per; };
+  const int64_t g = std::max({groups(grid_for(4ll * S.nnz), kDeepCornerBlocks),
+                              groups((S.ne + kDeepEdges - 1) / kDeepEdges, kDeepEdgeBlocks),
+                              groups(V.runs.blocks, kDeepVertexBlocks)});
+  k_final_deep<false><<<(unsigned)(g * kDeepGroup), kBlock, 0, st>>>(V);
+}
 
 constexpr int64_t kLakFormBlocks = 4096;  // 16 per CU
 

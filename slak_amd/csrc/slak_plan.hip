@@ -194,7 +194,9 @@ void Plan::upload_tables(int l0, int l1, Staging& staging, bool zero_state) {
   auto table_bytes = [&](const FinalTable& T) -> size_t {
     return final_table(T) ? align(T.segs.size() * sizeof(FinalSeg)) + align(T.units.size() * sizeof(int4)) : 0;
   };
-  auto fin_bytes = [&](const LevelPlan& L) -> size_t { return table_bytes(L.fin) + table_bytes(L.pos); };
+  auto fin_bytes = [&](const LevelPlan& L) -> size_t {
+    return table_bytes(L.fin) + table_bytes(L.pos) + table_bytes(L.deep);
+  };
   // a level of one mesh is described in its launches' arguments
   auto nblocks = [](int64_t items) { return (size_t)((items + kBlockItems - 1) / kBlockItems); };
   for (int l = l0; l < l1; ++l) {
@@ -253,7 +255,7 @@ void Plan::upload_tables(int l0, int l1, Staging& staging, bool zero_state) {
       }
       o = align(o + at * sizeof(int32_t));
     }
-    for (FinalTable* T : {&L.fin, &L.pos}) {
+    for (FinalTable* T : {&L.fin, &L.pos, &L.deep}) {
       if (!final_table(*T)) continue;
       std::memcpy(staging.p + o, T->segs.data(), T->segs.size() * sizeof(FinalSeg));
       T->d_segs = reinterpret_cast<FinalSeg*>(d + o);
@@ -629,14 +631,25 @@ void Plan::prepare() {
   {
     const char* e = std::getenv("SLAK_FUSED_FINAL");
     const bool allow = !e || std::atoi(e) != 0;
-    fused_final_ = false;
+    // k_final_deep: closed LAK meshes whose mesh three levels back is a
+    // refined one (it gathers a third of what k_final does, and the level
+    // before the last two writes no structure)
+    const char* d = std::getenv("SLAK_FINAL_DEEP");
+    const char* q = std::getenv("SLAK_FUSED_POS");
+    const bool allow_deep = allow && scheme_ == kLAK && (!d || std::atoi(d) != 0) && (!q || std::atoi(q) != 0);
     for (int j : levels_[0].jobs) {
       MeshJob& J = jobs_[j];
       J.fused = allow && J.levels >= 2 && (J.levels >= 3 || levels_[0].quad);
+      J.deep = allow_deep && J.levels >= 4 && 2 * J.ne[0] == J.nnz[0];
       J.p1 = nullptr;
-      fused_final_ |= J.fused;
+      J.p2 = nullptr;
+      J.own_base = -1;
     }
   }
+  // whether level l of a mesh hands on its positions alone
+  auto positions_only = [](const MeshJob& J, int l) {
+    return (J.fused && J.levels == l + 1) || (J.deep && J.levels == l + 2);
+  };
   // one arena block for the level buffers that follow (positions and ids
   // handed on, the positions for k_final, the alternating structure, the
   // boundary flags and their scan, the tables), from the closed-form sizes
@@ -650,7 +663,7 @@ void Plan::prepare() {
       int64_t nv = 0, pad = 0, ids = 0, snv = 0, snnz = 0, ne = 0;
       for (int j : levels_[0].jobs) {
         const MeshJob& J = jobs_[j];
-        const bool to_final = J.fused && J.levels == l + 1;
+        const bool to_final = positions_only(J, l);
         if (J.levels > l) {  // positions handed on (to the union or to k_final)
           nv += J.nv[l];
           pad += 8;
@@ -688,12 +701,17 @@ void Plan::prepare() {
       int64_t vb = 0, fb = 0, cb = 0, eb = 0;
       L.fin = FinalTable{};
       L.pos = FinalTable{};
+      L.deep = FinalTable{};
       L.pos_fused = false;
       for (int j : prev.jobs) {
         MeshJob& J = jobs_[j];
         if (J.levels < l) continue;
         if (J.fused && J.levels == l) {  // formed by k_final, outside the union
           L.fin.jobs.push_back(j);
+          continue;
+        }
+        if (J.deep && J.levels == l + 1) {  // positions here, then the output, both outside the union
+          L.deep.jobs.push_back(j);
           continue;
         }
         SegDesc S{};
@@ -728,7 +746,7 @@ void Plan::prepare() {
     }
     // destinations of this level's segments; a mesh whose next level is its
     // fused last one hands on its positions only, outside the next union
-    auto to_final = [l](const MeshJob& J) { return J.fused && J.levels == l + 1; };
+    auto to_final = [&](const MeshJob& J) { return positions_only(J, l); };
     int64_t nv_next = 0, nnz_next = 0;
     for (int j : L.jobs)
       if (jobs_[j].levels > l && !to_final(jobs_[j])) {
@@ -738,6 +756,7 @@ void Plan::prepare() {
     int64_t p1_total = 0, p1_off = 0;  // one block for the positions handed to k_final
     for (int j : L.jobs)
       if (to_final(jobs_[j])) p1_total += (jobs_[j].nv[l] + 7) & ~(int64_t)7;
+    for (int j : L.deep.jobs) p1_total += (jobs_[j].nv[l] + 7) & ~(int64_t)7;
     // the first level's positions of a single mesh: the buffer the early
     // numbering has written the face points into
     float4* early = l == 1 && early_faces_ && nv_next + p1_total <= early_p1_cap_ ? early_p1_ : nullptr;
@@ -745,11 +764,12 @@ void Plan::prepare() {
     float4* Un_P = nv_next ? (early ? early : arena_.get_n<float4>(nv_next)) : nullptr;
     int32_t* Un_ids = nnz_next ? arena_.get_n<int32_t>(nnz_next) : nullptr;
     float4* p1_block = p1_total ? (early ? early : arena_.get_n<float4>(p1_total)) : nullptr;
-    int64_t vbn = 0, cbn = 0, ebn = 0;
+    int64_t vbn = 0, cbn = 0, ebn = 0, own = 0;
     for (size_t k = 0; k < L.segs.size(); ++k) {
       MeshJob& J = jobs_[L.jobs[k]];
       SegDesc& S = L.segs[k];
       S.ne = J.ne[l - 1];
+      S.next_own = -1;
       if (l == 1) S.eb = bounds[k];
       L.boundary |= 2 * J.ne[l - 1] != J.nnz[l - 1];  // n_ext = 2 n_e - nnz
       if (J.levels == l) {
@@ -763,9 +783,9 @@ void Plan::prepare() {
         S.next_eb = -1;
         S.dst_final = 1;
       } else if (to_final(J)) {
-        J.p1 = p1_block + p1_off;
+        S.dst_verts = p1_block + p1_off;
         p1_off += (J.nv[l] + 7) & ~(int64_t)7;  // 128-byte lines
-        S.dst_verts = J.p1;
+        (J.levels == l + 1 ? J.p1 : J.p2) = S.dst_verts;
         S.dst_ids = nullptr;
         S.dst_ptr = nullptr;
         S.dst_vals = nullptr;
@@ -785,8 +805,17 @@ void Plan::prepare() {
         vbn += J.nv[l];
         cbn += J.nnz[l];
         ebn += J.ne[l];
+        if (J.deep && J.levels == l + 3) {  // a multiple of 4 edges: closed refined meshes only
+          S.next_own = J.own_base = own;
+          own += J.ne[l];
+        }
       }
     }
+    for (int j : L.deep.jobs) {
+      jobs_[j].p1 = p1_block + p1_off;
+      p1_off += (jobs_[j].nv[l] + 7) & ~(int64_t)7;
+    }
+    if (own > 0) levels_[l].own = arena_.get_n<int2>(own);
     if (l == 1) L.ne = bounds[nseg];
     L.next_nv = nv_next;
     L.next_nnz = nnz_next;
@@ -860,29 +889,37 @@ void Plan::prepare() {
     LevelPlan& L = levels_[l - 1];
     const LevelPlan& M = levels_[l - 2];
     for (size_t k = 0; k < M.jobs.size(); ++k) seg_in_m[M.jobs[k]] = (int)k;
+    auto segment = [&](int j, const float4* P) -> const SegDesc& {
+      if (seg_in_m[j] < 0 || !P) throw Error(SLAK_ERR_INTERNAL, "fused level without its input");
+      return M.segs[seg_in_m[j]];
+    };
     // meshes whose last level is l
-    for (int j : L.fin.jobs) {
-      const int k = seg_in_m[j];
-      if (k < 0 || !jobs_[j].p1) throw Error(SLAK_ERR_INTERNAL, "fused level without its input");
-      add_final_seg(L.fin, M.segs[k], jobs_[j].p1, jobs_[j], true);
-    }
-    if (final_table(L.fin)) build_final_units(l, L.fin);
-    // a level whose every segment hands its positions to k_final at the next
-    // level, with a quad mesh two levels back: its positions from that mesh's
-    // structure too (positions only)
+    for (int j : L.fin.jobs) add_final_seg(L.fin, j, segment(j, jobs_[j].p1), jobs_[j].p1, jobs_[j].out_verts);
+    if (final_table(L.fin)) build_units(l, L.fin, false);
+    // a level whose every segment hands on its positions alone, with a quad
+    // mesh two levels back: its positions from that mesh's structure too
     bool pos = allow_pos && !L.segs.empty() && (l >= 3 || levels_[0].quad);
-    for (int j : L.jobs) pos = pos && jobs_[j].fused && jobs_[j].levels == l + 1 && jobs_[j].p1;
+    for (int j : L.jobs) pos = pos && positions_only(jobs_[j], l);
     if (pos) {
       L.pos_fused = true;
       for (size_t k = 0; k < L.segs.size(); ++k) {
         const int j = L.jobs[k];
-        const int km = seg_in_m[j];
-        if (km < 0) throw Error(SLAK_ERR_INTERNAL, "fused level without its input");
+        const float4* P = L.P + L.segs[k].vb;
         L.pos.jobs.push_back(j);
-        add_final_seg(L.pos, M.segs[km], L.P + L.segs[k].vb, jobs_[j], false);
+        add_final_seg(L.pos, j, segment(j, P), P, L.segs[k].dst_verts);
       }
-      if (final_table(L.pos)) build_final_units(l, L.pos);
     }
+    // meshes whose last level is l + 1, from the mesh two levels before l
+    for (int j : L.deep.jobs) {
+      MeshJob& J = jobs_[j];
+      L.pos.jobs.push_back(j);
+      add_final_seg(L.pos, j, segment(j, J.p2), J.p2, J.p1);
+      add_final_seg(L.deep, j, segment(j, J.p1), J.p1, J.out_verts);
+      if (J.own_base < 0) throw Error(SLAK_ERR_INTERNAL, "deep final level without its edge owners");
+      L.deep.segs.back().eb = J.own_base;
+    }
+    if (final_table(L.pos)) build_units(l, L.pos, false);
+    if (final_table(L.deep)) build_units(l, L.deep, true);
   }
   // a level whose meshes all come from k_final runs no refine or vertex
   // items over its structure: only k_final reads its M^T rows, and it needs
@@ -928,51 +965,47 @@ static std::vector<int64_t> vertex_classes(const MeshJob& J, int l) {
   return cls;
 }
 
-// k_final over several meshes: work units of at most one block each, mesh by
-// mesh. A mesh's corner units (consecutive corners) and the units of each of
-// its vertex classes (consecutive vertices of the class) are interleaved by
-// their relative position in their list, so that every class advances over
-// the surface together with the corner items (each class is numbered in the
-// order of the original faces) and the positions a mesh's vertex items gather
-// are still in the L2 its corner items filled.
-void Plan::build_final_units(int l, FinalTable& T) {
+// k_final (k_final_deep) over several meshes: work units of at most one block
+// each, mesh by mesh. A mesh's corner units (consecutive corners), edge units
+// (deep: consecutive edges) and the units of each of its vertex classes
+// (consecutive vertices of the class) are interleaved by their relative
+// position in their list, so that every list advances over the surface
+// together (each is numbered in the order of the original faces) and what one
+// kind gathers is still in the L2 that another has filled. The deep form's
+// corners are M's, four per corner of the N its segments describe.
+void Plan::build_units(int l, FinalTable& T, bool deep) {
   T.units.clear();
   struct Key {
     int64_t num, den;  // relative position (2j + 1) / (2 nch) of the chunk
-    int c;             // -1: corners, else the vertex class
-    int64_t j;
+    int4 unit;
   };
   std::vector<Key> keys;
   for (size_t i = 0; i < T.jobs.size(); ++i) {
-    const std::vector<int64_t> cls = vertex_classes(jobs_[T.jobs[i]], l);
-    std::vector<int64_t> off(cls.size() + 1, 0);
-    for (size_t c = 0; c < cls.size(); ++c) off[c + 1] = off[c] + cls[c];
     keys.clear();
-    const int64_t ncc = (T.segs[i].nnz + kBlockItems - 1) / kBlockItems;
-    for (int64_t j = 0; j < ncc; ++j) keys.push_back(Key{2 * j + 1, 2 * ncc, -1, j});
-    for (size_t c = 0; c < cls.size(); ++c) {
-      const int64_t nch = (cls[c] + kBlockItems - 1) / kBlockItems;
-      for (int64_t j = 0; j < nch; ++j) keys.push_back(Key{2 * j + 1, 2 * nch, (int)c, j});
+    auto list = [&](int kind, int64_t first, int64_t n, int64_t per) {
+      const int64_t nch = (n + per - 1) / per;
+      for (int64_t j = 0; j < nch; ++j)
+        keys.push_back(Key{2 * j + 1, 2 * nch,
+                           make_int4((int)i, (int)(first + j * per), (int)std::min(per, n - j * per), kind)});
+    };
+    list(0, 0, deep ? 4 * (int64_t)T.segs[i].nnz : T.segs[i].nnz, kBlockItems);
+    if (deep) list(2, 0, T.segs[i].ne, kDeepEdgeUnit);
+    int64_t first = 0;
+    for (int64_t n : vertex_classes(jobs_[T.jobs[i]], l)) {
+      list(1, first, n, kBlockItems);
+      first += n;
     }
     std::stable_sort(keys.begin(), keys.end(),
                      [](const Key& a, const Key& b) { return a.num * b.den < b.num * a.den; });
-    for (const Key& k : keys) {
-      if (k.c < 0) {
-        const int64_t c0 = k.j * kBlockItems;
-        T.units.push_back(make_int4((int)i, (int)c0, (int)std::min<int64_t>(kBlockItems, T.segs[i].nnz - c0), 0));
-      } else {
-        const int64_t first = off[k.c] + k.j * kBlockItems;
-        const int64_t count = std::min<int64_t>(kBlockItems, cls[k.c] - k.j * kBlockItems);
-        T.units.push_back(make_int4((int)i, (int)first, (int)count, 1));
-      }
-    }
+    for (const Key& k : keys) T.units.push_back(k.unit);
   }
 }
 
-// One mesh of a k_final table: m is its segment of M, P1 the positions of
-// M1. The output level writes the job's outputs (quads, LAK form,
-// positions); the level before it writes the positions handed to k_final.
-void Plan::add_final_seg(FinalTable& T, const SegDesc& m, const float4* P1, const MeshJob& J, bool output_level) {
+// One mesh of a k_final table: m is its segment of M (of N for k_final_deep),
+// P1 the positions of M1. The output level also writes the job's quads and
+// LAK form; other levels positions alone.
+void Plan::add_final_seg(FinalTable& T, int job, const SegDesc& m, const float4* P1, float4* positions) {
+  const MeshJob& J = jobs_[job];
   FinalSeg F{};
   F.cb = m.cb;
   F.vb = m.vb;
@@ -981,10 +1014,9 @@ void Plan::add_final_seg(FinalTable& T, const SegDesc& m, const float4* P1, cons
   F.nf = m.nf;
   F.ne = (int32_t)m.ne;
   F.nnz = (int32_t)m.nnz;
-  F.id_off = 0;
   F.P1 = P1;
-  F.out_verts = output_level ? J.out_verts : J.p1;
-  if (output_level) {
+  F.out_verts = positions;
+  if (positions == J.out_verts) {
     F.out_ids = J.out_ids;
     F.out_ptr = J.out_ptr;
     F.out_vals = J.out_vals;
@@ -996,6 +1028,59 @@ void Plan::add_final_seg(FinalTable& T, const SegDesc& m, const float4* P1, cons
   T.segs.push_back(F);
   T.cb.push_back(T.cb.back() + m.nnz);
   T.vb.push_back(T.vb.back() + m.nv);
+}
+
+// k_final_deep over the meshes of table T, whose last level is l + 1, from the
+// structure of their mesh two levels before l (level l - 1's union) and their
+// positions of level l: launched right after those positions, before anything
+// of level l overwrites the structure.
+void Plan::launch_deep(int l, FinalTable& T) {
+  const LevelPlan& N = levels_[l - 2];
+  FinalView V{};
+  V.ids = N.ids;
+  V.ci = N.ci;
+  V.tptr = N.tptr;
+  V.trow = N.trow;
+  V.trow_x = N.rows_x ? reinterpret_cast<const int32_t*>(N.trow) : nullptr;
+  V.own = N.own;
+  V.nnz = T.cb.back();
+  V.nv = T.vb.back();
+  const bool multi = final_table(T);
+  if (multi) {
+    V.segs = T.d_segs;
+    V.units = T.d_units;
+    V.nunits = (int32_t)T.units.size();
+    V.nseg = (int32_t)T.segs.size();
+  } else {
+    V.one = T.segs[0];
+    V.nseg = 1;
+    std::vector<int64_t> cls = vertex_classes(jobs_[T.jobs[0]], l);
+    while (cls.size() > (size_t)kMaxVSeg) {
+      cls[1] += cls[0];
+      cls.erase(cls.begin());
+    }
+    V.runs.n = (int32_t)cls.size();
+    for (size_t i = 0; i < cls.size(); ++i) V.runs.first[i + 1] = V.runs.first[i] + (int32_t)cls[i];
+  }
+  // algorithmic bytes: reads N's ids, (edge, twin) pairs, edge owners, M^T
+  // rows and offsets and the positions of M1; writes the output positions and
+  // quads (and one mesh's LAK form)
+  double bytes = 0, lak_form = 0;
+  for (int j : T.jobs) {
+    const MeshJob& J = jobs_[j];
+    const double nnz = (double)J.nnz[l - 2], nnz1 = (double)J.nnz[l];
+    bytes += 12.0 * nnz + 8.0 * (double)J.ne[l - 2] + (N.rows_x ? 4.0 : 8.0) * nnz + 4.0 * (double)J.nv[l - 2] +
+             16.0 * (double)J.nv[l] + 16.0 * ((double)J.nv[l] + (double)J.nf[l] + (double)J.ne[l]) + 16.0 * nnz1;
+    if (J.out_ptr) (multi ? lak_form : bytes) += 4.0 * (nnz1 + 1) + 16.0 * nnz1;
+  }
+  {
+    ProfScope ps(st_, "refine_vertex_final_quad", bytes);
+    launch_final_deep(V, st_);
+  }
+  if (multi && lak_form > 0) {
+    ProfScope ps(st_, "lak_form", lak_form);
+    launch_final_lak_form(V, st_);
+  }
 }
 
 // k_final over the meshes of table T at level l, from the structure of their
@@ -1031,9 +1116,9 @@ void Plan::launch_final_table(int l, FinalTable& T, bool ids, const char* stage)
       cls[1] += cls[0];
       cls.erase(cls.begin());
     }
-    V.nvseg = (int32_t)cls.size();
-    V.vseg[0] = 0;
-    for (size_t i = 0; i < cls.size(); ++i) V.vseg[i + 1] = V.vseg[i] + (int32_t)cls[i];
+    V.runs.n = (int32_t)cls.size();
+    V.runs.first[0] = 0;
+    for (size_t i = 0; i < cls.size(); ++i) V.runs.first[i + 1] = V.runs.first[i] + (int32_t)cls[i];
   }
   // algorithmic bytes: reads the ids, (edge, twin) pairs, M^T rows and
   // offsets of M (boundary scan, SLAK positions) and the positions of M1;
@@ -1068,7 +1153,8 @@ void Plan::record_level(int l) {
   LevelPlan& L = levels_[l - 1];
   if (l > 1) {
     launch_final_table(l, L.fin, true, "refine_vertex_final_quad");
-    if (L.pos_fused) launch_final_table(l, L.pos, false, "refine_vertex_pos_quad");
+    launch_final_table(l, L.pos, false, "refine_vertex_pos_quad");
+    if (!L.deep.empty()) launch_deep(l, L.deep);
   }
   if (L.segs.empty()) return;  // every mesh of the level was fused
   const double poly_b = L.quad ? 0.0 : 4.0 * (L.nf + 1) + 4.0 * L.nnz;
@@ -1111,6 +1197,7 @@ void Plan::record_level(int l) {
   R.nci = L.nci;
   R.nbnd = L.nbnd;
   R.nmpos = L.nmpos;
+  R.nown = l < (int)levels_.size() ? levels_[l].own : nullptr;
   R.next_nv = (int32_t)L.next_nv;
   R.next_nnz = (int32_t)L.next_nnz;
   R.next_rows_x = l < (int)levels_.size() && levels_[l].rows_x ? 1 : 0;
@@ -1122,9 +1209,9 @@ void Plan::record_level(int l) {
       cls[1] += cls[0];
       cls.erase(cls.begin());
     }
-    R.nvseg = (int32_t)cls.size();
-    R.vseg[0] = 0;
-    for (size_t i = 0; i < cls.size(); ++i) R.vseg[i + 1] = R.vseg[i] + (int32_t)cls[i];
+    R.runs.n = (int32_t)cls.size();
+    R.runs.first[0] = 0;
+    for (size_t i = 0; i < cls.size(); ++i) R.runs.first[i + 1] = R.runs.first[i] + (int32_t)cls[i];
   }
   const bool next = L.ntptr != nullptr;
   {
@@ -1145,6 +1232,7 @@ void Plan::record_level(int l) {
         writes += (R.next_rows_x ? 48.0 : 64.0) * snnz + 4.0 * ((double)S.nv + (double)S.nf + sne) + (L.nbnd ? 4.0 * (snnz + 2.0 * sne) : 0.0) +
                   (scheme_ == kSLAK ? 16.0 * snnz : 0.0);
         if (scheme_ == kSLAK) reads += 4.0 * snnz;
+        if (S.next_own >= 0) writes += 32.0 * sne;
       }
     }
     ProfScope ps(st_, L.quad ? "refine_vertex_quad" : "refine_vertex_poly", reads + writes);

@@ -40,6 +40,12 @@ struct MeshJob {
   // p1: the positions of the level before the output (its only output)
   bool fused = false;
   float4* p1 = nullptr;
+  // ... or by k_final_deep from the quad mesh three levels back (closed LAK
+  // meshes of four levels or more): then the level before those two writes
+  // positions only too, to p2; own_base: the mesh's edge owners
+  bool deep = false;
+  float4* p2 = nullptr;
+  int64_t own_base = -1;
 };
 
 // Meshes whose level is formed by k_final from the structure of their mesh M
@@ -97,6 +103,10 @@ struct LevelPlan {
   // meshes whose last level is this one, formed by k_final (output quads,
   // LAK form, positions); they are not segments of this level's union
   FinalTable fin;
+  // meshes whose last level is the next one, formed by k_final_deep right
+  // after their positions of this level (in `pos`)
+  FinalTable deep;
+  int2* own = nullptr;  // edge owners of this level's meshes that k_final_deep starts from
   // every segment of this level hands its positions to k_final at the next
   // level: they are formed here by k_final's positions-only variant, and
   // this level launches no face points and no refine or vertex items
@@ -213,16 +223,13 @@ class Plan {
   hipStream_t capture_st_ = nullptr;  // stream the graph is captured on and replayed
   hipStream_t owned_st_ = nullptr;    // created when the caller's stream is the default one
   hipEvent_t order_ev_ = nullptr;
-  // some mesh refined two or more levels with a quad mesh two levels before
-  // its output: its last level is computed from that mesh's structure
-  // (k_final) and the level before it writes positions only
-  bool fused_final_ = false;
   // k_final's meshes come from a device table and work units (several meshes)
   bool force_final_table_ = false;
   bool final_table(const FinalTable& T) const { return T.segs.size() > 1 || (force_final_table_ && !T.empty()); }
-  void add_final_seg(FinalTable& T, const SegDesc& m, const float4* P1, const MeshJob& J, bool output_level);
+  void add_final_seg(FinalTable& T, int job, const SegDesc& m, const float4* P1, float4* positions);
   void launch_final_table(int l, FinalTable& T, bool ids, const char* stage);
-  void build_final_units(int l, FinalTable& T);
+  void launch_deep(int l, FinalTable& T);
+  void build_units(int l, FinalTable& T, bool deep);
   // single mesh: the first level's edge numbering ran during the analysis
   // read-back (the level then launches its face points only)
   bool number_early_ = false;
