@@ -592,7 +592,7 @@ struct RefineView {
 // two levels before the output and the positions of its refinement M1 (whose
 // structure is never written): M's bases in the union arrays of its level,
 // its sizes, its M1 positions and its outputs.
-struct FinalSeg {
+struct FinalMesh {
   int64_t cb, vb, eb;    // union bases of M's corners, vertices, edges
   int32_t nv, nf, ne;    // M sizes
   int32_t nnz;
@@ -601,6 +601,21 @@ struct FinalSeg {
   int32_t* out_ids;      // output quads: 4 per M1 corner, 16 per M corner
   int32_t* out_ptr;      // LAK form of the output (ptr[i] = 4i, vals cyclic 1..4), or null
   int32_t* out_vals;
+};
+
+// The mesh and its blocks of a launch: corner blocks, (k_final_deep) edge
+// blocks and vertex blocks in runs of one vertex class each, all spread over
+// the mesh's blocks in proportion, so that every list advances over the
+// surface together (each is numbered in the order of the original faces) and
+// what one kind gathers is still in the L2 that another has filled.
+struct FinalSeg {
+  FinalMesh m;
+  int32_t block0;        // its first block, and its first block of the LAK form's launch
+  int32_t lak0;
+  int32_t blocks;
+  uint64_t vratio;       // share of the vertex blocks, of the edge blocks among the others
+  uint64_t eratio;
+  VertexRuns runs;
 };
 
 struct FinalView {
@@ -614,21 +629,12 @@ struct FinalView {
   const int32_t* mpos;   // M^T position per corner (SLAK)
   const int2* own;       // k_final_deep, whose union and meshes are those of N, three levels before
                          // the output: (owner corner, twin) per edge, from base eb of each mesh
-  FinalSeg one;          // a single mesh (nseg == 1, no table)
-  const FinalSeg* segs;  // several meshes: device table
-  // several meshes: work units of one block each, (mesh, first mesh-local
-  // item, count, kind): kind 0 consecutive corners of one mesh, kind 1
-  // consecutive vertices of one class of one mesh, kind 2 consecutive edges
-  // (k_final_deep). Mesh by mesh, the corner
-  // units and every vertex class's units are interleaved by their relative
-  // position, so a mesh's vertex items run beside its corner items.
-  const int4* units;
-  int32_t nunits;
-  int32_t nseg;
-  int64_t nnz, nv;       // corner and vertex items of the launch
-  // the vertex items' runs (n 0: one run) and their share of the launch
-  VertexRuns runs;
-  uint64_t vratio;
+  FinalSeg one;          // a single mesh
+  const FinalSeg* segs;  // several meshes: device table, and the mesh of every block
+  const int32_t* block_seg;
+  const int32_t* lak_seg;
+  int32_t nblocks;       // several meshes: blocks of the launch, of the LAK form's launch
+  int32_t nlak;
 };
 
 // Face, successor and predecessor corner of corner t (quad: bit arithmetic;

@@ -84,6 +84,9 @@ void launch_spgemm_fde(bool quad, const LevelView& L, hipStream_t st);
 // refine (per corner) and vertex (per vertex) items of a level in one launch;
 // the refine items also write the LAK form of the segments with dst_ptr set
 void launch_level(bool quad, int scheme, const RefineView& R, hipStream_t st);
+// blocks of a mesh in a launch of k_final (of k_final_deep) and how they are
+// shared out (S.blocks, ratios, runs: runs.first holds its vertex classes)
+int64_t plan_final_blocks(FinalSeg& S, bool deep);
 // last level of one mesh or several (V.segs) from the quad mesh two levels
 // back; ids: also the output quads and LAK form (false: positions only)
 void launch_final(int scheme, const FinalView& V, bool ids, hipStream_t st);
@@ -91,7 +94,7 @@ void launch_final(int scheme, const FinalView& V, bool ids, hipStream_t st);
 // three levels back, whose structure V holds, and the positions of the level
 // before the output
 void launch_final_deep(const FinalView& V, hipStream_t st);
-constexpr int kDeepEdgeUnit = 64;  // edges per work unit of the several-mesh form
+constexpr int kDeepEdgeUnit = 64;  // edges per block
 // the LAK form (ptr, vals) of a several-mesh output level, after its k_final
 // launch (which leaves it out)
 void launch_final_lak_form(const FinalView& V, hipStream_t st);

@@ -1293,7 +1293,7 @@ struct Quads4 {
 // Corner t (mesh-local) of M in mesh S: returns its 16 output ids (IDS),
 // which the block stages in LDS.
 template <int SCHEME, bool BND, bool IDS, bool EARLY>
-__device__ __forceinline__ Quads4 final_corner(const FinalView& V, const FinalSeg& S, int32_t t) {
+__device__ __forceinline__ Quads4 final_corner(const FinalView& V, const FinalMesh& S, int32_t t) {
   // every lane of a quad runs (nnz = 4 nf, meshes and blocks hold whole quads)
   const int64_t cb = S.cb;
   const int32_t vb = (int32_t)S.vb;
@@ -1493,7 +1493,7 @@ __device__ __forceinline__ Quads4 final_corner(const FinalView& V, const FinalSe
 // of ep(e1(t)) across every boundary out-edge and of ep(e0(t)) across every
 // boundary in-edge
 template <int SCHEME, bool BND>
-__device__ __forceinline__ void final_vertex(const FinalView& V, const FinalSeg& S, int32_t v) {
+__device__ __forceinline__ void final_vertex(const FinalView& V, const FinalMesh& S, int32_t v) {
   const int32_t cb = (int32_t)S.cb;
   const int32_t ep0 = S.nv + S.nf;
   const int32_t emax = S.ne > 0 ? S.ne - 1 : 0;
@@ -1586,7 +1586,7 @@ __device__ __forceinline__ void final_vertex(const FinalView& V, const FinalSeg&
 // staged in LDS and stored with consecutive lanes on consecutive 16-byte
 // pieces; one mesh: their LAK form too.
 template <bool MULTI>
-__device__ __forceinline__ void store_quads(const FinalSeg& S, const Quads4& q4, int4* stage, int32_t t0, int32_t cnt,
+__device__ __forceinline__ void store_quads(const FinalMesh& S, const Quads4& q4, int4* stage, int32_t t0, int32_t cnt,
                                             int32_t nnz) {
   const int32_t t = t0 + (int32_t)threadIdx.x;
   if ((int)threadIdx.x < cnt) {
@@ -1628,47 +1628,37 @@ __device__ __forceinline__ void store_quads(const FinalSeg& S, const Quads4& q4,
   }
 }
 
-// Corner items and vertex items interleaved in proportion, as in k_level.
-// The vertex blocks are split the same way between the runs of V.runs (run s
-// against the runs after it): the vertex classes of M (the original vertices,
-// then the face points and edge points of every earlier level), each numbered
-// in the order of the original faces it descends from, so that every run
-// advances over the same part of the surface as the corner blocks and the
-// positions they gather are fetched once for both. Several meshes take their
-// blocks from V.units, which interleaves each mesh's corner and vertex units
-// the same way. A corner block stages its 16 KB of output quads in LDS and
-// stores them with consecutive lanes on consecutive 16-byte pieces.
+// the mesh of this block (block-uniform) and its descriptor
+template <bool MULTI>
+__device__ __forceinline__ FinalMesh block_mesh(const FinalView& V, const FinalSeg*& seg) {
+  if (!MULTI) {
+    seg = &V.one;
+    return V.one.m;
+  }
+  seg = V.segs + V.block_seg[block_index<kRemapFinal>()];
+  FinalMesh S = seg->m;
+  S.P1 = to_global(S.P1);
+  S.out_verts = to_global(S.out_verts);
+  S.out_ids = to_global(S.out_ids);
+  return S;
+}
+
+// Corner and vertex blocks interleaved (FinalSeg). A corner block stages its
+// 16 KB of output quads in LDS and stores them with consecutive lanes on
+// consecutive 16-byte pieces.
 template <int SCHEME, bool BND, bool MULTI, bool IDS>
 __global__ void __launch_bounds__(kBlock) k_final(FinalView V) {
-  const int32_t b = (int32_t)block_index<kRemapFinal>();
-  FinalSeg S;
-  int32_t t0, cnt;
-  if (MULTI) {  // work unit b (block-uniform): corners or vertices of one mesh
-    const int4 U = V.units[b];
-    S = V.segs[U.x];
-    S.P1 = to_global(S.P1);
-    S.out_verts = to_global(S.out_verts);
-    S.out_ids = to_global(S.out_ids);
-    S.out_ptr = to_global(S.out_ptr);
-    S.out_vals = to_global(S.out_vals);
-    if (U.w) {
-      if ((int)threadIdx.x < U.z) final_vertex<SCHEME, BND>(V, S, U.y + (int32_t)threadIdx.x);
-      return;
-    }
-    t0 = U.y;
-    cnt = U.z;
-  } else {
-    const int32_t before = share_of(b, V.vratio), after = share_of(b + 1, V.vratio);
-    if (after > before) {
-      int32_t end;
-      const int32_t v = run_block(V.runs, before, end) + (int32_t)threadIdx.x;
-      if (v < end) final_vertex<SCHEME, BND>(V, V.one, v);
-      return;
-    }
-    S = V.one;
-    t0 = (b - before) * kBlock;
-    cnt = (int32_t)min((int64_t)kBlock, V.nnz - t0);
+  const FinalSeg* seg;
+  const FinalMesh S = block_mesh<MULTI>(V, seg);
+  const int32_t b = (int32_t)block_index<kRemapFinal>() - (MULTI ? seg->block0 : 0);
+  const int32_t before = share_of(b, seg->vratio), after = share_of(b + 1, seg->vratio);
+  if (after > before) {
+    int32_t end;
+    const int32_t v = run_block(seg->runs, before, end) + (int32_t)threadIdx.x;
+    if (v < end) final_vertex<SCHEME, BND>(V, S, v);
+    return;
   }
+  const int32_t t0 = (b - before) * kBlock, cnt = min(kBlock, S.nnz - t0);
   const int32_t t = t0 + (int32_t)threadIdx.x;
   if (!IDS) {  // positions only
     if ((int)threadIdx.x < cnt) final_corner<SCHEME, BND, false, MULTI>(V, S, t);
@@ -1725,7 +1715,7 @@ struct DeepBase {
   int32_t eM;    // M1 vertex ep(M edge 0)
   int32_t fM1;   // output vertex fp(M1 face 0) = M1 vertices
   int32_t eM1;   // output vertex ep(M1 edge 0)
-  __device__ __forceinline__ explicit DeepBase(const FinalSeg& S) {
+  __device__ __forceinline__ explicit DeepBase(const FinalMesh& S) {
     epN = S.nv + S.nf;
     fM = epN + S.ne;
     eM = fM + S.nnz;
@@ -1754,7 +1744,7 @@ __device__ __forceinline__ void wave_lds_fence() {
 // float4. Returns the 16 output ids of M corner c.
 constexpr int kRowEx = 65;  // loaded 0-31, M1 face points 32-47, out-edge points 48-63, one pad
 
-__device__ __forceinline__ Quads4 deep_corner(const FinalView& V, const FinalSeg& S, int32_t c, float4* ex) {
+__device__ __forceinline__ Quads4 deep_corner(const FinalView& V, const FinalMesh& S, int32_t c, float4* ex) {
   const DeepBase B(S);
   const int i = threadIdx.x & 15, k = i & 3, j = i >> 2, jp = (j + 3) & 3;
   const int32_t t = c >> 2, f = c >> 4, q0 = t & ~3;
@@ -1854,7 +1844,7 @@ constexpr int kRowE = 33;                   // float4 of a row: p 0-15, psi 16-3
 constexpr int kRowX = 9 * kEdgeIter + 1;    // per edge: psi_1 and Y of j = 0 .. 3, X
 constexpr int kEdgeLds = (kRowE + kRowX) * kRows;  // float4
 
-__device__ __forceinline__ void deep_edges(const FinalView& V, const FinalSeg& S, int32_t first, int32_t cnt,
+__device__ __forceinline__ void deep_edges(const FinalView& V, const FinalMesh& S, int32_t first, int32_t cnt,
                                            float4* lds) {
   const DeepBase B(S);
   const int32_t cb = (int32_t)S.cb, vb = (int32_t)S.vb, emax = S.ne > 0 ? S.ne - 1 : 0;
@@ -1947,7 +1937,7 @@ __device__ __forceinline__ void deep_edges(const FinalView& V, const FinalSeg& S
 
 // vertex point of a vertex v of N in the output: M corners 4t of its row's
 // corners t, M1 faces (v, ep(4e1 + (v > w)), fp(M face t), ep(4e0 + (v > u)))
-__device__ __forceinline__ void deep_vertex(const FinalView& V, const FinalSeg& S, int32_t v) {
+__device__ __forceinline__ void deep_vertex(const FinalView& V, const FinalMesh& S, int32_t v) {
   const DeepBase B(S);
   const int32_t cb = (int32_t)S.cb, vb = (int32_t)S.vb;
   const int32_t emax = S.ne > 0 ? S.ne - 1 : 0;
@@ -2013,59 +2003,29 @@ __device__ __forceinline__ void deep_vertex(const FinalView& V, const FinalSeg& 
   S.out_verts[v] = f4div(f4add(f4div(s, nf), f4mul(Pv, nf - 2.0f)), nf);
 }
 
-// Blocks of one kind each: 256 M corners, kDeepEdges N edges, 256 N vertices.
-// One mesh: groups of kDeepGroup blocks, 32 of corners, 16 of edges and 2 of
-// vertices (a closed quad mesh has 4 M corners per N corner, N edges half and
-// N vertices about a quarter of its corners), so that the kinds advance over
-// the mesh together; several meshes take their blocks from V.units.
-constexpr int kDeepEdges = kDeepEdgeUnit;
-constexpr int kDeepCornerBlocks = 32, kDeepEdgeBlocks = 16, kDeepVertexBlocks = 2;
-constexpr int kDeepGroup = kDeepCornerBlocks + kDeepEdgeBlocks + kDeepVertexBlocks;
-
+// Blocks of one kind each: 256 M corners, kDeepEdgeUnit N edges, 256 N vertices
+// (FinalSeg).
 template <bool MULTI>
 __global__ void __launch_bounds__(kBlock) k_final_deep(FinalView V) {
-  const int32_t b = (int32_t)block_index<kRemapFinal>();
-  FinalSeg S;
-  int32_t first, cnt, kind;
-  if (MULTI) {
-    const int4 U = V.units[b];
-    S = V.segs[U.x];
-    S.P1 = to_global(S.P1);
-    S.out_verts = to_global(S.out_verts);
-    S.out_ids = to_global(S.out_ids);
-    first = U.y;
-    cnt = U.z;
-    kind = U.w;
-  } else {
-    S = V.one;
-    const int32_t g = b / kDeepGroup, r = b - g * kDeepGroup;
-    if (r < kDeepCornerBlocks) {
-      kind = 0;
-      first = (g * kDeepCornerBlocks + r) * kBlock;
-      cnt = min(kBlock, 4 * S.nnz - first);
-    } else if (r < kDeepCornerBlocks + kDeepEdgeBlocks) {
-      kind = 2;
-      first = (g * kDeepEdgeBlocks + (r - kDeepCornerBlocks)) * kDeepEdges;
-      cnt = min(kDeepEdges, S.ne - first);
-    } else {
-      kind = 1;
-      const int32_t u = g * kDeepVertexBlocks + (r - kDeepCornerBlocks - kDeepEdgeBlocks);
-      int32_t end = 0;
-      first = u < V.runs.blocks ? run_block(V.runs, u, end) : 0;
-      cnt = min(kBlock, end - first);
-    }
-    if (cnt <= 0) return;  // the last groups
-  }
-  if (kind == 1) {
-    if ((int)threadIdx.x < cnt) deep_vertex(V, S, first + (int32_t)threadIdx.x);
+  const FinalSeg* seg;
+  const FinalMesh S = block_mesh<MULTI>(V, seg);
+  const int32_t b = (int32_t)block_index<kRemapFinal>() - (MULTI ? seg->block0 : 0);
+  const int32_t before = share_of(b, seg->vratio), after = share_of(b + 1, seg->vratio);
+  if (after > before) {
+    int32_t end;
+    const int32_t v = run_block(seg->runs, before, end) + (int32_t)threadIdx.x;
+    if (v < end) deep_vertex(V, S, v);
     return;
   }
+  const int32_t b1 = b - before, edges = share_of(b1, seg->eratio);
   __shared__ int4 stage[std::max(kStageStride * kBlock, kEdgeLds)];
-  if (kind == 2) {
+  if (share_of(b1 + 1, seg->eratio) > edges) {
     static_assert(kEdgeIter == 4, "a quad of the row's lanes per edge of its X");
-    deep_edges(V, S, first, cnt, reinterpret_cast<float4*>(stage));
+    const int32_t first = edges * kDeepEdgeUnit;
+    deep_edges(V, S, first, min(kDeepEdgeUnit, S.ne - first), reinterpret_cast<float4*>(stage));
     return;
   }
+  const int32_t first = (b1 - edges) * kBlock, cnt = min(kBlock, 4 * S.nnz - first);
   Quads4 q4{};
   // (the exchange of a wave's rows lies in the LDS that the wave's own lanes stage their quads in)
   static_assert(4 * kRowEx <= 64 * kStageStride, "a wave's four rows in its staging area");
@@ -2077,34 +2037,32 @@ __global__ void __launch_bounds__(kBlock) k_final_deep(FinalView V) {
 
 
 // The LAK form of the output quads of a multi-mesh k_final launch
-// (createQuadColPtr / createQuadVals, LAKCatmullClarkKernels.cuh:396-431),
-// from the same corner units: a block writes the 1024 quads of its unit's
-// 256 corners, vals as int4 (1, 2, 3, 4), ptr as int4 16t + (0, 4, 8, 12).
-// A pure streaming write, apart from the gathers and scattered stores of
-// k_final; each block takes every gridDim.x-th unit (a block per unit spends
-// more on dispatch than on its 20 KB of stores).
+// (createQuadColPtr / createQuadVals, LAKCatmullClarkKernels.cuh:396-431): a
+// block writes the 1024 quads of 256 of its mesh's M corners, vals as int4
+// (1, 2, 3, 4), ptr as int4 16t + (0, 4, 8, 12). A pure streaming write, apart
+// from the gathers and scattered stores of k_final. XCD-chunked block order:
+// a fill of five 16-byte stores a thread reaches 6.6 TB/s that way, 5.8 to 6.2
+// with the blocks dealt round.
 __global__ void __launch_bounds__(kBlock) k_lak_form(FinalView V) {
-  for (int64_t u = block_index(); u < V.nunits; u += gridDim.x) {
-    const int4 U = V.units[u];
-    if (U.w) continue;  // vertex or edge unit
-    const FinalSeg& Sg = V.segs[U.x];
-    int32_t* const out_vals = to_global(Sg.out_vals);
-    int32_t* const out_ptr = to_global(Sg.out_ptr);
-    const int32_t t0 = U.y, cnt = U.z, nnz = V.own ? 4 * Sg.nnz : Sg.nnz;  // corners of M
-    const int32_t t = t0 + (int32_t)threadIdx.x;
-    const int nq = 4 * cnt;
-    if (out_vals) {
-      int32_t* __restrict__ vals = out_vals + 16 * (int64_t)t0;
+  const int32_t b = (int32_t)block_index<kRemapFinal>();
+  const FinalSeg& seg = V.segs[V.lak_seg[b]];
+  int32_t* const out_vals = to_global(seg.m.out_vals);
+  int32_t* const out_ptr = to_global(seg.m.out_ptr);
+  const int32_t nnz = V.own ? 4 * seg.m.nnz : seg.m.nnz;  // corners of M
+  const int32_t t0 = (b - seg.lak0) * kBlock, cnt = min(kBlock, nnz - t0);
+  const int32_t t = t0 + (int32_t)threadIdx.x;
+  const int nq = 4 * cnt;
+  if (out_vals) {
+    int32_t* __restrict__ vals = out_vals + 16 * (int64_t)t0;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int i = j * kBlock + threadIdx.x;
-        if (i < nq) store_nt(vals + 4 * i, 1, 2, 3, 4);
-      }
+    for (int j = 0; j < 4; ++j) {
+      const int i = j * kBlock + threadIdx.x;
+      if (i < nq) store_nt(vals + 4 * i, 1, 2, 3, 4);
     }
-    if (out_ptr) {
-      if ((int)threadIdx.x < cnt) store_nt(out_ptr + 4 * (int64_t)t, 16 * t, 16 * t + 4, 16 * t + 8, 16 * t + 12);
-      if (t == nnz - 1) store_nt(out_ptr + 4 * (int64_t)nnz, 16 * nnz);
-    }
+  }
+  if (out_ptr) {
+    if ((int)threadIdx.x < cnt) store_nt(out_ptr + 4 * (int64_t)t, 16 * t, 16 * t + 4, 16 * t + 8, 16 * t + 12);
+    if (t == nnz - 1) store_nt(out_ptr + 4 * (int64_t)nnz, 16 * nnz);
   }
 }
 
@@ -2596,30 +2554,39 @@ void launch_level(bool quad, int scheme, const RefineView& R0, hipStream_t st) {
   }
 }
 
-void launch_final(int scheme, const FinalView& V0, bool ids, hipStream_t st) {
-  FinalView V = V0;
-  const bool multi = V.segs != nullptr;
-  if (!multi) {
-    if (V.one.nnz <= 0 || (V.one.nnz & 3) || (int64_t)V.one.nnz != 4 * (int64_t)V.one.nf)
-      throw Error(5, "final level: the mesh two levels back must be quads");  // SLAK_ERR_INTERNAL
-    V.nnz = V.one.nnz;
-    V.nv = V.one.nv;
-  }
-  if (V.nnz <= 0) return;
-  if (V.nv > 0x7fffffffll) throw Error(1, "level too large for one launch");
+int64_t plan_final_blocks(FinalSeg& S, bool deep) {
   static const bool runs = [] {  // SLAK_FINAL_RUNS=0: vertex items in plain order
     const char* e = std::getenv("SLAK_FINAL_RUNS");
     return !e || std::atoi(e) != 0;
   }();
-  plan_runs(V.runs, runs && !multi, V.nv);
-  int64_t nblocks = (int64_t)grid_for(V.nnz) + V.runs.blocks;
-  if (multi) {  // one block per work unit of V.units
-    if (!V.units || V.nunits <= 0) throw Error(5, "final level: no work units");  // SLAK_ERR_INTERNAL
-    nblocks = V.nunits;
-  }
-  if (nblocks * kBlock > 0xffffffffll) throw Error(1, "level too large for one launch");
-  V.vratio = share_ratio(V.runs.blocks, nblocks);
-  const unsigned g = (unsigned)nblocks;
+  const FinalMesh& m = S.m;
+  if ((int64_t)m.nnz != 4 * (int64_t)m.nf)
+    throw Error(5, "final level: the mesh it starts from must be quads");  // SLAK_ERR_INTERNAL
+  if (deep && (2 * (int64_t)m.ne != m.nnz || 4ll * m.nnz > 0x7fffffff))
+    throw Error(5, "deep final level: a closed mesh expected");  // SLAK_ERR_INTERNAL
+  plan_runs(S.runs, runs, m.nv);
+  const int64_t corners = m.nnz > 0 ? grid_for((deep ? 4ll : 1ll) * m.nnz) : 0;  // (a mesh without faces)
+  const int64_t edges = deep ? ((int64_t)m.ne + kDeepEdgeUnit - 1) / kDeepEdgeUnit : 0;
+  const int64_t total = corners + edges + S.runs.blocks;
+  S.blocks = (int32_t)total;
+  S.vratio = share_ratio(S.runs.blocks, total);
+  S.eratio = share_ratio(edges, corners + edges);
+  return total;
+}
+
+// blocks of a launch of V's meshes (0: several meshes, all without faces)
+static unsigned final_grid(const FinalView& V) {
+  if (V.segs ? !V.block_seg : V.one.m.nnz <= 0)
+    throw Error(5, "final level: no blocks planned");  // SLAK_ERR_INTERNAL
+  const int64_t n = V.segs ? V.nblocks : V.one.blocks;
+  if (n * kBlock > 0xffffffffll) throw Error(1, "level too large for one launch");
+  return (unsigned)n;
+}
+
+void launch_final(int scheme, const FinalView& V, bool ids, hipStream_t st) {
+  const unsigned g = final_grid(V);
+  if (g == 0) return;
+  const bool multi = V.segs != nullptr;
   const bool bnd = V.blk != nullptr;
 #define SLAK_FINAL(S, B, M)                                                    \
   do {                                                                         \
@@ -2649,30 +2616,20 @@ void launch_final(int scheme, const FinalView& V0, bool ids, hipStream_t st) {
 }
 
 
-void launch_final_deep(const FinalView& V0, hipStream_t st) {
-  FinalView V = V0;
+void launch_final_deep(const FinalView& V, hipStream_t st) {
   if (!V.own || V.blk) throw Error(5, "deep final level: closed meshes with edge owners only");  // SLAK_ERR_INTERNAL
-  if (V.segs) {
-    if (!V.units || V.nunits <= 0) throw Error(5, "final level: no work units");  // SLAK_ERR_INTERNAL
-    k_final_deep<true><<<(unsigned)V.nunits, kBlock, 0, st>>>(V);
-    return;
-  }
-  const FinalSeg& S = V.one;
-  if (S.nnz <= 0 || (int64_t)S.nnz != 4 * (int64_t)S.nf || 2 * (int64_t)S.ne != S.nnz || 4ll * S.nnz > 0x7fffffff)
-    throw Error(5, "deep final level: a closed quad mesh expected");  // SLAK_ERR_INTERNAL
-  plan_runs(V.runs, true, S.nv);
-  auto groups = [](int64_t blocks, int per) { return (blocks + per - 1) / per; };
-  const int64_t g = std::max({groups(grid_for(4ll * S.nnz), kDeepCornerBlocks),
-                              groups((S.ne + kDeepEdges - 1) / kDeepEdges, kDeepEdgeBlocks),
-                              groups(V.runs.blocks, kDeepVertexBlocks)});
-  k_final_deep<false><<<(unsigned)(g * kDeepGroup), kBlock, 0, st>>>(V);
+  const unsigned g = final_grid(V);
+  if (g == 0) return;
+  if (V.segs)
+    k_final_deep<true><<<g, kBlock, 0, st>>>(V);
+  else
+    k_final_deep<false><<<g, kBlock, 0, st>>>(V);
 }
 
-constexpr int64_t kLakFormBlocks = 4096;  // 16 per CU
-
 void launch_final_lak_form(const FinalView& V, hipStream_t st) {
-  if (!V.segs || !V.units || V.nunits <= 0) throw Error(5, "final level: no work units");  // SLAK_ERR_INTERNAL
-  k_lak_form<<<(unsigned)std::min<int64_t>(V.nunits, kLakFormBlocks), kBlock, 0, st>>>(V);
+  if (!V.segs || !V.lak_seg) throw Error(5, "final level: no blocks planned");  // SLAK_ERR_INTERNAL
+  if (V.nlak <= 0) return;
+  k_lak_form<<<(unsigned)V.nlak, kBlock, 0, st>>>(V);
 }
 
 void launch_sort_faces(bool by_vals, const int32_t* ptr, int32_t stride, int32_t nf, int64_t nnz, int32_t* ids,

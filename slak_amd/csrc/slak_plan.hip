@@ -192,7 +192,9 @@ void Plan::upload_tables(int l0, int l1, Staging& staging, bool zero_state) {
   std::vector<size_t> offs;
   // k_final tables of several meshes: FinalSeg[n], corner and vertex item bases
   auto table_bytes = [&](const FinalTable& T) -> size_t {
-    return final_table(T) ? align(T.segs.size() * sizeof(FinalSeg)) + align(T.units.size() * sizeof(int4)) : 0;
+    return final_table(T) ? align(T.segs.size() * sizeof(FinalSeg)) +
+                                align((T.block_seg.size() + T.lak_seg.size()) * sizeof(int32_t))
+                          : 0;
   };
   auto fin_bytes = [&](const LevelPlan& L) -> size_t {
     return table_bytes(L.fin) + table_bytes(L.pos) + table_bytes(L.deep);
@@ -260,9 +262,12 @@ void Plan::upload_tables(int l0, int l1, Staging& staging, bool zero_state) {
       std::memcpy(staging.p + o, T->segs.data(), T->segs.size() * sizeof(FinalSeg));
       T->d_segs = reinterpret_cast<FinalSeg*>(d + o);
       o = align(o + T->segs.size() * sizeof(FinalSeg));
-      std::memcpy(staging.p + o, T->units.data(), T->units.size() * sizeof(int4));
-      T->d_units = reinterpret_cast<int4*>(d + o);
-      o = align(o + T->units.size() * sizeof(int4));
+      const size_t nb = T->block_seg.size() * sizeof(int32_t), nl = T->lak_seg.size() * sizeof(int32_t);
+      std::memcpy(staging.p + o, T->block_seg.data(), nb);
+      T->d_block_seg = reinterpret_cast<int32_t*>(d + o);
+      std::memcpy(staging.p + o + nb, T->lak_seg.data(), nl);
+      T->d_lak_seg = reinterpret_cast<int32_t*>(d + o + nb);
+      o = align(o + nb + nl);
     }
   }
   launch_setup(staging.p, d, (int64_t)total, zero_state ? d_state_ : nullptr, zero_state ? n_state_ : 0, st_);
@@ -894,8 +899,8 @@ void Plan::prepare() {
       return M.segs[seg_in_m[j]];
     };
     // meshes whose last level is l
-    for (int j : L.fin.jobs) add_final_seg(L.fin, j, segment(j, jobs_[j].p1), jobs_[j].p1, jobs_[j].out_verts);
-    if (final_table(L.fin)) build_units(l, L.fin, false);
+    for (int j : L.fin.jobs) add_final_seg(L.fin, l, j, segment(j, jobs_[j].p1), jobs_[j].p1, jobs_[j].out_verts);
+    plan_blocks(L.fin, false);
     // a level whose every segment hands on its positions alone, with a quad
     // mesh two levels back: its positions from that mesh's structure too
     bool pos = allow_pos && !L.segs.empty() && (l >= 3 || levels_[0].quad);
@@ -906,20 +911,20 @@ void Plan::prepare() {
         const int j = L.jobs[k];
         const float4* P = L.P + L.segs[k].vb;
         L.pos.jobs.push_back(j);
-        add_final_seg(L.pos, j, segment(j, P), P, L.segs[k].dst_verts);
+        add_final_seg(L.pos, l, j, segment(j, P), P, L.segs[k].dst_verts);
       }
     }
     // meshes whose last level is l + 1, from the mesh two levels before l
     for (int j : L.deep.jobs) {
       MeshJob& J = jobs_[j];
       L.pos.jobs.push_back(j);
-      add_final_seg(L.pos, j, segment(j, J.p2), J.p2, J.p1);
-      add_final_seg(L.deep, j, segment(j, J.p1), J.p1, J.out_verts);
+      add_final_seg(L.pos, l, j, segment(j, J.p2), J.p2, J.p1);
+      add_final_seg(L.deep, l, j, segment(j, J.p1), J.p1, J.out_verts);
       if (J.own_base < 0) throw Error(SLAK_ERR_INTERNAL, "deep final level without its edge owners");
-      L.deep.segs.back().eb = J.own_base;
+      L.deep.segs.back().m.eb = J.own_base;
     }
-    if (final_table(L.pos)) build_units(l, L.pos, false);
-    if (final_table(L.deep)) build_units(l, L.deep, true);
+    plan_blocks(L.pos, false);
+    plan_blocks(L.deep, true);
   }
   // a level whose meshes all come from k_final runs no refine or vertex
   // items over its structure: only k_final reads its M^T rows, and it needs
@@ -965,69 +970,70 @@ static std::vector<int64_t> vertex_classes(const MeshJob& J, int l) {
   return cls;
 }
 
-// k_final (k_final_deep) over several meshes: work units of at most one block
-// each, mesh by mesh. A mesh's corner units (consecutive corners), edge units
-// (deep: consecutive edges) and the units of each of its vertex classes
-// (consecutive vertices of the class) are interleaved by their relative
-// position in their list, so that every list advances over the surface
-// together (each is numbered in the order of the original faces) and what one
-// kind gathers is still in the L2 that another has filled. The deep form's
-// corners are M's, four per corner of the N its segments describe.
-void Plan::build_units(int l, FinalTable& T, bool deep) {
-  T.units.clear();
-  struct Key {
-    int64_t num, den;  // relative position (2j + 1) / (2 nch) of the chunk
-    int4 unit;
-  };
-  std::vector<Key> keys;
-  for (size_t i = 0; i < T.jobs.size(); ++i) {
-    keys.clear();
-    auto list = [&](int kind, int64_t first, int64_t n, int64_t per) {
-      const int64_t nch = (n + per - 1) / per;
-      for (int64_t j = 0; j < nch; ++j)
-        keys.push_back(Key{2 * j + 1, 2 * nch,
-                           make_int4((int)i, (int)(first + j * per), (int)std::min(per, n - j * per), kind)});
-    };
-    list(0, 0, deep ? 4 * (int64_t)T.segs[i].nnz : T.segs[i].nnz, kBlockItems);
-    if (deep) list(2, 0, T.segs[i].ne, kDeepEdgeUnit);
-    int64_t first = 0;
-    for (int64_t n : vertex_classes(jobs_[T.jobs[i]], l)) {
-      list(1, first, n, kBlockItems);
-      first += n;
-    }
-    std::stable_sort(keys.begin(), keys.end(),
-                     [](const Key& a, const Key& b) { return a.num * b.den < b.num * a.den; });
-    for (const Key& k : keys) T.units.push_back(k.unit);
+// vertex classes as runs (leading ones merged past kMaxVSeg)
+static void set_runs(VertexRuns& R, std::vector<int64_t> cls) {
+  while (cls.size() > (size_t)kMaxVSeg) {
+    cls[1] += cls[0];
+    cls.erase(cls.begin());
   }
+  R.n = (int32_t)cls.size();
+  R.first[0] = 0;
+  for (size_t i = 0; i < cls.size(); ++i) R.first[i + 1] = R.first[i] + (int32_t)cls[i];
+}
+
+// The blocks of a table's meshes, mesh by mesh, and (several meshes) the mesh
+// of every block.
+void Plan::plan_blocks(FinalTable& T, bool deep) {
+  int64_t blocks = 0, lak = 0;
+  const bool table = final_table(T);
+  for (size_t k = 0; k < T.segs.size(); ++k) {
+    FinalSeg& F = T.segs[k];
+    F.block0 = (int32_t)blocks;
+    F.lak0 = (int32_t)lak;
+    blocks += plan_final_blocks(F, deep);
+    if (F.m.out_vals) lak += ((deep ? 4 : 1) * (int64_t)F.m.nnz + kBlockItems - 1) / kBlockItems;
+    check_i32(blocks * kBlockItems / 2, "items of a final level");
+    if (!table) continue;
+    T.block_seg.resize((size_t)blocks, (int32_t)k);
+    T.lak_seg.resize((size_t)lak, (int32_t)k);
+  }
+}
+
+// the meshes of a table as a launch's arguments
+void Plan::set_final_table(FinalView& V, const FinalTable& T) const {
+  if (!final_table(T)) {
+    V.one = T.segs[0];
+    return;
+  }
+  V.segs = T.d_segs;
+  V.block_seg = T.d_block_seg;
+  V.lak_seg = T.d_lak_seg;
+  V.nblocks = (int32_t)T.block_seg.size();
+  V.nlak = (int32_t)T.lak_seg.size();
 }
 
 // One mesh of a k_final table: m is its segment of M (of N for k_final_deep),
 // P1 the positions of M1. The output level also writes the job's quads and
 // LAK form; other levels positions alone.
-void Plan::add_final_seg(FinalTable& T, int job, const SegDesc& m, const float4* P1, float4* positions) {
+void Plan::add_final_seg(FinalTable& T, int l, int job, const SegDesc& m, const float4* P1, float4* positions) {
   const MeshJob& J = jobs_[job];
   FinalSeg F{};
-  F.cb = m.cb;
-  F.vb = m.vb;
-  F.eb = m.eb;
-  F.nv = m.nv;
-  F.nf = m.nf;
-  F.ne = (int32_t)m.ne;
-  F.nnz = (int32_t)m.nnz;
-  F.P1 = P1;
-  F.out_verts = positions;
+  F.m.cb = m.cb;
+  F.m.vb = m.vb;
+  F.m.eb = m.eb;
+  F.m.nv = m.nv;
+  F.m.nf = m.nf;
+  F.m.ne = (int32_t)m.ne;
+  F.m.nnz = (int32_t)m.nnz;
+  F.m.P1 = P1;
+  F.m.out_verts = positions;
   if (positions == J.out_verts) {
-    F.out_ids = J.out_ids;
-    F.out_ptr = J.out_ptr;
-    F.out_vals = J.out_vals;
+    F.m.out_ids = J.out_ids;
+    F.m.out_ptr = J.out_ptr;
+    F.m.out_vals = J.out_vals;
   }
-  if (T.segs.empty()) {
-    T.cb.assign(1, 0);
-    T.vb.assign(1, 0);
-  }
+  set_runs(F.runs, vertex_classes(J, l));
   T.segs.push_back(F);
-  T.cb.push_back(T.cb.back() + m.nnz);
-  T.vb.push_back(T.vb.back() + m.nv);
 }
 
 // k_final_deep over the meshes of table T, whose last level is l + 1, from the
@@ -1043,25 +1049,8 @@ void Plan::launch_deep(int l, FinalTable& T) {
   V.trow = N.trow;
   V.trow_x = N.rows_x ? reinterpret_cast<const int32_t*>(N.trow) : nullptr;
   V.own = N.own;
-  V.nnz = T.cb.back();
-  V.nv = T.vb.back();
+  set_final_table(V, T);
   const bool multi = final_table(T);
-  if (multi) {
-    V.segs = T.d_segs;
-    V.units = T.d_units;
-    V.nunits = (int32_t)T.units.size();
-    V.nseg = (int32_t)T.segs.size();
-  } else {
-    V.one = T.segs[0];
-    V.nseg = 1;
-    std::vector<int64_t> cls = vertex_classes(jobs_[T.jobs[0]], l);
-    while (cls.size() > (size_t)kMaxVSeg) {
-      cls[1] += cls[0];
-      cls.erase(cls.begin());
-    }
-    V.runs.n = (int32_t)cls.size();
-    for (size_t i = 0; i < cls.size(); ++i) V.runs.first[i + 1] = V.runs.first[i] + (int32_t)cls[i];
-  }
   // algorithmic bytes: reads N's ids, (edge, twin) pairs, edge owners, M^T
   // rows and offsets and the positions of M1; writes the output positions and
   // quads (and one mesh's LAK form)
@@ -1099,27 +1088,7 @@ void Plan::launch_final_table(int l, FinalTable& T, bool ids, const char* stage)
   V.trow_x = M.rows_x ? reinterpret_cast<const int32_t*>(M.trow) : nullptr;
   V.blk = M.blk;
   V.mpos = M.mpos;
-  V.nnz = T.cb.back();
-  V.nv = T.vb.back();
-  if (final_table(T)) {
-    V.segs = T.d_segs;
-    V.units = T.d_units;
-    V.nunits = (int32_t)T.units.size();
-    V.nseg = (int32_t)T.segs.size();
-  } else {
-    V.one = T.segs[0];
-    V.nseg = 1;
-    // vertex classes of M: the original vertices, then the face points and
-    // edge points of every level before M (leading ones merged past kMaxVSeg)
-    std::vector<int64_t> cls = vertex_classes(jobs_[T.jobs[0]], l);
-    while (cls.size() > (size_t)kMaxVSeg) {
-      cls[1] += cls[0];
-      cls.erase(cls.begin());
-    }
-    V.runs.n = (int32_t)cls.size();
-    V.runs.first[0] = 0;
-    for (size_t i = 0; i < cls.size(); ++i) V.runs.first[i + 1] = V.runs.first[i] + (int32_t)cls[i];
-  }
+  set_final_table(V, T);
   // algorithmic bytes: reads the ids, (edge, twin) pairs, M^T rows and
   // offsets of M (boundary scan, SLAK positions) and the positions of M1;
   // writes every output position and, for the output level, the quads (and
@@ -1204,14 +1173,7 @@ void Plan::record_level(int l) {
   if (L.segs.size() == 1 && l >= 2) {
     // one mesh: its vertex classes (the original vertices, then the face and
     // edge points of every earlier level) as runs in step with the corners
-    std::vector<int64_t> cls = vertex_classes(jobs_[L.jobs[0]], l + 1);
-    while (cls.size() > (size_t)kMaxVSeg) {
-      cls[1] += cls[0];
-      cls.erase(cls.begin());
-    }
-    R.runs.n = (int32_t)cls.size();
-    R.runs.first[0] = 0;
-    for (size_t i = 0; i < cls.size(); ++i) R.runs.first[i + 1] = R.runs.first[i] + (int32_t)cls[i];
+    set_runs(R.runs, vertex_classes(jobs_[L.jobs[0]], l + 1));
   }
   const bool next = L.ntptr != nullptr;
   {

@@ -49,15 +49,15 @@ struct MeshJob {
 };
 
 // Meshes whose level is formed by k_final from the structure of their mesh M
-// two levels before it: per mesh its segment of M, the positions of M1 and
-// the outputs; item bases; work units of the table path (several meshes).
+// two levels before it (k_final_deep: N, three levels before): per mesh its
+// segment of M, the positions of M1, the outputs and its blocks; several
+// meshes: the mesh of every block of the launch and of the LAK form's.
 struct FinalTable {
   std::vector<int> jobs;
   std::vector<FinalSeg> segs;
-  std::vector<int64_t> cb, vb;  // corner and vertex item bases (n + 1)
-  std::vector<int4> units;
+  std::vector<int32_t> block_seg, lak_seg;
   FinalSeg* d_segs = nullptr;
-  int4* d_units = nullptr;
+  int32_t *d_block_seg = nullptr, *d_lak_seg = nullptr;
   bool empty() const { return segs.empty(); }
 };
 
@@ -223,13 +223,14 @@ class Plan {
   hipStream_t capture_st_ = nullptr;  // stream the graph is captured on and replayed
   hipStream_t owned_st_ = nullptr;    // created when the caller's stream is the default one
   hipEvent_t order_ev_ = nullptr;
-  // k_final's meshes come from a device table and work units (several meshes)
+  // k_final's meshes come from a device table (several meshes)
   bool force_final_table_ = false;
   bool final_table(const FinalTable& T) const { return T.segs.size() > 1 || (force_final_table_ && !T.empty()); }
-  void add_final_seg(FinalTable& T, int job, const SegDesc& m, const float4* P1, float4* positions);
+  void add_final_seg(FinalTable& T, int l, int job, const SegDesc& m, const float4* P1, float4* positions);
   void launch_final_table(int l, FinalTable& T, bool ids, const char* stage);
   void launch_deep(int l, FinalTable& T);
-  void build_units(int l, FinalTable& T, bool deep);
+  void plan_blocks(FinalTable& T, bool deep);
+  void set_final_table(FinalView& V, const FinalTable& T) const;
   // single mesh: the first level's edge numbering ran during the analysis
   // read-back (the level then launches its face points only)
   bool number_early_ = false;
