@@ -5,7 +5,6 @@
 #include <stdint.h>
 
 #include <exception>
-#include <initializer_list>
 #include <mutex>
 #include <stdexcept>
 #include <string>
@@ -79,6 +78,9 @@ void launch_seg_bounds(const LevelView& L, hipStream_t st);
 // points in one launch, after the symbolic pass; a single mesh's launch also
 // fills L.report (if set), which several meshes take from launch_report
 void launch_report(const LevelView& L, hipStream_t st);
+// a small single mesh: all of the above in one launch (no zeroed state needed)
+bool first_level_is_small(const LevelView& L);
+void launch_first_small(bool quad, int scheme, bool use_vals, const LevelView& L, bool faces, hipStream_t st);
 void launch_number_faces(bool quad, int scheme, const LevelView& L, bool faces, hipStream_t st);
 void launch_spgemm_fde(bool quad, const LevelView& L, hipStream_t st);
 // refine (per corner) and vertex (per vertex) items of a level in one launch;
@@ -220,9 +222,11 @@ class Profiler {
 struct ProfScope {
   hipStream_t st;
   bool on;
-  ProfScope(hipStream_t s, const char* name, double bytes) : ProfScope(s, {{name, bytes}}) {}
-  ProfScope(hipStream_t s, std::initializer_list<StageBytes> stages) : st(s), on(Profiler::get().enabled()) {
-    if (on) Profiler::get().begin(st, stages);
+  ProfScope(hipStream_t s, const char* name, double bytes) : st(s), on(Profiler::get().enabled()) {
+    if (on) Profiler::get().begin(st, {{name, bytes}});
+  }
+  ProfScope(hipStream_t s, std::vector<StageBytes> stages) : st(s), on(Profiler::get().enabled()) {
+    if (on) Profiler::get().begin(st, std::move(stages));
   }
   ~ProfScope() {
     if (on) Profiler::get().end(st);

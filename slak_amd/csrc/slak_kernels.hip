@@ -761,6 +761,128 @@ __global__ void __launch_bounds__(kBlock) k_number_faces(LevelView L, int32_t nb
     for (int i = threadIdx.x; i < len; i += kBlock) L.trow[s0 + i] = tile_out[i];
 }
 
+// The whole first level of a small mesh (at most kSmallItems faces and
+// vertices, four times as many corners) in one block: gather, row sizing,
+// report, numbering and face points, one item per thread, phases apart by
+// barriers; counters and offsets stay in LDS. A call on such a mesh is bound
+// by its chain of dependent launches, and this is one of them in place of
+// four (zeroed state, gather, sizing, numbering). Whole calls: cube, 3 levels
+// 59.8 -> 51.3 us; torus of 512 quads, 3 levels 62.5 -> 55.5; of 1024 quads
+// 62.7 -> 60.8; 968 triangles, 2 levels 68.4 -> 64.0; open grid of 930 quads
+// 70.5 -> 61.6. The line is the largest block: beyond it one compute unit
+// would do in turn what the launches spread. Same rows, numbers and points as
+// theirs: both run the same row and face code.
+constexpr int kSmallItems = 1024;
+
+template <bool QUAD, int SCHEME>
+__global__ void __launch_bounds__(kSmallItems) k_first_small(LevelView L, int use_vals, int faces) {
+  constexpr int REGS = QUAD ? 4 : kGatherRegs;
+  __shared__ int32_t cnt[kSmallItems], head[kSmallItems];  // blockDim.x used: one per thread
+  __shared__ uint64_t wave_sum[kSmallItems / 64];
+  __shared__ int32_t pool;
+  __shared__ int32_t flags;
+  const int tid = threadIdx.x;
+  cnt[tid] = 0;
+  if (tid == 0) {
+    pool = 0;
+    flags = 0;
+    L.seg.mflags[0] = 0;
+  }
+  __syncthreads();
+  const RowBuild rb{cnt, L.slots, head, L.next};
+  FaceCorners<REGS> fc;
+#pragma unroll
+  for (int i = 0; i < REGS; ++i) fc.v[i] = -1;
+  if (tid < L.nf)
+    gather_face<QUAD, true>(L.seg, tid, L.nf, use_vals, const_cast<int32_t*>(L.ids), const_cast<int32_t*>(L.fptr),
+                            const_cast<int32_t*>(L.cface), &flags, rb, fc);
+#pragma unroll
+  for (int i = 0; i < REGS; ++i)
+    if (fc.v[i] >= 0) put_row(rb, fc.v[i], atomicAdd(&cnt[fc.v[i]], 1), fc.c[i]);
+  __syncthreads();
+  const bool valid = !(flags & kFlagsInput);  // the sizing sets no input flag: the same for every thread
+  const int32_t v = tid;
+  const bool active = valid && v < L.nv;
+  const int n = active ? cnt[v] : 0;
+  int32_t* row = L.slots + (int64_t)kRowSlots * v;
+  int32_t owned = 0, bcount = 0;
+  int bad = 0;
+  if (active) {
+    if (n <= L.row_cap) {
+      with_row<QUAD>(L, row, n, [&](auto& r) __attribute__((always_inline)) {
+        row_symbolic<SCHEME>(r, v, owned, bcount, bad);
+      });
+    } else {
+      if (n > kRowSlots) {  // the whole row to a run of the pool
+        int32_t* const run = L.tids + atomicAdd(&pool, n);
+        for (int i = 0; i < kRowSlots; ++i) run[i] = row[i];
+        int32_t c = head[v];
+        for (int i = kRowSlots; i < n; ++i) {
+          run[i] = c;
+          c = L.next[c];
+        }
+        row[0] = (int32_t)(run - L.tids);
+        row = run;
+      }
+      sort_row_in_place(row, n);
+      const MemRow<QUAD> r(L, row, n);
+      row_symbolic<SCHEME>(r, v, owned, bcount, bad);
+    }
+    (void)bcount;
+    if (bad) {
+      atomicOr(&flags, bad);
+      atomicOr(L.seg.mflags, bad);
+    }
+  }
+  const uint64_t own = pack_row(n, owned);
+  const uint64_t inc = (uint64_t)wave_scan64((int64_t)own);
+  if ((tid & 63) == 63) wave_sum[tid >> 6] = inc;
+  __syncthreads();  // (also: L.next is read before the numbering overwrites it)
+  uint64_t at = inc - own, total = 0;
+  for (int w = 0; w < (int)(blockDim.x >> 6); ++w) {
+    at += w < (tid >> 6) ? wave_sum[w] : 0;
+    total += wave_sum[w];
+  }
+  static_assert(2 + kRowHistBins + 2 <= 64);
+  if (tid < 2 + kRowHistBins + 2) {  // one wave; the host goes on from here
+    int32_t x = 0;                   // (no histogram: it tunes launches that a small mesh does not have)
+    if (tid == 0) *L.flags = flags;
+    if (tid == 1) x = flags;
+    if (tid == 2 + kRowHistBins + 1) x = (int32_t)(total & kOwnedMask);
+    if (tid > 0) L.report[tid] = x;
+    __threadfence_system();
+    if (tid == 0) __hip_atomic_store(L.report, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);  // (after the wave's stores)
+  }
+  if (!valid) return;
+  if (active) {
+    const int32_t s = (int32_t)(at >> 31), e0 = (int32_t)(at & kOwnedMask);
+    L.tptr[v] = s;
+    L.eptr[v] = e0;
+    if (v == L.nv - 1) {
+      L.tptr[L.nv] = s + n;
+      L.eptr[L.nv] = e0 + owned;
+    }
+    auto put = [&](int i, int32_t t, int32_t u) __attribute__((always_inline)) {
+      L.trow[s + i] = make_int2(t, u);
+      if (SCHEME == kSLAK) L.mpos[t] = s + i;
+    };
+    if (n <= L.row_cap) {
+      with_row<QUAD>(L, row, n, [&](auto& r) __attribute__((always_inline)) {
+        constexpr int C = std::decay_t<decltype(r)>::kCap;
+#pragma unroll
+        for (int i = 0; i < C; ++i)
+          if (i < n) put(i, r.T(i), r.U(i));
+        row_number<SCHEME, true>(r, L, v, e0);
+      });
+    } else {
+      MemRow<QUAD> r(L, row, n);  // sorted above
+      for (int i = 0; i < n; ++i) put(i, r.T(i), r.U(i));
+      row_number<SCHEME, true>(r, L, v, e0);
+    }
+  }
+  if (faces) faces_item<QUAD, true>(L.ids, L.fptr, L.P, L.nf, L.seg, tid);
+}
+
 template <bool QUAD>
 __global__ void __launch_bounds__(kBlock) k_spgemm_fde(LevelView L) {
   int32_t v = (int32_t)(block_index() * blockDim.x + threadIdx.x);
@@ -2484,6 +2606,23 @@ void launch_number_faces(bool quad, int scheme, const LevelView& L, bool faces, 
 }
 
 void launch_report(const LevelView& L, hipStream_t st) { k_report<<<1, kBlock, 0, st>>>(L); }
+
+bool first_level_is_small(const LevelView& L) {
+  return L.seg.n == 1 && L.nv <= kSmallItems && L.nf <= kSmallItems && L.nnz <= 4 * kSmallItems;
+}
+
+void launch_first_small(bool quad, int scheme, bool use_vals, const LevelView& L, bool faces, hipStream_t st) {
+  if (!first_level_is_small(L) || !L.report) throw Error(5, "not a small first level");  // SLAK_ERR_INTERNAL
+  const int vals = use_vals ? 1 : 0, fp = faces ? 1 : 0;
+  const int threads = (std::max({L.nv, L.nf, 1}) + 63) & ~63;  // one per vertex and face
+  if (quad) {
+    if (scheme == kLAK) k_first_small<true, kLAK><<<1, threads, 0, st>>>(L, vals, fp);
+    else k_first_small<true, kSLAK><<<1, threads, 0, st>>>(L, vals, fp);
+  } else {
+    if (scheme == kLAK) k_first_small<false, kLAK><<<1, threads, 0, st>>>(L, vals, fp);
+    else k_first_small<false, kSLAK><<<1, threads, 0, st>>>(L, vals, fp);
+  }
+}
 
 void launch_spgemm_fde(bool quad, const LevelView& L, hipStream_t st) {
   if (L.nv <= 0) return;

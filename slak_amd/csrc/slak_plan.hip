@@ -420,10 +420,7 @@ LevelView LevelPlan::view(int* flags, int* late) const {
 
 // Validation, position order, valences and the rows' corners in one launch.
 void Plan::record_gather(LevelPlan& L) {
-  ProfScope ps(st_, {{"gather", 4.0 * (L.nf + 1) + 12.0 * L.nnz + (L.quad ? 0.0 : 8.0 * L.nnz + 4.0 * L.nf)},
-                     {L.quad ? "count_quad" : "count_poly", 4.0 * L.nnz + 8.0 * L.nv + (L.quad ? 0.0 : 4.0 * L.nf)},
-                     {L.quad ? "transpose_quad" : "transpose_poly",
-                      8.0 * L.nnz + 12.0 * L.nv + (L.quad ? 0.0 : 4.0 * L.nf)}});
+  ProfScope ps(st_, gather_stages(L));
   launch_gather(L.quad, L.table(), scheme_ == kLAK, const_cast<int32_t*>(L.ids), L.view(d_flags_, late_), st_);
 }
 
@@ -431,16 +428,45 @@ void Plan::record_gather(LevelPlan& L) {
 // offsets, owned-edge counts and offsets (later levels receive their structure
 // from the level before).
 void Plan::record_analysis(LevelPlan& L) {
-  const double poly_b = L.quad ? 0.0 : 4.0 * (L.nf + 1) + 4.0 * L.nnz;
   LevelView V = L.view(d_flags_, late_);
   V.hist_rows = d_state_ + kStateRowHist;
   V.bounds = d_state_ + kStateBounds;
-  ProfScope ps(st_, {{"scan", 8.0 * L.nv + 4},
-                     {L.quad ? "spgemm_symbolic_quad" : "spgemm_symbolic_poly",
-                      8.0 * L.nnz + 8.0 * L.nv + 8.0 * L.nnz + poly_b},
-                     {"scan", 8.0 * L.nv + 4}});
+  ProfScope ps(st_, analysis_stages(L));
   launch_symbolic(L.quad, scheme_, V, st_);
   if (L.segs.size() > 1) launch_seg_bounds(V, st_);
+}
+
+std::vector<StageBytes> Plan::gather_stages(const LevelPlan& L) const {
+  return {{"gather", 4.0 * (L.nf + 1) + 12.0 * L.nnz + (L.quad ? 0.0 : 8.0 * L.nnz + 4.0 * L.nf)},
+          {L.quad ? "count_quad" : "count_poly", 4.0 * L.nnz + 8.0 * L.nv + (L.quad ? 0.0 : 4.0 * L.nf)},
+          {L.quad ? "transpose_quad" : "transpose_poly", 8.0 * L.nnz + 12.0 * L.nv + (L.quad ? 0.0 : 4.0 * L.nf)}};
+}
+
+std::vector<StageBytes> Plan::analysis_stages(const LevelPlan& L) const {
+  const double poly_b = L.quad ? 0.0 : 4.0 * (L.nf + 1) + 4.0 * L.nnz;
+  return {{"scan", 8.0 * L.nv + 4},
+          {L.quad ? "spgemm_symbolic_quad" : "spgemm_symbolic_poly", 8.0 * L.nnz + 8.0 * L.nv + 8.0 * L.nnz + poly_b},
+          {"scan", 8.0 * L.nv + 4}};
+}
+
+StageBytes Plan::number_stage(const LevelPlan& L, bool faces) const {
+  const double poly_b = L.quad ? 0.0 : 4.0 * (L.nf + 1) + 4.0 * L.nnz;
+  return {faces ? (L.quad ? "number_facepoints_quad" : "number_facepoints_poly") : "number",
+          12.0 * L.nv + 12.0 * L.nnz + 8.0 * L.nnz + (L.bnd ? 4.0 * (double)L.ne : 0.0) + poly_b +
+              (faces ? 4.0 * L.nnz + 16.0 * L.nv + 16.0 * L.nf : 0.0)};
+}
+
+// A small mesh's first level: gather, analysis and numbering in one launch.
+void Plan::record_small(LevelPlan& L, bool faces) {
+  LevelView V = L.view(d_flags_, late_);
+  V.ci = reinterpret_cast<int32_t*>(L.ci);
+  V.bnd = L.bnd;
+  V.report = report_;
+  std::vector<StageBytes> stages = gather_stages(L);
+  for (const StageBytes& s : analysis_stages(L)) stages.push_back(s);
+  stages.push_back(number_stage(L, faces));
+  ProfScope ps(st_, std::move(stages));
+  launch_first_small(L.quad, scheme_, scheme_ == kLAK, V, faces, st_);
 }
 
 void Plan::prepare() {
@@ -493,11 +519,15 @@ void Plan::prepare() {
   report_ = late_ + kReportAt;
   *late_ = 0;
   *report_ = 0;
-  upload_tables(0, 1, staging_first_, true);
+  // a small mesh's first level is one launch, which zeroes what it needs
+  const bool small = early && first_level_is_small(L1.view(nullptr, nullptr));
+  upload_tables(0, 1, staging_first_, !small);
 
   // 1. validate + gather (the state block is zeroed with the table upload)
-  record_gather(L1);
-  if (P1_) launch_gather_verts(L1.table(), (int32_t)L1.nv, P1_, st_);
+  if (!small) {
+    record_gather(L1);
+    if (P1_) launch_gather_verts(L1.table(), (int32_t)L1.nv, P1_, st_);
+  }
   auto fail_if = [&](int fl) {
     if (!fl) return;
     std::vector<int> mf(nseg, 0);
@@ -513,12 +543,17 @@ void Plan::prepare() {
   // 2. first-level analysis: M^T, owned-edge counts, per-mesh edge totals
   // (its kernels do nothing on an input the gather flagged; the flags come
   // back with the edge counts in one round trip)
-  record_analysis(L1);
+  if (small)
+    record_small(L1, early_p1_ != nullptr);
+  else
+    record_analysis(L1);
   std::vector<int64_t> hb(kRowHistBins + nseg + 1, 0);
   bool have_hist = false;
   if (!all_known) {
     // a single mesh numbers its edges (and forms its face points) meanwhile
-    if (early) {
+    if (small) {
+      // (in the one launch)
+    } else if (early) {
       launch_number(L1, early_p1_ != nullptr, true);
     } else {
       LevelView V = L1.view(d_flags_, late_);
@@ -939,8 +974,6 @@ void Plan::prepare() {
 // of every half-edge, boundary flags), with its face points in the same
 // launch when faces is set.
 void Plan::launch_number(LevelPlan& L, bool faces, bool rep) {
-  const double poly_b = L.quad ? 0.0 : 4.0 * (L.nf + 1) + 4.0 * L.nnz;
-  const double ne = (double)L.ne;
   LevelView V = L.view(d_flags_, late_);
   V.ci = reinterpret_cast<int32_t*>(L.ci);
   V.bnd = L.bnd;
@@ -949,9 +982,7 @@ void Plan::launch_number(LevelPlan& L, bool faces, bool rep) {
     V.hist_rows = d_state_ + kStateRowHist;
     V.ngroups = (int32_t)n_groups_;
   }
-  ProfScope ps(st_, faces ? (L.quad ? "number_facepoints_quad" : "number_facepoints_poly") : "number",
-               12.0 * L.nv + 12.0 * L.nnz + 8.0 * L.nnz + (L.bnd ? 4.0 * ne : 0.0) + poly_b +
-                   (faces ? 4.0 * L.nnz + 16.0 * L.nv + 16.0 * L.nf : 0.0));
+  ProfScope ps(st_, std::vector<StageBytes>{number_stage(L, faces)});
   launch_number_faces(L.quad, scheme_, V, faces, st_);
 }
 

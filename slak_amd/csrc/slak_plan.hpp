@@ -189,6 +189,11 @@ class Plan {
   };
   void upload_tables(int l0, int l1, Staging& staging, bool zero_state = false);
   void record_gather(LevelPlan& L);
+  void record_small(LevelPlan& L, bool faces);
+  // algorithmic bytes of the first level's stages
+  std::vector<StageBytes> gather_stages(const LevelPlan& L) const;
+  std::vector<StageBytes> analysis_stages(const LevelPlan& L) const;
+  StageBytes number_stage(const LevelPlan& L, bool faces) const;
   int read_flags();
   void wait_report();
   void launch_number(LevelPlan& L, bool faces, bool rep = false);
