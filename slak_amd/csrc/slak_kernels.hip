@@ -1480,7 +1480,10 @@ __device__ __forceinline__ Quads4 final_corner(const FinalView& V, const FinalMe
   // face point of M1 face t = (v, ep(e1), fp(F), ep(e0)), as k_faces forms it;
   // it is an output position too
   const float4 fpt = face_point(Pv, Pe, PF, Pu);
-  out[nv1 + t] = fpt;
+  if (IDS)
+    store_nt(out + (nv1 + t), fpt);  // (1 KB a wave; the partial lines of the others stay cached)
+  else
+    out[nv1 + t] = fpt;
   const float4 fptn = quad_next(fpt);
   // vertex point of fp(F): row 4t'+2 for the corners t' of F in order,
   // in-neighbours ep(e1(t')); never on the boundary. Every lane of the quad
@@ -1816,6 +1819,14 @@ __global__ void __launch_bounds__(kBlock) k_final(FinalView V) {
 //                 vertex points of the four M edge points and of X
 //   vertex items  one lane per N vertex
 // Every sum adds the same terms in the same order as k_final's: same bits.
+// Face points leave by non-temporal stores (whole lines of a wave), edge points
+// (64 bytes per quad of lanes) only when the launch's positions exceed what the
+// 256 MB last-level cache holds (FinalView.stream, kStreamBytes): they would
+// displace the positions still to be gathered, but below that line the cache
+// takes them faster. Whole calls, cached -> non-temporal edge points: torus
+// 256 x 256, 4 levels (268 MB of positions) 291 -> 271 us, 400 x 200 with a
+// quarter triangles (300 MB) 433 -> 351, 4096 meshes 10497 -> 10366; but
+// 256 x 192 (201 MB) 194 -> 207. Face points: 300 meshes 763 -> 742.
 
 template <int N>
 __device__ __forceinline__ int32_t row_ror_i(int32_t x) {  // lane i of a row of 16 reads lane i - N
@@ -1931,7 +1942,7 @@ __device__ __forceinline__ Quads4 deep_corner(const FinalView& V, const FinalMes
     sV = sV + q[64 + 52];
     sV = (sV / 4.0f + xf[32 + k] * 2.0f) / 4.0f;
   }
-  out[B.fM1 + c] = fpt;
+  store_nt(out + (B.fM1 + c), fpt);
   outf[4 * (int64_t)(B.fM + t) + k] = sF;
   if (j == 0) outf[4 * (int64_t)(S.nv + f) + k] = sV;
   // M1 edges of corners 4c .. 4c + 3, then the four output quads
@@ -2017,7 +2028,12 @@ __device__ __forceinline__ void deep_edges(const FinalView& V, const FinalMesh& 
     re[i] = p;
     re[16 + i] = psi;
     if (m) rx[9 * it + (m == 3 ? 8 : m == 2 ? 4 + j : j)] = f4sel(m == 1, psi, p);
-    out[B.eM1 + 4 * Y_id + slot] = f4mul(f4add(f4add(f4add(nbr, Y), psi), quad_prev(psi)), 0.25f);
+    const float4 q = f4mul(f4add(f4add(f4add(nbr, Y), psi), quad_prev(psi)), 0.25f);
+    float4* const d = out + (B.eM1 + 4 * Y_id + slot);
+    if (V.stream)
+      store_nt(d, q);
+    else
+      *d = q;
     wave_lds_fence();
     // vertex point of Y_j, component m: the row's corners are those of the
     // lower M face first; in Z_j A_j's comes before X's, in Z_{j-1} when j is odd

@@ -64,3 +64,13 @@ def test_mixed_batch_with_deep_meshes(monkeypatch):
     finally:
         for d in dev:
             d.freeAndReset()
+
+
+def test_output_beyond_the_last_level_cache(monkeypatch):
+    """276 MB of positions: the edge points are stored past the caches."""
+    m = g.torus(270, 250, seed=6)
+    monkeypatch.setenv("SLAK_FINAL_DEEP", "0")
+    want, _ = subdivide_host(m, 4, LAK)
+    monkeypatch.delenv("SLAK_FINAL_DEEP")
+    got, _ = subdivide_host(m, 4, LAK)
+    _assert_same(got, want)
