@@ -588,12 +588,13 @@ struct RefineView {
   uint64_t vratio;
 };
 
-// One mesh of a final level computed from the structure of the quad mesh M
+// One mesh of a final level computed from the structure of the mesh M
 // two levels before the output and the positions of its refinement M1 (whose
 // structure is never written): M's bases in the union arrays of its level,
 // its sizes, its M1 positions and its outputs.
 struct FinalMesh {
   int64_t cb, vb, eb;    // union bases of M's corners, vertices, edges
+  int64_t fb;            // and faces (polygons)
   int32_t nv, nf, ne;    // M sizes
   int32_t nnz;
   const float4* P1;      // M1 positions = [M vertices | M face points | M edge points]
@@ -610,8 +611,7 @@ struct FinalMesh {
 // what one kind gathers is still in the L2 that another has filled.
 struct FinalSeg {
   FinalMesh m;
-  int32_t block0;        // its first block, and its first block of the LAK form's launch
-  int32_t lak0;
+  int32_t block0;        // its first block
   int32_t blocks;
   uint64_t vratio;       // share of the vertex blocks, of the edge blocks among the others
   uint64_t eratio;
@@ -622,6 +622,8 @@ struct FinalView {
   // union arrays of M's level
   const int32_t* ids;    // corners -> vertices
   const int2* ci;        // (mesh-local edge id, twin corner or -1) per corner
+  const int32_t* fptr;   // polygons: corners of each face, face of each corner (null: quads)
+  const int32_t* cface;
   const int32_t* tptr;   // M^T row offsets
   const int2* trow;      // M^T rows (corner, in-neighbour), sorted
   const int32_t* trow_x; // or the rows' corners alone (int32), or null
@@ -633,9 +635,16 @@ struct FinalView {
   FinalSeg one;          // a single mesh
   const FinalSeg* segs;  // several meshes: device table, and the mesh of every block
   const int32_t* block_seg;
-  const int32_t* lak_seg;
-  int32_t nblocks;       // several meshes: blocks of the launch, of the LAK form's launch
-  int32_t nlak;
+  int32_t nblocks;       // several meshes: blocks of the launch
+};
+
+// One mesh of the LAK form's launch: its first block, a fourth of its output
+// quads, and the arrays.
+struct LakSeg {
+  int32_t block0;
+  int32_t n;
+  int32_t* vals;
+  int32_t* ptr;  // or null
 };
 
 // Face, successor and predecessor corner of corner t (quad: bit arithmetic;

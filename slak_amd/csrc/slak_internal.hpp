@@ -88,18 +88,18 @@ void launch_spgemm_fde(bool quad, const LevelView& L, hipStream_t st);
 void launch_level(bool quad, int scheme, const RefineView& R, hipStream_t st);
 // blocks of a mesh in a launch of k_final (of k_final_deep) and how they are
 // shared out (S.blocks, ratios, runs: runs.first holds its vertex classes)
-int64_t plan_final_blocks(FinalSeg& S, bool deep);
-// last level of one mesh or several (V.segs) from the quad mesh two levels
-// back; ids: also the output quads and LAK form (false: positions only)
+int64_t plan_final_blocks(FinalSeg& S, bool quad, bool deep);
+// last level of one mesh or several (V.segs) from the mesh two levels back
+// (V.fptr: polygons); ids: also the output quads and LAK form (false: positions only)
 void launch_final(int scheme, const FinalView& V, bool ids, hipStream_t st);
 // last level of one closed LAK mesh or several (V.segs) from the quad mesh
 // three levels back, whose structure V holds, and the positions of the level
 // before the output
 void launch_final_deep(const FinalView& V, hipStream_t st);
 constexpr int kDeepEdgeUnit = 64;  // edges per block
-// the LAK form (ptr, vals) of a several-mesh output level, after its k_final
-// launch (which leaves it out)
-void launch_final_lak_form(const FinalView& V, hipStream_t st);
+// the LAK form (ptr, vals) of the meshes that share their last level's launch
+// (which leaves it out)
+void launch_lak_form(const LakSeg* segs, const int32_t* block_seg, int64_t nblocks, hipStream_t st);
 // homogeneous-mesh conversions: per-face reorder of (ids, vals) by vals or by
 // ids (faces by ptr, or stride when ptr is null; 3 or 4 corners); fills of
 // stride ptr / 1-based positions

@@ -944,9 +944,8 @@ __device__ __forceinline__ int32_t quad_prev_i(int32_t x) { return __builtin_amd
 
 // entry k of the next level's M^T rows: (corner, in-neighbour), or the corner
 // alone when those rows are read by the last level's kernel only
-template <bool QUAD>
 __device__ __forceinline__ void put_next_row(const RefineView& R, int64_t k, int2 x) {
-  if (QUAD && R.next_rows_x)  // (only a quad level writes such rows)
+  if (R.next_rows_x)
     reinterpret_cast<int32_t*>(R.ntrow)[k] = x.x;
   else
     R.ntrow[k] = x;
@@ -1115,7 +1114,7 @@ __device__ __forceinline__ void corner_store(const RefineView& R, const SegK& K,
   // face point row: corner 2 of each refined quad of f, in corner order;
   // in-neighbour ep(e1)
   const int32_t nep = nvb + snv + snf;
-  put_next_row<QUAD>(R, ncb + snnz + lt, make_int2(c4 + 2, nep + c.e1));
+  put_next_row(R, ncb + snnz + lt, make_int2(c4 + 2, nep + c.e1));
   bool first;
   if (QUAD) first = (c.t & 3) == 0;
   else first = c.t == R.fptr[c.f];
@@ -1144,7 +1143,7 @@ __device__ __forceinline__ void corner_store(const RefineView& R, const SegK& K,
       a0 = a1;
       a1 = x;
     }
-    auto q = [&](int k, int2 x) __attribute__((always_inline)) { put_next_row<QUAD>(R, row1 + k, x); };
+    auto q = [&](int k, int2 x) __attribute__((always_inline)) { put_next_row(R, row1 + k, x); };
     if (c.s1 < 0) {
       q(0, a0);
       q(1, a1);
@@ -1285,7 +1284,7 @@ __device__ __forceinline__ void vertex_item(const RefineView& R, int32_t v) {
   };
   // the in-half-edges give the refined row's in-neighbours (and the boundary
   // rule): not needed when the next level's rows are corners alone
-  const bool load_cp = BND || (NEXT && !(QUAD && R.next_rows_x));
+  const bool load_cp = BND || (NEXT && !R.next_rows_x);
   int2 e[kVertexRegs], cp[kVertexRegs], co[kVertexRegs];
   float4 a[kVertexRegs], b[kVertexRegs];
 #pragma unroll
@@ -1348,12 +1347,12 @@ __device__ __forceinline__ void vertex_item(const RefineView& R, int32_t v) {
 #pragma unroll
   for (int i = 0; i < kVertexRegs; ++i)
     if (i < n) {
-      put_next_row<QUAD>(R, nrow + i, make_int2(ncb + 4 * (e[i].x - cb), load_cp ? nep + clampi(cp[i].x, emax) : 0));
+      put_next_row(R, nrow + i, make_int2(ncb + 4 * (e[i].x - cb), load_cp ? nep + clampi(cp[i].x, emax) : 0));
       if (nbnd) nbnd[neb + pos + i] = co[i].y < 0 ? 1 : 0;
     }
   for (int i = kVertexRegs; i < n; ++i) {
     const int32_t t = row[i].x;
-    put_next_row<QUAD>(R, nrow + i, make_int2(ncb + 4 * (t - cb), load_cp ? nep + clampi(ci[prevc(t)].x, emax) : 0));
+    put_next_row(R, nrow + i, make_int2(ncb + 4 * (t - cb), load_cp ? nep + clampi(ci[prevc(t)].x, emax) : 0));
     if (nbnd) nbnd[neb + pos + i] = ci[t].y < 0 ? 1 : 0;
   }
 }
@@ -1377,8 +1376,8 @@ __global__ void __launch_bounds__(kBlock) k_level(RefineView R) {
 }
 
 // ---------------------------------------------------------------------------
-// A level in closed form from the quad mesh M two levels before it (one mesh,
-// or several through a device table and work units): the output level (IDS:
+// A level in closed form from the mesh M two levels before it (one mesh,
+// or several through a device table): the output level (IDS:
 // quads, LAK form, positions) or the level before it (positions only). M1
 // (the refinement of M, whose positions P1 are in hand; its ids and
 // structure are never written) has corners 4t + k for the corners t of M:
@@ -1398,6 +1397,14 @@ __global__ void __launch_bounds__(kBlock) k_level(RefineView R) {
 // point of fp(F) from its four lanes. Vertex items remain only for the
 // vertices of M. Every sum adds the same terms in the same order as the
 // refine and vertex items of M1 would: the results are the same bits.
+// M may be the caller's polygons (second level): the same closed forms with
+// the neighbours of a corner through cface / fptr instead of lane exchange,
+// and one more run of items for the vertex points of the face points. Against
+// the refine and vertex items of M1, which read M1's structure (4 corners for
+// each of M's) and needed it written: 4096 meshes of levels 1 to 4, second
+// level 1340 (face points, items) -> 880 us and first level 1000 -> 749 (meshes
+// of two levels write no structure, the others rows of corners alone); 16
+// serve meshes 2950 -> 2680 us a call; no difference on calls of one small mesh.
 
 __device__ __forceinline__ float4 f4sel(bool c, float4 a, float4 b) { return c ? a : b; }
 // face point of a quad from its corners' positions in corner order (the sum
@@ -1412,31 +1419,57 @@ struct Quads4 {
   int4 a, b, c, d;
 };
 
+// face, successor and predecessor of a mesh's corner t (all mesh-local)
+template <bool QUAD>
+__device__ __forceinline__ void final_nbrs(const FinalView& V, const FinalMesh& S, int32_t t, int32_t& f, int32_t& tn,
+                                           int32_t& tp) {
+  if (QUAD) {
+    corner_nbrs<true>(nullptr, nullptr, t, f, tn, tp);
+  } else {
+    const int32_t cb = (int32_t)S.cb;
+    corner_nbrs<false>(V.fptr, V.cface, cb + t, f, tn, tp);
+    f -= (int32_t)S.fb;
+    tn -= cb;
+    tp -= cb;
+  }
+}
+
 // Corner t (mesh-local) of M in mesh S: returns its 16 output ids (IDS),
 // which the block stages in LDS.
-template <int SCHEME, bool BND, bool IDS, bool EARLY>
+template <bool QUAD, int SCHEME, bool BND, bool IDS, bool EARLY>
 __device__ __forceinline__ Quads4 final_corner(const FinalView& V, const FinalMesh& S, int32_t t) {
-  // every lane of a quad runs (nnz = 4 nf, meshes and blocks hold whole quads)
+  // QUAD: every lane of a quad runs (nnz = 4 nf, meshes and blocks hold whole
+  // quads): the quad's four lanes load their own corner once; w (next corner's
+  // vertex), u and the in-half-edge's (edge, twin) come from the
+  // neighbouring lanes. Polygons: each lane loads its neighbours' itself (they
+  // are in the lines the neighbouring lanes load).
   const int64_t cb = S.cb;
   const int32_t vb = (int32_t)S.vb;
-  const int32_t F = t >> 2, q0 = t & ~3;
-  const int32_t tn = q0 | ((t + 1) & 3);
+  int32_t F, tn, tp;
+  final_nbrs<QUAD>(V, S, t, F, tn, tp);
   const int32_t* __restrict__ ids = V.ids + cb;
   const int2* __restrict__ ci = V.ci + cb;
-  // the quad's four lanes load their own corner once; w (next corner's
-  // vertex), u and the in-half-edge's (edge, twin) come from the
-  // neighbouring lanes
   const int32_t v = ids[t] - vb;
-  const int32_t w = quad_next_i(v), u = quad_prev_i(v);
+  const int32_t w = QUAD ? quad_next_i(v) : ids[tn] - vb;
+  const int32_t u = QUAD ? quad_prev_i(v) : IDS && SCHEME == kLAK ? ids[tp] - vb : 0;
   const int2 c1 = ci[t];
-  const int2 c0 = make_int2(quad_prev_i(c1.x), quad_prev_i(c1.y));
+  const int2 c0 = QUAD ? make_int2(quad_prev_i(c1.x), quad_prev_i(c1.y)) : ci[tp];
   const int32_t emax = S.ne > 0 ? S.ne - 1 : 0;
   const int32_t e1 = clampi(c1.x, emax), e0 = clampi(c0.x, emax);
   // twins are union corners
   const int32_t s1 = c1.y >= 0 ? (int32_t)(c1.y - cb) : -1, s0 = c0.y >= 0 ? (int32_t)(c0.y - cb) : -1;
-  const int32_t g1 = s1 >= 0 ? (s1 >> 2) : F, g0 = s0 >= 0 ? (s0 >> 2) : F;
-  const int32_t n1 = s1 >= 0 ? ((s1 & ~3) | ((s1 + 1) & 3)) : 0;  // next(s1)
   const bool own = s1 < 0 || t < s1;
+  // faces across e1 and e0, next(s1) and prev(s1)
+  int32_t g1 = F, g0 = F, n1 = 0, p1 = 0;
+  if (QUAD) {
+    g1 = s1 >= 0 ? (s1 >> 2) : F;
+    g0 = s0 >= 0 ? (s0 >> 2) : F;
+    n1 = s1 >= 0 ? ((s1 & ~3) | ((s1 + 1) & 3)) : 0;
+    p1 = (s1 & ~3) | ((s1 + 3) & 3);
+  } else {
+    if (s1 >= 0 && (own || (IDS && SCHEME == kLAK))) final_nbrs<QUAD>(V, S, s1, g1, n1, p1);
+    if (s0 >= 0 && IDS && SCHEME == kLAK) g0 = V.cface[cb + s0] - (int32_t)S.fb;
+  }
   const int32_t nv = S.nv, nnz = S.nnz;
   const int32_t ep0 = nv + S.nf;     // M1 vertex of the edge point of edge 0 of M
   const int32_t nv1 = ep0 + S.ne;    // M1 vertices
@@ -1459,38 +1492,50 @@ __device__ __forceinline__ Quads4 final_corner(const FinalView& V, const FinalMe
   }
   int2 cs0 = make_int2(0, 0), cn1 = make_int2(0, 0);  // (edge, twin) of prev(s1) and next(s1)
   if (own && s1 >= 0) {
-    cs0 = ci[(s1 & ~3) | ((s1 + 3) & 3)];
+    cs0 = ci[p1];
     cn1 = ci[n1];
   }
+  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
   const float4 Pe = P1[ep0 + e1];   // ep(e1)
   const float4 Pv = P1[v];
   const float4 PF = P1[nv + F];     // fp(F)
   // across e1: fp(G) and the edge points of prev(s1) and next(s1). EARLY:
   // loaded before the first store, since a wait for a load also waits for
   // the stores issued before it (more registers: one wave fewer per SIMD)
-  float4 PG = make_float4(0.f, 0.f, 0.f, 0.f), Pa = PG, Pb = PG;
+  float4 PG = zero, Pa = zero, Pb = zero;
   if (EARLY && own && s1 >= 0) {
     PG = P1[nv + g1];
     Pa = P1[ep0 + clampi(cs0.x, emax)];
     Pb = P1[ep0 + clampi(cn1.x, emax)];
   }
-  // from the other lanes of the quad (all four run this): w is the vertex of
-  // the next corner, ep(e0) the edge point of the previous one
-  const float4 Pw = quad_next(Pv), Pu = quad_prev(Pe);
+  // w is the vertex of the next corner, ep(e0) the edge point of the previous
+  // one; the M1 face of the next corner is needed around ep(e1)
+  const bool next_face = own || SCHEME == kSLAK;
+  float4 Pw = zero, Pu, fptn = zero;
+  if (QUAD) {
+    Pw = quad_next(Pv);
+    Pu = quad_prev(Pe);
+  } else {
+    Pu = P1[ep0 + e0];
+    if (next_face) {
+      Pw = P1[w];
+      fptn = face_point(Pw, P1[ep0 + clampi(ci[tn].x, emax)], PF, Pe);
+    }
+  }
   // face point of M1 face t = (v, ep(e1), fp(F), ep(e0)), as k_faces forms it;
   // it is an output position too
   const float4 fpt = face_point(Pv, Pe, PF, Pu);
+  if (QUAD) fptn = quad_next(fpt);
   if (IDS)
     store_nt(out + (nv1 + t), fpt);  // (1 KB a wave; the partial lines of the others stay cached)
   else
     out[nv1 + t] = fpt;
-  const float4 fptn = quad_next(fpt);
   // vertex point of fp(F): row 4t'+2 for the corners t' of F in order,
   // in-neighbours ep(e1(t')); never on the boundary. Every lane of the quad
   // forms the sum from the quad's lanes in corner order (each term consumed
-  // as it arrives), lane 0 stores it.
-  {
-    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+  // as it arrives), lane 0 stores it (polygons: final_face).
+  if (QUAD) {
+    float4 s = zero;
     s = f4add(s, quad_lane<0>(fpt));
     s = f4add(s, quad_lane<1>(fpt));
     s = f4add(s, quad_lane<2>(fpt));
@@ -1503,7 +1548,7 @@ __device__ __forceinline__ Quads4 final_corner(const FinalView& V, const FinalMe
   }
   // across e1: M1 faces s1 = (w, ep(e1), fp(G), ep(e0(s1))) and
   // next(s1) = (v, ep(e1(next(s1))), fp(G), ep(e1))
-  float4 fps = make_float4(0.f, 0.f, 0.f, 0.f), fpsn = fps;
+  float4 fps = zero, fpsn = zero;
   if (own && s1 >= 0) {
     if (!EARLY) {
       PG = P1[nv + g1];
@@ -1617,7 +1662,7 @@ __device__ __forceinline__ Quads4 final_corner(const FinalView& V, const FinalMe
 // order, faces t, in-neighbours ep(e0(t)); on the boundary 3/4 P1[v] plus 1/8
 // of ep(e1(t)) across every boundary out-edge and of ep(e0(t)) across every
 // boundary in-edge
-template <int SCHEME, bool BND>
+template <bool QUAD, int SCHEME, bool BND>
 __device__ __forceinline__ void final_vertex(const FinalView& V, const FinalMesh& S, int32_t v) {
   const int32_t cb = (int32_t)S.cb;
   const int32_t ep0 = S.nv + S.nf;
@@ -1631,10 +1676,17 @@ __device__ __forceinline__ void final_vertex(const FinalView& V, const FinalMesh
   const int32_t* __restrict__ rx = V.trow_x ? V.trow_x + p0 : reinterpret_cast<const int32_t*>(V.trow + p0);
   const int rs = V.trow_x ? 1 : 2;
   const float4 Pv = P1[v];
-  auto prevc = [](int32_t t) __attribute__((always_inline)) { return (t & ~3) | ((t + 3) & 3); };
+  auto face = [&](int32_t t) __attribute__((always_inline)) {
+    return QUAD ? t >> 2 : V.cface[cb + t] - (int32_t)S.fb;
+  };
+  auto prevc = [&](int32_t t) __attribute__((always_inline)) {
+    int32_t f, tn, tp;
+    final_nbrs<QUAD>(V, S, t, f, tn, tp);
+    return tp;
+  };
   // face point of M1 face t = (v, ep(e1(t)), fp(face of t), ep(e0(t)))
   auto fp_of = [&](int32_t t, int2 c1, float4 pe0) __attribute__((always_inline)) {
-    return face_point(Pv, P1[ep0 + clampi(c1.x, emax)], P1[S.nv + (t >> 2)], pe0);
+    return face_point(Pv, P1[ep0 + clampi(c1.x, emax)], P1[S.nv + face(t)], pe0);
   };
   int32_t tt[kVertexRegs];
   int2 cp[kVertexRegs], co[kVertexRegs];
@@ -1665,7 +1717,7 @@ __device__ __forceinline__ void final_vertex(const FinalView& V, const FinalMesh
 #pragma unroll
       for (int j = 1; j < kVertexRegs; ++j) e1 = f4sel(m == j, b[j], e1);
       if (m < 0) e1 = P1[ep0 + clampi(co[i].x, emax)];
-      a[i] = face_point(Pv, e1, P1[S.nv + (tt[i] >> 2)], b[i]);
+      a[i] = face_point(Pv, e1, P1[S.nv + face(tt[i])], b[i]);
     }
   bool boundary = false;
   if (BND) {
@@ -1707,6 +1759,46 @@ __device__ __forceinline__ void final_vertex(const FinalView& V, const FinalMesh
   S.out_verts[v] = q;
 }
 
+// vertex point of the face point of a polygon f of M: row 4t + 2 for its
+// corners t in order, faces t, in-neighbours ep(e1(t)); never on the boundary.
+// (A lane per face: the corners of a polygon do not fill lanes of one wave as
+// a quad's do.)
+__device__ __forceinline__ void final_face(const FinalView& V, const FinalMesh& S, int32_t f) {
+  const int32_t vb = (int32_t)S.vb, ep0 = S.nv + S.nf;
+  const int32_t emax = S.ne > 0 ? S.ne - 1 : 0;
+  const float4* __restrict__ P1 = S.P1;
+  const int32_t t0 = V.fptr[S.fb + f], n = V.fptr[S.fb + f + 1] - t0;  // union corners
+  const float4 PF = P1[S.nv + f];
+  auto edge = [&](int32_t i) __attribute__((always_inline)) { return P1[ep0 + clampi(V.ci[t0 + i].x, emax)]; };
+  auto vert = [&](int32_t i) __attribute__((always_inline)) { return P1[V.ids[t0 + i] - vb]; };
+  float4 a[kVertexRegs], b[kVertexRegs];
+  float4 last = edge(n - 1);
+#pragma unroll
+  for (int i = 0; i < kVertexRegs; ++i)
+    if (i < n) {
+      a[i] = vert(i);
+      b[i] = edge(i);
+    }
+  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+  for (int i = 0; i < kVertexRegs; ++i)
+    if (i < n) {
+      s = f4add(s, face_point(a[i], b[i], PF, last));
+      last = b[i];
+    }
+  for (int i = kVertexRegs; i < n; ++i) {
+    const float4 e = edge(i);
+    s = f4add(s, face_point(vert(i), e, PF, last));
+    last = e;
+  }
+#pragma unroll
+  for (int i = 0; i < kVertexRegs; ++i)
+    if (i < n) s = f4add(s, b[i]);
+  for (int i = kVertexRegs; i < n; ++i) s = f4add(s, edge(i));
+  const float nf = (float)n;
+  S.out_verts[S.nv + f] = f4div(f4add(f4div(s, nf), f4mul(PF, nf - 2.0f)), nf);
+}
+
 // The output quads of a block's corners t0 .. t0 + cnt (of nnz in the mesh):
 // staged in LDS and stored with consecutive lanes on consecutive 16-byte
 // pieces; one mesh: their LAK form too.
@@ -1737,7 +1829,7 @@ __device__ __forceinline__ void store_quads(const FinalMesh& S, const Quads4& q4
   // LAK form of the block's 4 x 256 output quads (createQuadColPtr /
   // createQuadVals): every int4 of vals is (1, 2, 3, 4) and int4 q of ptr
   // is 16q + (0, 4, 8, 12), so consecutive lanes take consecutive pieces.
-  // Several meshes: written by k_lak_form after this launch instead.
+  // Several meshes: written by k_lak_form instead.
   if (MULTI) return;
   if (S.out_vals) {
     int32_t* __restrict__ vals = S.out_vals + 16 * (int64_t)t0;
@@ -1771,7 +1863,7 @@ __device__ __forceinline__ FinalMesh block_mesh(const FinalView& V, const FinalS
 // Corner and vertex blocks interleaved (FinalSeg). A corner block stages its
 // 16 KB of output quads in LDS and stores them with consecutive lanes on
 // consecutive 16-byte pieces.
-template <int SCHEME, bool BND, bool MULTI, bool IDS>
+template <bool QUAD, int SCHEME, bool BND, bool MULTI, bool IDS>
 __global__ void __launch_bounds__(kBlock) k_final(FinalView V) {
   const FinalSeg* seg;
   const FinalMesh S = block_mesh<MULTI>(V, seg);
@@ -1780,18 +1872,22 @@ __global__ void __launch_bounds__(kBlock) k_final(FinalView V) {
   if (after > before) {
     int32_t end;
     const int32_t v = run_block(seg->runs, before, end) + (int32_t)threadIdx.x;
-    if (v < end) final_vertex<SCHEME, BND>(V, S, v);
+    if (v >= end) return;
+    if (QUAD || v < S.nv)
+      final_vertex<QUAD, SCHEME, BND>(V, S, v);
+    else
+      final_face(V, S, v - S.nv);  // (polygons: a run of their own after the vertices)
     return;
   }
   const int32_t t0 = (b - before) * kBlock, cnt = min(kBlock, S.nnz - t0);
   const int32_t t = t0 + (int32_t)threadIdx.x;
   if (!IDS) {  // positions only
-    if ((int)threadIdx.x < cnt) final_corner<SCHEME, BND, false, MULTI>(V, S, t);
+    if ((int)threadIdx.x < cnt) final_corner<QUAD, SCHEME, BND, false, MULTI>(V, S, t);
     return;
   }
   __shared__ int4 stage[kStageStride * kBlock];
   Quads4 q4{};
-  if ((int)threadIdx.x < cnt) q4 = final_corner<SCHEME, BND, true, MULTI>(V, S, t);
+  if ((int)threadIdx.x < cnt) q4 = final_corner<QUAD, SCHEME, BND, true, MULTI>(V, S, t);
   store_quads<MULTI>(S, q4, stage, t0, cnt, S.nnz);
 }
 
@@ -2174,34 +2270,31 @@ __global__ void __launch_bounds__(kBlock) k_final_deep(FinalView V) {
 }
 
 
-// The LAK form of the output quads of a multi-mesh k_final launch
-// (createQuadColPtr / createQuadVals, LAKCatmullClarkKernels.cuh:396-431): a
-// block writes the 1024 quads of 256 of its mesh's M corners, vals as int4
-// (1, 2, 3, 4), ptr as int4 16t + (0, 4, 8, 12). A pure streaming write, apart
-// from the gathers and scattered stores of k_final. XCD-chunked block order:
-// a fill of five 16-byte stores a thread reaches 6.6 TB/s that way, 5.8 to 6.2
-// with the blocks dealt round.
-__global__ void __launch_bounds__(kBlock) k_lak_form(FinalView V) {
+// The LAK form of the output quads of the meshes that share their last level's
+// launch (createQuadColPtr / createQuadVals, LAKCatmullClarkKernels.cuh:396-431),
+// whatever their levels: a block writes the 1024 quads of 256 items of its mesh,
+// vals as int4 (1, 2, 3, 4), ptr as int4 16t + (0, 4, 8, 12). A pure streaming
+// write, apart from the gathers and scattered stores of k_final. XCD-chunked
+// block order: a fill of five 16-byte stores a thread reaches 6.6 TB/s that
+// way, 5.8 to 6.2 with the blocks dealt round. One launch for all levels: two
+// launches less on a batch of levels 1 to 4, about 6 us each when it is small.
+__global__ void __launch_bounds__(kBlock) k_lak_form(const LakSeg* __restrict__ segs,
+                                                     const int32_t* __restrict__ block_seg) {
   const int32_t b = (int32_t)block_index<kRemapFinal>();
-  const FinalSeg& seg = V.segs[V.lak_seg[b]];
-  int32_t* const out_vals = to_global(seg.m.out_vals);
-  int32_t* const out_ptr = to_global(seg.m.out_ptr);
-  const int32_t nnz = V.own ? 4 * seg.m.nnz : seg.m.nnz;  // corners of M
-  const int32_t t0 = (b - seg.lak0) * kBlock, cnt = min(kBlock, nnz - t0);
+  const LakSeg& seg = segs[block_seg[b]];
+  const int32_t t0 = (b - seg.block0) * kBlock, cnt = min(kBlock, seg.n - t0);
   const int32_t t = t0 + (int32_t)threadIdx.x;
   const int nq = 4 * cnt;
-  if (out_vals) {
-    int32_t* __restrict__ vals = out_vals + 16 * (int64_t)t0;
+  int32_t* __restrict__ vals = to_global(seg.vals) + 16 * (int64_t)t0;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int i = j * kBlock + threadIdx.x;
-      if (i < nq) store_nt(vals + 4 * i, 1, 2, 3, 4);
-    }
+  for (int j = 0; j < 4; ++j) {
+    const int i = j * kBlock + threadIdx.x;
+    if (i < nq) store_nt(vals + 4 * i, 1, 2, 3, 4);
   }
-  if (out_ptr) {
-    if ((int)threadIdx.x < cnt) store_nt(out_ptr + 4 * (int64_t)t, 16 * t, 16 * t + 4, 16 * t + 8, 16 * t + 12);
-    if (t == nnz - 1) store_nt(out_ptr + 4 * (int64_t)nnz, 16 * nnz);
-  }
+  int32_t* const ptr = to_global(seg.ptr);
+  if (!ptr) return;
+  if ((int)threadIdx.x < cnt) store_nt(ptr + 4 * (int64_t)t, 16 * t, 16 * t + 4, 16 * t + 8, 16 * t + 12);
+  if (t == seg.n - 1) store_nt(ptr + 4 * (int64_t)seg.n, 16 * seg.n);
 }
 
 // ---------------------------------------------------------------------------
@@ -2709,17 +2802,17 @@ void launch_level(bool quad, int scheme, const RefineView& R0, hipStream_t st) {
   }
 }
 
-int64_t plan_final_blocks(FinalSeg& S, bool deep) {
+int64_t plan_final_blocks(FinalSeg& S, bool quad, bool deep) {
   static const bool runs = [] {  // SLAK_FINAL_RUNS=0: vertex items in plain order
     const char* e = std::getenv("SLAK_FINAL_RUNS");
     return !e || std::atoi(e) != 0;
   }();
   const FinalMesh& m = S.m;
-  if ((int64_t)m.nnz != 4 * (int64_t)m.nf)
+  if (quad ? (int64_t)m.nnz != 4 * (int64_t)m.nf : deep)
     throw Error(5, "final level: the mesh it starts from must be quads");  // SLAK_ERR_INTERNAL
   if (deep && (2 * (int64_t)m.ne != m.nnz || 4ll * m.nnz > 0x7fffffff))
     throw Error(5, "deep final level: a closed mesh expected");  // SLAK_ERR_INTERNAL
-  plan_runs(S.runs, runs, m.nv);
+  plan_runs(S.runs, runs, (int64_t)m.nv + (quad ? 0 : m.nf));  // (polygons: final_face)
   const int64_t corners = m.nnz > 0 ? grid_for((deep ? 4ll : 1ll) * m.nnz) : 0;  // (a mesh without faces)
   const int64_t edges = deep ? ((int64_t)m.ne + kDeepEdgeUnit - 1) / kDeepEdgeUnit : 0;
   const int64_t total = corners + edges + S.runs.blocks;
@@ -2738,38 +2831,35 @@ static unsigned final_grid(const FinalView& V) {
   return (unsigned)n;
 }
 
+template <bool QUAD, int SCHEME, bool BND>
+static void launch_final_t(const FinalView& V, bool ids, unsigned g, hipStream_t st) {
+  if (V.segs) {
+    if (ids) k_final<QUAD, SCHEME, BND, true, true><<<g, kBlock, 0, st>>>(V);
+    else k_final<QUAD, SCHEME, BND, true, false><<<g, kBlock, 0, st>>>(V);
+  } else {
+    if (ids) k_final<QUAD, SCHEME, BND, false, true><<<g, kBlock, 0, st>>>(V);
+    else k_final<QUAD, SCHEME, BND, false, false><<<g, kBlock, 0, st>>>(V);
+  }
+}
+
+template <bool QUAD>
+static void launch_final_t(int scheme, const FinalView& V, bool ids, unsigned g, hipStream_t st) {
+  const bool bnd = V.blk != nullptr;
+  if (scheme == kLAK) {
+    if (bnd) launch_final_t<QUAD, kLAK, true>(V, ids, g, st);
+    else launch_final_t<QUAD, kLAK, false>(V, ids, g, st);
+  } else {
+    if (bnd) launch_final_t<QUAD, kSLAK, true>(V, ids, g, st);
+    else launch_final_t<QUAD, kSLAK, false>(V, ids, g, st);
+  }
+}
+
 void launch_final(int scheme, const FinalView& V, bool ids, hipStream_t st) {
   const unsigned g = final_grid(V);
   if (g == 0) return;
-  const bool multi = V.segs != nullptr;
-  const bool bnd = V.blk != nullptr;
-#define SLAK_FINAL(S, B, M)                                                    \
-  do {                                                                         \
-    if (ids)                                                                   \
-      k_final<S, B, M, true><<<g, kBlock, 0, st>>>(V);  \
-    else                                                                       \
-      k_final<S, B, M, false><<<g, kBlock, 0, st>>>(V); \
-  } while (0)
-  if (scheme == kLAK) {
-    if (multi) {
-      if (bnd) SLAK_FINAL(kLAK, true, true);
-      else SLAK_FINAL(kLAK, false, true);
-    } else {
-      if (bnd) SLAK_FINAL(kLAK, true, false);
-      else SLAK_FINAL(kLAK, false, false);
-    }
-  } else {
-    if (multi) {
-      if (bnd) SLAK_FINAL(kSLAK, true, true);
-      else SLAK_FINAL(kSLAK, false, true);
-    } else {
-      if (bnd) SLAK_FINAL(kSLAK, true, false);
-      else SLAK_FINAL(kSLAK, false, false);
-    }
-  }
-#undef SLAK_FINAL
+  if (V.fptr) launch_final_t<false>(scheme, V, ids, g, st);
+  else launch_final_t<true>(scheme, V, ids, g, st);
 }
-
 
 void launch_final_deep(const FinalView& V, hipStream_t st) {
   if (!V.own || V.blk) throw Error(5, "deep final level: closed meshes with edge owners only");  // SLAK_ERR_INTERNAL
@@ -2781,10 +2871,11 @@ void launch_final_deep(const FinalView& V, hipStream_t st) {
     k_final_deep<false><<<g, kBlock, 0, st>>>(V);
 }
 
-void launch_final_lak_form(const FinalView& V, hipStream_t st) {
-  if (!V.segs || !V.lak_seg) throw Error(5, "final level: no blocks planned");  // SLAK_ERR_INTERNAL
-  if (V.nlak <= 0) return;
-  k_lak_form<<<(unsigned)V.nlak, kBlock, 0, st>>>(V);
+void launch_lak_form(const LakSeg* segs, const int32_t* block_seg, int64_t nblocks, hipStream_t st) {
+  if (nblocks <= 0) return;
+  if (!segs || !block_seg) throw Error(5, "LAK form: no blocks planned");  // SLAK_ERR_INTERNAL
+  if (nblocks * kBlock > 0xffffffffll) throw Error(1, "LAK form too large for one launch");
+  k_lak_form<<<(unsigned)nblocks, kBlock, 0, st>>>(segs, block_seg);
 }
 
 void launch_sort_faces(bool by_vals, const int32_t* ptr, int32_t stride, int32_t nf, int64_t nnz, int32_t* ids,

@@ -192,9 +192,7 @@ void Plan::upload_tables(int l0, int l1, Staging& staging, bool zero_state) {
   std::vector<size_t> offs;
   // k_final tables of several meshes: FinalSeg[n], corner and vertex item bases
   auto table_bytes = [&](const FinalTable& T) -> size_t {
-    return final_table(T) ? align(T.segs.size() * sizeof(FinalSeg)) +
-                                align((T.block_seg.size() + T.lak_seg.size()) * sizeof(int32_t))
-                          : 0;
+    return final_table(T) ? align(T.segs.size() * sizeof(FinalSeg)) + align(T.block_seg.size() * sizeof(int32_t)) : 0;
   };
   auto fin_bytes = [&](const LevelPlan& L) -> size_t {
     return table_bytes(L.fin) + table_bytes(L.pos) + table_bytes(L.deep);
@@ -210,6 +208,9 @@ void Plan::upload_tables(int l0, int l1, Staging& staging, bool zero_state) {
               align((nblocks(L.nv) + nblocks(L.nf) + nblocks(L.nnz)) * sizeof(int32_t));
     total += fin_bytes(L);
   }
+  // (planned with the last levels: empty when the first level's tables go up)
+  const size_t lak_bytes = lak_.segs.empty() ? 0 : align(lak_.segs.size() * sizeof(LakSeg)) + align(lak_.block_seg.size() * sizeof(int32_t));
+  total += lak_bytes;
   for (int l = l0; l < l1; ++l)
     if (!levels_[l].d_mflags)
       levels_[l].d_mflags = l == 0 ? d_state_ + kStateBounds + (levels_[l].segs.size() + 1)
@@ -262,13 +263,19 @@ void Plan::upload_tables(int l0, int l1, Staging& staging, bool zero_state) {
       std::memcpy(staging.p + o, T->segs.data(), T->segs.size() * sizeof(FinalSeg));
       T->d_segs = reinterpret_cast<FinalSeg*>(d + o);
       o = align(o + T->segs.size() * sizeof(FinalSeg));
-      const size_t nb = T->block_seg.size() * sizeof(int32_t), nl = T->lak_seg.size() * sizeof(int32_t);
+      const size_t nb = T->block_seg.size() * sizeof(int32_t);
       std::memcpy(staging.p + o, T->block_seg.data(), nb);
       T->d_block_seg = reinterpret_cast<int32_t*>(d + o);
-      std::memcpy(staging.p + o + nb, T->lak_seg.data(), nl);
-      T->d_lak_seg = reinterpret_cast<int32_t*>(d + o + nb);
-      o = align(o + nb + nl);
+      o = align(o + nb);
     }
+  }
+  if (lak_bytes) {
+    size_t o = total - lak_bytes;
+    std::memcpy(staging.p + o, lak_.segs.data(), lak_.segs.size() * sizeof(LakSeg));
+    lak_.d_segs = reinterpret_cast<LakSeg*>(d + o);
+    o = align(o + lak_.segs.size() * sizeof(LakSeg));
+    std::memcpy(staging.p + o, lak_.block_seg.data(), lak_.block_seg.size() * sizeof(int32_t));
+    lak_.d_block_seg = reinterpret_cast<int32_t*>(d + o);
   }
   launch_setup(staging.p, d, (int64_t)total, zero_state ? d_state_ : nullptr, zero_state ? n_state_ : 0, st_);
 }
@@ -666,8 +673,6 @@ void Plan::prepare() {
     force_final_table_ = e && std::atoi(e) != 0;
   }
   // k_final computes the last level of every mesh refined two or more levels
-  // whose mesh two levels before the output is a quad mesh of a quad level
-  // (levels >= 2 are; the first is when every input is a quad mesh)
   {
     const char* e = std::getenv("SLAK_FUSED_FINAL");
     const bool allow = !e || std::atoi(e) != 0;
@@ -679,7 +684,7 @@ void Plan::prepare() {
     const bool allow_deep = allow && scheme_ == kLAK && (!d || std::atoi(d) != 0) && (!q || std::atoi(q) != 0);
     for (int j : levels_[0].jobs) {
       MeshJob& J = jobs_[j];
-      J.fused = allow && J.levels >= 2 && (J.levels >= 3 || levels_[0].quad);
+      J.fused = allow && J.levels >= 2;
       J.deep = allow_deep && J.levels >= 4 && 2 * J.ne[0] == J.nnz[0];
       J.p1 = nullptr;
       J.p2 = nullptr;
@@ -925,6 +930,7 @@ void Plan::prepare() {
   std::vector<int> seg_in_m(jobs_.size(), -1);  // job -> its segment of M
   const char* pe = std::getenv("SLAK_FUSED_POS");
   const bool allow_pos = !pe || std::atoi(pe) != 0;
+  lak_ = LakTable{};
   for (int l = 2; l <= Lmax; ++l) {
     LevelPlan& L = levels_[l - 1];
     const LevelPlan& M = levels_[l - 2];
@@ -935,10 +941,10 @@ void Plan::prepare() {
     };
     // meshes whose last level is l
     for (int j : L.fin.jobs) add_final_seg(L.fin, l, j, segment(j, jobs_[j].p1), jobs_[j].p1, jobs_[j].out_verts);
-    plan_blocks(L.fin, false);
-    // a level whose every segment hands on its positions alone, with a quad
-    // mesh two levels back: its positions from that mesh's structure too
-    bool pos = allow_pos && !L.segs.empty() && (l >= 3 || levels_[0].quad);
+    plan_blocks(L.fin, M.quad, false);
+    // a level whose every segment hands on its positions alone: its positions
+    // from the structure two levels back too
+    bool pos = allow_pos && !L.segs.empty();
     for (int j : L.jobs) pos = pos && positions_only(jobs_[j], l);
     if (pos) {
       L.pos_fused = true;
@@ -958,14 +964,14 @@ void Plan::prepare() {
       if (J.own_base < 0) throw Error(SLAK_ERR_INTERNAL, "deep final level without its edge owners");
       L.deep.segs.back().m.eb = J.own_base;
     }
-    plan_blocks(L.pos, false);
-    plan_blocks(L.deep, true);
+    plan_blocks(L.pos, M.quad, false);
+    plan_blocks(L.deep, M.quad, true);
   }
   // a level whose meshes all come from k_final runs no refine or vertex
   // items over its structure: only k_final reads its M^T rows, and it needs
   // their corners alone
   for (size_t i = 1; i < levels_.size(); ++i)
-    levels_[i].rows_x = levels_[i - 1].quad && (levels_[i].segs.empty() || levels_[i].pos_fused);
+    levels_[i].rows_x = levels_[i].segs.empty() || levels_[i].pos_fused;
   upload_tables(0, (int)levels_.size(), staging_all_);
   prepared_ = true;
 }
@@ -1014,19 +1020,27 @@ static void set_runs(VertexRuns& R, std::vector<int64_t> cls) {
 
 // The blocks of a table's meshes, mesh by mesh, and (several meshes) the mesh
 // of every block.
-void Plan::plan_blocks(FinalTable& T, bool deep) {
-  int64_t blocks = 0, lak = 0;
+void Plan::plan_blocks(FinalTable& T, bool quad, bool deep) {
+  int64_t blocks = 0;
   const bool table = final_table(T);
   for (size_t k = 0; k < T.segs.size(); ++k) {
     FinalSeg& F = T.segs[k];
     F.block0 = (int32_t)blocks;
-    F.lak0 = (int32_t)lak;
-    blocks += plan_final_blocks(F, deep);
-    if (F.m.out_vals) lak += ((deep ? 4 : 1) * (int64_t)F.m.nnz + kBlockItems - 1) / kBlockItems;
+    blocks += plan_final_blocks(F, quad, deep);
     check_i32(blocks * kBlockItems / 2, "items of a final level");
     if (!table) continue;
     T.block_seg.resize((size_t)blocks, (int32_t)k);
-    T.lak_seg.resize((size_t)lak, (int32_t)k);
+    if (!F.m.out_vals) continue;
+    LakSeg A{};
+    A.block0 = (int32_t)lak_.block_seg.size();
+    A.n = (deep ? 4 : 1) * F.m.nnz;
+    A.vals = F.m.out_vals;
+    A.ptr = F.m.out_ptr;
+    const int64_t lak = (int64_t)A.block0 + ((int64_t)A.n + kBlockItems - 1) / kBlockItems;
+    check_i32(lak * kBlockItems / 2, "items of the LAK form");
+    lak_.block_seg.resize((size_t)lak, (int32_t)lak_.segs.size());
+    lak_.segs.push_back(A);
+    lak_.bytes += 4.0 * (A.ptr ? 4.0 * A.n + 1 : 0.0) + 64.0 * A.n;
   }
 }
 
@@ -1038,9 +1052,7 @@ void Plan::set_final_table(FinalView& V, const FinalTable& T) const {
   }
   V.segs = T.d_segs;
   V.block_seg = T.d_block_seg;
-  V.lak_seg = T.d_lak_seg;
   V.nblocks = (int32_t)T.block_seg.size();
-  V.nlak = (int32_t)T.lak_seg.size();
 }
 
 // One mesh of a k_final table: m is its segment of M (of N for k_final_deep),
@@ -1052,6 +1064,7 @@ void Plan::add_final_seg(FinalTable& T, int l, int job, const SegDesc& m, const 
   F.m.cb = m.cb;
   F.m.vb = m.vb;
   F.m.eb = m.eb;
+  F.m.fb = m.fb;
   F.m.nv = m.nv;
   F.m.nf = m.nf;
   F.m.ne = (int32_t)m.ne;
@@ -1063,7 +1076,9 @@ void Plan::add_final_seg(FinalTable& T, int l, int job, const SegDesc& m, const 
     F.m.out_ptr = J.out_ptr;
     F.m.out_vals = J.out_vals;
   }
-  set_runs(F.runs, vertex_classes(J, l));
+  std::vector<int64_t> cls = vertex_classes(J, l);
+  if (!levels_[l - 2].quad) cls.push_back(m.nf);  // polygons' face points have items of their own
+  set_runs(F.runs, cls);
   T.segs.push_back(F);
 }
 
@@ -1090,23 +1105,19 @@ void Plan::launch_deep(int l, FinalTable& T) {
   // algorithmic bytes: reads N's ids, (edge, twin) pairs, edge owners, M^T
   // rows and offsets and the positions of M1; writes the output positions and
   // quads (and one mesh's LAK form)
-  double bytes = 0, lak_form = 0, positions = 0;
+  double bytes = 0, positions = 0;
   for (int j : T.jobs) {
     const MeshJob& J = jobs_[j];
     const double nnz = (double)J.nnz[l - 2], nnz1 = (double)J.nnz[l];
     bytes += 12.0 * nnz + 8.0 * (double)J.ne[l - 2] + (N.rows_x ? 4.0 : 8.0) * nnz + 4.0 * (double)J.nv[l - 2] +
              16.0 * (double)J.nv[l] + 16.0 * ((double)J.nv[l] + (double)J.nf[l] + (double)J.ne[l]) + 16.0 * nnz1;
-    if (J.out_ptr) (multi ? lak_form : bytes) += 4.0 * (nnz1 + 1) + 16.0 * nnz1;
+    if (J.out_ptr && !multi) bytes += 4.0 * (nnz1 + 1) + 16.0 * nnz1;
     positions += 16.0 * ((double)J.nv[l] + (double)J.nf[l] + (double)J.ne[l]);
   }
   V.stream = positions > kStreamBytes;
   {
     ProfScope ps(st_, "refine_vertex_final_quad", bytes);
     launch_final_deep(V, st_);
-  }
-  if (multi && lak_form > 0) {
-    ProfScope ps(st_, "lak_form", lak_form);
-    launch_final_lak_form(V, st_);
   }
 }
 
@@ -1121,6 +1132,10 @@ void Plan::launch_final_table(int l, FinalTable& T, bool ids, const char* stage)
   FinalView V{};
   V.ids = M.ids;
   V.ci = M.ci;
+  if (!M.quad) {
+    V.fptr = M.fptr;
+    V.cface = M.cface;
+  }
   V.tptr = M.tptr;
   V.trow = M.trow;
   V.trow_x = M.rows_x ? reinterpret_cast<const int32_t*>(M.trow) : nullptr;
@@ -1131,36 +1146,33 @@ void Plan::launch_final_table(int l, FinalTable& T, bool ids, const char* stage)
   // offsets of M (boundary scan, SLAK positions) and the positions of M1;
   // writes every output position and, for the output level, the quads (and
   // the LAK form)
-  // (several meshes: the LAK form is written by a launch of its own after it)
+  // (several meshes: the LAK form is written by a launch of its own)
   const bool multi = final_table(T);
-  double reads = 0, writes = 0, lak_form = 0;
+  double reads = 0, writes = 0;
   for (int j : T.jobs) {
     const MeshJob& J = jobs_[j];
     const double mnnz = (double)J.nnz[l - 2], mnv = (double)J.nv[l - 2], mne = (double)J.ne[l - 2];
     const double nnz1 = (double)J.nnz[l - 1], nv1 = (double)J.nv[l - 1], nf1 = (double)J.nf[l - 1];
     const double ne1 = (double)J.ne[l - 1];
-    reads += (M.rows_x ? 16.0 : 20.0) * mnnz + 4.0 * mnv + (M.blk ? 4.0 * mne : 0.0) + (scheme_ == kSLAK ? 4.0 * mnnz : 0.0) + 16.0 * nv1;
+    reads += (M.rows_x ? 16.0 : 20.0) * mnnz + (M.quad ? 0.0 : 4.0 * mnnz + 4.0 * ((double)J.nf[l - 2] + 1)) + 4.0 * mnv + (M.blk ? 4.0 * mne : 0.0) + (scheme_ == kSLAK ? 4.0 * mnnz : 0.0) + 16.0 * nv1;
     writes += 16.0 * nv1 + 16.0 * nf1 + 16.0 * ne1;
     if (ids) {
       writes += 16.0 * nnz1;
-      if (J.out_ptr) (multi ? lak_form : writes) += 4.0 * (nnz1 + 1) + 16.0 * nnz1;
+      if (J.out_ptr && !multi) writes += 4.0 * (nnz1 + 1) + 16.0 * nnz1;
     }
   }
   {
     ProfScope ps(st_, stage, reads + writes);
     launch_final(scheme_, V, ids, st_);
   }
-  if (multi && lak_form > 0) {
-    ProfScope ps(st_, "lak_form", lak_form);
-    launch_final_lak_form(V, st_);
-  }
 }
 
 void Plan::record_level(int l) {
   LevelPlan& L = levels_[l - 1];
   if (l > 1) {
-    launch_final_table(l, L.fin, true, "refine_vertex_final_quad");
-    launch_final_table(l, L.pos, false, "refine_vertex_pos_quad");
+    const bool quad = levels_[l - 2].quad;
+    launch_final_table(l, L.fin, true, quad ? "refine_vertex_final_quad" : "refine_vertex_final_poly");
+    launch_final_table(l, L.pos, false, quad ? "refine_vertex_pos_quad" : "refine_vertex_pos_poly");
     if (!L.deep.empty()) launch_deep(l, L.deep);
   }
   if (L.segs.empty()) return;  // every mesh of the level was fused
@@ -1255,6 +1267,10 @@ void Plan::launch(bool include_analysis) {
     record_analysis(L1);
   }
   for (int l = 1; l <= (int)levels_.size(); ++l) record_level(l);
+  if (!lak_.segs.empty()) {
+    ProfScope ps(st_, "lak_form", lak_.bytes);
+    launch_lak_form(lak_.d_segs, lak_.d_block_seg, (int64_t)lak_.block_seg.size(), st_);
+  }
 }
 
 void Plan::run_graph() {

@@ -55,10 +55,19 @@ struct MeshJob {
 struct FinalTable {
   std::vector<int> jobs;
   std::vector<FinalSeg> segs;
-  std::vector<int32_t> block_seg, lak_seg;
+  std::vector<int32_t> block_seg;
   FinalSeg* d_segs = nullptr;
-  int32_t *d_block_seg = nullptr, *d_lak_seg = nullptr;
+  int32_t* d_block_seg = nullptr;
   bool empty() const { return segs.empty(); }
+};
+
+// The LAK forms of every mesh of those tables that has one, in one launch.
+struct LakTable {
+  std::vector<LakSeg> segs;
+  std::vector<int32_t> block_seg;
+  LakSeg* d_segs = nullptr;
+  int32_t* d_block_seg = nullptr;
+  double bytes = 0;
 };
 
 // rows per block and LDS row tile (entries) of the first level's numbering
@@ -234,7 +243,8 @@ class Plan {
   void add_final_seg(FinalTable& T, int l, int job, const SegDesc& m, const float4* P1, float4* positions);
   void launch_final_table(int l, FinalTable& T, bool ids, const char* stage);
   void launch_deep(int l, FinalTable& T);
-  void plan_blocks(FinalTable& T, bool deep);
+  LakTable lak_;
+  void plan_blocks(FinalTable& T, bool quad, bool deep);
   void set_final_table(FinalView& V, const FinalTable& T) const;
   // single mesh: the first level's edge numbering ran during the analysis
   // read-back (the level then launches its face points only)
