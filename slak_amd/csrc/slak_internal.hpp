@@ -96,7 +96,7 @@ void launch_final(int scheme, const FinalView& V, bool ids, hipStream_t st);
 // three levels back, whose structure V holds, and the positions of the level
 // before the output
 void launch_final_deep(const FinalView& V, hipStream_t st);
-constexpr int kDeepEdgeUnit = 64;  // edges per block
+constexpr int kDeepEdgeUnit = 32;  // edges per block
 // the LAK form (ptr, vals) of the meshes that share their last level's launch
 // (which leaves it out)
 void launch_lak_form(const LakSeg* segs, const int32_t* block_seg, int64_t nblocks, hipStream_t st);

@@ -2062,14 +2062,21 @@ __device__ __forceinline__ Quads4 deep_corner(const FinalView& V, const FinalMes
 //   psi_0 = (A_j, Y_j, Z_j, Bin_j)        psi_1 = (X, Y_{j+1}, Z_j, Y_j)
 //   psi_2 = (X, Y_j, Z_{j-1}, Y_{j-1})    psi_3 = (A_j, Bout_j, Z_{j-1}, Y_j)
 // after each, Bin_j and Bout_j being the edge points of A_j's other M edges in
-// Z_j and Z_{j-1}. The row loads the four Y (64 contiguous bytes), Z, A and X, and
-// the eight Bin / Bout (pairs of neighbours). Lane 4j + m then forms psi_m and the
-// edge point of M1's edge from Y_j to its neighbour m, (neighbour + Y_j + psi_m +
-// psi_{m-1}) / 4; the vertex points of the Y_j and of X are formed one component
-// per lane, their terms picked in row order by address.
+// Z_j and Z_{j-1}. Lane 4j + m loads the four corners of psi_m (the quads of
+// lanes share lines; its neighbour of Y_j and Y_j itself are among them) and
+// forms psi_m and the edge point of M1's edge from Y_j to its neighbour m,
+// (neighbour + Y_j + psi_m + psi_{m-1}) / 4; the vertex points of the Y_j and of
+// X are formed one component per lane, their terms picked in row order by
+// address. What the kernel waits for is latency: seven waves a SIMD, each for
+// its chain of half-edges, corners, positions and for the stores before its
+// next loads (sending all positions' stores to a few lines, so without their
+// HBM writes, gave 1.1 of 3.9 ms; half the vector instructions gave nothing).
+// So a block takes two edges a row with every load before the first store:
+// 4096 meshes 3.90 -> 3.69 ms. Four edges a row (79 registers instead of 61)
+// 3.82, one or four without loads ahead 3.90.
 constexpr int kRows = kBlock / 16;
 constexpr int kEdgeIter = kDeepEdgeUnit / kRows;  // edges per row and unit
-constexpr int kRowE = 33;                   // float4 of a row: p 0-15, psi 16-31, one pad (rows start 4 banks apart)
+constexpr int kRowE = 33;                   // float4 of a row: neighbours of the Y 0-15, psi 16-31, one pad (rows start 4 banks apart)
 constexpr int kRowX = 9 * kEdgeIter + 1;    // per edge: psi_1 and Y of j = 0 .. 3, X
 constexpr int kEdgeLds = (kRowE + kRowX) * kRows;  // float4
 
@@ -2080,50 +2087,76 @@ __device__ __forceinline__ void deep_edges(const FinalView& V, const FinalMesh& 
   const float4* __restrict__ P1 = S.P1;
   float4* __restrict__ out = S.out_verts;
   float* __restrict__ outf = reinterpret_cast<float*>(S.out_verts);
-  const int row = threadIdx.x >> 4, i = threadIdx.x & 15, m = i & 3, j = i >> 2, jp = (j + 3) & 3;
+  const int row = threadIdx.x >> 4, i = threadIdx.x & 15, m = i & 3, j = i >> 2;
   const bool odd = (j & 1) != 0, side = (j & 2) != 0;
   float4* const re = lds + row * kRowE;
   float4* const rx = lds + kRows * kRowE + row * kRowX;
   const float* const ref = reinterpret_cast<const float*>(re);
   uint32_t order = 0;  // per edge: t before next(t), s before next(s)
+  // All loads of an edge come before the stores of the edge before it (a wait
+  // for a load also waits for the stores issued before it): the half-edges and
+  // their corners for the unit, the positions one edge ahead. A row beyond the
+  // unit's edges repeats the last one and stores nothing.
+  int32_t tq[kEdgeIter], sq[kEdgeIter], idq[kEdgeIter];
+  int2 cq[kEdgeIter];
 #pragma unroll
   for (int it = 0; it < kEdgeIter; ++it) {
-    const int r = row + it * kRows;
-    if (r >= cnt) break;
-    const int32_t e = first + r;
-    const int2 o = V.own[S.eb + e];
-    const int32_t t = o.x - cb, s1 = o.y - cb;
-    const bool tt = (t & 3) != 3, ss = (s1 & 3) != 3;
-    order |= ((tt ? 1u : 0u) | (ss ? 2u : 0u)) << (2 * it);
+    const int2 o = V.own[S.eb + first + min(row + it * kRows, cnt - 1)];
+    tq[it] = o.x - cb;
+    sq[it] = o.y - cb;
+  }
+#pragma unroll
+  for (int it = 0; it < kEdgeIter; ++it) {
     // the row's halves hold the face of t and the face of its twin, each quad
     // the face's corners from the half-edge's own on
-    const int32_t a = side ? s1 : t, h = a >> 2;
+    const int32_t a = side ? sq[it] : tq[it];
     const int32_t corner = cb + ((a & ~3) | ((a + m) & 3));
-    const int32_t id = V.ids[corner] - vb;
-    const int2 cc = V.ci[corner];
-    const int32_t ce = clampi(cc.x, emax), cg = (cc.y - cb) >> 2;  // edge, face across it
+    idq[it] = V.ids[corner] - vb;
+    cq[it] = V.ci[corner];
+  }
+  struct Row {
+    int32_t Y_id;
+    float4 r1, r2, r3, r4;  // the four corners of psi_m, in order
+  };
+  const bool even = (m & 1) == 0;
+  auto load = [&](int it) __attribute__((always_inline)) {
+    Row R;
+    const int32_t e = first + min(row + it * kRows, cnt - 1);
+    const int32_t a = side ? sq[it] : tq[it], h = a >> 2, id = idq[it];
+    const int32_t ce = clampi(cq[it].x, emax), cg = (cq[it].y - cb) >> 2;  // edge, face across it
     const int32_t I0 = quad_lane_i<0>(id), I1 = quad_lane_i<1>(id), I2 = quad_lane_i<2>(id), I3 = quad_lane_i<3>(id);
     const int32_t C1 = quad_lane_i<1>(ce), C3 = quad_lane_i<3>(ce);
     const int32_t gc = quad_lane_i<1>(cg), gd = quad_lane_i<3>(cg);
     const int32_t Zc = odd ? ((a & ~3) | ((a + 1) & 3)) : a;
-    const int32_t Y_id = 4 * e + (odd ? (side ? 3 : 2) : (I0 > I1 ? 1 : 0));
+    R.Y_id = 4 * e + (odd ? (side ? 3 : 2) : (I0 > I1 ? 1 : 0));
     const int32_t across = row_ror_i<8>(4 * C1 + (I1 > I2 ? 1 : 0));  // the other half's
     const int32_t Bin = odd ? 4 * C1 + 2 + (h > gc ? 1 : 0) : 4 * C3 + (I0 > I3 ? 1 : 0);
     const int32_t Bout = odd ? 4 * C3 + 2 + (h > gd ? 1 : 0) : across;
-    const float4 p = P1[m == 0 ? (odd ? S.nv + h : I0) : m == 1 ? B.fM + Zc : m == 2 ? B.eM + Y_id : B.epN + e];
-    float4 b = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (m == 0 || m == 3) b = P1[B.eM + (m == 0 ? Bin : Bout)];
-    const float4 A = quad_lane<0>(p), Z = quad_lane<1>(p), Y = quad_lane<2>(p), X = quad_lane<3>(p);
-    const float4 Zp = row_ror<4>(Z), Yn = row_ror<12>(Y), Yp = row_ror<4>(Y);
-    const bool atA = m == 0 || m == 3;
-    const float4 psi = face_point(f4sel(atA, A, X), f4sel(m == 1, Yn, f4sel(m == 3, b, Y)), f4sel(m < 2, Z, Zp),
-                                  f4sel(m == 0, b, f4sel(m == 2, Yp, Y)));
-    const float4 nbr = f4sel(m == 0, A, f4sel(m == 1, Z, f4sel(m == 2, X, Zp)));
+    const int32_t Zq = row_ror_i<4>(Zc), Yn_id = row_ror_i<12>(R.Y_id), Yp_id = row_ror_i<4>(R.Y_id);
+    R.r1 = P1[m == 0 || m == 3 ? (odd ? S.nv + h : I0) : B.epN + e];
+    R.r2 = P1[B.eM + (even ? R.Y_id : m == 1 ? Yn_id : Bout)];
+    R.r3 = P1[B.fM + (m < 2 ? Zc : Zq)];
+    R.r4 = P1[B.eM + (!even ? R.Y_id : m == 0 ? Bin : Yp_id)];
+    return R;
+  };
+  Row ahead = load(0);
+#pragma unroll
+  for (int it = 0; it < kEdgeIter; ++it) {
+    const int r = row + it * kRows;
+    const Row R = ahead;
+    if (it + 1 < kEdgeIter) ahead = load(it + 1);
+    if (r >= cnt) break;
+    const bool tt = (tq[it] & 3) != 3, ss = (sq[it] & 3) != 3;
+    order |= ((tt ? 1u : 0u) | (ss ? 2u : 0u)) << (2 * it);
+    const float4 r1 = R.r1, r2 = R.r2, r3 = R.r3, r4 = R.r4;
+    const int32_t Y_id = R.Y_id;
+    const float4 psi = face_point(r1, r2, r3, r4);
+    const float4 nbr = f4sel(even, r1, r3), Y = f4sel(even, r2, r4);
     const bool zfirst = j == 0 || (j == 1 && !tt) || (j == 3 && !ss);  // Z_j before Z_{j-1}
     const int32_t slot = m == 0 ? 0 : m == 2 ? 1 : ((m == 1) == zfirst ? 2 : 3);
-    re[i] = p;
+    re[i] = nbr;
     re[16 + i] = psi;
-    if (m) rx[9 * it + (m == 3 ? 8 : m == 2 ? 4 + j : j)] = f4sel(m == 1, psi, p);
+    if (m) rx[9 * it + (m == 2 ? 8 : m == 3 ? 4 + j : j)] = f4sel(m == 1, psi, f4sel(m == 2, nbr, Y));
     const float4 q = f4mul(f4add(f4add(f4add(nbr, Y), psi), quad_prev(psi)), 0.25f);
     float4* const d = out + (B.eM1 + 4 * Y_id + slot);
     if (V.stream)
@@ -2136,8 +2169,7 @@ __device__ __forceinline__ void deep_edges(const FinalView& V, const FinalMesh& 
     {
       const int f = 16 * j + m, g = 64 + f;
       const int r0 = odd ? 8 : 12, r1 = odd ? 12 : 8;
-      const int z = 16 * jp + 4 + m;  // Z_{j-1}
-      const int n0 = odd ? f + 12 : z, n1 = odd ? z : f + 12;
+      const int n0 = odd ? f + 8 : f + 12, n1 = odd ? f + 12 : f + 8;  // X and Z_{j-1}
       float sum = 0.f;
       sum = sum + ref[g + (zfirst ? 0 : r0)];
       sum = sum + ref[g + (zfirst ? 4 : r1)];
@@ -2147,13 +2179,14 @@ __device__ __forceinline__ void deep_edges(const FinalView& V, const FinalMesh& 
       sum = sum + ref[zfirst ? f + 4 : n1];
       sum = sum + ref[zfirst ? n0 : f];
       sum = sum + ref[zfirst ? n1 : f + 4];
-      outf[4 * (int64_t)(B.eM + Y_id) + m] = (sum / 4.0f + ref[f + 8] * 2.0f) / 4.0f;
+      const float y = m < 2 ? (m == 0 ? Y.x : Y.y) : (m == 2 ? Y.z : Y.w);
+      outf[4 * (int64_t)(B.eM + Y_id) + m] = (sum / 4.0f + y * 2.0f) / 4.0f;
     }
     wave_lds_fence();  // read before the next edge writes
   }
   // vertex points of the X: lane i forms component m of the row's edge j
   const int r = row + j * kRows;
-  if (r < cnt) {
+  if (j < kEdgeIter && r < cnt) {
     const float* const x = reinterpret_cast<const float*>(rx + 9 * j) + m;
     const int tt = (order >> (2 * j)) & 1 ? 0 : 4, ss = (order >> (2 * j)) & 2 ? 8 : 12;
     float sum = 0.f;
@@ -2254,7 +2287,7 @@ __global__ void __launch_bounds__(kBlock) k_final_deep(FinalView V) {
   const int32_t b1 = b - before, edges = share_of(b1, seg->eratio);
   __shared__ int4 stage[std::max(kStageStride * kBlock, kEdgeLds)];
   if (share_of(b1 + 1, seg->eratio) > edges) {
-    static_assert(kEdgeIter == 4, "a quad of the row's lanes per edge of its X");
+    static_assert(kEdgeIter <= 4, "a quad of the row's lanes per edge of its X");
     const int32_t first = edges * kDeepEdgeUnit;
     deep_edges(V, S, first, min(kDeepEdgeUnit, S.ne - first), reinterpret_cast<float4*>(stage));
     return;
