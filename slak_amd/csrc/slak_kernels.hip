@@ -939,6 +939,10 @@ __device__ __forceinline__ float4 quad_prev(float4 x) {
                      __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x.z), ctrl, 0xF, 0xF, false)),
                      __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x.w), ctrl, 0xF, 0xF, false)));
 }
+template <int K>
+__device__ __forceinline__ int32_t quad_lane_i(int32_t x) {
+  return __builtin_amdgcn_mov_dpp(x, K * 0x55, 0xF, 0xF, false);
+}
 __device__ __forceinline__ int32_t quad_next_i(int32_t x) { return __builtin_amdgcn_mov_dpp(x, 0x39, 0xF, 0xF, false); }
 __device__ __forceinline__ int32_t quad_prev_i(int32_t x) { return __builtin_amdgcn_mov_dpp(x, 0x93, 0xF, 0xF, false); }
 
@@ -1419,6 +1423,14 @@ struct Quads4 {
   int4 a, b, c, d;
 };
 
+// Lanes exchange positions through LDS (quads or rows of 16 lanes, so inside one wave):
+// orders the accesses for the compiler, the hardware keeps a wave's in order.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // face, successor and predecessor of a mesh's corner t (all mesh-local)
 template <bool QUAD>
 __device__ __forceinline__ void final_nbrs(const FinalView& V, const FinalMesh& S, int32_t t, int32_t& f, int32_t& tn,
@@ -1436,8 +1448,9 @@ __device__ __forceinline__ void final_nbrs(const FinalView& V, const FinalMesh& 
 
 // Corner t (mesh-local) of M in mesh S: returns its 16 output ids (IDS),
 // which the block stages in LDS.
+// rows: this lane's quad of lanes' 4 x kStageStride float4 of LDS (QUAD, LAK).
 template <bool QUAD, int SCHEME, bool BND, bool IDS, bool EARLY>
-__device__ __forceinline__ Quads4 final_corner(const FinalView& V, const FinalMesh& S, int32_t t) {
+__device__ __forceinline__ Quads4 final_corner(const FinalView& V, const FinalMesh& S, int32_t t, float4* rows) {
   // QUAD: every lane of a quad runs (nnz = 4 nf, meshes and blocks hold whole
   // quads): the quad's four lanes load their own corner once; w (next corner's
   // vertex), u and the in-half-edge's (edge, twin) come from the
@@ -1598,7 +1611,8 @@ __device__ __forceinline__ Quads4 final_corner(const FinalView& V, const FinalMe
     else
       *d = q;
   }
-  if (!own) return q4;
+  constexpr bool kGroups = QUAD && SCHEME == kLAK;  // whole quads of lanes store the groups below
+  if (!kGroups && !own) return q4;
   // edge points of the M1 edges around ep(e1), by lower end point then the
   // faces of the half-edges lower -> upper and upper -> lower
   const bool inner = !BND || s1 >= 0;
@@ -1623,7 +1637,32 @@ __device__ __forceinline__ Quads4 final_corner(const FinalView& V, const FinalMe
   // (cached when the next kernel reads them)
   float4* __restrict__ eo = out + epb2;
   const float4 q_fG = f4mul(f4add(f4add(f4add(PG, Pe), fpsn), fps), 0.25f);
-  if (SCHEME == kLAK) {
+  if (kGroups) {
+    // an owner's points are one group of 64 contiguous bytes: the four lanes
+    // of the quad store them side by side, one owner after the other. (A lane
+    // storing its own four takes four times as many L1 accesses, 128 of about
+    // 600 per 64 corners, and the L1's are what the kernel is bound by.)
+    const int32_t base1 = 4 * e1 - bl1;
+    const int lane = threadIdx.x & 3;
+    float4* const mine = rows + kStageStride * lane;
+    if (own) {
+      mine[i_vh - base1] = q_vh;
+      mine[i_wh - base1] = q_wh;
+      mine[i_fF - base1] = q_fF;
+      if (inner) mine[i_fG - base1] = q_fG;
+    }
+    wave_lds_fence();
+    const int32_t len = own ? (inner ? 4 : 3) : 0;
+    auto put = [&](int k, int32_t b, int32_t n) __attribute__((always_inline)) {
+      if (lane < n) eo[b + lane] = rows[kStageStride * k + lane];
+    };
+    put(0, quad_lane_i<0>(base1), quad_lane_i<0>(len));
+    put(1, quad_lane_i<1>(base1), quad_lane_i<1>(len));
+    put(2, quad_lane_i<2>(base1), quad_lane_i<2>(len));
+    put(3, quad_lane_i<3>(base1), quad_lane_i<3>(len));
+    wave_lds_fence();  // read before the block's quads overwrite it
+    if (!own) return q4;
+  } else if (SCHEME == kLAK) {
     eo[i_vh] = q_vh;
     eo[i_wh] = q_wh;
     eo[i_fF] = q_fF;
@@ -1881,13 +1920,14 @@ __global__ void __launch_bounds__(kBlock) k_final(FinalView V) {
   }
   const int32_t t0 = (b - before) * kBlock, cnt = min(kBlock, S.nnz - t0);
   const int32_t t = t0 + (int32_t)threadIdx.x;
+  __shared__ int4 stage[IDS || (QUAD && SCHEME == kLAK) ? kStageStride * kBlock : 1];
+  float4* const rows = reinterpret_cast<float4*>(stage) + (QUAD && SCHEME == kLAK ? kStageStride * (threadIdx.x & ~3) : 0);
   if (!IDS) {  // positions only
-    if ((int)threadIdx.x < cnt) final_corner<QUAD, SCHEME, BND, false, MULTI>(V, S, t);
+    if ((int)threadIdx.x < cnt) final_corner<QUAD, SCHEME, BND, false, MULTI>(V, S, t, rows);
     return;
   }
-  __shared__ int4 stage[kStageStride * kBlock];
   Quads4 q4{};
-  if ((int)threadIdx.x < cnt) q4 = final_corner<QUAD, SCHEME, BND, true, MULTI>(V, S, t);
+  if ((int)threadIdx.x < cnt) q4 = final_corner<QUAD, SCHEME, BND, true, MULTI>(V, S, t, rows);
   store_quads<MULTI>(S, q4, stage, t0, cnt, S.nnz);
 }
 
@@ -1933,10 +1973,6 @@ __device__ __forceinline__ float4 row_ror(float4 x) {
   return make_float4(__int_as_float(row_ror_i<N>(__float_as_int(x.x))), __int_as_float(row_ror_i<N>(__float_as_int(x.y))),
                      __int_as_float(row_ror_i<N>(__float_as_int(x.z))), __int_as_float(row_ror_i<N>(__float_as_int(x.w))));
 }
-template <int K>
-__device__ __forceinline__ int32_t quad_lane_i(int32_t x) {
-  return __builtin_amdgcn_mov_dpp(x, K * 0x55, 0xF, 0xF, false);
-}
 // sizes of N, M and M1 of one mesh, as vertex bases of the output
 struct DeepBase {
   int32_t epN;   // M vertex ep(edge 0 of N) = N vertices + N faces
@@ -1952,14 +1988,6 @@ struct DeepBase {
     eM1 = fM1 + 4 * S.nnz;
   }
 };
-
-// Lanes exchange positions through LDS (rows of 16 lanes, so inside one wave):
-// orders the accesses for the compiler, the hardware keeps a wave's in order.
-__device__ __forceinline__ void wave_lds_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // What the vector memory unit pays for is lines per four neighbouring lanes:
 // a gather whose every lane has its own line takes four times as long as one
