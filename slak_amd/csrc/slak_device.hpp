@@ -631,7 +631,7 @@ struct FinalView {
   const int32_t* mpos;   // M^T position per corner (SLAK)
   const int2* own;       // k_final_deep, whose union and meshes are those of N, three levels before
                          // the output: (owner corner, twin) per edge, from base eb of each mesh
-  int32_t stream;        // k_final_deep: the launch's positions exceed kStreamBytes
+  int32_t stream;        // the launch's positions exceed kStreamBytes
   FinalSeg one;          // a single mesh
   const FinalSeg* segs;  // several meshes: device table, and the mesh of every block
   const int32_t* block_seg;

@@ -1084,7 +1084,7 @@ void Plan::add_final_seg(FinalTable& T, int l, int job, const SegDesc& m, const 
 
 // Output positions above which a launch's edge points bypass the caches: 7/8
 // of the 256 MB last-level cache (measured between 201 MB, where it costs 4 %,
-// and 268 MB, where it gives 7 %).
+// and 268 MB, where it gives 7 % (k_final_deep) and 13 % (k_final)).
 constexpr double kStreamBytes = 224.0 * (1 << 20);
 
 // k_final_deep over the meshes of table T, whose last level is l + 1, from the
@@ -1148,7 +1148,7 @@ void Plan::launch_final_table(int l, FinalTable& T, bool ids, const char* stage)
   // the LAK form)
   // (several meshes: the LAK form is written by a launch of its own)
   const bool multi = final_table(T);
-  double reads = 0, writes = 0;
+  double reads = 0, writes = 0, positions = 0;
   for (int j : T.jobs) {
     const MeshJob& J = jobs_[j];
     const double mnnz = (double)J.nnz[l - 2], mnv = (double)J.nv[l - 2], mne = (double)J.ne[l - 2];
@@ -1156,11 +1156,13 @@ void Plan::launch_final_table(int l, FinalTable& T, bool ids, const char* stage)
     const double ne1 = (double)J.ne[l - 1];
     reads += (M.rows_x ? 16.0 : 20.0) * mnnz + (M.quad ? 0.0 : 4.0 * mnnz + 4.0 * ((double)J.nf[l - 2] + 1)) + 4.0 * mnv + (M.blk ? 4.0 * mne : 0.0) + (scheme_ == kSLAK ? 4.0 * mnnz : 0.0) + 16.0 * nv1;
     writes += 16.0 * nv1 + 16.0 * nf1 + 16.0 * ne1;
+    positions += 16.0 * (nv1 + nf1 + ne1);
     if (ids) {
       writes += 16.0 * nnz1;
       if (J.out_ptr && !multi) writes += 4.0 * (nnz1 + 1) + 16.0 * nnz1;
     }
   }
+  V.stream = ids && positions > kStreamBytes;
   {
     ProfScope ps(st_, stage, reads + writes);
     launch_final(scheme_, V, ids, st_);

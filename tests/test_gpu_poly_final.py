@@ -71,3 +71,12 @@ def test_mixed_batch_from_polygons(scheme, deepest, monkeypatch):
     finally:
         for d in dev:
             d.freeAndReset()
+
+
+@pytest.mark.parametrize("shape", ["closed", "open"])
+def test_output_beyond_the_last_level_cache(shape, monkeypatch):
+    """More than 224 MiB of positions: k_final's edge points are stored past
+    the caches, in whole groups and in the boundary's groups of three."""
+    m = g.torus(510, 505, seed=6) if shape == "closed" else g.open_grid(505, 510, sigma=1e-3)
+    want = _chain(monkeypatch, lambda: subdivide_host(m, 3, LAK)[0])
+    _assert_same(subdivide_host(m, 3, LAK)[0], want, LAK)
