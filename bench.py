@@ -85,19 +85,20 @@ def stage_roofline(prof, stage=None):
 
 
 def output_level_roofline(prof):
-    """The several-mesh output level as one unit: k_final (refine_vertex_final_quad)
-    and the LAK-form launch that follows it (lak_form), their algorithmic
-    bytes over their summed HIP-event durations. None when no LAK form is
-    written separately (SLAK, or one mesh)."""
+    """The several-mesh output levels as one unit: their k_final launches
+    (refine_vertex_final_quad, and _poly for meshes of two levels) and the
+    LAK-form launch of all of them (lak_form), their algorithmic bytes over
+    their summed HIP-event durations. None when no LAK form is written
+    separately (SLAK, or one mesh)."""
     st = {s["name"]: s for s in prof["stages"]}
     if CFG4_STAGE not in st or "lak_form" not in st:
         return None
-    a, b = st[CFG4_STAGE], st["lak_form"]
-    n = a["launches"]
-    byts = (a["bytes"] + b["bytes"]) / n
-    ms = (a["total_ms"] + b["total_ms"]) / n
+    finals = [n for n in (CFG4_STAGE, CFG4_STAGE.replace("_quad", "_poly")) if n in st]
+    n = sum(st[k]["launches"] for k in finals)
+    byts = sum(st[k]["bytes"] for k in finals + ["lak_form"]) / n
+    ms = sum(st[k]["total_ms"] for k in finals + ["lak_form"]) / n
     gbps = byts / (ms * 1e-3) / 1e9
-    return {"stages": [CFG4_STAGE, "lak_form"], "bytes_per_launch": int(byts), "us_per_launch": round(ms * 1e3, 2),
+    return {"stages": finals + ["lak_form"], "bytes_per_launch": int(byts), "us_per_launch": round(ms * 1e3, 2),
             "achieved": round(gbps, 1), "frac": round(gbps / HBM_PEAK_GBPS, 4)}
 
 
@@ -308,22 +309,24 @@ def serve_leg(n_requests, qps_fraction, scheme, seed=5, keep=()):
 
 # kernel of each roofline stage ({s}: 0 LAK, 1 SLAK; multi: the table path)
 STAGE_KERNELS = {
-    "refine_vertex_final_quad": r"k_final<{s}, \w+, {multi}, true>",
-    "refine_vertex_pos_quad": r"k_final<{s}, \w+, {multi}, false>",
+    "refine_vertex_final_quad": r"k_final<true, {s}, \w+, {multi}, true>|k_final_deep<{multi}>",
+    "refine_vertex_final_poly": r"k_final<false, {s}, \w+, {multi}, true>",
+    "refine_vertex_pos_quad": r"k_final<true, {s}, \w+, {multi}, false>",
+    "refine_vertex_pos_poly": r"k_final<false, {s}, \w+, {multi}, false>",
     "refine_vertex_quad": r"k_level<true, {s},",
     "refine_vertex_poly": r"k_level<false, {s},",
-    "facepoints_quad": r"k_faces<true>",
-    "facepoints_poly": r"k_faces<false>",
+    "facepoints_quad": r"k_faces<true,",
+    "facepoints_poly": r"k_faces<false,",
     "gather": r"k_gather<",  # the gather, count and transpose stages are one launch
-    "count_quad": r"k_gather<true>",
-    "count_poly": r"k_gather<false>",
+    "count_quad": r"k_gather<true,",
+    "count_poly": r"k_gather<false,",
     "lak_form": r"k_lak_form",
-    "transpose_quad": r"k_gather<true>",
-    "transpose_poly": r"k_gather<false>",
+    "transpose_quad": r"k_gather<true,",
+    "transpose_poly": r"k_gather<false,",
     "spgemm_symbolic_quad": r"k_symbolic<true, {s}>",
     "spgemm_symbolic_poly": r"k_symbolic<false, {s}>",
-    "number_facepoints_quad": r"k_number_faces<true, {s}>",
-    "number_facepoints_poly": r"k_number_faces<false, {s}>",
+    "number_facepoints_quad": r"k_number_faces<true, {s},",
+    "number_facepoints_poly": r"k_number_faces<false, {s},",
 }
 PMC_WORKLOADS = ("cfg4", "cfg2", "cfg3")
 

@@ -5,12 +5,13 @@
 //                 (sortKeyValuePairsSegmentedInPlace, LAKCatmullClarkKernels.cuh:147-180);
 //                 valence per vertex (spmv_right with ones, LAKCatmullClarkImpl.cu:347-356)
 //                 and the corners of M^T's rows into fixed slots per vertex
-//   symbolic      M^T (csr2cscEx2, LAKCatmullClarkImpl.cu:381-423) and row sizing
-//                 of the mapped SpGEMM -> edges owned per vertex; rows sorted and
-//                 stored with their in-neighbours at offsets scanned in the same
-//                 pass (scan_exclusive, cub_wrappers.cuh:30-43)
-//   number        mapped SpGEMM rows -> E numbering: edge id and twin of
-//                 every corner's half-edge, boundary flags
+//   symbolic      row sizing of the mapped SpGEMM -> edges owned per vertex;
+//                 corner and edge counts summed per tile of vertices
+//   number        offsets from those sums (scan_exclusive, cub_wrappers.cuh:30-43),
+//                 M^T's rows sorted, with their in-neighbours (csr2cscEx2,
+//                 LAKCatmullClarkImpl.cu:381-423); mapped SpGEMM rows -> E numbering:
+//                 edge id and twin of every corner's half-edge, boundary flags
+//   first_small   all of it in one block for a small mesh
 // Every level:
 //   face points   left mapped SpMV fp = M^T P / order (spmv.cuh:64-81)
 //   refine        per corner: edge points (calculateInternal/ExternalEdgepoints),
@@ -22,15 +23,16 @@
 //                 (LAKCatmullClarkImpl.cu:200-235) and boundary rule
 //                 (LAKCatmullClarkKernels.cuh:464-511); the vertex rows of the
 //                 refined M^T
-// Last two levels of a quad chain:
-//   final         from the quad mesh M two levels back: the output quads,
-//                 edge, face and vertex points of the level (or its positions
-//                 only, for the level before it); several meshes per launch
-//                 through work-unit tables
+// Last levels of a chain:
+//   final         from the mesh M two levels back (quads, or the caller's
+//                 polygons): the output quads, edge, face and vertex points of
+//                 the level (or its positions only, for the level before it);
+//                 several meshes per launch through a table
+//   final_deep    the output level of a closed LAK mesh from three levels back
 //   LAK form      several meshes: the output level's ptr / vals in a launch
 //                 of their own (createQuadColPtr / createQuadVals)
 // All kernels are pull-based and atomic-free except the integer valence
-// count and transpose slots, whose result does not depend on atomic order,
+// count and row slots, whose result does not depend on atomic order,
 // so every output is bitwise deterministic.
 #include <hip/hip_runtime.h>
 
