@@ -576,7 +576,7 @@ struct RefineView {
   int32_t* ntptr;
   int2* ntrow;
   int2* nci;
-  int32_t* nbnd;         // next level's union edge boundary flags, or null: closed
+  int32_t* nbnd;         // next level's union edge boundary flags (LAK: ranks, its blk), or null: closed
   int32_t* nmpos;        // next level's M^T positions (SLAK)
   int2* nown;            // next level's edge owners (owner corner, twin), for the meshes with next_own >= 0
   int32_t next_nv;       // next level's union vertices and corners (end of its M^T)

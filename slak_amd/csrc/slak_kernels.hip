@@ -1176,11 +1176,15 @@ __device__ __forceinline__ void corner_store(const RefineView& R, const SegK& K,
       const int32_t nlast = neb + snnz + 2 * (K.emax + 1) - 1;
       if (SCHEME == kLAK) {
         const int32_t base1 = min(neb + 4 * c.e1 - c.bl1, nlast - (c.s1 < 0 ? 2 : 3));
-        const int32_t b = c.s1 < 0 ? 1 : 0;
-        nbnd[base1] = b;
-        nbnd[base1 + 1] = b;
-        nbnd[base1 + 2] = 0;
-        if (c.s1 >= 0) nbnd[base1 + 3] = 0;
+        // the next level's boundary ranks, not its flags: the halves of the
+        // bl(e) boundary edges before e, and e's own two come first. (Against
+        // flags and a scan launch per level: open grid 301 x 203, 3 levels 124 ->
+        // 118 us a call, 64 x 64, 4 levels 108 -> 100, 500 x 400 unchanged.)
+        const int32_t b = c.s1 < 0 ? 1 : 0, bl = 2 * c.bl1;
+        nbnd[base1] = bl;
+        nbnd[base1 + 1] = bl + b;
+        nbnd[base1 + 2] = bl + 2 * b;
+        if (c.s1 >= 0) nbnd[base1 + 3] = bl;
       } else if (c.s1 < 0) {
         nbnd[min(neb + 2 * snnz + c.bl1, nlast)] = 1;
       }
@@ -1200,6 +1204,7 @@ __device__ __forceinline__ void corner_store(const RefineView& R, const SegK& K,
 //                  4t+2 -> 4 prev(t) + 1, 4t+3 -> 4 s0
 //   LAK edge ids   edge point e owns its edges to the two end points, then to
 //                  the face points, ranked by the smaller id: base(e) = 4e - bl(e)
+//   LAK bl(e)      of its edges: 2 bl(e), for a boundary edge e + 0, 1, 2
 //   SLAK edge ids  vertices own one edge per corner, numbered by the corner's
 //                  M^T storage position; face points one per corner
 //                  (nnz + corner); boundary edge points one (2 nnz + bl(e))

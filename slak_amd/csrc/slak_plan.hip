@@ -726,7 +726,7 @@ void Plan::prepare() {
       mne = std::max(mne, ne);
     }
     est += 2 * (line(mnv + 1, 4) + 2 * line(mnnz, 8) + line(mnnz, 4));
-    est += 2 * line(mne + 1, 4) + line(scan_partials_len(mne), 8);
+    est += (lak_scheme ? 4 : 2) * line(mne + 1, 4) + line(scan_partials_len(mne), 8);
     est += (size_t)1 << 20;
     if (Lmax >= 1) arena_.reserve(est);
   }
@@ -905,9 +905,19 @@ void Plan::prepare() {
   if (max_ne > 0) {
     int32_t* bnd = arena_.get_n<int32_t>(max_ne);
     int32_t* blk = arena_.get_n<int32_t>(max_ne + 1);
+    // LAK: later levels receive their ranks from the level before, which reads
+    // its own meanwhile (two alternating buffers)
+    int32_t* ranks[2] = {nullptr, nullptr};
+    if (lak_scheme && Lstruct >= 2) ranks[0] = arena_.get_n<int32_t>(max_ne + 1);
+    if (lak_scheme && Lstruct >= 3) ranks[1] = arena_.get_n<int32_t>(max_ne + 1);
     for (int l = 1; l <= Lstruct; ++l) {
       LevelPlan& L = levels_[l - 1];
       if (!L.boundary) continue;
+      if (lak_scheme && l >= 2) {
+        L.blk = ranks[l % 2];
+        levels_[l - 2].nbnd = L.blk;
+        continue;
+      }
       if (!(l == 1 && number_early_)) L.bnd = bnd;  // the early numbering wrote level 1's own
       L.blk = blk;
       if (l >= 2) levels_[l - 2].nbnd = bnd;
@@ -1189,7 +1199,7 @@ void Plan::record_level(int l) {
                  4.0 * L.nnz + 16.0 * L.nv + 16.0 * L.nf + (L.quad ? 0.0 : 4.0 * (L.nf + 1)));
     launch_faces(L.quad, L.ids, L.fptr, L.P, (int32_t)L.nf, L.table(), st_);
   }
-  if (L.blk) {
+  if (L.blk && (l == 1 || scheme_ == kSLAK)) {
     ProfScope ps(st_, "scan", 8.0 * ne + 4);
     launch_scan(L.bnd, L.blk, L.ne, d_partial_, late_, st_);
   }

@@ -156,3 +156,21 @@ def test_output_level_from_three_levels_back(name, make):
         c, d = (2, 3) if ss else (3, 2)
         assert [r[0] >> 2 for r in row(X)] == [psi[j, 1] for j in (a, b, c, d)]
         assert [r[1] for r in row(X)] == [eM + Y[j] for j in (a, b, c, d)]
+
+
+@pytest.mark.parametrize("name,make", POLYGONS + CLOSED[:1], ids=[m[0] for m in POLYGONS + CLOSED[:1]])
+def test_boundary_ranks_of_the_refined_mesh(name, make):
+    """The boundary edges before each refined edge, as the owners of the edges
+    hand them on (LAK), over two refinements."""
+    mesh = make()
+    S = M.structure_of(mesh.face_ptr(), mesh.ids, mesh.nverts, M.LAK)
+    for _ in range(2):
+        S1 = M.refine_structure(S, M.LAK)
+        blk = np.concatenate([[0], np.cumsum(S.bnd)]).astype(np.int64)
+        got = np.full(len(S1.bnd), -1, dtype=np.int64)
+        for e in range(len(S.bnd)):
+            b, bl = int(S.bnd[e] != 0), int(blk[e])
+            ranks = [2 * bl, 2 * bl + b, 2 * bl + 2 * b] + ([] if b else [2 * bl])
+            got[4 * e - bl: 4 * e - bl + len(ranks)] = ranks
+        np.testing.assert_array_equal(got, np.concatenate([[0], np.cumsum(S1.bnd)])[:-1])
+        S = S1
