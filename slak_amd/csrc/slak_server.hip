@@ -92,7 +92,7 @@ ChainBound chain_bound(const slak_mesh& m, int levels) {
 // launch per kernel per level over the union of the requests still active at
 // that level, the first level's analysis once per request, every later
 // level's structure in closed form from the level before it, the last level
-// from the quad mesh two levels back. Each slot has its own worker thread
+// from the mesh two or three levels back. Each slot has its own worker thread
 // and stream, so a step starts as soon as requests are pending and a slot is
 // free: requests that arrive while another step is on the GPU run beside it.
 struct slak_server {

@@ -80,3 +80,13 @@ def test_output_beyond_the_last_level_cache(shape, monkeypatch):
     m = g.torus(510, 505, seed=6) if shape == "closed" else g.open_grid(505, 510, sigma=1e-3)
     want = _chain(monkeypatch, lambda: subdivide_host(m, 3, LAK)[0])
     _assert_same(subdivide_host(m, 3, LAK)[0], want, LAK)
+
+
+@pytest.mark.parametrize("scheme", [LAK, SLAK], ids=["LAK", "SLAK"])
+def test_two_levels_of_a_mesh_without_faces(scheme):
+    """Isolated vertices only: accepted by the level-by-level chain, so not
+    handed to the fused level, which has no blocks for it."""
+    none = np.zeros(0, np.int32)
+    m = g.HostMesh(g.TRI, None, none, none, np.ones((5, 4), np.float32))
+    r, _ = subdivide_host(m, 2, scheme)
+    assert len(r.verts) == 5 and len(r.ids) == 0
