@@ -166,7 +166,7 @@ int slak_scan_exclusive_noalloc(const int32_t* in, int32_t* out, uint64_t n, voi
  * one mesh per call) ----
  * slak_batch_create validates the meshes (device pointers, kept by pointer:
  * they must stay valid and unchanged in topology until destroy), runs the
- * first level's analysis for all of them (two blocking round trips) and
+ * first level's analysis for all of them (one blocking round trip) and
  * allocates every buffer of the whole chain, sized in closed form.
  * slak_batch_run recomputes the full chain from the current inputs (positions
  * may change between runs) with one launch per kernel per level over the union
@@ -200,7 +200,7 @@ int slak_batch_destroy(slak_batch* batch);
  * requests to the target level in the batched kernels (one launch per kernel
  * per level over the union of the requests still active at that level; the
  * first level's analysis once, later levels' structure in closed form, the
- * last level from the quad mesh two levels back). Up to `slots` steps run at
+ * last level from the mesh two or three levels back). Up to `slots` steps run at
  * once, each on its own stream, so requests that arrive while others are on
  * the GPU start beside them as soon as a slot and memory are free.
  * Intermediate levels stay resident on the device. The submitted mesh must

@@ -36,7 +36,7 @@ struct MeshJob {
   int32_t* out_ptr = nullptr;
   int32_t* out_vals = nullptr;
   int bad_flags = 0;
-  // the last level is formed by k_final from the quad mesh two levels back;
+  // the last level is formed by k_final from the mesh two levels back;
   // p1: the positions of the level before the output (its only output)
   bool fused = false;
   float4* p1 = nullptr;

@@ -4,7 +4,7 @@
 // CatmullClarkImpl.cu:457-515). Sizes of every level after the first follow
 // from the first level's edge count in closed form (a manifold quad level
 // with n_ext boundary edges refines to n_ext' = 2 n_ext, n_e' = 2 nnz + n_ext),
-// so a call needs two blocking round trips (input validation, first-level
+// so a call needs one blocking round trip (input validation and first-level
 // edge count) plus the final synchronization; levels 2.. are launched back
 // to back on one stream.
 #include <hip/hip_runtime.h>
