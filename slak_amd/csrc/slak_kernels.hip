@@ -1223,7 +1223,6 @@ __device__ __forceinline__ void refine_item(const RefineView& R, int64_t t64) {
   c.t = (int32_t)t64;
   corner_nbrs<QUAD>(R.fptr, R.cface, c.t, c.f, c.tn, c.tp);
   const SegK K = seg_consts<ONE>(R.seg, c.t);
-  if (R.ntptr && t64 == R.nnz - 1) R.ntptr[R.next_nv] = R.next_nnz;  // end of the next level's M^T
   c.v = R.ids[c.t];
   const int2 c1 = R.ci[c.t];
   if (QUAD) {
@@ -1342,6 +1341,9 @@ __device__ __forceinline__ void vertex_item(const RefineView& R, int32_t v) {
     for (int i = 0; i < n; ++i)
       if (ci[prevc(row[i].x)].y < 0) q = f4add(q, f4mul(P[row[i].y], 0.125f));
   }
+  // end of the next level's M^T: written with the last vertex, which every
+  // union that feeds a level has (a union without faces has no corner items)
+  if (NEXT && v == R.nv - 1) R.ntptr[R.next_nv] = R.next_nnz;
   if (!next && dst_final) {
     store_nt(dst + (v - vb), q);
     return;
