@@ -2901,10 +2901,10 @@ int64_t plan_final_blocks(FinalSeg& S, bool quad, bool deep) {
   return total;
 }
 
-// blocks of a launch of V's meshes (0: several meshes, all without faces)
+// blocks of a launch of V's meshes (a mesh without faces has vertex blocks
+// alone, one without vertices none)
 static unsigned final_grid(const FinalView& V) {
-  if (V.segs ? !V.block_seg : V.one.m.nnz <= 0)
-    throw Error(5, "final level: no blocks planned");  // SLAK_ERR_INTERNAL
+  if (V.segs && !V.block_seg) throw Error(5, "final level: no blocks planned");  // SLAK_ERR_INTERNAL
   const int64_t n = V.segs ? V.nblocks : V.one.blocks;
   if (n * kBlock > 0xffffffffll) throw Error(1, "level too large for one launch");
   return (unsigned)n;

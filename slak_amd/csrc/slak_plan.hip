@@ -684,8 +684,8 @@ void Plan::prepare() {
     const bool allow_deep = allow && scheme_ == kLAK && (!d || std::atoi(d) != 0) && (!q || std::atoi(q) != 0);
     for (int j : levels_[0].jobs) {
       MeshJob& J = jobs_[j];
-      J.fused = allow && J.levels >= 2 && (J.levels >= 3 || levels_[0].quad || J.nnz[0] > 0);  // (no faces: nothing to fuse)
-      J.deep = allow_deep && J.levels >= 4 && 2 * J.ne[0] == J.nnz[0];
+      J.fused = allow && J.levels >= 2;
+      J.deep = allow_deep && J.levels >= 4 && J.nnz[0] > 0 && 2 * J.ne[0] == J.nnz[0];  // (no faces: no edge owners)
       J.p1 = nullptr;
       J.p2 = nullptr;
       J.own_base = -1;
