@@ -689,6 +689,7 @@ void Plan::prepare() {
       J.p1 = nullptr;
       J.p2 = nullptr;
       J.own_base = -1;
+      if (J.nnz[0] == 0) faceless_.push_back(j);
     }
   }
   // whether level l of a mesh hands on its positions alone
@@ -1279,6 +1280,10 @@ void Plan::launch(bool include_analysis) {
     record_analysis(L1);
   }
   for (int l = 1; l <= (int)levels_.size(); ++l) record_level(l);
+  // the LAK form of a mesh without faces is the single offset 0, which no
+  // corner item writes
+  for (int j : faceless_)
+    if (jobs_[j].out_ptr) launch_fill_i32(jobs_[j].out_ptr, 1, 0, st_);
   if (!lak_.segs.empty()) {
     ProfScope ps(st_, "lak_form", lak_.bytes);
     launch_lak_form(lak_.d_segs, lak_.d_block_seg, (int64_t)lak_.block_seg.size(), st_);

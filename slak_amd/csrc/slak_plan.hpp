@@ -254,7 +254,7 @@ class Plan {
   bool early_faces_ = false;
   float4* early_p1_ = nullptr;
   int64_t early_p1_cap_ = 0;
-  std::vector<void*> pooled_outputs_;
+  std::vector<int> faceless_;  // jobs without faces
 };
 
 std::string flags_message(int f);
