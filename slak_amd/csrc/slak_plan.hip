@@ -1268,9 +1268,10 @@ void Plan::record_level(int l) {
 void Plan::launch(bool include_analysis) {
   if (levels_.empty()) return;
   replayed_ = include_analysis;
-  if (include_analysis) number_early_ = false;  // the analysis runs again: number in order
   LevelPlan& L1 = levels_[0];
   if (include_analysis) {
+    number_early_ = false;  // the analysis runs again: number in order
+    *late_ = 0;             // (no earlier run is in flight: finish() waits for each)
     launch_setup(nullptr, nullptr, 0, d_state_, n_state_, st_);  // a fill kernel: graph-safe
     record_gather(L1);
     if (P1_) {
@@ -1333,6 +1334,7 @@ void Plan::run_graph() {
     SLAK_HIP_CHECK(hipGraphInstantiate(&exec_, graph_, nullptr, nullptr, 0));
   }
   replayed_ = true;
+  *late_ = 0;
   SLAK_HIP_CHECK(hipGraphLaunch(exec_, st_));
   if (owned_st_) {
     // later work on the caller's default stream sees the results
