@@ -37,6 +37,7 @@ enum : int {
   kFlagDupHalfEdge = 32,
   kFlagDegenerate = 64,
   kFlagOverflow = 128,
+  kFlagChanged = 256,  // a replay found another number of edges than the plan is sized for
 };
 // flags the first-level gather raises for an invalid input mesh; the analysis
 // kernels after it do nothing once one is set (their indices would come from
@@ -192,7 +193,14 @@ struct LevelView {
   int32_t row_cap;         // rows up to this length are processed in registers (4 or 8)
   int32_t rows_per_block;  // numbering: M^T rows per block (64, 128 or 256)
   int32_t tile_entries;    // numbering: entries of the block's LDS row tile
+  int32_t planned;         // 1: the meshes' edges must be those of their descriptors (kFlagChanged)
 };
+
+// The kernels after a replayed analysis: stop is its flags word, null for a
+// chain whose analysis the host has already checked. Once a flag is set the
+// rows, ids and edge pairs they would follow are those of no mesh, or were
+// never written, so they do nothing (the run ends in an error).
+__device__ __forceinline__ bool stopped(const int* stop) { return stop && *stop != 0; }
 
 __device__ __forceinline__ float4 f4add(float4 a, float4 b) {
   return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
@@ -586,6 +594,7 @@ struct RefineView {
   // proportion over the launch; n 0: one run), and their share of the launch
   VertexRuns runs;
   uint64_t vratio;
+  const int* stop;       // see stopped()
 };
 
 // One mesh of a final level computed from the structure of the mesh M
@@ -636,6 +645,7 @@ struct FinalView {
   const FinalSeg* segs;  // several meshes: device table, and the mesh of every block
   const int32_t* block_seg;
   int32_t nblocks;       // several meshes: blocks of the launch
+  const int* stop;       // see stopped()
 };
 
 // One mesh of the LAK form's launch: its first block, a fourth of its output

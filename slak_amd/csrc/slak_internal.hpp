@@ -68,7 +68,7 @@ void launch_copy_probe(const float4* a, float4* b, int64_t n, hipStream_t st);
 // *out = order-sensitive 64-bit digest of bytes at p (out: device, 8 bytes)
 void launch_digest(const void* p, int64_t bytes, uint64_t* out, hipStream_t st);
 void launch_faces(bool quad, const int32_t* ids, const int32_t* fptr, const float4* P, int32_t nf, const SegTable& seg,
-                  hipStream_t st);
+                  const int* stop, hipStream_t st);
 // validates and sizes the rows the gather has placed: owned edges per vertex
 // (L.ecnt) and the sums of tiles and groups (L.pool and L.group_sum zeroed before)
 void launch_symbolic(bool quad, int scheme, const LevelView& L, hipStream_t st);

@@ -461,7 +461,8 @@ __device__ __forceinline__ void faces_item(const int32_t* __restrict__ ids, cons
 
 template <bool QUAD, bool ONE>
 __global__ void k_faces(const int32_t* __restrict__ ids, const int32_t* __restrict__ fptr, const float4* __restrict__ P,
-                        int32_t nf, SegTable seg) {
+                        int32_t nf, SegTable seg, const int* stop) {
+  if (stopped(stop)) return;
   faces_item<QUAD, ONE>(ids, fptr, P, nf, seg, (int32_t)(block_index() * blockDim.x + threadIdx.x));
 }
 
@@ -640,7 +641,12 @@ __global__ void __launch_bounds__(kBlock) k_seg_bounds(LevelView L) {
   uint64_t acc = tiles_before(L, tile, lane, 64) & kOwnedMask;
   for (int32_t v = tile * kBlock + lane; v < b; v += 64) acc += (uint64_t)L.ecnt[v];
   for (int d = 32; d > 0; d >>= 1) acc += __shfl_xor(acc, d, 64);
-  if (lane == 0) L.bounds[k] = (int32_t)acc;
+  if (lane) return;
+  L.bounds[k] = (int32_t)acc;
+  if (L.planned) {
+    const SegDesc& S = L.seg.d[k < L.seg.n ? k : L.seg.n - 1];
+    if ((int64_t)acc != S.eb + (k < L.seg.n ? 0 : S.ne)) atomicOr(L.flags, kFlagChanged);
+  }
 }
 
 // What the host waits for, written straight to its memory by one block (a
@@ -727,8 +733,10 @@ __global__ void __launch_bounds__(kBlock) k_number_faces(LevelView L, int32_t nb
     L.tptr[v] = s;
     L.eptr[v] = e0;
     if (v == L.nv - 1) {
+      const int32_t edges = (int32_t)(row_at[r0 + threadIdx.x + 1] & kOwnedMask);
       L.tptr[L.nv] = s + n;
-      L.eptr[L.nv] = (int32_t)(row_at[r0 + threadIdx.x + 1] & kOwnedMask);
+      L.eptr[L.nv] = edges;
+      if (ONE && L.planned && edges != L.seg.one.ne) atomicOr(L.flags, kFlagChanged);
     }
     // the sorted row to the LDS tile, or straight to its place
     // (by a branch around each store: a pointer that may address LDS or
@@ -1377,6 +1385,7 @@ __device__ __forceinline__ void vertex_item(const RefineView& R, int32_t v) {
 // machine (share_ratio).
 template <bool QUAD, int SCHEME, bool NEXT, bool BND, bool ONE>
 __global__ void __launch_bounds__(kBlock) k_level(RefineView R) {
+  if (stopped(R.stop)) return;
   const int32_t b = (int32_t)(NEXT ? block_index<kRemapLevel>() : block_index<kRemapPositions>());
   const int32_t before = share_of(b, R.vratio), after = share_of(b + 1, R.vratio);
   if (after > before) {
@@ -1922,6 +1931,7 @@ __device__ __forceinline__ FinalMesh block_mesh(const FinalView& V, const FinalS
 // consecutive 16-byte pieces.
 template <bool QUAD, int SCHEME, bool BND, bool MULTI, bool IDS>
 __global__ void __launch_bounds__(kBlock) k_final(FinalView V) {
+  if (stopped(V.stop)) return;
   const FinalSeg* seg;
   const FinalMesh S = block_mesh<MULTI>(V, seg);
   const int32_t b = (int32_t)block_index<kRemapFinal>() - (MULTI ? seg->block0 : 0);
@@ -2320,6 +2330,7 @@ __device__ __forceinline__ void deep_vertex(const FinalView& V, const FinalMesh&
 // (FinalSeg).
 template <bool MULTI>
 __global__ void __launch_bounds__(kBlock) k_final_deep(FinalView V) {
+  if (stopped(V.stop)) return;
   const FinalSeg* seg;
   const FinalMesh S = block_mesh<MULTI>(V, seg);
   const int32_t b = (int32_t)block_index<kRemapFinal>() - (MULTI ? seg->block0 : 0);
@@ -2732,15 +2743,15 @@ void launch_digest(const void* p, int64_t bytes, uint64_t* out, hipStream_t st) 
 }
 
 void launch_faces(bool quad, const int32_t* ids, const int32_t* fptr, const float4* P, int32_t nf, const SegTable& seg,
-                  hipStream_t st) {
+                  const int* stop, hipStream_t st) {
   if (nf <= 0) return;
   const bool one = seg.n == 1;
   if (quad) {
-    if (one) k_faces<true, true><<<grid_for(nf), kBlock, 0, st>>>(ids, fptr, P, nf, seg);
-    else k_faces<true, false><<<grid_for(nf), kBlock, 0, st>>>(ids, fptr, P, nf, seg);
+    if (one) k_faces<true, true><<<grid_for(nf), kBlock, 0, st>>>(ids, fptr, P, nf, seg, stop);
+    else k_faces<true, false><<<grid_for(nf), kBlock, 0, st>>>(ids, fptr, P, nf, seg, stop);
   } else {
-    if (one) k_faces<false, true><<<grid_for(nf), kBlock, 0, st>>>(ids, fptr, P, nf, seg);
-    else k_faces<false, false><<<grid_for(nf), kBlock, 0, st>>>(ids, fptr, P, nf, seg);
+    if (one) k_faces<false, true><<<grid_for(nf), kBlock, 0, st>>>(ids, fptr, P, nf, seg, stop);
+    else k_faces<false, false><<<grid_for(nf), kBlock, 0, st>>>(ids, fptr, P, nf, seg, stop);
   }
 }
 

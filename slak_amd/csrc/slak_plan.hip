@@ -21,6 +21,7 @@ std::string flags_message(int f) {
     m += " non-manifold: a directed edge occurs twice (inconsistent orientation or >2 faces on an edge);";
   if (f & kFlagDegenerate) m += " degenerate face (repeated vertex along a face);";
   if (f & kFlagOverflow) m += " index overflow (counts exceed int32);";
+  if (f & kFlagChanged) m += " the number of edges differs from the one the batch was created with;";
   return m;
 }
 
@@ -438,6 +439,7 @@ void Plan::record_analysis(LevelPlan& L) {
   LevelView V = L.view(d_flags_, late_);
   V.hist_rows = d_state_ + kStateRowHist;
   V.bounds = d_state_ + kStateBounds;
+  V.planned = replayed_ ? 1 : 0;
   ProfScope ps(st_, analysis_stages(L));
   launch_symbolic(L.quad, scheme_, V, st_);
   if (L.segs.size() > 1) launch_seg_bounds(V, st_);
@@ -994,6 +996,7 @@ void Plan::launch_number(LevelPlan& L, bool faces, bool rep) {
   LevelView V = L.view(d_flags_, late_);
   V.ci = reinterpret_cast<int32_t*>(L.ci);
   V.bnd = L.bnd;
+  V.planned = replayed_ ? 1 : 0;
   if (rep) {
     V.report = report_;
     V.hist_rows = d_state_ + kStateRowHist;
@@ -1111,6 +1114,7 @@ void Plan::launch_deep(int l, FinalTable& T) {
   V.trow = N.trow;
   V.trow_x = N.rows_x ? reinterpret_cast<const int32_t*>(N.trow) : nullptr;
   V.own = N.own;
+  V.stop = stop();
   set_final_table(V, T);
   const bool multi = final_table(T);
   // algorithmic bytes: reads N's ids, (edge, twin) pairs, edge owners, M^T
@@ -1152,6 +1156,7 @@ void Plan::launch_final_table(int l, FinalTable& T, bool ids, const char* stage)
   V.trow_x = M.rows_x ? reinterpret_cast<const int32_t*>(M.trow) : nullptr;
   V.blk = M.blk;
   V.mpos = M.mpos;
+  V.stop = stop();
   set_final_table(V, T);
   // algorithmic bytes: reads the ids, (edge, twin) pairs, M^T rows and
   // offsets of M (boundary scan, SLAK positions) and the positions of M1;
@@ -1198,7 +1203,7 @@ void Plan::record_level(int l) {
   if (l == 1 && number_early_ && !early_faces_) {
     ProfScope ps(st_, L.quad ? "facepoints_quad" : "facepoints_poly",
                  4.0 * L.nnz + 16.0 * L.nv + 16.0 * L.nf + (L.quad ? 0.0 : 4.0 * (L.nf + 1)));
-    launch_faces(L.quad, L.ids, L.fptr, L.P, (int32_t)L.nf, L.table(), st_);
+    launch_faces(L.quad, L.ids, L.fptr, L.P, (int32_t)L.nf, L.table(), stop(), st_);
   }
   if (L.blk && (l == 1 || scheme_ == kSLAK)) {
     ProfScope ps(st_, "scan", 8.0 * ne + 4);
@@ -1208,7 +1213,7 @@ void Plan::record_level(int l) {
   if (l > 1) {
     ProfScope ps(st_, L.quad ? "facepoints_quad" : "facepoints_poly",
                  4.0 * L.nnz + 16.0 * L.nv + 16.0 * L.nf + (L.quad ? 0.0 : 4.0 * (L.nf + 1)));
-    launch_faces(L.quad, L.ids, L.fptr, L.P, (int32_t)L.nf, L.table(), st_);
+    launch_faces(L.quad, L.ids, L.fptr, L.P, (int32_t)L.nf, L.table(), stop(), st_);
   }
   RefineView R{};
   R.ids = L.ids;
@@ -1224,6 +1229,7 @@ void Plan::record_level(int l) {
   R.blk = L.blk;
   R.mpos = L.mpos;
   R.seg = L.table();
+  R.stop = stop();
   R.ntptr = L.ntptr;
   R.ntrow = L.ntrow;
   R.nci = L.nci;

@@ -227,6 +227,7 @@ class Plan {
   int32_t* late_ = nullptr;
   int32_t* report_ = nullptr;
   bool replayed_ = false;  // the last launch ran the analysis again
+  const int* stop() const { return replayed_ ? d_flags_ : nullptr; }  // see stopped()
   // first-level union gather (multi-mesh)
   float4* P1_ = nullptr;
   bool prepared_ = false;

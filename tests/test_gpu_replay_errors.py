@@ -7,7 +7,7 @@ import pytest
 from slak_amd import capi, meshgen as g
 from slak_amd.batch import Batch
 from slak_amd.capi import SlakError
-from slak_amd.mesh import MeshInfo
+from slak_amd.mesh import MeshInfo, subdivide_host
 
 pytestmark = pytest.mark.gpu
 LAK, SLAK = capi.SLAK_SCHEME_LAK, capi.SLAK_SCHEME_SLAK
@@ -58,3 +58,54 @@ def test_an_error_ends_with_its_run(scheme, copies, graph):
     finally:
         for d in dev:
             d.freeAndReset()
+
+
+def changed(kind):
+    """A mesh and ids that break the contract: (mesh, other ids, flag text)."""
+    if kind == "more_edges":
+        m, ids = spare_cube()
+        return m, ids, "number of edges"
+    if kind == "fewer_edges":  # the open cube and the quad become the cube
+        m, ids = spare_cube()
+        return g.HostMesh(m.type, m.ptr, ids, m.vals, m.verts), m.ids, "number of edges"
+    m = g.uv_sphere(12, 5)  # rows beyond their eight slots
+    ids = m.ids.copy()
+    if kind == "bad_id":
+        ids[5] = m.nverts
+        return m, ids, "vertex id out of range"
+    assert kind == "turned_face"
+    ids[:3] = ids[:3][::-1]
+    return m, ids, "non-manifold"
+
+
+@pytest.mark.parametrize("graph", [False, True], ids=["eager", "graph"])
+@pytest.mark.parametrize("levels", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("kind", ["more_edges", "fewer_edges", "bad_id", "turned_face"])
+@pytest.mark.parametrize("scheme", [LAK, SLAK], ids=["LAK", "SLAK"])
+def test_nothing_is_refined_from_a_failed_analysis(scheme, kind, levels, graph):
+    """Changed before the first run (nothing a level reads has been written
+    then) and after a good one: the run reports the flag, the kernels after the
+    analysis write nothing, and the original ids give the same result again.
+    Alone and between other meshes."""
+    m, ids, text = changed(kind)
+    want = subdivide_host(m, levels, scheme)[0]
+    for hosts in ([m], [g.torus(6, 5, seed=2), m, g.open_grid(4, 3, sigma=1e-3)]):
+        at = len(hosts) // 2
+        dev = [MeshInfo.from_host(h) for h in hosts]
+        try:
+            with Batch(dev, [levels] * len(hosts), scheme) as b:
+                for again in range(2):
+                    set_ids(dev[at], ids)
+                    before = [b.result(k).to_host() for k in range(len(hosts))]
+                    with pytest.raises(SlakError) as ei:
+                        b.run(use_graph=graph)
+                    assert ei.value.code == 5 and text in str(ei.value)
+                    if again and levels > 1:
+                        for k in range(len(hosts)):
+                            assert_same(b.result(k).to_host(), before[k])
+                    set_ids(dev[at], m.ids)
+                    b.run(use_graph=graph)
+                    assert_same(b.result(at).to_host(), want)
+        finally:
+            for d in dev:
+                d.freeAndReset()
