@@ -206,7 +206,7 @@ void Plan::upload_tables(int l0, int l1, Staging& staging, bool zero_state) {
     offs.push_back(total);
     if (n > 1)
       total = align(total + n * sizeof(SegDesc)) + align(3 * (n + 1) * sizeof(int64_t)) +
-              align((nblocks(L.nv) + nblocks(L.nf) + nblocks(L.nnz)) * sizeof(int32_t));
+              align((nblocks(L.nv) + nblocks(L.nf) + nblocks(L.nnz) + 3) * sizeof(int32_t));
     total += fin_bytes(L);
   }
   // (planned with the last levels: empty when the first level's tables go up)
@@ -255,7 +255,8 @@ void Plan::upload_tables(int l0, int l1, Staging& staging, bool zero_state) {
           while (k + 1 < n && base[k + 1] <= (int64_t)b * kBlockItems) ++k;
           blk[b] = (int32_t)k;
         }
-        at += nb;
+        blk[nb] = (int32_t)n - 1;
+        at += nb + 1;
       }
       o = align(o + at * sizeof(int32_t));
     }
