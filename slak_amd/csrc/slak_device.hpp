@@ -539,8 +539,9 @@ __device__ __forceinline__ void row_number(Row& r, const LevelView& L, int32_t v
 // b - share(b) of the rest. With ratio = ceil(n 2^32 / T) and T < 2^31, share
 // rises by 0 or 1 per block and ends at n: the lists are covered exactly. (A
 // 64-bit division in its place is more than a hundred scalar instructions.)
-inline uint64_t share_ratio(int64_t n, int64_t T) {
-  return T > 0 ? (uint64_t)((((__uint128_t)n << 32) + (__uint128_t)(T - 1)) / (__uint128_t)T) : 0;
+inline uint64_t share_ratio(int64_t n, int64_t T) {  // 0 <= n <= T: the numerator stays below 2^64
+  if (n == 0 || T <= 0) return 0;
+  return n == T ? 1ull << 32 : (((uint64_t)n << 32) + (uint64_t)(T - 1)) / (uint64_t)T;
 }
 __device__ __forceinline__ int32_t share_of(int32_t b, uint64_t ratio) {
   return (int32_t)(((uint64_t)(uint32_t)b * ratio) >> 32);

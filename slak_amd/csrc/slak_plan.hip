@@ -225,7 +225,6 @@ void Plan::upload_tables(int l0, int l1, Staging& staging, bool zero_state) {
     pinned_release(staging.p, staging.cap);
     staging.p = pinned_acquire(total, staging.cap);
   }
-  std::memset(staging.p, 0, total);
   char* d = arena_.get_n<char>((int64_t)total);
   for (int l = l0; l < l1; ++l) {
     LevelPlan& L = levels_[l];
@@ -953,6 +952,8 @@ void Plan::prepare() {
       if (seg_in_m[j] < 0 || !P) throw Error(SLAK_ERR_INTERNAL, "fused level without its input");
       return M.segs[seg_in_m[j]];
     };
+    L.fin.segs.reserve(L.fin.jobs.size());
+    L.deep.segs.reserve(L.deep.jobs.size());
     // meshes whose last level is l
     for (int j : L.fin.jobs) add_final_seg(L.fin, l, j, segment(j, jobs_[j].p1), jobs_[j].p1, jobs_[j].out_verts);
     plan_blocks(L.fin, M.quad, false);
@@ -960,6 +961,7 @@ void Plan::prepare() {
     // from the structure two levels back too
     bool pos = allow_pos && !L.segs.empty();
     for (int j : L.jobs) pos = pos && positions_only(jobs_[j], l);
+    L.pos.segs.reserve((pos ? L.jobs.size() : 0) + L.deep.jobs.size());
     if (pos) {
       L.pos_fused = true;
       for (size_t k = 0; k < L.segs.size(); ++k) {
@@ -1007,30 +1009,35 @@ void Plan::launch_number(LevelPlan& L, bool faces, bool rep) {
   launch_number_faces(L.quad, scheme_, V, faces, st_);
 }
 
-// Vertex classes of the mesh two levels before job J's level l (the mesh M
-// of its k_final): the original vertices, then the face points and edge
-// points of every level before M; one class if the sizes do not add up.
-static std::vector<int64_t> vertex_classes(const MeshJob& J, int l) {
-  std::vector<int64_t> cls{J.nv[0]};
-  for (int k = 0; k + 2 < l; ++k) {
-    cls.push_back(J.nf[k]);
-    cls.push_back(J.ne[k]);
-  }
-  int64_t sum = 0;
-  for (int64_t c : cls) sum += c;
-  if (sum != J.nv[l - 2]) cls.assign(1, J.nv[l - 2]);
-  return cls;
-}
-
-// vertex classes as runs (leading ones merged past kMaxVSeg)
-static void set_runs(VertexRuns& R, std::vector<int64_t> cls) {
-  while (cls.size() > (size_t)kMaxVSeg) {
-    cls[1] += cls[0];
-    cls.erase(cls.begin());
-  }
-  R.n = (int32_t)cls.size();
+// Vertex runs of the mesh two levels before job J's level l (the mesh M of its
+// k_final): the original vertices, then the face points and edge points of
+// every level before M (the leading classes as one past kMaxVSeg); one run if
+// the sizes do not add up. more: items that follow, a run of their own.
+static void set_runs(VertexRuns& R, const MeshJob& J, int l, int32_t more = 0) {
+  const int levels = std::max(l - 2, 0), classes = 1 + 2 * levels + (more ? 1 : 0);
+  int skip = std::max(classes - kMaxVSeg, 0);
+  int64_t end = 0;
+  R.n = 0;
   R.first[0] = 0;
-  for (size_t i = 0; i < cls.size(); ++i) R.first[i + 1] = R.first[i] + (int32_t)cls[i];
+  auto add = [&](int64_t c) {
+    end += c;
+    if (skip > 0)
+      --skip;
+    else
+      R.first[++R.n] = (int32_t)end;
+  };
+  add(J.nv[0]);
+  for (int k = 0; k < levels; ++k) {
+    add(J.nf[k]);
+    add(J.ne[k]);
+  }
+  if (end != J.nv[levels]) {
+    skip = 0;
+    R.n = 0;
+    end = 0;
+    add(J.nv[levels]);
+  }
+  if (more) add(more);
 }
 
 // The blocks of a table's meshes, mesh by mesh, and (several meshes) the mesh
@@ -1038,6 +1045,7 @@ static void set_runs(VertexRuns& R, std::vector<int64_t> cls) {
 void Plan::plan_blocks(FinalTable& T, bool quad, bool deep) {
   int64_t blocks = 0;
   const bool table = final_table(T);
+  if (table) T.block_seg.reserve(2 * T.segs.size());  // (a corner and a vertex block of each mesh at least)
   for (size_t k = 0; k < T.segs.size(); ++k) {
     FinalSeg& F = T.segs[k];
     F.block0 = (int32_t)blocks;
@@ -1091,9 +1099,7 @@ void Plan::add_final_seg(FinalTable& T, int l, int job, const SegDesc& m, const 
     F.m.out_ptr = J.out_ptr;
     F.m.out_vals = J.out_vals;
   }
-  std::vector<int64_t> cls = vertex_classes(J, l);
-  if (!levels_[l - 2].quad) cls.push_back(m.nf);  // polygons' face points have items of their own
-  set_runs(F.runs, cls);
+  set_runs(F.runs, J, l, levels_[l - 2].quad ? 0 : m.nf);  // (polygons' face points have items of their own)
   T.segs.push_back(F);
 }
 
@@ -1243,7 +1249,7 @@ void Plan::record_level(int l) {
   if (L.segs.size() == 1 && l >= 2) {
     // one mesh: its vertex classes (the original vertices, then the face and
     // edge points of every earlier level) as runs in step with the corners
-    set_runs(R.runs, vertex_classes(jobs_[L.jobs[0]], l + 1));
+    set_runs(R.runs, jobs_[L.jobs[0]], l + 1);
   }
   const bool next = L.ntptr != nullptr;
   {
