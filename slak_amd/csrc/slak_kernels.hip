@@ -603,7 +603,7 @@ __global__ void __launch_bounds__(kBlock) k_symbolic(LevelView L) {
         int32_t* const run = L.tids + atomicAdd(L.pool, n);
         for (int i = 0; i < kRowSlots; ++i) run[i] = row[i];
         int32_t c = L.head[v];
-        for (int i = kRowSlots; i < n; ++i) {
+        for (int i = n - 1; i >= kRowSlots; --i) {  // (the list is last in, first out: nearly ascending this way)
           run[i] = c;
           c = L.next[c];
         }
@@ -827,7 +827,7 @@ __global__ void __launch_bounds__(kSmallItems) k_first_small(LevelView L, int us
         int32_t* const run = L.tids + atomicAdd(&pool, n);
         for (int i = 0; i < kRowSlots; ++i) run[i] = row[i];
         int32_t c = head[v];
-        for (int i = kRowSlots; i < n; ++i) {
+        for (int i = n - 1; i >= kRowSlots; --i) {  // (the list is last in, first out: nearly ascending this way)
           run[i] = c;
           c = L.next[c];
         }
