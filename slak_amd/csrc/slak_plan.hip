@@ -540,6 +540,9 @@ void Plan::prepare() {
   auto fail_if = [&](int fl) {
     if (!fl) return;
     std::vector<int> mf(nseg, 0);
+    // the report may have come from a launch that is still running (a small
+    // mesh's), and the copy does not wait for a non-blocking stream
+    SLAK_HIP_CHECK(hipStreamSynchronize(st_));
     SLAK_HIP_CHECK(hipMemcpy(mf.data(), L1.d_mflags, nseg * sizeof(int), hipMemcpyDeviceToHost));
     for (int k = 0; k < nseg; ++k) jobs_[L1.jobs[k]].bad_flags = mf[k];
     throw Error(SLAK_ERR_INVALID_MESH, describe_failure(fl));

@@ -1,13 +1,16 @@
-"""Batches whose inputs change between runs against their contract (same
+"""Errors of the first level's analysis: what a call on an invalid mesh reports,
+and batches whose inputs change between runs against their contract (same
 topology): the run reports it, and a later run on the restored inputs is as
 good as the first."""
+import ctypes
+
 import numpy as np
 import pytest
 
 from slak_amd import capi, meshgen as g
 from slak_amd.batch import Batch
 from slak_amd.capi import SlakError
-from slak_amd.mesh import MeshInfo, subdivide_host
+from slak_amd.mesh import LAKCatmullClark, MeshInfo, subdivide_host
 
 pytestmark = pytest.mark.gpu
 LAK, SLAK = capi.SLAK_SCHEME_LAK, capi.SLAK_SCHEME_SLAK
@@ -109,3 +112,25 @@ def test_nothing_is_refined_from_a_failed_analysis(scheme, kind, levels, graph):
         finally:
             for d in dev:
                 d.freeAndReset()
+
+
+@pytest.mark.parametrize("shape", ["small", "launches"])
+@pytest.mark.parametrize("kind", ["bad_id", "turned_face"])
+def test_an_error_names_its_mesh_on_any_stream(kind, shape):
+    """The flags of each mesh are read after the kernel that writes them, also
+    on a stream that copies do not wait for."""
+    m = g.uv_sphere(12, 5) if shape == "small" else g.uv_sphere(12, 200)
+    ids = m.ids.copy()
+    ids[:3] = (m.nverts, ids[1], ids[2]) if kind == "bad_id" else ids[:3][::-1]
+    text = "vertex id out of range" if kind == "bad_id" else "non-manifold"
+    bad = MeshInfo.from_host(g.HostMesh(m.type, m.ptr, ids, m.vals, m.verts))
+    st = ctypes.c_void_p()
+    assert capi.lib().hipStreamCreateWithFlags(ctypes.byref(st), ctypes.c_uint(1)) == 0  # non-blocking
+    try:
+        for _ in range(20):
+            with pytest.raises(SlakError) as ei:
+                LAKCatmullClark.subdivideIteratively(bad, MeshInfo(), 2, st.value)
+            assert ei.value.code == 2 and "mesh 0:" in str(ei.value) and text in str(ei.value)
+    finally:
+        capi.lib().hipStreamDestroy(st)
+        bad.freeAndReset()
