@@ -507,7 +507,7 @@ void Plan::prepare() {
   const int nseg = (int)L1.segs.size();
   // a single mesh numbers its edges before the read-back: the first upload
   // gives it nnz >= ne as the edge-id bound and a flag buffer of that size
-  const bool early = nseg == 1 && jobs_.size() == 1 && jobs_[L1.jobs[0]].known_ne < 0;
+  const bool early = nseg == 1 && jobs_.size() == 1;
   early_p1_ = nullptr;
   early_faces_ = false;
   if (early) {
@@ -547,11 +547,6 @@ void Plan::prepare() {
     for (int k = 0; k < nseg; ++k) jobs_[L1.jobs[k]].bad_flags = mf[k];
     throw Error(SLAK_ERR_INVALID_MESH, describe_failure(fl));
   };
-  bool all_trusted = true, all_known = true;
-  for (int k = 0; k < nseg; ++k) {
-    all_trusted &= jobs_[L1.jobs[k]].trusted;
-    all_known &= jobs_[L1.jobs[k]].known_ne >= 0;
-  }
   // 2. first-level analysis: M^T, owned-edge counts, per-mesh edge totals
   // (its kernels do nothing on an input the gather flagged; the flags come
   // back with the edge counts in one round trip)
@@ -560,37 +555,29 @@ void Plan::prepare() {
   else
     record_analysis(L1);
   std::vector<int64_t> hb(kRowHistBins + nseg + 1, 0);
-  bool have_hist = false;
-  if (!all_known) {
-    // a single mesh numbers its edges (and forms its face points) meanwhile
-    if (small) {
-      // (in the one launch)
-    } else if (early) {
-      launch_number(L1, early_p1_ != nullptr, true);
-    } else {
-      LevelView V = L1.view(d_flags_, late_);
-      V.hist_rows = d_state_ + kStateRowHist;
-      V.bounds = d_state_ + kStateBounds;
-      V.report = report_;
-      V.ngroups = (int32_t)n_groups_;
-      launch_report(V, st_);
-    }
-    wait_report();
-    fail_if(report_[1]);
-    for (int b = 0; b < kRowHistBins; ++b) hb[b] = report_[2 + b];
-    for (int k = 0; k <= nseg; ++k) hb[kRowHistBins + k] = report_[2 + kRowHistBins + k];
-    // the early numbering was recorded before its edge count was known: its
-    // boundary-flag writes (4 bytes per edge) join its algorithmic bytes now
-    if (early && Profiler::get().enabled())
-      Profiler::get().amend_last(L1.quad ? "number_facepoints_quad" : "number_facepoints_poly",
-                                 4.0 * (double)hb[kRowHistBins + 1]);
-    number_early_ = early;
-    early_faces_ = early && early_p1_ != nullptr;
-    have_hist = true;
+  // a single mesh numbers its edges (and forms its face points) meanwhile (a
+  // small one in that one launch)
+  if (early) {
+    if (!small) launch_number(L1, early_p1_ != nullptr, true);
   } else {
-    if (!all_trusted) fail_if(read_flags());
-    for (int k = 0; k < nseg; ++k) hb[kRowHistBins + k + 1] = hb[kRowHistBins + k] + jobs_[L1.jobs[k]].known_ne;
+    LevelView V = L1.view(d_flags_, late_);
+    V.hist_rows = d_state_ + kStateRowHist;
+    V.bounds = d_state_ + kStateBounds;
+    V.report = report_;
+    V.ngroups = (int32_t)n_groups_;
+    launch_report(V, st_);
   }
+  wait_report();
+  fail_if(report_[1]);
+  for (int b = 0; b < kRowHistBins; ++b) hb[b] = report_[2 + b];
+  for (int k = 0; k <= nseg; ++k) hb[kRowHistBins + k] = report_[2 + kRowHistBins + k];
+  // the early numbering was recorded before its edge count was known: its
+  // boundary-flag writes (4 bytes per edge) join its algorithmic bytes now
+  if (early && Profiler::get().enabled())
+    Profiler::get().amend_last(L1.quad ? "number_facepoints_quad" : "number_facepoints_poly",
+                               4.0 * (double)hb[kRowHistBins + 1]);
+  number_early_ = early;
+  early_faces_ = early && early_p1_ != nullptr;
   const int64_t* bounds = hb.data() + kRowHistBins;
   // 3. closed-form sizes of every later level
   int Lmax = 0;
@@ -961,7 +948,7 @@ void Plan::prepare() {
   // the first level's rows per block, now with the row-length spread (the
   // numbering after the read-back and every graph replay use it)
   {
-    const RowTiling rt = autotune_rows(levels_[0].nv, levels_[0].nnz, have_hist ? hb.data() : nullptr);
+    const RowTiling rt = autotune_rows(levels_[0].nv, levels_[0].nnz, hb.data());
     levels_[0].rows = rt.rows;
     levels_[0].tile = rt.tile;
   }
