@@ -65,6 +65,11 @@ ChainBound chain_bound(const slak_mesh& m, int levels) {
   double nv = (double)m.nverts, nf = (double)m.nfaces, nnz = (double)m.nnz;
   double held = 16 * nv + 4 * nnz;  // the caller's input (gathered once)
   double peak = 0;
+  // What the plan holds at once. The first level's arrays: union positions, row
+  // slots, lists, counts and offsets per vertex, ids, edge pairs, rows and lists
+  // per corner (polygons: face offsets and faces); the positions of its result.
+  double first = 68 * nv + 4 * nf + 36 * nnz;
+  double handed = 0, structure = 0;  // positions and ids handed on; two buffers of a level's structure
   for (int l = 0; l < std::max(levels, 1); ++l) {
     const double ne = nnz;  // bound
     const double nv2 = nv + nf + ne, nnz2 = 4 * nnz;
@@ -76,6 +81,16 @@ ChainBound chain_bound(const slak_mesh& m, int levels) {
     const double level = 28 * nnz + 8 * nv + 16 * nv2 + 4 * nnz2 * 2 + 4 * nnz;
     peak = std::max(peak, held + level);
     held += 16 * nv2 + 4 * nnz2;  // a level stays resident while the next one runs
+    if (l + 1 < levels) {
+      if (l == 0) first += 16 * nv2;
+      handed += 16 * nv2;
+      if (l + 2 < levels) {
+        handed += 4 * nnz2;
+        structure = 8 * nv2 + 40 * nnz2;
+      }
+    } else {  // boundary flags and ranks, the result (LAK form)
+      peak = std::max(peak, first + handed + structure + 16 * ne + 16 * nv2 + 9 * nnz2);
+    }
     nv = nv2;
     nf = nnz;
     nnz = nnz2;

@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 
 from slak_amd import capi, meshgen as g
+from slak_amd.batch import Batch
 from slak_amd.capi import SlakError
 from slak_amd.mesh import MeshInfo, subdivide_host, to_host
 from slak_amd.serve import Server
@@ -134,3 +135,33 @@ def test_concurrent_submitters():
     finally:
         for d in dev:
             d.freeAndReset()
+
+
+def quad_soup(n):
+    """n quads that share no vertex: the most vertices and edges per corner."""
+    corner = np.array([[0, 0, 0, 1], [1, 0, 0, 1], [1, 1, 0, 1], [0, 1, 0, 1]], np.float32)
+    verts = np.tile(corner, (n, 1))
+    verts[:, 2] = np.repeat(np.arange(n), 4)
+    ids = np.arange(4 * n, dtype=np.int32)
+    return g.HostMesh(g.QUAD, np.arange(0, 4 * n + 1, 4, dtype=np.int32), ids, ids % 4 + 1, verts)
+
+
+@pytest.mark.parametrize("levels", [1, 2, 3])
+@pytest.mark.parametrize("shape", ["soup", "closed", "triangles"])
+def test_footprint_covers_what_a_request_takes(shape, levels):
+    """A budget just below the device memory that the request's chain holds
+    (less 2 MiB, which the fixed part of a plan is rounded from) refuses it."""
+    n = 60000 >> 2 * (levels - 1)
+    side = int(n ** 0.5)
+    m = {"soup": lambda: quad_soup(n), "closed": lambda: g.torus(side, side, seed=1),
+         "triangles": lambda: g.torus_mixed(side, side, 1.0, seed=1)}[shape]()
+    d = MeshInfo.from_host(m)
+    try:
+        with Batch([d], [levels], LAK) as b:
+            need = int(b.info().device_bytes)
+        with Server(LAK, memory_budget_bytes=need - (2 << 20)) as srv:
+            with pytest.raises(SlakError) as ei:
+                srv.submit(d, levels)
+            assert ei.value.code == 6
+    finally:
+        d.freeAndReset()
