@@ -58,10 +58,10 @@ def cpu_model() -> str:
 
 
 def stage_roofline(prof, stage=None):
-    """Roofline of one stage of a library profile (the slowest one by
-    default): its algorithmic bytes per launch over its mean HIP-event launch
-    duration, against the 8 TB/s HBM peak; plus the whole chain's figure."""
-    stages = prof["stages"]
+    """Roofline of one launch of a library profile (the slowest one by
+    default): its algorithmic bytes over its mean HIP-event duration, against
+    the 8 TB/s HBM peak; plus the whole chain's figure."""
+    stages = prof["launches"]
     total_ms = sum(s["total_ms"] for s in stages)
     total_b = sum(s["bytes"] for s in stages)
     dom = max(stages, key=lambda s: s["total_ms"]) if stage is None else next(s for s in stages if s["name"] == stage)
@@ -90,7 +90,7 @@ def output_level_roofline(prof):
     LAK-form launch of all of them (lak_form), their algorithmic bytes over
     their summed HIP-event durations. None when no LAK form is written
     separately (SLAK, or one mesh)."""
-    st = {s["name"]: s for s in prof["stages"]}
+    st = {s["name"]: s for s in prof["launches"]}
     if CFG4_STAGE not in st or "lak_form" not in st:
         return None
     finals = [n for n in (CFG4_STAGE, CFG4_STAGE.replace("_quad", "_poly")) if n in st]
@@ -105,7 +105,7 @@ def output_level_roofline(prof):
 def stage_table(prof):
     return [{"name": s["name"], "launches": s["launches"], "us": round(s["total_ms"] * 1e3, 1),
              "bytes": int(s["bytes"]), "gbps": round(s["bytes"] / (s["total_ms"] * 1e-3) / 1e9, 1)}
-            for s in prof["stages"]]
+            for s in prof["launches"]]
 
 
 # ---------------------------------------------------------------------------
@@ -307,7 +307,7 @@ def serve_leg(n_requests, qps_fraction, scheme, seed=5, keep=()):
 # ---------------------------------------------------------------------------
 # HBM counters (rocprofv3 in child processes, before this process touches the GPU)
 
-# kernel of each roofline stage ({s}: 0 LAK, 1 SLAK; multi: the table path)
+# kernel of each launch of a profile ({s}: 0 LAK, 1 SLAK; multi: the table path)
 STAGE_KERNELS = {
     "refine_vertex_final_quad": r"k_final<true, {s}, \w+, {multi}, true>|k_final_deep<{multi}>",
     "refine_vertex_final_poly": r"k_final<false, {s}, \w+, {multi}, true>",
@@ -317,14 +317,10 @@ STAGE_KERNELS = {
     "refine_vertex_poly": r"k_level<false, {s},",
     "facepoints_quad": r"k_faces<true,",
     "facepoints_poly": r"k_faces<false,",
-    "gather": r"k_gather<",  # the gather, count and transpose stages are one launch
-    "count_quad": r"k_gather<true,",
-    "count_poly": r"k_gather<false,",
+    "gather": r"k_gather<",
     "lak_form": r"k_lak_form",
-    "transpose_quad": r"k_gather<true,",
-    "transpose_poly": r"k_gather<false,",
-    "spgemm_symbolic_quad": r"k_symbolic<true, {s}>",
-    "spgemm_symbolic_poly": r"k_symbolic<false, {s}>",
+    "symbolic_quad": r"k_symbolic<true, {s}>",
+    "symbolic_poly": r"k_symbolic<false, {s}>",
     "number_facepoints_quad": r"k_number_faces<true, {s},",
     "number_facepoints_poly": r"k_number_faces<false, {s},",
 }
@@ -720,7 +716,7 @@ def main():
                     "host_syncs": int(st.host_syncs),
                 }
                 if w == "cfg3":
-                    # GB/s of every SpGEMM / SpMV stage of the chain
+                    # GB/s of every SpGEMM / SpMV launch of the chain
                     tab = stage_table(prof)
                     for row in tab:
                         t = stage_traffic(traffic, w, row["name"], sname, False) if sname == args.scheme else None

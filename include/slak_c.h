@@ -101,8 +101,11 @@ int slak_pool_stats(uint64_t* in_use, uint64_t* cached, uint64_t* peak);
 /* ---- per-stage timing (TimeProfileIndividual, LibInclude/profiling.h:182-200) ----
  * slak_profile_enable(1) clears the record and brackets every later kernel
  * launch with a HIP event pair on its stream; slak_profile_report writes
- * {"stages": [{"name", "launches", "total_ms", "bytes"}]} as JSON text, where
- * bytes are the stage's algorithmic (compulsory) bytes summed over launches. */
+ * {"stages": [{"name", "launches", "total_ms", "bytes"}], "launches": [...]}
+ * as JSON text, where bytes are algorithmic (compulsory) bytes summed over
+ * launches. "launches" is what was measured. A launch that runs several stages
+ * (of the first level) is one entry there; under "stages" its time is shared
+ * among them in proportion to their bytes. */
 int slak_profile_enable(int32_t on);
 int slak_profile_report(char* buf, uint64_t len);
 /* HBM reference: `iters` float4 stream copies of `bytes` (k_copy_probe);

@@ -187,8 +187,10 @@ class Arena {
 // when enabled, every launch site records an event pair on its stream and the
 // stage's algorithmic bytes (compulsory reads + writes of distinct arrays).
 
-// A launch that runs several stages records them all; the report shares its
-// time among them in proportion to their algorithmic bytes.
+// A launch that runs several stages records them all, under a name and with
+// algorithmic bytes of its own (what the stages hand each other inside it does
+// not reach memory). The report lists the launches as they were measured; under
+// the stages it shares a launch's time in proportion to their bytes.
 
 struct StageBytes {
   const char* name;
@@ -200,15 +202,17 @@ class Profiler {
   static Profiler& get();
   bool enabled() const { return enabled_; }
   void set_enabled(bool on) { enabled_ = on; }
-  void begin(hipStream_t st, std::vector<StageBytes> stages);
+  void begin(hipStream_t st, StageBytes launch, std::vector<StageBytes> stages);
   void end(hipStream_t st);
   // adds `bytes` to the latest record of stage `name` (names compare by text)
+  // and to its launch
   void amend_last(const char* name, double bytes);
   void reset();
   std::string report();  // JSON
 
  private:
   struct Rec {
+    StageBytes launch;
     std::vector<StageBytes> stages;
     hipEvent_t a, b;
   };
@@ -223,10 +227,11 @@ struct ProfScope {
   hipStream_t st;
   bool on;
   ProfScope(hipStream_t s, const char* name, double bytes) : st(s), on(Profiler::get().enabled()) {
-    if (on) Profiler::get().begin(st, {{name, bytes}});
+    if (on) Profiler::get().begin(st, {name, bytes}, {{name, bytes}});
   }
-  ProfScope(hipStream_t s, std::vector<StageBytes> stages) : st(s), on(Profiler::get().enabled()) {
-    if (on) Profiler::get().begin(st, std::move(stages));
+  ProfScope(hipStream_t s, StageBytes launch, std::vector<StageBytes> stages)
+      : st(s), on(Profiler::get().enabled()) {
+    if (on) Profiler::get().begin(st, launch, std::move(stages));
   }
   ~ProfScope() {
     if (on) Profiler::get().end(st);

@@ -428,7 +428,7 @@ LevelView LevelPlan::view(int* flags, int* late) const {
 
 // Validation, position order, valences and the rows' corners in one launch.
 void Plan::record_gather(LevelPlan& L) {
-  ProfScope ps(st_, gather_stages(L));
+  ProfScope ps(st_, {"gather", gather_bytes(L)}, gather_stages(L));
   launch_gather(L.quad, L.table(), scheme_ == kLAK, const_cast<int32_t*>(L.ids), L.view(d_flags_, late_), st_);
 }
 
@@ -440,9 +440,18 @@ void Plan::record_analysis(LevelPlan& L) {
   V.hist_rows = d_state_ + kStateRowHist;
   V.bounds = d_state_ + kStateBounds;
   V.planned = replayed_ ? 1 : 0;
-  ProfScope ps(st_, analysis_stages(L));
+  // reads the rows and their corners' neighbours, writes the owned counts
+  ProfScope ps(st_, {L.quad ? "symbolic_quad" : "symbolic_poly",
+                     8.0 * L.nnz + 8.0 * L.nv + (L.quad ? 0.0 : 4.0 * L.nnz + 4.0 * (L.nf + 1))},
+               analysis_stages(L));
   launch_symbolic(L.quad, scheme_, V, st_);
   if (L.segs.size() > 1) launch_seg_bounds(V, st_);
+}
+
+// reads face offsets, ids and vals, writes the ids in position order, the
+// rows' corners and the valences (polygons: face offsets and corner faces)
+double Plan::gather_bytes(const LevelPlan& L) const {
+  return 4.0 * (L.nf + 1) + 16.0 * L.nnz + 4.0 * L.nv + (L.quad ? 0.0 : 4.0 * L.nnz + 4.0 * (L.nf + 1));
 }
 
 std::vector<StageBytes> Plan::gather_stages(const LevelPlan& L) const {
@@ -474,7 +483,10 @@ void Plan::record_small(LevelPlan& L, bool faces) {
   std::vector<StageBytes> stages = gather_stages(L);
   for (const StageBytes& s : analysis_stages(L)) stages.push_back(s);
   stages.push_back(number_stage(L, faces));
-  ProfScope ps(st_, std::move(stages));
+  // the inputs, what the gather writes, M^T's rows and offsets and the (edge,
+  // twin) pairs; face points
+  const double bytes = gather_bytes(L) + 16.0 * L.nnz + 4.0 * L.nv + (faces ? 16.0 * L.nv + 16.0 * L.nf : 0.0);
+  ProfScope ps(st_, {L.quad ? "first_level_small_quad" : "first_level_small_poly", bytes}, std::move(stages));
   launch_first_small(L.quad, scheme_, scheme_ == kLAK, V, faces, st_);
 }
 
@@ -1019,7 +1031,8 @@ void Plan::launch_number(LevelPlan& L, bool faces, bool rep) {
     V.hist_rows = d_state_ + kStateRowHist;
     V.ngroups = (int32_t)n_groups_;
   }
-  ProfScope ps(st_, std::vector<StageBytes>{number_stage(L, faces)});
+  const StageBytes stage = number_stage(L, faces);
+  ProfScope ps(st_, stage.name, stage.bytes);
   launch_number_faces(L.quad, scheme_, V, faces, st_);
 }
 

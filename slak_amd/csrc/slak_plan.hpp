@@ -194,8 +194,9 @@ class Plan {
   void upload_tables(int l0, int l1, Staging& staging, bool zero_state = false);
   void record_gather(LevelPlan& L);
   void record_small(LevelPlan& L, bool faces);
-  // algorithmic bytes of the first level's stages
+  // algorithmic bytes of the first level's stages; of the gather's launch
   std::vector<StageBytes> gather_stages(const LevelPlan& L) const;
+  double gather_bytes(const LevelPlan& L) const;
   std::vector<StageBytes> analysis_stages(const LevelPlan& L) const;
   StageBytes number_stage(const LevelPlan& L, bool faces) const;
   int read_flags();

@@ -166,9 +166,9 @@ hipEvent_t Profiler::event() {
   return e;
 }
 
-void Profiler::begin(hipStream_t st, std::vector<StageBytes> stages) {
+void Profiler::begin(hipStream_t st, StageBytes launch, std::vector<StageBytes> stages) {
   std::lock_guard<std::mutex> g(mu_);
-  Rec r{std::move(stages), event(), event()};
+  Rec r{launch, std::move(stages), event(), event()};
   SLAK_HIP_CHECK(hipEventRecord(r.a, st));
   recs_.push_back(r);
 }
@@ -184,6 +184,7 @@ void Profiler::amend_last(const char* name, double bytes) {
     for (StageBytes& s : it->stages)
       if (std::strcmp(s.name, name) == 0) {
         s.bytes += bytes;
+        it->launch.bytes += bytes;
         return;
       }
 }
@@ -204,32 +205,40 @@ std::string Profiler::report() {
     int64_t n = 0;
     double ms = 0, bytes = 0;
   };
-  std::vector<std::pair<std::string, Agg>> agg;
+  using List = std::vector<std::pair<std::string, Agg>>;  // in order of first use
+  List stages, launches;
+  auto add = [](List& list, const StageBytes& x, double ms) {
+    auto it = std::find_if(list.begin(), list.end(), [&](auto& kv) { return kv.first == x.name; });
+    if (it == list.end()) {
+      list.push_back({x.name, Agg{}});
+      it = list.end() - 1;
+    }
+    it->second.n += 1;
+    it->second.ms += ms;
+    it->second.bytes += x.bytes;
+  };
   for (auto& r : recs_) {
     SLAK_HIP_CHECK(hipEventSynchronize(r.b));
     float ms = 0;
     SLAK_HIP_CHECK(hipEventElapsedTime(&ms, r.a, r.b));
     double all = 0;
     for (const StageBytes& x : r.stages) all += x.bytes;
-    for (const StageBytes& x : r.stages) {
-      auto it = std::find_if(agg.begin(), agg.end(), [&](auto& kv) { return kv.first == x.name; });
-      if (it == agg.end()) {
-        agg.push_back({x.name, Agg{}});
-        it = agg.end() - 1;
-      }
-      it->second.n += 1;
-      it->second.ms += all > 0 ? ms * x.bytes / all : ms / r.stages.size();
-      it->second.bytes += x.bytes;
+    for (const StageBytes& x : r.stages) add(stages, x, all > 0 ? ms * x.bytes / all : ms / r.stages.size());
+    add(launches, r.launch, ms);
+  }
+  std::string js = "{";
+  for (const auto& [title, list] : {std::pair<const char*, const List&>{"stages", stages}, {"launches", launches}}) {
+    js += std::string(js.size() > 1 ? ", " : "") + "\"" + title + "\": [";
+    for (size_t i = 0; i < list.size(); ++i) {
+      char buf[256];
+      snprintf(buf, sizeof(buf), "%s{\"name\": \"%s\", \"launches\": %lld, \"total_ms\": %.6f, \"bytes\": %.0f}",
+               i ? ", " : "", list[i].first.c_str(), (long long)list[i].second.n, list[i].second.ms,
+               list[i].second.bytes);
+      js += buf;
     }
+    js += "]";
   }
-  std::string js = "{\"stages\": [";
-  for (size_t i = 0; i < agg.size(); ++i) {
-    char buf[256];
-    snprintf(buf, sizeof(buf), "%s{\"name\": \"%s\", \"launches\": %lld, \"total_ms\": %.6f, \"bytes\": %.0f}",
-             i ? ", " : "", agg[i].first.c_str(), (long long)agg[i].second.n, agg[i].second.ms, agg[i].second.bytes);
-    js += buf;
-  }
-  js += "]}";
+  js += "}";
   return js;
 }
 

@@ -61,3 +61,38 @@ def test_profile_disabled_records_nothing():
     capi.profile_enable(False)
     subdivide_host(g.cube(), 2, capi.SLAK_SCHEME_LAK)
     assert capi.profile_report()["stages"] == []
+
+
+def test_launches_are_listed_as_measured():
+    """A launch that runs several stages is one entry of "launches", with bytes
+    of its own; its stages share its time and no other."""
+    m = g.torus_mixed(60, 40, 0.3, seed=3)  # beyond the small meshes' one launch
+    nv, nf, nnz = m.nverts, m.nfaces, m.nnz
+    capi.profile_enable(True)
+    try:
+        subdivide_host(m, 2, capi.SLAK_SCHEME_LAK)
+        rep = capi.profile_report()
+    finally:
+        capi.profile_enable(False)
+    stages = {s["name"]: s for s in rep["stages"]}
+    launches = {s["name"]: s for s in rep["launches"]}
+    assert all(s["launches"] == 1 and s["total_ms"] > 0 for s in rep["launches"])
+    assert int(launches["gather"]["bytes"]) == 8 * (nf + 1) + 20 * nnz + 4 * nv
+    assert int(launches["symbolic_poly"]["bytes"]) == 12 * nnz + 8 * nv + 4 * (nf + 1)
+    fused = {"gather": ["gather", "count_poly", "transpose_poly"], "symbolic_poly": ["scan", "spgemm_symbolic_poly"]}
+    for name, parts in fused.items():
+        assert launches[name]["total_ms"] == pytest.approx(sum(stages[p]["total_ms"] for p in parts), abs=1e-5)
+    single = [n for n in launches if n not in fused]
+    assert sorted(single) == sorted(n for n in stages if n not in sum(fused.values(), []))
+    for n in single:
+        assert launches[n] == stages[n]
+
+
+def test_the_small_first_level_is_one_launch():
+    capi.profile_enable(True)
+    try:
+        subdivide_host(g.config1(), 1, capi.SLAK_SCHEME_LAK)
+        names = [s["name"] for s in capi.profile_report()["launches"]]
+    finally:
+        capi.profile_enable(False)
+    assert names == ["first_level_small_quad", "facepoints_quad", "refine_vertex_quad"]
