@@ -74,14 +74,15 @@ void launch_faces(bool quad, const int32_t* ids, const int32_t* fptr, const floa
 void launch_symbolic(bool quad, int scheme, const LevelView& L, hipStream_t st);
 // L.bounds of several meshes, from the symbolic pass's sums
 void launch_seg_bounds(const LevelView& L, hipStream_t st);
+// L.report of several meshes (the symbolic pass's histogram, the bounds)
+void launch_report(const LevelView& L, hipStream_t st);
 // first level: row offsets, sorted rows, edge numbering and (faces set) face
 // points in one launch, after the symbolic pass; a single mesh's launch also
-// fills L.report (if set), which several meshes take from launch_report
-void launch_report(const LevelView& L, hipStream_t st);
-// a small single mesh: all of the above in one launch (no zeroed state needed)
+// fills L.report (if set)
+void launch_number_faces(bool quad, int scheme, const LevelView& L, bool faces, hipStream_t st);
+// a small single mesh: gather to numbering in one launch (no zeroed state needed)
 bool first_level_is_small(const LevelView& L);
 void launch_first_small(bool quad, int scheme, bool use_vals, const LevelView& L, bool faces, hipStream_t st);
-void launch_number_faces(bool quad, int scheme, const LevelView& L, bool faces, hipStream_t st);
 void launch_spgemm_fde(bool quad, const LevelView& L, hipStream_t st);
 // refine (per corner) and vertex (per vertex) items of a level in one launch;
 // the refine items also write the LAK form of the segments with dst_ptr set

@@ -513,8 +513,12 @@ __device__ __forceinline__ int32_t* row_corners(const LevelView& L, int32_t v, i
 // Row lengths and owned-edge counts are summed per tile of kBlock vertices
 // (packed: corners << 31 | edges; a level's totals stay below 2^31) and per
 // kTilesPerGroup tiles, so that any later block adds up the offsets of its
-// rows from a few hundred sums: no scan launches, and no block waits for
-// another. (A decoupled look-back in the sizing pass measured slower: its
+// rows from the sums before it, one group sum for 16384 vertices and at most 64
+// tile sums, 256 at a time: no scan launches, and no block waits for another.
+// The sums grow with the square of the vertices, but int32 corners end a quad
+// mesh at 134 M vertices, where they are 32 loads a thread: one level of quad
+// tori of 5, 20, 40 and 80 M vertices takes 0.81, 2.97, 5.93 and 12.1 ms a call
+// (with scan launches 0.97, 3.64, 7.35, 14.7), the last 2 % above linear. (A decoupled look-back in the sizing pass measured slower: its
 // ticket, one atomic per block on one address, takes about 20 ns a block --
 // 89 against 31 us on 4096 blocks.)
 __device__ __forceinline__ uint64_t pack_row(int32_t n, int32_t owned) {
@@ -2157,6 +2161,7 @@ __device__ __forceinline__ void deep_edges(const FinalView& V, const FinalMesh& 
   int2 cq[kEdgeIter];
 #pragma unroll
   for (int it = 0; it < kEdgeIter; ++it) {
+    // (written whole for a closed mesh, and a replay whose edges differ stops before)
     const int2 o = V.own[S.eb + first + min(row + it * kRows, cnt - 1)];
     tq[it] = o.x - cb;
     sq[it] = o.y - cb;

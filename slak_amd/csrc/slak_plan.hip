@@ -184,14 +184,14 @@ void Plan::wait_report() {
   ++syncs_;
 }
 
-// Uploads the segment tables (SegDesc, vertex, face and corner bases) of levels
-// [l0, l1) in one copy from a plan-owned staging buffer (one per call site,
+// Uploads the segment tables (SegDesc, vertex, face and corner bases, first
+// segment of every block) of levels [l0, l1) in one copy from a plan-owned staging buffer (one per call site,
 // so a pending copy never sees its source rewritten).
 void Plan::upload_tables(int l0, int l1, Staging& staging, bool zero_state) {
   auto align = [](size_t x) { return (x + 255) & ~(size_t)255; };
   size_t total = 0;
   std::vector<size_t> offs;
-  // k_final tables of several meshes: FinalSeg[n], corner and vertex item bases
+  // k_final tables of several meshes: FinalSeg[n] and the mesh of every block
   auto table_bytes = [&](const FinalTable& T) -> size_t {
     return final_table(T) ? align(T.segs.size() * sizeof(FinalSeg)) + align(T.block_seg.size() * sizeof(int32_t)) : 0;
   };
