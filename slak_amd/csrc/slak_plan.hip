@@ -209,9 +209,10 @@ void Plan::upload_tables(int l0, int l1, Staging& staging, bool zero_state) {
     const LevelPlan& L = levels_[l];
     const size_t n = L.segs.size();
     offs.push_back(total);
-    if (n > 1)
-      total = align(total + n * sizeof(SegDesc)) + align(3 * (n + 1) * sizeof(int64_t)) +
-              align((nblocks(L.nv) + nblocks(L.nf) + nblocks(L.nnz) + 3) * sizeof(int32_t));
+    if (n > 1) total = align(total + n * sizeof(SegDesc));
+    if (n > 1 && !L.d_vblk)  // (the first level's second upload changes its descriptors alone)
+      total += align(3 * (n + 1) * sizeof(int64_t)) +
+               align((nblocks(L.nv) + nblocks(L.nf) + nblocks(L.nnz) + 3) * sizeof(int32_t));
     total += fin_bytes(L);
   }
   // (planned with the last levels: empty when the first level's tables go up)
@@ -239,6 +240,8 @@ void Plan::upload_tables(int l0, int l1, Staging& staging, bool zero_state) {
       std::memcpy(staging.p + o, L.segs.data(), n * sizeof(SegDesc));
       L.d_segs = reinterpret_cast<SegDesc*>(d + o);
       o = align(o + n * sizeof(SegDesc));
+    }
+    if (n > 1 && !L.d_vblk) {
       const std::vector<int64_t>* bases[3] = {&L.vbase, &L.fbase, &L.cbase};
       int64_t** d_bases[3] = {&L.d_vbase, &L.d_fbase, &L.d_cbase};
       for (int i = 0; i < 3; ++i) {
@@ -254,11 +257,7 @@ void Plan::upload_tables(int l0, int l1, Staging& staging, bool zero_state) {
         *d_blks[i] = reinterpret_cast<int32_t*>(d + o) + at;
         const std::vector<int64_t>& base = *bases[i];
         const size_t nb = nblocks(base.back());
-        size_t k = 0;
-        for (size_t b = 0; b < nb; ++b) {
-          while (k + 1 < n && base[k + 1] <= (int64_t)b * kBlockItems) ++k;
-          blk[b] = (int32_t)k;
-        }
+        for (size_t k = 0; k < n; ++k) std::fill(blk + nblocks(base[k]), blk + nblocks(base[k + 1]), (int32_t)k);
         blk[nb] = (int32_t)n - 1;
         at += nb + 1;
       }
