@@ -170,17 +170,12 @@ int Plan::read_flags() {
 }
 
 // Waits until the analysis has filled the report. The host looks at the done
-// word itself (an event wait returns about 5 us later); now and then, every
-// millisecond or two, it asks for the stream's state, which ends the wait if the
-// work has failed. (The question takes about 20 us, in which the report may
-// arrive: asked every 4096 looks, without a pause between looks, the building of
-// a batch of 29 tori of 60000 quads took 227 us instead of 214, of 3 62 instead
-// of 58.)
+// word itself (an event wait returns about 5 us later); now and then it asks
+// for the stream's state, which ends the wait if the work has failed.
 void Plan::wait_report() {
   auto done = [this] { return __atomic_load_n(report_, __ATOMIC_ACQUIRE) != 0; };
   for (int64_t i = 1; !done(); ++i) {
-    __builtin_ia32_pause();
-    if (i % 65536) continue;
+    if (i % 4096) continue;
     const hipError_t e = hipStreamQuery(st_);
     if (e == hipErrorNotReady) continue;
     if (e != hipSuccess) SLAK_HIP_CHECK(e);
